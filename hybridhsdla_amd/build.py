@@ -24,8 +24,8 @@ LIB = LIBDIR / "libhsgen.so"
 ORACLE_DIR = ROOT / "oracle"
 ORACLE_LIB = ORACLE_DIR / "liborc.so"
 
-HIP_SOURCES = ["abgen.hip", "zgemm.hip", "ozaki.hip", "context.hip", "fp64_path.hip", "split_path.hip",
-               "tune_eig.hip", "noalloc.hip"]
+HIP_SOURCES = ["sphere.hip", "abgen.hip", "zgemm.hip", "ozaki.hip", "context.hip", "fp64_path.hip", "sphere_path.hip",
+               "split_path.hip", "tune_eig.hip", "noalloc.hip"]
 # host-only set-up code (radial solver, T assembly), linked into the same library
 HOST_SOURCES = ["radial.cpp", "tmat.cpp"]
 HOST_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-Wall", "-ffp-contract=off"]

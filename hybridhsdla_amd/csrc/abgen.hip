@@ -24,76 +24,9 @@
 //             columns >= ng are written as zeros (tile padding).
 //   ref:      A[col*L*natoms + a*L + lm], B likewise, rows lm >= nlm_a zero
 //             (the reference's arma::cx_cube(L, natoms, G) layout).
-#include "hsgen_internal.h"
+#include "sphere_dev.h"
 
 namespace hsgen {
-
-
-// Fleur sphbes (sphbes.f:7-76) + dsphbs (dsphbs.f:11-47) for one x; writes
-// fj[l], dfj[l] for l = 0..lmax into strided LDS slots.  lmax >= 1, x >= 0.
-__device__ inline void bessel_lds(int lmax, double x, double* fj, double* dfj)
-{
-    const double small = 1.0e-3;
-    double xx = x * x;
-    if (x >= small) {
-        double xinv = 1.0 / x;
-        double s, c;
-        sincos(x, &s, &c);
-        double f0 = s * xinv;
-        double f1 = (f0 - c) * xinv;
-        fj[0] = f0;
-        fj[1] = f1;
-        if ((double)lmax < x) {
-            double fm2 = f0, fm1 = f1;
-            for (int l = 2; l <= lmax; ++l) {
-                double f = (2 * l - 1) * xinv * fm1 - fm2;
-                fj[l] = f;
-                fm2 = fm1;
-                fm1 = f;
-            }
-        } else if (lmax >= 2) {
-            // Miller: aux(n) = 0, aux(n-1) = 1, aux(i-1) = (2i+1)/x aux(i) - aux(i+1).
-            // n - 1 >= lmax + 9, so every aux(l), l <= lmax, comes out of the loop;
-            // they are parked in fj[] and rescaled afterwards.
-            int n = (int)(lmax + 10 + x);
-            double anext = 0.0, acur = 1.0;
-            for (int i = n - 1; i >= 1; --i) {
-                double aprev = (2 * i + 1) * xinv * acur - anext;   // aux(i-1)
-                if (i - 1 <= lmax) fj[i - 1] = aprev;
-                anext = acur;
-                acur = aprev;
-            }
-            // normalise with j0 or j1, whichever is larger in magnitude
-            int mn = (fabs(f0) < fabs(f1)) ? 1 : 0;
-            double quot = mn ? f1 / fj[1] : f0 / fj[0];
-            fj[0] = f0;
-            fj[1] = f1;
-            for (int l = 2; l <= lmax; ++l) fj[l] = fj[l] * quot;
-        }
-        // x >= 1e-3 > 1e-4: dsphbs recurrence branch
-        dfj[0] = -fj[1];
-        for (int l = 1; l <= lmax; ++l) dfj[l] = fj[l - 1] - (l + 1) * fj[l] / x;
-    } else {
-        fj[0] = 1.0 - xx / 6.0 * (1.0 - xx / 20.0 * (1.0 - xx / 42.0));
-        fj[1] = (x / 3.0) * (1.0 - xx / 10.0 * (1.0 - xx / 28.0));
-        double fac = xx / 15.0;
-        for (int l = 2; l <= lmax; ++l) {
-            fj[l] = fac * (1.0 - xx / (4 * l + 6));
-            fac = x * fac / (2 * l + 3);
-        }
-        dfj[0] = -fj[1];
-        if (x < 1.0e-4) {
-            double x2 = 0.5 * x * x;
-            double f = 1.0 / 3.0;
-            for (int l = 1; l <= lmax; ++l) {
-                dfj[l] = f * (l - x2 * (l + 2) / (2 * l + 3));
-                f = x * f / (2 * l + 3);
-            }
-        } else {
-            for (int l = 1; l <= lmax; ++l) dfj[l] = fj[l - 1] - (l + 1) * fj[l] / x;
-        }
-    }
-}
 
 template <bool kCompact>
 __global__ __launch_bounds__(256) void k_abgen(AbgenParams p)
@@ -331,15 +264,6 @@ __device__ inline void ylm_column(int m, int lmax, double cth, double sth, doubl
             yl[lm0 - m] = make_double2(yr * nm, yi * nm);    // conj(Y_{l,-m})
         }
     }
-}
-
-// l of lm = l(l+1)+m, |m| <= l
-__device__ inline int l_of_lm(int lm)
-{
-    int l = (int)sqrtf((float)lm + 0.5f);
-    if ((l + 1) * (l + 1) <= lm) ++l;
-    if (l * l > lm) --l;
-    return l;
 }
 
 // Class-shared generator: Y_lm depends on the atom only through its

@@ -205,6 +205,9 @@ hsgen_status upload_M(hsgen_ctx* ctx, hsgen_sys* s, const int32_t* nlm, const do
 
 hsgen_status ensure_M(hsgen_ctx* ctx, hsgen_sys* s, int bk, int bm)
 {
+    std::lock_guard<std::mutex> lk(s->m_mu);
+    s->pad_bk = bk;
+    s->pad_bm = bm;
     if (s->d_M && s->m_bk == bk && s->m_bm == bm) return HSGEN_OK;
     const int na = s->natoms;
     std::vector<const double*> pa(na), pb(na), pc(na);
@@ -387,13 +390,12 @@ hsgen_status hsgen_release_workspace(hsgen_ctx* ctx)
     for (DevBuf* b : {&ctx->Z, &ctx->Zs, &ctx->W, &ctx->Htmp, &ctx->Stmp, &ctx->A, &ctx->B, &ctx->g,
                       &ctx->probs, &ctx->work, &ctx->unorm2, &ctx->atoms_tmp, &ctx->oz_e, &ctx->oz_res,
                       &ctx->oz_out, &ctx->oz_fprob, &ctx->oz_probs, &ctx->oz_work, &ctx->oz_smp, &ctx->btmp, &ctx->eig_a,
-                      &ctx->eig_b, &ctx->eig_d})
+                      &ctx->eig_b, &ctx->eig_d, &ctx->sph_ph, &ctx->sph_rs, &ctx->sph_y, &ctx->sph_w})
         release(*b);
     for (auto& bg : ctx->bgraphs) {
         if (bg.exec) (void)hipGraphExecDestroy(bg.exec);
         release(bg.g);
-        release(bg.probs);
-        release(bg.work);
+        release(bg.ks);
     }
     ctx->bgraphs.clear();
     for (auto& og : ctx->ozgraphs) destroy_oz_graph(og);
@@ -541,8 +543,10 @@ hsgen_status hsgen_system_create(hsgen_ctx* ctx, const hsgen_system* d, hsgen_sy
         cp(xtab[a], d->t_ab[a]);
         cp(xtbb[a], d->t_bb[a]);
     }
-    Geometry geo = geometry(0, s->kdim, 1);
-    st = ensure_M(ctx, s, geo.t.bk, geo.t.bm);
+    const Geometry geo = geometry(0, s->kdim, 1);
+    s->pad_bk = geo.t.bk;
+    s->pad_bm = geo.t.bm;
+    st = sphere_setup(ctx, s, rad.data());
     if (st != HSGEN_OK) {
         hsgen_system_destroy(ctx, s);
         return st;
@@ -559,6 +563,7 @@ hsgen_status hsgen_system_destroy(hsgen_ctx* ctx, hsgen_sys* s)
     if (s->d_rad) (void)hipFree(s->d_rad);
     if (s->d_ynorm) (void)hipFree(s->d_ynorm);
     if (s->d_M) (void)hipFree(s->d_M);
+    if (s->d_sphere) (void)hipFree(s->d_sphere);
     delete s;
     return HSGEN_OK;
 }

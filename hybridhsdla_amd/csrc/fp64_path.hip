@@ -337,16 +337,125 @@ hsgen_status finish_hs(hsgen_ctx* ctx, hsgen_sys* s, const Geometry& geo, int ng
     return HSGEN_OK;
 }
 
+// create_hs on the general operands: A/B generator -> T application -> S and
+// H.  o.tile is the call's tile; ng > 0.
+hsgen_status create_hs_general(hsgen_ctx* ctx, hsgen_sys* s, const hsgen_kpoint* kp, const hsgen_opts& o, double* H,
+                               double* S, int64_t ld, hsgen_report* rep)
+{
+    const int ng = kp->ng;
+    Geometry geo = geometry(o.precision == HSGEN_PREC_FP64 ? o.tile : fp64_tile_by_size(ctx, ng), s->kdim, ng,
+                            o.precision == HSGEN_PREC_FP64 ? 1 : split_col_align(o.precision, o.tile));
+    geo.fold = s->fold;
+    hsgen_status st = upload_g(ctx, kp);
+    if (st) return st;
+    const size_t zbytes = sizeof(double2) * (size_t)geo.ldz * geo.gp;
+    st = ensure(ctx, ctx->Z, zbytes, false);
+    if (st) return st;
+    if (!geo.fold) {
+        st = ensure(ctx, ctx->Zs, zbytes, false);
+        if (st) return st;
+    }
+    AbgenParams p = abgen_params(s, kp, (const int32_t*)ctx->g.p);
+    p.ncols = (int32_t)geo.gp;
+    p.Z = (double2*)ctx->Z.p;
+    p.Zs = geo.fold ? nullptr : (double2*)ctx->Zs.p;
+    p.ldz = geo.ldz;
+    p.fold = geo.fold;
+    HIPCHK(hipEventRecord(ctx->ev[0], ctx->stream));
+    HIPCHK(launch_abgen(p, true, ctx->stream));
+    HIPCHK(hipEventRecord(ctx->ev[1], ctx->stream));
+    st = finish_hs(ctx, s, geo, ng, o, H, S, ld, rep, 0.0);
+    if (st) return st;
+    if (rep) {
+        float t0 = 0;
+        HIPCHK(hipEventElapsedTime(&t0, ctx->ev[0], ctx->ev[1]));
+        rep->ms_abgen = t0;
+        rep->ms_total += t0;
+        rep->bytes_abgen = (geo.fold ? 1.0 : 2.0) * 2.0 * 16.0 * (double)ng * s->kdim;   // Y, or Z and Zs
+    }
+    return HSGEN_OK;
+}
+
 namespace {
 
+// FP64 H and S of one k-point (ng > 0) from the system: sphere_path.hip.
+// Every tile gives the same bits, so o.tile is only reported.
+hsgen_status create_hs_sphere(hsgen_ctx* ctx, hsgen_sys* s, const hsgen_kpoint* kp, const hsgen_opts& o, double* H,
+                              double* S, int64_t ld, hsgen_report* rep)
+{
+    const int ng = kp->ng;
+    const bool do_h = !(o.flags & HSGEN_SKIP_H), do_s = !(o.flags & HSGEN_SKIP_S);
+    const Geometry geo = geometry(o.tile, s->kdim, ng);
+    {
+        std::lock_guard<std::mutex> lk(s->m_mu);
+        s->pad_bk = geo.t.bk;
+        s->pad_bm = geo.t.bm;
+    }
+    hsgen_status st = upload_g(ctx, kp);
+    if (st) return st;
+    const SphereLayout l = sphere_layout(ctx, s, {ng}, do_h);
+    if ((st = ensure(ctx, ctx->sph_ph, l.b_ph, false)) || (st = ensure(ctx, ctx->sph_rs, l.b_rs, false))) return st;
+    if (do_h && ((st = ensure(ctx, ctx->sph_y, l.b_y, false)) || (st = ensure(ctx, ctx->sph_w, l.b_w, false)))) return st;
+    const bool hdev = !do_h || is_device_ptr(H), sdev = !do_s || is_device_ptr(S);
+    double2* dH = (double2*)H;
+    double2* dS = (double2*)S;
+    int64_t ldH = ld, ldS = ld;
+    if (!hdev) {
+        st = ensure(ctx, ctx->Htmp, sizeof(double2) * (size_t)ng * ng, false);
+        if (st) return st;
+        dH = (double2*)ctx->Htmp.p;
+        ldH = ng;
+    }
+    if (!sdev) {
+        st = ensure(ctx, ctx->Stmp, sizeof(double2) * (size_t)ng * ng, false);
+        if (st) return st;
+        dS = (double2*)ctx->Stmp.p;
+        ldS = ng;
+    }
+    SphereArgs p = sphere_args(s, l, ctx->sph_ph.p, ctx->sph_rs.p, do_h ? ctx->sph_y.p : nullptr,
+                               do_h ? ctx->sph_w.p : nullptr);
+    p.one = sphere_ks(l, {kp}, {(const int32_t*)ctx->g.p}, {dH}, {dS}, {ldH}, {ldS})[0];
+    HIPCHK(hipEventRecord(ctx->ev[0], ctx->stream));
+    HIPCHK(sphere_launch(p, l, s, do_h, do_s, rep ? ctx->ev[1] : nullptr, rep ? ctx->ev[3] : nullptr, ctx->stream));
+    if (o.flags & HSGEN_FILL_UPPER) {
+        if (do_h) HIPCHK(launch_fill_upper(dH, ldH, ng, ctx->stream));
+        if (do_s) HIPCHK(launch_fill_upper(dS, ldS, ng, ctx->stream));
+    }
+    HIPCHK(hipEventRecord(ctx->ev[4], ctx->stream));
+    HIPCHK(hipEventSynchronize(ctx->ev[4]));
+    const bool full = (o.flags & HSGEN_FILL_UPPER) != 0;
+    if (!hdev) {
+        st = copy_lower_to_host(ctx, dH, ng, H, ld, full);
+        if (st) return st;
+    }
+    if (!sdev) {
+        st = copy_lower_to_host(ctx, dS, ng, S, ld, full);
+        if (st) return st;
+    }
+    if (rep) {
+        float t0 = 0, t1 = 0, t2 = 0;
+        HIPCHK(hipEventElapsedTime(&t0, ctx->ev[0], ctx->ev[1]));
+        HIPCHK(hipEventElapsedTime(&t1, ctx->ev[1], ctx->ev[3]));
+        HIPCHK(hipEventElapsedTime(&t2, ctx->ev[3], ctx->ev[4]));
+        rep->ms_abgen = t0;
+        rep->ms_tmul = t1;
+        rep->ms_contract = t2;
+        rep->ms_total = t0 + t1 + t2;
+        rep->ng = ng;
+        rep->kdim = s->kdim;
+        rep->flops_alg = 16.0 * (double)ng * ng * s->kdim + 32.0 * (double)ng * (double)s->sum_nlm2;
+        rep->bytes_abgen = sphere_gen_bytes(s) * ng;
+        rep->tile_used = geo.cfg;
+    }
+    return HSGEN_OK;
+}
+
 // ---------------------------------------------------------------------------
-// Batched k-points, FP64: per batch of k-points that fits in memory, A/B
-// generation per k into one column-concatenated Z/Zs, ONE grouped launch for
-// the T application of all their columns and ONE persistent grouped launch
-// for the S and H tiles of all of them (largest k first).  The launch
-// sequence is captured in a hipGraph and replayed while the call signature
-// (system, k-points and their G lists, outputs, workspace) is unchanged, as
-// in repeated SCF iterations over one k-set.
+// Batched k-points, FP64: per batch of k-points that fits in memory one launch
+// each of the generator, the T application and the H and S tiles over all of
+// them.  The launch sequence is captured in a hipGraph and replayed while the
+// call signature (system, k-points and their G lists, outputs, workspace) is
+// unchanged, as in repeated SCF iterations over one k-set.
 // ---------------------------------------------------------------------------
 uint64_t hash_words(const void* data, size_t bytes, uint64_t h)
 {
@@ -362,12 +471,13 @@ hsgen_status batched_fp64(hsgen_ctx* ctx, hsgen_sys* s, int nk, const hsgen_kpoi
     const bool do_s = !(flags & HSGEN_SKIP_S), do_h = !(flags & HSGEN_SKIP_H);
     int max_ng = 1;
     for (int i = 0; i < nk; ++i) max_ng = std::max(max_ng, kps[i].ng);
-    Geometry geo = geometry(o.tile, s->kdim, max_ng);
-    geo.fold = s->fold;
-    const int64_t tm = std::max(geo.t.bm, geo.t.bn);
-    const int tc = tapp_cfg(geo);
-    hsgen_status st = ensure_M(ctx, s, geo.t.bk, geo.t.bm);
-    if (st) return st;
+    const Geometry geo = geometry(o.tile, s->kdim, max_ng);
+    {
+        std::lock_guard<std::mutex> lk(s->m_mu);
+        s->pad_bk = geo.t.bk;
+        s->pad_bm = geo.t.bm;
+    }
+    hsgen_status st;
     // largest k first; k-points without G-vectors have nothing to compute
     std::vector<int> order;
     for (int i = 0; i < nk; ++i)
@@ -378,13 +488,13 @@ hsgen_status batched_fp64(hsgen_ctx* ctx, hsgen_sys* s, int nk, const hsgen_kpoi
         hdev[i] = !do_h || is_device_ptr(H[i]);
         sdev[i] = !do_s || is_device_ptr(S[i]);
     }
-    // batches: operands (Y, W or Z, Zs, W) plus device copies of host outputs within
-    // 90% of the memory the call may use (the rest of the call's device memory,
-    // the graph's problem and tile lists, is a few MB)
-    if (geo.fold) release(ctx->Zs);   // folded operands need no Zs
+    // batches: operands plus device copies of host outputs within 90% of the
+    // memory the call may use (the rest of the call's device memory, the
+    // graph's G lists, is small)
     size_t fr = 0, tot = 0;
     HIPCHK(hipMemGetInfo(&fr, &tot));
-    size_t budget = (size_t)(0.9 * (double)(fr + ctx->Z.bytes + ctx->Zs.bytes + ctx->W.bytes + ctx->btmp.bytes));
+    size_t budget = (size_t)(0.9 * (double)(fr + ctx->sph_ph.bytes + ctx->sph_rs.bytes + ctx->sph_y.bytes +
+                                            ctx->sph_w.bytes + ctx->btmp.bytes));
     if (const char* e = std::getenv("HSGEN_BATCH_BYTES"))   // cap (tuning and tests)
         if (std::strtoull(e, nullptr, 10) > 0) budget = std::min<size_t>(budget, std::strtoull(e, nullptr, 10));
     std::vector<std::vector<int>> batches;
@@ -392,8 +502,8 @@ hsgen_status batched_fp64(hsgen_ctx* ctx, hsgen_sys* s, int nk, const hsgen_kpoi
         size_t used = 0;
         std::vector<int> cur;
         for (int i : order) {
-            const size_t gp = (size_t)roundup(std::max(kps[i].ng, 1), tm);
-            const size_t need = n_operands(geo) * sizeof(double2) * (size_t)geo.ldz * gp +
+            const SphereLayout lk = sphere_layout(ctx, s, {kps[i].ng}, do_h);
+            const size_t need = lk.b_ph + lk.b_rs + lk.b_y + lk.b_w +
                                 sizeof(double2) * (size_t)kps[i].ng * kps[i].ng * ((!hdev[i]) + (!sdev[i]));
             if (!cur.empty() && used + need > budget) {
                 batches.push_back(cur);
@@ -406,39 +516,26 @@ hsgen_status batched_fp64(hsgen_ctx* ctx, hsgen_sys* s, int nk, const hsgen_kpoi
         if (!cur.empty()) batches.push_back(cur);
     }
     if (ctx->bgraphs.size() < batches.size()) ctx->bgraphs.resize(batches.size());
-    // persistent grids: every workgroup slot of every CU (one for the default
-    // tile, whose 128 KiB of LDS fill a CU)
-    const int ncu = ctx->n_cu > 0 ? ctx->n_cu : 256;
     double ms_all = 0.0;
     for (size_t b = 0; b < batches.size(); ++b) {
         const std::vector<int>& ks = batches[b];
-        std::vector<int64_t> col0(ks.size()), tmp0(ks.size());
-        int64_t ncols = 0, ntmp = 0;
+        std::vector<int64_t> tmp0(ks.size());
+        std::vector<int> ngs;
+        int64_t ntmp = 0;
         for (size_t q = 0; q < ks.size(); ++q) {
             const int i = ks[q];
-            col0[q] = ncols;
-            ncols += roundup(std::max(kps[i].ng, 1), tm);
+            ngs.push_back(kps[i].ng);
             tmp0[q] = ntmp;
             ntmp += (int64_t)kps[i].ng * kps[i].ng * ((!hdev[i]) + (!sdev[i]));
         }
-        const size_t zbytes = sizeof(double2) * (size_t)geo.ldz * ncols;
-        st = ensure(ctx, ctx->Z, zbytes, false);
-        if (st) return st;
-        if (!geo.fold) {
-            st = ensure(ctx, ctx->Zs, zbytes, false);
-            if (st) return st;
-        }
-        if (do_h) {
-            st = ensure(ctx, ctx->W, zbytes, true);
-            if (st) return st;
-        }
+        const SphereLayout l = sphere_layout(ctx, s, ngs, do_h);
+        if ((st = ensure(ctx, ctx->sph_ph, l.b_ph, false)) || (st = ensure(ctx, ctx->sph_rs, l.b_rs, false))) return st;
+        if (do_h && ((st = ensure(ctx, ctx->sph_y, l.b_y, false)) || (st = ensure(ctx, ctx->sph_w, l.b_w, false))))
+            return st;
         if (ntmp > 0) {
             st = ensure(ctx, ctx->btmp, sizeof(double2) * (size_t)ntmp, false);
             if (st) return st;
         }
-        double2* Z = (double2*)ctx->Z.p;
-        double2* Zs = zs_ptr(ctx, geo);
-        double2* W = (double2*)ctx->W.p;
         // device outputs of every k of the batch (the caller's, or scratch)
         std::vector<double2*> dH(ks.size(), nullptr), dS(ks.size(), nullptr);
         std::vector<int64_t> ldH(ks.size()), ldS(ks.size());
@@ -453,9 +550,9 @@ hsgen_status batched_fp64(hsgen_ctx* ctx, hsgen_sys* s, int nk, const hsgen_kpoi
             ldS[q] = ts ? kps[i].ng : ld[i];
         }
         // call signature
-        std::vector<int64_t> sig{(int64_t)s->serial, (int64_t)flags, geo.cfg, tc, (int64_t)(intptr_t)Z,
-                                 (int64_t)(intptr_t)Zs, (int64_t)(intptr_t)W, (int64_t)(intptr_t)s->d_M,
-                                 (int64_t)(intptr_t)ctx->btmp.p, (int64_t)ks.size()};
+        std::vector<int64_t> sig{(int64_t)s->serial, (int64_t)flags, (int64_t)(intptr_t)ctx->sph_ph.p,
+                                 (int64_t)(intptr_t)ctx->sph_rs.p, (int64_t)(intptr_t)ctx->sph_y.p,
+                                 (int64_t)(intptr_t)ctx->sph_w.p, (int64_t)(intptr_t)ctx->btmp.p, (int64_t)ks.size()};
         for (size_t q = 0; q < ks.size(); ++q) {
             const int i = ks[q];
             int64_t kb[3];
@@ -480,63 +577,28 @@ hsgen_status batched_fp64(hsgen_ctx* ctx, hsgen_sys* s, int nk, const hsgen_kpoi
             }
             st = ensure(ctx, bg.g, sizeof(int32_t) * std::max<size_t>(gall.size(), 3), false);
             if (st) return st;
-            // problems: T application over all columns, then S and H per k
-            std::vector<GemmProblem> probs;
-            std::vector<TileWork> tw_t, tw_c;
-            if (do_h) add_tmul_problems(probs, tw_t, s, geo, zgemm_cfg(tc), ncols, Z, W);
+            std::vector<const hsgen_kpoint*> kpp;
+            std::vector<const int32_t*> gpp;
             for (size_t q = 0; q < ks.size(); ++q) {
-                const int i = ks[q];
-                const size_t p0 = probs.size();
-                add_hs_problems(probs, tw_c, geo, kps[i].ng, Z + col0[q] * geo.ldz, Zs + col0[q] * geo.ldz,
-                                W + col0[q] * geo.ldz, dH[q], dS[q], 0, flags);
-                for (size_t pi = p0; pi < probs.size(); ++pi) {
-                    probs[pi].ldl = geo.ldz;
-                    probs[pi].ldr = geo.ldz;
-                    probs[pi].kdepth = (int32_t)geo.kpad;
-                    probs[pi].ldc = probs[pi].C == dH[q] ? ldH[q] : ldS[q];
-                }
+                kpp.push_back(&kps[ks[q]]);
+                gpp.push_back((const int32_t*)bg.g.p + goff[q]);
             }
-            xcd_permute(tw_c);
-            std::vector<TileWork> work(tw_t);
-            work.insert(work.end(), tw_c.begin(), tw_c.end());
-            st = ensure(ctx, bg.probs, sizeof(GemmProblem) * std::max<size_t>(probs.size(), 1), false);
+            const std::vector<SphereK> sk = sphere_ks(l, kpp, gpp, dH, dS, ldH, ldS);
+            st = ensure(ctx, bg.ks, sizeof(SphereK) * sk.size(), false);
             if (st) return st;
-            st = ensure(ctx, bg.work, sizeof(TileWork) * std::max<size_t>(work.size(), 1), false);
-            if (st) return st;
-            if (!gall.empty())
-                HIPCHK(hipMemcpyAsync(bg.g.p, gall.data(), sizeof(int32_t) * gall.size(), hipMemcpyHostToDevice,
-                                      ctx->stream));
-            HIPCHK(hipMemcpyAsync(bg.probs.p, probs.data(), sizeof(GemmProblem) * probs.size(),
-                                  hipMemcpyHostToDevice, ctx->stream));
-            if (!work.empty())
-                HIPCHK(hipMemcpyAsync(bg.work.p, work.data(), sizeof(TileWork) * work.size(),
-                                      hipMemcpyHostToDevice, ctx->stream));
+            HIPCHK(hipMemcpyAsync(bg.g.p, gall.data(), sizeof(int32_t) * gall.size(), hipMemcpyHostToDevice,
+                                  ctx->stream));
+            HIPCHK(hipMemcpyAsync(bg.ks.p, sk.data(), sizeof(SphereK) * sk.size(), hipMemcpyHostToDevice, ctx->stream));
             // the host vectors must outlive the copies
             HIPCHK(hipStreamSynchronize(ctx->stream));
-            const int grid_t = tc == geo.cfg ? ncu * zgemm_blocks_per_cu(tc) : 0;
-            const int grid_c = ncu * zgemm_blocks_per_cu(geo.cfg);
+            SphereArgs p = sphere_args(s, l, ctx->sph_ph.p, ctx->sph_rs.p, do_h ? ctx->sph_y.p : nullptr,
+                                       do_h ? ctx->sph_w.p : nullptr);
+            p.nk = (int32_t)sk.size();
+            p.one = sk[0];
+            p.many = (const SphereK*)bg.ks.p;
             // capture the launch sequence
             HIPCHK(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
-            hipError_t ce = hipSuccess;
-            for (size_t q = 0; q < ks.size() && ce == hipSuccess; ++q) {
-                const int i = ks[q];
-                AbgenParams p = abgen_params(s, &kps[i], (const int32_t*)bg.g.p + goff[q]);
-                p.ncols = (int32_t)roundup(std::max(kps[i].ng, 1), tm);
-                p.Z = Z + col0[q] * geo.ldz;
-                p.Zs = geo.fold ? nullptr : Zs + col0[q] * geo.ldz;
-                p.ldz = geo.ldz;
-                p.fold = geo.fold;
-                ce = launch_abgen(p, true, ctx->stream);
-            }
-            const GemmProblem* dp = (const GemmProblem*)bg.probs.p;
-            const TileWork* dw = (const TileWork*)bg.work.p;
-            if (ce == hipSuccess && do_h) {
-                ce = launch_zgemm(tc, dp, dw, (int)tw_t.size(), ctx->stream, grid_t);
-                if (ce == hipSuccess)
-                    ce = launch_clear_rows(W, geo.ldz, 2 * (int64_t)s->kdim, geo.ldz, (int)ncols, ctx->stream);
-            }
-            if (ce == hipSuccess)
-                ce = launch_zgemm(geo.cfg, dp, dw + tw_t.size(), (int)tw_c.size(), ctx->stream, grid_c);
+            hipError_t ce = sphere_launch(p, l, s, do_h, do_s, nullptr, nullptr, ctx->stream);
             for (size_t q = 0; q < ks.size() && ce == hipSuccess && (flags & HSGEN_FILL_UPPER); ++q) {
                 if (do_h) ce = launch_fill_upper(dH[q], ldH[q], kps[ks[q]].ng, ctx->stream);
                 if (ce == hipSuccess && do_s) ce = launch_fill_upper(dS[q], ldS[q], kps[ks[q]].ng, ctx->stream);
@@ -583,7 +645,7 @@ hsgen_status batched_fp64(hsgen_ctx* ctx, hsgen_sys* s, int nk, const hsgen_kpoi
             r.ng = kps[i].ng;
             r.kdim = s->kdim;
             r.flops_alg = 16.0 * (double)kps[i].ng * kps[i].ng * s->kdim + 32.0 * (double)kps[i].ng * (double)s->sum_nlm2;
-            r.bytes_abgen = (geo.fold ? 1.0 : 2.0) * 2.0 * 16.0 * (double)kps[i].ng * s->kdim;
+            r.bytes_abgen = sphere_gen_bytes(s) * kps[i].ng;
             r.tile_used = geo.cfg;
         }
         if (nk > 0) rep[0].ms_total = ms_all;
@@ -655,37 +717,8 @@ hsgen_status hsgen_create_hs(hsgen_ctx* ctx, const hsgen_sys* sc, const hsgen_kp
     if (rep) std::memset(rep, 0, sizeof *rep);
     if (ng == 0) return HSGEN_OK;
     HIPCHK(hipSetDevice(ctx->device));
-    Geometry geo = geometry(o.precision == HSGEN_PREC_FP64 ? o.tile : fp64_tile_by_size(ctx, ng), s->kdim, ng,
-                            o.precision == HSGEN_PREC_FP64 ? 1 : split_col_align(o.precision, o.tile));
-    geo.fold = s->fold;
-    st = upload_g(ctx, kp);
-    if (st) return st;
-    const size_t zbytes = sizeof(double2) * (size_t)geo.ldz * geo.gp;
-    st = ensure(ctx, ctx->Z, zbytes, false);
-    if (st) return st;
-    if (!geo.fold) {
-        st = ensure(ctx, ctx->Zs, zbytes, false);
-        if (st) return st;
-    }
-    AbgenParams p = abgen_params(s, kp, (const int32_t*)ctx->g.p);
-    p.ncols = (int32_t)geo.gp;
-    p.Z = (double2*)ctx->Z.p;
-    p.Zs = geo.fold ? nullptr : (double2*)ctx->Zs.p;
-    p.ldz = geo.ldz;
-    p.fold = geo.fold;
-    HIPCHK(hipEventRecord(ctx->ev[0], ctx->stream));
-    HIPCHK(launch_abgen(p, true, ctx->stream));
-    HIPCHK(hipEventRecord(ctx->ev[1], ctx->stream));
-    st = finish_hs(ctx, s, geo, ng, o, H, S, ld, rep, 0.0);
-    if (st) return st;
-    if (rep) {
-        float t0 = 0;
-        HIPCHK(hipEventElapsedTime(&t0, ctx->ev[0], ctx->ev[1]));
-        rep->ms_abgen = t0;
-        rep->ms_total += t0;
-        rep->bytes_abgen = (geo.fold ? 1.0 : 2.0) * 2.0 * 16.0 * (double)ng * s->kdim;   // Y, or Z and Zs
-    }
-    return HSGEN_OK;
+    if (is_split(o.precision)) return create_hs_general(ctx, s, kp, o, H, S, ld, rep);
+    return create_hs_sphere(ctx, s, kp, o, H, S, ld, rep);
 }
 
 hsgen_status hsgen_create_hs_batched(hsgen_ctx* ctx, const hsgen_sys* sys, int32_t nk,

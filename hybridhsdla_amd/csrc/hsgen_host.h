@@ -6,8 +6,11 @@
 //                   and batched
 //   tune_eig.hip    the tile autotuner and the generalized eigensolve
 //   noalloc.hip     the allocation-free FP64 entry point
+//   sphere_path.hip FP64 H and S from a system (kernels: sphere.hip, whose
+//                   operands sphere.h describes)
 //
-// Operand layout in HBM, per k-point (complex128, column-major, ld = ldz).
+// Operand layout of the other paths (split precision, the contraction of
+// given coefficients) in HBM, per k-point (complex128, column-major, ld = ldz).
 // Folded (every ||u_dot_l||^2 > 0, the usual case):
 //   Y  = [A_1; N_1^1/2 B_1; A_2; ...]   rows 2*off_a .. 2*off_a + 2*nlm_a - 1
 //   W  = [M'_1 Y_1; M'_2 Y_2; ...]      M'_a = D_a^-1/2 M_a D_a^-1/2
@@ -24,6 +27,7 @@
 #include <cstdarg>
 #include <list>
 #include <map>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -31,6 +35,7 @@
 
 #include "../../include/hsgen.h"
 #include "hsgen_internal.h"
+#include "sphere.h"
 
 namespace hsgen {
 
@@ -73,6 +78,8 @@ struct hsgen_ctx {
     std::string err;
     // workspace
     hsgen::DevBuf Z, Zs, W, Htmp, Stmp, A, B, g, probs, work, unorm2, atoms_tmp;
+    // FP64 from a system: phases, radial factors, real vectors (W, host-output copies above)
+    hsgen::DevBuf sph_ph, sph_rs, sph_y, sph_w;
     // split precision
     hsgen::DevBuf oz_e, oz_res, oz_out, oz_probs, oz_work, oz_smp, oz_fprob;
     hipEvent_t oz_ev[2 * hsgen::kMaxModuli] = {};   // INT8 GEMM start/stop per residue group
@@ -82,7 +89,7 @@ struct hsgen_ctx {
     struct BatchGraph {
         std::vector<int64_t> sig;
         hipGraphExec_t exec = nullptr;
-        hsgen::DevBuf g, probs, work;
+        hsgen::DevBuf g, ks;
     };
     std::vector<BatchGraph> bgraphs;
     hsgen::DevBuf btmp;                              // device H, S of host-output k-points
@@ -116,6 +123,11 @@ struct hsgen_sys {
     std::vector<int32_t> m_ld;         // per atom: leading dim of M_a
     std::vector<int32_t> m_cols;       // per atom: padded column count
     int m_bk = 0, m_bm = 0;            // tile geometry M was padded for
+    // M is built by the first call that reads it (calls on contexts that share
+    // the system may be the first together); pad_bk, pad_bm: the tile geometry
+    // of the last call, which the allocation-free entry point asks for
+    std::mutex m_mu;
+    int pad_bk = 0, pad_bm = 0;
     int64_t sum_nlm2 = 0;              // sum_a nlm_a^2
     // folded operands: Y = [A_a; sqrt(N_a) B_a] per atom (S = Y^H Y,
     // H = Y^H M' Y) when every N_l = ||u_dot_l||^2 is positive; otherwise
@@ -131,6 +143,15 @@ struct hsgen_sys {
     // geometry
     std::vector<std::vector<std::complex<double>>> h_taa, h_tab, h_tbb;
     std::vector<int> h_owner;          // per atom: the atom whose copies hold its T
+    // FP64 path (sphere.h): one allocation, d_sphere
+    void* d_sphere = nullptr;
+    double2* d_mt = nullptr;
+    hsgen::KindDev* d_kinds = nullptr;
+    int32_t* d_order = nullptr;
+    int32_t* d_ksteps = nullptr;
+    int64_t* d_mtoff = nullptr;
+    int nkinds = 0, nksteps = 0, ldr = 0, rt64 = 0, rt32 = 0;
+    int64_t ldy = 0, ldw = 0;
     // first atom of each rotation class and of each rmt class (AtomDev::cls)
     std::vector<int32_t> rot_rep, rmt_rep;
 };
@@ -206,6 +227,32 @@ void add_tmul_problems(std::vector<GemmProblem>& probs, std::vector<TileWork>& w
 hsgen_status run_grouped(hsgen_ctx* ctx, int cfg, std::vector<GemmProblem>& probs, std::vector<TileWork>& work);
 hsgen_status finish_hs(hsgen_ctx* ctx, hsgen_sys* s, const Geometry& geo, int ng, const hsgen_opts& o, double* H,
                        double* S, int64_t ld, hsgen_report* rep, double ms_front);
+
+// create_hs on the general operands (split precision; the autotuner's FP64 runs)
+hsgen_status create_hs_general(hsgen_ctx* ctx, hsgen_sys* s, const hsgen_kpoint* kp, const hsgen_opts& o, double* H,
+                               double* S, int64_t ld, hsgen_report* rep);
+
+// ---- sphere_path.hip ----
+struct SphereLayout {
+    int64_t gtot = 0;                       // operand columns, 64 per tile column of every k-point
+    int64_t ngcols = 0, npatch = 0, nstiles = 0;
+    int htile = 64, ttile = 64, stile = 64, pside = 1;
+    size_t b_ph = 0, b_rs = 0, b_y = 0, b_w = 0;   // bytes of the operand arrays
+};
+hsgen_status sphere_setup(hsgen_ctx* ctx, hsgen_sys* s, const RadDev* rad);
+SphereLayout sphere_layout(const hsgen_ctx* ctx, const hsgen_sys* s, const std::vector<int>& ngs, bool do_h);
+SphereArgs sphere_args(const hsgen_sys* s, const SphereLayout& l, void* ph, void* rs, void* y, void* w);
+std::vector<SphereK> sphere_ks(const SphereLayout& l, const std::vector<const hsgen_kpoint*>& kps,
+                               const std::vector<const int32_t*>& gs, const std::vector<double2*>& H,
+                               const std::vector<double2*>& S, const std::vector<int64_t>& ldH,
+                               const std::vector<int64_t>& ldS);
+hipError_t sphere_launch(const SphereArgs& p, const SphereLayout& l, const hsgen_sys* s, bool do_h, bool do_s,
+                         hipEvent_t ev_gen, hipEvent_t ev_tapp, hipStream_t st);
+// Bytes of the operands per plane wave (reports).
+inline double sphere_gen_bytes(const hsgen_sys* s)
+{
+    return 16.0 * s->natoms + 16.0 * s->ldr + 8.0 * s->ldy;
+}
 
 // ---- split_path.hip ----
 struct OzResult {

@@ -1,0 +1,98 @@
+// FP64 H and S from a system description: declarations of the kernels in
+// sphere.hip and of the tables they share with the host.
+//
+// A matching coefficient of atom a at plane wave K factors into a phase and
+// a real number: with real spherical harmonics y (cos / sin of m phi in place
+// of e^{i m phi})
+//   A_lm = ph_a(K) (D y_a(K))_lm, B_lm likewise,   ph_a = e^{i 2 pi K.tau_a},
+// D the constant map from real to complex harmonics and y_a real, the same
+// for all atoms of one "kind" (equal l cutoff, radius, radial data and
+// rotation, bit for bit).  So
+//   H_ij = sum_a conj(ph_a(i)) [ y_a(i)^T W_a(j) ],   W_a = ph_a (D^H M_a D) y_a
+//   S_ij = sum_kind F(i, j) sum_l (2l+1)/4pi (a_l a_l' + N_l b_l b_l') P_l(cos),
+//          F(i, j) = sum_{a of the kind} conj(ph_a(i)) ph_a(j)
+// (the addition theorem): H takes one real-by-complex product per depth, half
+// the operations of a complex one, and S next to none.
+#pragma once
+
+#include "hsgen_internal.h"
+
+namespace hsgen {
+
+// Atoms of one kind share the real vector y and the radial factors.
+struct KindDev {
+    int32_t lmax, nlm;
+    int32_t r4;          // rows of y and of one W_a: 2 nlm rounded up to the MFMA depth of 4
+    int32_t rep;         // first atom of the kind (system order): RadDev row
+    int32_t yoff;        // first row of y
+    int32_t rsoff;       // first row of the radial factors
+    int32_t woff;        // first row of W
+    int32_t ldm;         // leading dimension of Mt: 2 nlm rounded up to the stage depth of 16
+    int32_t rt64, rt32;  // T-application row tiles of the kinds before this one, for tiles of 64 and 32
+    int32_t first, count;   // its atoms, in kind order
+    double rmt;
+    double rot[9];       // column-major R_atom * bmat
+};
+
+// One k-point of a launch.
+struct SphereK {
+    double k[3];
+    const int32_t* g;    // [ng][3], device memory
+    double2* H;
+    double2* S;
+    int64_t ldH, ldS;
+    int64_t col0;        // first column in the operand arrays (a multiple of the tile side)
+    int32_t ng;
+    int32_t gcol0;       // plane waves of the k-points before this one
+    int32_t stile0;      // S tiles before this one
+    int32_t hpatch0;     // H patches before this one
+};
+
+// One T block to turn into real harmonics (device pointers).
+struct MtJob {
+    const double2* taa;
+    const double2* tab;
+    const double2* tbb;
+    int64_t off;         // of its Mt (complex units)
+    int32_t nlm, rows, ldm;
+    int32_t pad;
+};
+
+// Everything the kernels read; one k-point travels in `one`, more in `many`.
+struct SphereArgs {
+    const KindDev* kinds;
+    const AtomDev* atoms;      // system order
+    const int32_t* order;      // [natoms] atoms in kind order
+    const RadDev* rad;
+    const double* ynorm;
+    double bmat[9];
+    double vol_prefac;
+    int32_t natoms, nkinds, max_lmax, nl, L;
+    int32_t chunk;             // kinds per LDS chunk of the generator
+    int32_t nk, ngcols;        // k-points; plane waves of all of them
+    SphereK one;
+    const SphereK* many;
+    int64_t gtot;              // columns of the operand arrays
+    double2* ph;               // [natoms + 1][gtot] phases, kind order (the last row is not used)
+    double2* rs;               // [gtot][ldr] radial factors (a_l, b_l)
+    int32_t ldr;
+    double* y;                 // [gtot][ldy] real vectors of all kinds, or null (S alone)
+    double2* W;                // [gtot][ldw]
+    int64_t ldy, ldw;
+    const double2* mt;
+    const int64_t* mtoff;      // [natoms] Mt of each atom, kind order
+    const int32_t* ksteps;     // per k-step of H: row of y (a multiple of 4), bit 0 set in an atom's last
+    int32_t nksteps;
+    int32_t pside, npatch;     // H patches
+};
+
+int sphere_chunk(int nl, int L);
+hipError_t launch_build_mt(const MtJob* jobs, int njobs, int64_t max_elems, double2* mt, hipStream_t st);
+hipError_t launch_sphere_gen(const SphereArgs& p, hipStream_t st);
+// S tile side by the number of lower tiles; the bits do not depend on it
+int overlap_tile(int64_t tiles64, int n_cu);
+hipError_t launch_sphere_tapp(const SphereArgs& p, int tile, int rtiles, hipStream_t st);
+hipError_t launch_sphere_h(const SphereArgs& p, int tile, hipStream_t st);
+hipError_t launch_overlap(const SphereArgs& p, int tile, int64_t ntiles, hipStream_t st);
+
+}  // namespace hsgen

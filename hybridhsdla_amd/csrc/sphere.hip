@@ -1,0 +1,852 @@
+// FP64 kernels of the path from a system description to H and S that use the
+// form of the matching coefficients: a phase per atom times real numbers that
+// atoms of one kind share (sphere.h).
+#include "sphere.h"
+#include "sphere_dev.h"
+
+namespace hsgen {
+
+namespace {
+
+// Largest i in [0, n) with key(i) <= v; key ascending, key(0) <= v.
+template <class Key>
+__device__ __forceinline__ int find_last(int n, int v, Key key)
+{
+    int lo = 0, hi = n;
+    while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (key(mid) <= v) lo = mid;
+        else hi = mid;
+    }
+    return lo;
+}
+
+// Row of the lower triangle that element t of its row-by-row list is in.
+__device__ __forceinline__ int tri_row(int t)
+{
+    int r = (int)((sqrt(8.0 * (double)t + 1.0) - 1.0) * 0.5);
+    while ((int64_t)(r + 1) * (r + 2) / 2 <= t) ++r;
+    while ((int64_t)r * (r + 1) / 2 > t) --r;
+    return r;
+}
+
+// Real harmonics of one m >= 0 by the ylm4 recurrences (ylm4.f:194-217):
+// Y_l0, and for m > 0 Re and Im of Y_lm at l(l+1)+m and l(l+1)-m, so that
+// conj(Y_lm) = re - i im and conj(Y_l,-m) = (-1)^m (re + i im).
+__device__ inline void ylm_real(int m, int lmax, const DirAngles& dir, const double* __restrict__ ynorm, double* yl)
+{
+    double cm = 1.0, sm = 0.0;
+    if (m >= 1) {
+        double cmm1 = 1.0, smm1 = 0.0;
+        cm = dir.cph;
+        sm = dir.sph;
+        const double cph2 = dir.cph + dir.cph;
+        for (int mm = 2; mm <= m; ++mm) {
+            const double cn = cph2 * cm - cmm1;
+            const double sn = cph2 * sm - smm1;
+            cmm1 = cm;
+            smm1 = sm;
+            cm = cn;
+            sm = sn;
+        }
+    }
+    double fac = 1.0;
+    for (int mm = 0; mm < m; ++mm) {
+        fac = -(mm + mm - 1) * fac;
+        fac = fac * dir.sth;
+    }
+    fac = -(m + m - 1) * fac;
+    double pl2 = 0.0, pl1 = fac;
+    for (int l = m; l <= lmax; ++l) {
+        double pv;
+        if (l == m) pv = fac;
+        else if (l == m + 1) pv = (m + m + 1) * dir.cth * fac;
+        else pv = ((l + l - 1) * dir.cth * pl1 - (l + m - 1) * pl2) / (l - m);
+        if (l > m) {
+            pl2 = pl1;
+            pl1 = pv;
+        }
+        const int lm0 = l * (l + 1);
+        const double v = ynorm[lm0 + m] * pv;
+        if (m == 0) {
+            yl[lm0] = v;
+        } else {
+            yl[lm0 + m] = v * cm;
+            yl[lm0 - m] = v * sm;
+        }
+    }
+}
+
+}  // namespace
+
+// ---------------------------------------------------------------------------
+// Generator: one workgroup per plane wave.  Phases of all atoms, then per
+// chunk of kinds the Bessel values and the direction (one lane per kind), the
+// real radial factors a_l, b_l (A and B without phase and harmonic), the real
+// harmonics (one lane per kind and m) and, with y, the real vectors
+// [a_l Y_lm; b_l Y_lm].
+// ---------------------------------------------------------------------------
+__global__ __launch_bounds__(256) void k_sphere_gen(SphereArgs p)
+{
+    extern __shared__ double smem[];
+    const int tid = threadIdx.x;
+    const int nl = p.nl;
+    const int L = p.L;
+    double* s_bes = smem;                              // [chunk][2 nl]  fj, dfj
+    double2* s_ab = (double2*)(s_bes + p.chunk * 2 * nl);   // [chunk][nl] (a_l, b_l)
+    double* s_y = (double*)(s_ab + p.chunk * nl);      // [chunk][L]     real harmonics
+    DirAngles* s_dir = (DirAngles*)(s_y + p.chunk * L);     // [chunk]
+    unsigned char* s_l = (unsigned char*)(s_dir + p.chunk); // [L]       l of lm
+    const int c = blockIdx.x;
+    const SphereK* kp = &p.one;
+    if (p.nk > 1) kp = p.many + find_last(p.nk, c, [&](int i) { return p.many[i].gcol0; });
+    const int gi = c - kp->gcol0;
+    const int64_t col = kp->col0 + gi;
+    const double K0 = kp->k[0] + kp->g[3 * gi + 0];
+    const double K1 = kp->k[1] + kp->g[3 * gi + 1];
+    const double K2 = kp->k[2] + kp->g[3 * gi + 2];
+    const double c0 = p.bmat[0] * K0 + p.bmat[3] * K1 + p.bmat[6] * K2;
+    const double c1 = p.bmat[1] * K0 + p.bmat[4] * K1 + p.bmat[7] * K2;
+    const double c2 = p.bmat[2] * K0 + p.bmat[5] * K1 + p.bmat[8] * K2;
+    const double Knorm = sqrt(c0 * c0 + c1 * c1 + c2 * c2);
+
+    for (int lm = tid; lm < L; lm += blockDim.x) s_l[lm] = (unsigned char)l_of_lm(lm);
+    // phases e^{i 2 pi K.tau}; the lanes with the Bessel recurrences come last
+    for (int a = blockDim.x - 1 - tid; a < p.natoms; a += blockDim.x) {
+        const AtomDev& at = p.atoms[p.order[a]];
+        const double kt = K0 * at.pos[0] + K1 * at.pos[1] + K2 * at.pos[2];
+        double ps, pc;
+        sincos(2.0 * kPi * kt, &ps, &pc);
+        p.ph[(int64_t)a * p.gtot + col] = make_double2(pc, ps);
+    }
+    for (int k0 = 0; k0 < p.nkinds; k0 += p.chunk) {
+        const int nk = min(p.chunk, p.nkinds - k0);
+        if (tid < nk) {
+            double* fj = s_bes + tid * 2 * nl;
+            bessel_lds(p.max_lmax, p.kinds[k0 + tid].rmt * Knorm, fj, fj + nl);
+        } else if (p.y && tid >= 64 && tid - 64 < nk) {
+            s_dir[tid - 64] = dir_angles(p.kinds[k0 + tid - 64].rot, K0, K1, K2);
+        }
+        __syncthreads();
+        for (int q = tid; q < nk * nl; q += blockDim.x) {
+            const int t = q / nl;
+            const int l = q - t * nl;
+            const KindDev& kd = p.kinds[k0 + t];
+            if (l > kd.lmax) continue;
+            const double* fj = s_bes + t * 2 * nl;
+            const double* dfj = fj + nl;
+            const RadDev m = p.rad[(int64_t)kd.rep * nl + l];
+            const double pref = p.vol_prefac * m.inv_wronk;
+            const double au = m.dE_u * Knorm * dfj[l] - m.dE_u_dr * fj[l];
+            const double bu = -m.u * Knorm * dfj[l] + m.u_dr * fj[l];
+            const double2 ab = make_double2(pref * au, pref * bu);
+            s_ab[t * nl + l] = ab;
+            p.rs[col * p.ldr + kd.rsoff + l] = ab;
+        }
+        if (p.y) {
+            for (int q = tid; q < nk * nl; q += blockDim.x) {
+                const int t = q / nl;
+                const int m = q - t * nl;
+                if (m <= p.kinds[k0 + t].lmax) ylm_real(m, p.kinds[k0 + t].lmax, s_dir[t], p.ynorm, s_y + t * L);
+            }
+            __syncthreads();
+            double* yc = p.y + col * p.ldy;
+            for (int t = 0; t < nk; ++t) {
+                const KindDev& kd = p.kinds[k0 + t];
+                for (int r = tid; r < kd.r4; r += blockDim.x) {
+                    double v = 0.0;
+                    if (r < kd.nlm) v = s_ab[t * nl + s_l[r]].x * s_y[t * L + r];
+                    else if (r < 2 * kd.nlm) v = s_ab[t * nl + s_l[r - kd.nlm]].y * s_y[t * L + r - kd.nlm];
+                    yc[kd.yoff + r] = v;
+                }
+            }
+        }
+        __syncthreads();
+    }
+}
+
+static size_t sphere_gen_lds(int chunk, int nl, int L)
+{
+    return sizeof(double) * (size_t)chunk * (2 * nl + 2 * nl + L) + sizeof(DirAngles) * (size_t)chunk + (size_t)L;
+}
+
+// Kinds per pass of the generator: as many as 32 KiB of LDS hold, at most 16
+// (5 workgroups per CU; 16 kinds of lmax 12 take 28 KiB).
+int sphere_chunk(int nl, int L)
+{
+    int chunk = 16;
+    while (chunk > 1 && sphere_gen_lds(chunk, nl, L) > 32 * 1024) chunk /= 2;
+    return chunk;
+}
+
+hipError_t launch_sphere_gen(const SphereArgs& p, hipStream_t st)
+{
+    if (p.ngcols <= 0) return hipSuccess;
+    const size_t lds = sphere_gen_lds(p.chunk, p.nl, p.L);
+    hipLaunchKernelGGL(k_sphere_gen, dim3(p.ngcols), dim3(256), lds, st, p);
+    return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------
+// S by the addition theorem.  One workgroup per lower tile of 16 M x 16 M,
+// M x MJ elements per thread (rows tx + 16 m: stores of 16 consecutive rows).  Per kind, per element: the Legendre sum (7 FP64
+// operations per l) and 4 fused operations per atom of the kind, against
+// 8 (2 L) per atom of the contraction S = Y^H Y it replaces; vector FP64 and
+// the LDS reads (M + MJ of 16 bytes per M MJ elements) bound it.  Measured:
+// 6.1 ms at N_G 12007 (128 atoms of 8 kinds, lmax 12), where the contraction
+// took about 350 ms; 0.10 ms at N_G 2003 (32 atoms, 4 kinds, lmax 10).
+//
+// P_l comes from t = 1 - |cos| = |n -+ n'|^2 / 2, formed from the difference
+// (sum, where the cosine is negative) of the unit vectors, by
+//   P_l+1 - P_l = (l (P_l - P_l-1) - (2l+1) t P_l) / (l+1):
+// near parallel and antiparallel vectors, where P_l varies fastest, t keeps
+// its relative accuracy, which a cosine would lose.  Odd l carry the sign.
+// ---------------------------------------------------------------------------
+constexpr int kOvAtoms = 8;     // atoms whose phases are staged at a time
+
+struct LegendreCoef {
+    double a[kMaxLmax + 1], b[kMaxLmax + 1];
+};
+constexpr LegendreCoef legendre_coef()
+{
+    LegendreCoef c{};
+    for (int l = 0; l <= kMaxLmax; ++l) {
+        c.a[l] = (double)l / (double)(l + 1);
+        c.b[l] = (double)(2 * l + 1) / (double)(l + 1);
+    }
+    return c;
+}
+__constant__ const LegendreCoef kLegendre = legendre_coef();
+
+template <int M, int MJ>
+__global__ __launch_bounds__(256 * M / MJ) void k_overlap(SphereArgs p)
+{
+    // one rounding per written operation: every tile gives the same bits
+#pragma clang fp contract(off)
+    constexpr int T = 16 * M, TY = T / MJ, NT = 16 * TY;
+    extern __shared__ double smem[];
+    double2* s_ri = (double2*)smem;               // [nl][T] (a_l, b_l) of the rows
+    double2* s_rj = s_ri + p.nl * T;              // [nl][T] weighted, of the columns
+    double2* s_pi = s_rj + p.nl * T;              // [kOvAtoms][T] phases
+    double2* s_pj = s_pi + kOvAtoms * T;
+    double* s_n = (double*)(s_pj + kOvAtoms * T); // [2][3][T] unit vectors
+
+    const int tid = threadIdx.x;
+    const int tx = tid & 15, ty = tid >> 4;
+    const SphereK* kp = &p.one;
+    if (p.nk > 1) kp = p.many + find_last(p.nk, (int)blockIdx.x, [&](int i) { return p.many[i].stile0; });
+    const int tile = (int)blockIdx.x - kp->stile0;
+    const int bi = tri_row(tile);
+    const int bj = tile - (int)((int64_t)bi * (bi + 1) / 2);
+    const int I0 = bi * T, J0 = bj * T;
+    const int ng = kp->ng;
+    const int64_t ci = kp->col0 + I0, cj = kp->col0 + J0;
+
+    double sr[M][MJ], si[M][MJ], t[M][MJ], sg[M][MJ];
+#pragma unroll
+    for (int m = 0; m < M; ++m)
+#pragma unroll
+        for (int n = 0; n < MJ; ++n) {
+            sr[m][n] = 0.0;
+            si[m][n] = 0.0;
+            t[m][n] = 0.0;
+            sg[m][n] = 1.0;
+        }
+
+    for (int kk = 0; kk < p.nkinds; ++kk) {
+        const KindDev& kd = p.kinds[kk];
+        const int nlk = kd.lmax + 1;
+        const int count = kd.count;
+        // the direction of a column is kept while the rotation stays
+        bool newrot = kk == 0;
+        if (kk > 0)
+            for (int q = 0; q < 9; ++q)
+                newrot |= __double_as_longlong(kd.rot[q]) != __double_as_longlong(p.kinds[kk - 1].rot[q]);
+        __syncthreads();
+        for (int q = tid; q < nlk * T; q += NT) {
+            const int c = q / nlk, l = q - c * nlk;
+            s_ri[l * T + c] = p.rs[(ci + c) * p.ldr + kd.rsoff + l];
+        }
+        for (int q = tid; q < nlk * T; q += NT) {
+            const int c = q / nlk, l = q - c * nlk;
+            const double wl = (2 * l + 1) / (4.0 * kPi);
+            const double2 r = p.rs[(cj + c) * p.ldr + kd.rsoff + l];
+            const double wb = wl * p.rad[(int64_t)kd.rep * p.nl + l].dE_u_norm;
+            s_rj[l * T + c] = make_double2(wl * r.x, wb * r.y);
+        }
+        if (newrot && tid < 2 * T) {
+            const int side = tid / T, c = tid - side * T;
+            const int gi = min((side ? J0 : I0) + c, ng - 1);
+            const DirAngles d = dir_angles(kd.rot, kp->k[0] + kp->g[3 * gi], kp->k[1] + kp->g[3 * gi + 1],
+                                           kp->k[2] + kp->g[3 * gi + 2]);
+            double* s = s_n + side * 3 * T + c;
+            s[0] = d.sth * d.cph;
+            s[T] = d.sth * d.sph;
+            s[2 * T] = d.cth;
+        }
+        const int n0 = min(kOvAtoms, count);
+        for (int q = tid; q < n0 * T; q += NT) {
+            const int a = q / T, c = q - a * T;
+            const double2* ph = p.ph + (int64_t)(kd.first + a) * p.gtot;
+            s_pi[q] = ph[ci + c];
+            s_pj[q] = ph[cj + c];
+        }
+        __syncthreads();
+        if (newrot) {
+#pragma unroll
+            for (int m = 0; m < M; ++m)
+#pragma unroll
+                for (int n = 0; n < MJ; ++n) {
+                    const double* a = s_n + tx + 16 * m;
+                    const double* b = s_n + 3 * T + ty + TY * n;
+                    const double dot = __builtin_fma(a[2 * T], b[2 * T], __builtin_fma(a[T], b[T], a[0] * b[0]));
+                    sg[m][n] = dot < 0.0 ? -1.0 : 1.0;
+                    const double x = __builtin_fma(-sg[m][n], b[0], a[0]);
+                    const double y = __builtin_fma(-sg[m][n], b[T], a[T]);
+                    const double z = __builtin_fma(-sg[m][n], b[2 * T], a[2 * T]);
+                    t[m][n] = 0.5 * __builtin_fma(z, z, __builtin_fma(y, y, x * x));
+                }
+        }
+        // sum over l, even and odd apart
+        double rad[M][MJ];
+        {
+            double P[M][MJ], d[M][MJ], ev[M][MJ], od[M][MJ];
+#pragma unroll
+            for (int m = 0; m < M; ++m)
+#pragma unroll
+                for (int n = 0; n < MJ; ++n) {
+                    P[m][n] = 1.0;
+                    d[m][n] = 0.0;
+                    ev[m][n] = 0.0;
+                    od[m][n] = 0.0;
+                }
+            auto step = [&](int l, double(&acc)[M][MJ]) {
+                double2 ri[M], rj[MJ];
+#pragma unroll
+                for (int m = 0; m < M; ++m) ri[m] = s_ri[l * T + tx + 16 * m];
+#pragma unroll
+                for (int n = 0; n < MJ; ++n) rj[n] = s_rj[l * T + ty + TY * n];
+                const double ca = kLegendre.a[l], cb = kLegendre.b[l];
+#pragma unroll
+                for (int m = 0; m < M; ++m)
+#pragma unroll
+                    for (int n = 0; n < MJ; ++n) {
+                        const double w = __builtin_fma(ri[m].y, rj[n].y, ri[m].x * rj[n].x);
+                        acc[m][n] = __builtin_fma(w, P[m][n], acc[m][n]);
+                        d[m][n] = __builtin_fma(-cb, t[m][n] * P[m][n], ca * d[m][n]);
+                        P[m][n] += d[m][n];
+                    }
+            };
+            for (int l = 0; l < nlk; l += 2) {
+                step(l, ev);
+                if (l + 1 < nlk) step(l + 1, od);
+            }
+#pragma unroll
+            for (int m = 0; m < M; ++m)
+#pragma unroll
+                for (int n = 0; n < MJ; ++n) rad[m][n] = __builtin_fma(sg[m][n], od[m][n], ev[m][n]);
+        }
+        // structure factor of the kind's atoms
+        double fr[M][MJ], fi[M][MJ];
+#pragma unroll
+        for (int m = 0; m < M; ++m)
+#pragma unroll
+            for (int n = 0; n < MJ; ++n) {
+                fr[m][n] = 0.0;
+                fi[m][n] = 0.0;
+            }
+        for (int a0 = 0; a0 < count; a0 += kOvAtoms) {
+            const int na = min(kOvAtoms, count - a0);
+            if (a0 > 0) {
+                __syncthreads();
+                for (int q = tid; q < na * T; q += NT) {
+                    const int a = q / T, c = q - a * T;
+                    const double2* ph = p.ph + (int64_t)(kd.first + a0 + a) * p.gtot;
+                    s_pi[q] = ph[ci + c];
+                    s_pj[q] = ph[cj + c];
+                }
+                __syncthreads();
+            }
+            for (int a = 0; a < na; ++a) {
+                double2 u[M], v[MJ];
+#pragma unroll
+                for (int m = 0; m < M; ++m) u[m] = s_pi[a * T + tx + 16 * m];
+#pragma unroll
+                for (int n = 0; n < MJ; ++n) v[n] = s_pj[a * T + ty + TY * n];
+#pragma unroll
+                for (int m = 0; m < M; ++m)
+#pragma unroll
+                    for (int n = 0; n < MJ; ++n) {
+                        fr[m][n] = __builtin_fma(u[m].y, v[n].y, __builtin_fma(u[m].x, v[n].x, fr[m][n]));
+                        fi[m][n] = __builtin_fma(-u[m].y, v[n].x, __builtin_fma(u[m].x, v[n].y, fi[m][n]));
+                    }
+            }
+        }
+#pragma unroll
+        for (int m = 0; m < M; ++m)
+#pragma unroll
+            for (int n = 0; n < MJ; ++n) {
+                sr[m][n] = __builtin_fma(fr[m][n], rad[m][n], sr[m][n]);
+                si[m][n] = __builtin_fma(fi[m][n], rad[m][n], si[m][n]);
+            }
+    }
+#pragma unroll
+    for (int n = 0; n < MJ; ++n)
+#pragma unroll
+        for (int m = 0; m < M; ++m) {
+            const int i = I0 + tx + 16 * m, j = J0 + ty + TY * n;
+            if (i < ng && i >= j) kp->S[(int64_t)j * kp->ldS + i] = make_double2(sr[m][n], i == j ? 0.0 : si[m][n]);
+        }
+}
+
+int overlap_tile(int64_t tiles64, int n_cu)
+{
+    // 64 x 64 tiles once they give every CU two workgroups, 32 x 32 once
+    // those do, else 16 x 16: a smaller tile reads its columns more often but
+    // spreads a small triangle over more CUs
+    if (tiles64 >= 2 * (int64_t)n_cu) return 64;
+    return 4 * tiles64 >= 2 * (int64_t)n_cu ? 32 : 16;
+}
+
+hipError_t launch_overlap(const SphereArgs& p, int tile, int64_t ntiles, hipStream_t st)
+{
+    if (ntiles <= 0) return hipSuccess;
+    const size_t lds = sizeof(double2) * (size_t)tile * 2 * (p.nl + kOvAtoms) + sizeof(double) * 6 * tile;
+    const dim3 grid((unsigned)ntiles), block(tile == 64 ? 512 : 256);
+    if (tile == 64) {
+        const hipError_t e =
+            hipFuncSetAttribute((const void*)(k_overlap<4, 2>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) return e;
+        hipLaunchKernelGGL((k_overlap<4, 2>), grid, block, lds, st, p);
+    } else if (tile == 32) {
+        hipLaunchKernelGGL((k_overlap<2, 2>), grid, block, lds, st, p);
+    } else {
+        hipLaunchKernelGGL((k_overlap<1, 1>), grid, block, lds, st, p);
+    }
+    return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------
+// T in real harmonics: Mt = D^H M D of one atom's M = [[T_aa, T_ab],
+// [T_ab^H, T_bb]] (T_aa, T_bb from their lower triangles), rows contiguous:
+// Mt[r * ldm + k] = (D^H M D)_rk, zero for r or k past 2 nlm.  D maps real to
+// complex harmonics with entries 1 and +-i, so an element is a sum of at most
+// four elements of M.
+// ---------------------------------------------------------------------------
+namespace {
+
+__device__ __forceinline__ double2 t_elem(const double2* taa, const double2* tab, const double2* tbb, int n, int r,
+                                          int c)
+{
+    const bool rb = r >= n, cb = c >= n;
+    const int i = rb ? r - n : r, j = cb ? c - n : c;
+    double2 v;
+    if (rb == cb) {
+        const double2* t = rb ? tbb : taa;
+        if (i >= j) {
+            v = t[i + (int64_t)n * j];
+        } else {
+            v = t[j + (int64_t)n * i];
+            v.y = -v.y;
+        }
+        if (i == j) v.y = 0.0;
+    } else if (cb) {
+        v = tab[i + (int64_t)n * j];
+    } else {
+        v = tab[j + (int64_t)n * i];
+        v.y = -v.y;
+    }
+    return v;
+}
+
+}  // namespace
+
+__global__ __launch_bounds__(256) void k_build_mt(const MtJob* __restrict__ jobs, double2* __restrict__ mt)
+{
+#pragma clang fp contract(off)
+    const MtJob jb = jobs[blockIdx.y];
+    const int n = jb.nlm, n2 = 2 * n;
+    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int r = (int)(e / jb.ldm), k = (int)(e - (int64_t)r * jb.ldm);
+    if (r >= jb.rows) return;
+    double2 out = make_double2(0.0, 0.0);
+    if (r < n2 && k < n2) {
+        // D column of x = (l, +-m): entries at (l, m) and (l, -m)
+        auto terms = [&](int x, int idx[2], double2 co[2]) {
+            const int blk = x >= n ? n : 0;
+            const int lm = x - blk;
+            const int l = l_of_lm(lm);
+            const int m = lm - l * (l + 1);
+            if (m == 0) {
+                idx[0] = x;
+                co[0] = make_double2(1.0, 0.0);
+                return 1;
+            }
+            const int am = m > 0 ? m : -m;
+            const double s = (am & 1) ? -1.0 : 1.0;
+            idx[0] = blk + l * (l + 1) + am;
+            idx[1] = blk + l * (l + 1) - am;
+            // cos: (1, s); sin: (-i, s i)
+            co[0] = m > 0 ? make_double2(1.0, 0.0) : make_double2(0.0, -1.0);
+            co[1] = m > 0 ? make_double2(s, 0.0) : make_double2(0.0, s);
+            return 2;
+        };
+        int ir[2], ik[2];
+        double2 cr[2], ck[2];
+        const int nr = terms(r, ir, cr), nk = terms(k, ik, ck);
+        for (int a = 0; a < nr; ++a)
+            for (int b = 0; b < nk; ++b) {
+                const double2 v = t_elem(jb.taa, jb.tab, jb.tbb, n, ir[a], ik[b]);
+                // conj(cr) ck is a power of i
+                const double fr = cr[a].x * ck[b].x + cr[a].y * ck[b].y;
+                const double fi = cr[a].x * ck[b].y - cr[a].y * ck[b].x;
+                if (fr != 0.0) {
+                    out.x += fr * v.x;
+                    out.y += fr * v.y;
+                } else {
+                    out.x -= fi * v.y;
+                    out.y += fi * v.x;
+                }
+            }
+    }
+    mt[jb.off + e] = out;
+}
+
+hipError_t launch_build_mt(const MtJob* jobs, int njobs, int64_t max_elems, double2* mt, hipStream_t st)
+{
+    if (njobs <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_build_mt, dim3((unsigned)((max_elems + 255) / 256), njobs), dim3(256), 0, st, jobs, mt);
+    return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------
+// Complex-by-real products on v_mfma_f64_16x16x4.
+//
+// One tile is B x B: rows are columns of a complex operand X, columns are
+// columns of a real operand y, both contiguous along the depth:
+//   T[r][c] = sum_k X[k, r] y[k, c]       two real MFMAs per 16 x 16 x 4.
+// kH: X = W of the tile's H columns j, y of the tile's H rows i.  The depth
+//   runs over all atoms; where an atom ends (a k-step of 4, marked in the
+//   k-step table) T is multiplied by conj(ph_a(i)) into the result C and
+//   cleared: 4 fused operations per element and atom on the vector pipe next
+//   to 4 (2 L_a) on the matrix pipe.  The table also gives the row of y of
+//   each k-step, so atoms of one kind read the same y.
+// !kH (T application): X = rows of Mt of one kind's atoms side by side, y of
+//   the kind; W = ph_a(g) T is stored.
+//
+// Bound by FP64 MFMA.  Waves own 16 x 32 of the tile (16 x 16 of the 32 x 32
+// tile): T and C take 64 VGPRs, so four waves per SIMD fit (two workgroups of
+// 64 x 64 per CU, whose barriers do not wait for each other).  The operands go
+// from global memory straight into a two-stage LDS ring (16 rows per stage);
+// X's columns are 16 chunks of 16 bytes, chunk q stored at q ^ (column % 16),
+// y's 8 chunks, chunk q at q ^ (column / 2 % 8): 16 lanes that read one row
+// hit distinct banks.  The fragments of the next k-step are read before the
+// MFMAs of the current one, across the stage barrier too.
+// Measured (whole call, complex-by-complex contraction of S and H before, now):
+// 713 -> 244 ms at N_G 12007 (128 atoms, lmax 12), 33.4 -> 12.3 ms at 6002 and
+// 5.42 -> 2.35 ms at 2003 (32 atoms, lmax 10).
+// ---------------------------------------------------------------------------
+namespace {
+
+typedef double d4 __attribute__((ext_vector_type(4)));
+typedef double v2d __attribute__((ext_vector_type(2)));
+typedef int i4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(4))) const i4* ctab;
+
+// s_waitcnt immediates (vmcnt bits [3:0] and [15:14], expcnt [6:4], lgkmcnt [11:8])
+constexpr int kWaitVm0 = (0 & 15) | (7 << 4) | (15 << 8);
+constexpr int kWaitVm0Lgkm0 = (0 & 15) | (7 << 4) | (0 << 8);
+
+}  // namespace
+
+template <int B>
+struct SphereTile {
+    static constexpr int kRB = 1;                 // 16-row blocks per wave
+    static constexpr int kCB = B == 64 ? 2 : 1;   // 16-column blocks per wave
+    static constexpr int kWR = B / (16 * kRB);    // waves along the rows
+    static constexpr int kWC = B / (16 * kCB);
+    static constexpr int kWaves = kWR * kWC;
+    static constexpr int kThreads = 64 * kWaves;
+    static constexpr int kXBytes = B * 256;       // one stage of X, of y
+    static constexpr int kYBytes = B * 128;
+    static constexpr int kStage = kXBytes + kYBytes;
+    static constexpr int kLoads = kStage / 1024 / kWaves;   // 1 KiB wave loads per wave and stage
+    static_assert(kStage / 1024 % kWaves == 0, "a stage splits evenly over the waves");
+};
+
+template <int B, bool kH>
+__global__ __launch_bounds__(SphereTile<B>::kThreads, B == 64 ? 4 : 2) void k_sphere_gemm(SphereArgs p)
+{
+#pragma clang fp contract(off)
+    using Tl = SphereTile<B>;
+    constexpr int RB = Tl::kRB, CB = Tl::kCB, LPW = Tl::kLoads;
+    extern __shared__ __attribute__((aligned(1024))) char lds[];
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wr = wave % Tl::kWR, wc = wave / Tl::kWR;
+
+    // ---- the tile ----
+    const SphereK* kp = &p.one;
+    const KindDev* kd = nullptr;
+    int R0, C0;             // first row (X column), first column (y column) of the tile
+    int nsteps;             // k-steps of 4
+    if constexpr (kH) {
+        // Workgroups go to the 8 XCDs in turn: XCD x takes the patches x,
+        // x + 8, ... of pside x pside tiles, so that the tiles in flight on
+        // one L2 share their panels.
+        const int pp = p.pside * p.pside;
+        const int slot = (int)blockIdx.x / 8;
+        const int patch = slot / pp * 8 + (int)blockIdx.x % 8;
+        if (patch >= p.npatch) return;
+        const int in = slot % pp;
+        if (p.nk > 1) kp = p.many + find_last(p.nk, patch, [&](int i) { return p.many[i].hpatch0; });
+        const int lp = patch - kp->hpatch0;
+        const int pi = tri_row(lp);
+        const int pj = lp - (int)((int64_t)pi * (pi + 1) / 2);
+        const int bi = pi * p.pside + in % p.pside, bj = pj * p.pside + in / p.pside;
+        if (bj > bi || bi * B >= kp->ng) return;
+        R0 = bj * B;
+        C0 = bi * B;
+        nsteps = p.nksteps;
+    } else {
+        // kinds in turn; per kind its tiles of rows, per row tile all columns
+        const int ntc = (int)((p.gtot + B - 1) / B);
+        const int tr = (int)blockIdx.x / ntc;
+        const int kk = find_last(p.nkinds, tr, [&](int i) { return B == 64 ? p.kinds[i].rt64 : p.kinds[i].rt32; });
+        kd = p.kinds + kk;
+        R0 = (tr - (B == 64 ? kd->rt64 : kd->rt32)) * B;
+        C0 = ((int)blockIdx.x - tr * ntc) * B;
+        nsteps = kd->r4 / 4;
+    }
+    const int nst = (nsteps + 3) / 4;
+
+    // ---- this lane's loads: X columns of 16 chunks, then y columns of 8 ----
+    const char* src[LPW];
+    bool isy[LPW];
+    int sel[LPW];
+#pragma unroll
+    for (int r = 0; r < LPW; ++r) {
+        const int g = wave * LPW + r;
+        const int slot = g * 64 + lane;
+        isy[r] = g >= Tl::kXBytes / 1024;
+        if (!isy[r]) {
+            const int c = slot / 16;
+            const int q = (slot % 16) ^ (c & 15);
+            const double2* x;
+            if constexpr (kH) {
+                x = p.W + (kp->col0 + R0 + c) * p.ldw;
+            } else {
+                // row R0 + c of the kind's stacked Mt; past its last row the last one again
+                const int row = min(R0 + c, kd->count * kd->r4 - 1);
+                const int a = row / kd->r4;
+                x = p.mt + p.mtoff[kd->first + a] + (int64_t)(row - a * kd->r4) * kd->ldm;
+            }
+            src[r] = (const char*)(x + q);
+            sel[r] = 0;
+        } else {
+            const int s2 = slot - B * 16;
+            const int c = s2 / 8;
+            const int q = (s2 % 8) ^ ((c >> 1) & 7);
+            const int64_t col = (kH ? kp->col0 : 0) + C0 + c;
+            const double* y = p.y + col * p.ldy + 2 * (q & 1);
+            if constexpr (!kH) y += kd->yoff;
+            src[r] = (const char*)y;
+            sel[r] = q >> 1;
+        }
+    }
+    typedef __attribute__((address_space(3))) char lchar;
+    lchar* lbase = (lchar*)lds;
+    // constant address space: the table's entries come by scalar loads
+    const ctab tab = (ctab)(const void*)p.ksteps;
+    // the k-step entries of stage s (for T: none)
+    auto entries = [&](int s) -> i4 {
+        if constexpr (kH) return tab[__builtin_amdgcn_readfirstlane(s)];
+        else return i4{0, 0, 0, 0};
+    };
+    auto issue = [&](int s, int buf, i4 e) {
+#pragma unroll
+        for (int r = 0; r < LPW; ++r) {
+            const char* gb;
+            if (!isy[r]) {
+                gb = src[r] + (int64_t)s * 256;
+            } else if constexpr (kH) {
+                const int lo = sel[r] & 1 ? e.y : e.x, hi = sel[r] & 1 ? e.w : e.z;
+                const int row = sel[r] & 2 ? hi : lo;
+                gb = src[r] + (int64_t)(row & ~3) * 8;
+            } else {
+                gb = src[r] + (int64_t)(16 * s + 4 * sel[r]) * 8;
+            }
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)gb,
+                                             (__attribute__((address_space(3))) void*)(lbase + buf * Tl::kStage +
+                                                                                       (wave * LPW + r) * 1024),
+                                             16, 0, 0);
+        }
+    };
+
+    d4 tr_[RB][CB], ti_[RB][CB];
+    d4 cr[RB][CB], ci[RB][CB];
+#pragma unroll
+    for (int i = 0; i < RB; ++i)
+#pragma unroll
+        for (int j = 0; j < CB; ++j) {
+            tr_[i][j] = ti_[i][j] = d4{0.0, 0.0, 0.0, 0.0};
+            if constexpr (kH) cr[i][j] = ci[i][j] = d4{0.0, 0.0, 0.0, 0.0};
+        }
+
+    int rowX[RB], colY[CB];
+#pragma unroll
+    for (int i = 0; i < RB; ++i) rowX[i] = wr * 16 * RB + i * 16 + (lane & 15);
+#pragma unroll
+    for (int j = 0; j < CB; ++j) colY[j] = wc * 16 * CB + j * 16 + (lane & 15);
+    const int q0 = lane >> 4;
+    auto read_frags = [&](int buf, int ks, v2d* x, double* y) {
+        const char* lb = lds + buf * Tl::kStage;
+#pragma unroll
+        for (int i = 0; i < RB; ++i) x[i] = *(const v2d*)&lb[rowX[i] * 256 + 16 * ((q0 + 4 * ks) ^ (rowX[i] & 15))];
+#pragma unroll
+        for (int j = 0; j < CB; ++j)
+            y[j] = *(const double*)&lb[Tl::kXBytes + colY[j] * 128 +
+                                       16 * (((q0 >> 1) + 2 * ks) ^ ((colY[j] >> 1) & 7)) + 8 * (q0 & 1)];
+    };
+    // phases of the current atom at this lane's H rows
+    double2 ph[CB];
+    const double2* phsrc = nullptr;
+    if constexpr (kH) {
+        phsrc = p.ph + kp->col0 + C0;
+#pragma unroll
+        for (int j = 0; j < CB; ++j) ph[j] = phsrc[colY[j]];
+    }
+    auto flush = [&]() {
+#pragma unroll
+        for (int i = 0; i < RB; ++i)
+#pragma unroll
+            for (int j = 0; j < CB; ++j)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const double a = tr_[i][j][q], b = ti_[i][j][q];
+                    cr[i][j][q] = __builtin_fma(ph[j].y, b, __builtin_fma(ph[j].x, a, cr[i][j][q]));
+                    ci[i][j][q] = __builtin_fma(-ph[j].y, a, __builtin_fma(ph[j].x, b, ci[i][j][q]));
+                    tr_[i][j][q] = 0.0;
+                    ti_[i][j][q] = 0.0;
+                }
+        // the next atom's (after the last: a spare row, unused)
+        phsrc += p.gtot;
+#pragma unroll
+        for (int j = 0; j < CB; ++j) ph[j] = phsrc[colY[j]];
+    };
+
+    // ---- main loop ----
+    i4 e0 = entries(0), e1 = entries(min(1, nst - 1));
+    issue(0, 0, e0);
+    __builtin_amdgcn_s_waitcnt(kWaitVm0);
+    asm volatile("s_barrier" ::: "memory");
+    issue(min(1, nst - 1), 1, e1);
+    v2d fx[RB];
+    double fy[CB];
+    read_frags(0, 0, fx, fy);
+    for (int s = 0; s < nst; ++s) {
+        const i4 e2 = entries(min(s + 2, nst - 1));
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) {
+            v2d x[RB];
+            double y[CB];
+#pragma unroll
+            for (int i = 0; i < RB; ++i) x[i] = fx[i];
+#pragma unroll
+            for (int j = 0; j < CB; ++j) y[j] = fy[j];
+            if (ks < 3) {
+                read_frags(s & 1, ks + 1, fx, fy);
+            } else if (s + 1 < nst) {
+                // this wave's loads of stage s+1 landed and its reads of stage
+                // s are done; after the barrier that holds for every wave, and
+                // stage s+2 (at the end the last again: in bounds, unused) may
+                // overwrite stage s
+                __builtin_amdgcn_s_waitcnt(kWaitVm0Lgkm0);
+                asm volatile("s_barrier" ::: "memory");
+                issue(min(s + 2, nst - 1), s & 1, e2);
+                read_frags((s + 1) & 1, 0, fx, fy);
+            }
+            // rows past the depth (in the last stage) are not multiplied
+            if (!kH && 4 * s + ks >= nsteps) break;
+#pragma unroll
+            for (int i = 0; i < RB; ++i)
+#pragma unroll
+                for (int j = 0; j < CB; ++j)
+                    tr_[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[i].x, y[j], tr_[i][j], 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < RB; ++i)
+#pragma unroll
+                for (int j = 0; j < CB; ++j)
+                    ti_[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[i].y, y[j], ti_[i][j], 0, 0, 0);
+            if constexpr (kH) {
+                const int f = ks == 0 ? e0.x : ks == 1 ? e0.y : ks == 2 ? e0.z : e0.w;
+                if (f & 1) flush();
+            }
+        }
+        e0 = e1;
+        e1 = e2;
+    }
+    __builtin_amdgcn_s_waitcnt(0);
+
+    // ---- store: lane holds rows (lane >> 4) + 4 q of column lane & 15 ----
+    if constexpr (kH) {
+        const int ng = kp->ng;
+#pragma unroll
+        for (int i = 0; i < RB; ++i)
+#pragma unroll
+            for (int j = 0; j < CB; ++j) {
+                const int gi = C0 + colY[j];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const int gj = R0 + wr * 16 * RB + i * 16 + q0 + 4 * q;
+                    if (gi < ng && gi >= gj)
+                        kp->H[(int64_t)gj * kp->ldH + gi] = make_double2(cr[i][j][q], gi == gj ? 0.0 : ci[i][j][q]);
+                }
+            }
+    } else {
+        const int nrow = kd->count * kd->r4;
+#pragma unroll
+        for (int i = 0; i < RB; ++i)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int row = R0 + wr * 16 * RB + i * 16 + q0 + 4 * q;
+                if (row < nrow) {
+                    const double2* phr = p.ph + (int64_t)(kd->first + row / kd->r4) * p.gtot;
+#pragma unroll
+                    for (int j = 0; j < CB; ++j) {
+                        const int64_t col = C0 + colY[j];
+                        if (col < p.gtot) {
+                            const double2 f = phr[col];
+                            const double a = tr_[i][j][q], b = ti_[i][j][q];
+                            p.W[col * p.ldw + kd->woff + row] =
+                                make_double2(__builtin_fma(f.x, a, -(f.y * b)), __builtin_fma(f.x, b, f.y * a));
+                        }
+                    }
+                }
+            }
+    }
+}
+
+template <int B, bool kH>
+static hipError_t launch_sphere_gemm(const SphereArgs& p, int64_t nblk, hipStream_t st)
+{
+    if (nblk <= 0) return hipSuccess;
+    constexpr int lds = 2 * SphereTile<B>::kStage;
+    hipLaunchKernelGGL((k_sphere_gemm<B, kH>), dim3((unsigned)nblk), dim3(SphereTile<B>::kThreads), lds, st, p);
+    return hipGetLastError();
+}
+
+hipError_t launch_sphere_tapp(const SphereArgs& p, int tile, int rtiles, hipStream_t st)
+{
+    const int64_t n = (int64_t)rtiles * ((p.gtot + tile - 1) / tile);
+    return tile == 64 ? launch_sphere_gemm<64, false>(p, n, st) : launch_sphere_gemm<32, false>(p, n, st);
+}
+
+hipError_t launch_sphere_h(const SphereArgs& p, int tile, hipStream_t st)
+{
+    const int64_t n = (int64_t)((p.npatch + 7) / 8) * 8 * p.pside * p.pside;
+    return tile == 64 ? launch_sphere_gemm<64, true>(p, n, st) : launch_sphere_gemm<32, true>(p, n, st);
+}
+
+}  // namespace hsgen

@@ -1,0 +1,271 @@
+// Host side of the FP64 path from a system description (sphere.h, sphere.hip):
+// tables of a system, operand layout of a call and its launch sequence
+//   generator (phases, radial factors, real vectors) -> T application -> H, S
+// shared by hsgen_create_hs, hsgen_create_hs_batched and
+// hsgen_create_hs_noalloc.
+#include <algorithm>
+#include <cstring>
+#include <map>
+
+#include "hsgen_host.h"
+
+namespace hsgen {
+
+namespace {
+
+// The bits that make two atoms one kind.
+std::string kind_key(const hsgen_sys* s, int a, const RadDev* rad)
+{
+    const AtomDev& at = s->atoms[a];
+    std::string k((const char*)&at.lmax, sizeof at.lmax);
+    k.append((const char*)&at.rmt, sizeof at.rmt);
+    k.append((const char*)at.rot, sizeof at.rot);
+    k.append((const char*)(rad + (size_t)a * s->nl), sizeof(RadDev) * (size_t)(at.lmax + 1));
+    return k;
+}
+
+int64_t lower(int64_t n) { return n * (n + 1) / 2; }
+
+}  // namespace
+
+// Kinds, their tables and the T blocks in real harmonics.  rad: the radial
+// data as uploaded to s->d_rad.
+hsgen_status sphere_setup(hsgen_ctx* ctx, hsgen_sys* s, const RadDev* rad)
+{
+    const int na = s->natoms;
+    std::map<std::string, int> id;
+    std::vector<std::vector<int>> members;
+    for (int a = 0; a < na; ++a) {
+        const auto it = id.emplace(kind_key(s, a, rad), (int)members.size());
+        if (it.second) members.emplace_back();
+        members[it.first->second].push_back(a);
+    }
+    // kinds of one rotation next to each other: S keeps its directions over them
+    std::stable_sort(members.begin(), members.end(), [&](const std::vector<int>& x, const std::vector<int>& y) {
+        return (s->atoms[x[0]].cls & 0xffff) < (s->atoms[y[0]].cls & 0xffff);
+    });
+    std::vector<KindDev> kinds(members.size());
+    std::vector<int32_t> order;
+    std::vector<int32_t> steps;
+    int64_t ry = 0, rw = 0, rr = 0, rt64 = 0, rt32 = 0;
+    for (size_t i = 0; i < members.size(); ++i) {
+        KindDev& k = kinds[i];
+        const AtomDev& at = s->atoms[members[i][0]];
+        std::memset(&k, 0, sizeof k);
+        k.lmax = at.lmax;
+        k.nlm = at.nlm;
+        k.r4 = (int32_t)roundup(2 * at.nlm, 4);
+        k.rep = members[i][0];
+        k.yoff = (int32_t)ry;
+        k.rsoff = (int32_t)rr;
+        k.woff = (int32_t)rw;
+        k.ldm = (int32_t)roundup(2 * at.nlm, 16);
+        k.rt64 = (int32_t)rt64;
+        k.rt32 = (int32_t)rt32;
+        k.first = (int32_t)order.size();
+        k.count = (int32_t)members[i].size();
+        k.rmt = at.rmt;
+        std::memcpy(k.rot, at.rot, sizeof k.rot);
+        for (int a : members[i]) {
+            order.push_back(a);
+            for (int r = 0; r < k.r4; r += 4) steps.push_back(k.yoff + r + (r + 4 == k.r4));
+        }
+        ry += k.r4;
+        rr += at.lmax + 1;
+        rw += (int64_t)k.count * k.r4;
+        rt64 += ((int64_t)k.count * k.r4 + 63) / 64;
+        rt32 += ((int64_t)k.count * k.r4 + 31) / 32;
+    }
+    if (rw > INT32_MAX - 64) return fail(ctx, HSGEN_ERR_UNSUPPORTED, "contraction depth too large");
+    s->nksteps = (int)steps.size();
+    while (steps.size() % 4) steps.push_back(0);    // the last stage reads four entries
+    s->nkinds = (int)kinds.size();
+    s->ldr = (int)rr;
+    s->rt64 = (int)rt64;
+    s->rt32 = (int)rt32;
+    // whole stages of 16 rows can be read at the end of a column, from any
+    // kind's first row; the odd multiple of 16 spreads the columns over the
+    // memory channels
+    s->ldy = (roundup(ry, 16) + 16) | 16;
+    s->ldw = roundup(rw, 16) | 16;
+    // T blocks in real harmonics, one per distinct T (h_owner)
+    std::vector<int64_t> off(na, 0), traw(na, 0);
+    int64_t total = 0, raw = 0, most = 0;
+    std::vector<int> owners;
+    for (int a = 0; a < na; ++a) {
+        if (s->h_owner[a] != a) continue;
+        const int64_t n = s->atoms[a].nlm;
+        off[a] = total;
+        total += roundup(2 * n, 4) * roundup(2 * n, 16);
+        most = std::max(most, roundup(2 * n, 4) * roundup(2 * n, 16));
+        traw[a] = raw;
+        raw += 3 * n * n;
+        owners.push_back(a);
+    }
+    std::vector<int64_t> mtoff(na);
+    for (int i = 0; i < na; ++i) mtoff[i] = off[s->h_owner[order[i]]];
+    auto up = [](size_t b) { return (size_t)roundup((int64_t)b, 256); };
+    const size_t b_mt = up(sizeof(double2) * (size_t)total), b_k = up(sizeof(KindDev) * kinds.size()),
+                 b_o = up(sizeof(int32_t) * order.size()), b_s = up(sizeof(int32_t) * steps.size()),
+                 b_m = up(sizeof(int64_t) * mtoff.size());
+    HIPCHK(hipMalloc(&s->d_sphere, b_mt + b_k + b_o + b_s + b_m));
+    char* p = (char*)s->d_sphere;
+    s->d_mt = (double2*)p;
+    s->d_kinds = (KindDev*)(p += b_mt);
+    s->d_order = (int32_t*)(p += b_k);
+    s->d_ksteps = (int32_t*)(p += b_o);
+    s->d_mtoff = (int64_t*)(p += b_s);
+    HIPCHK(hipMemcpyAsync(s->d_kinds, kinds.data(), sizeof(KindDev) * kinds.size(), hipMemcpyHostToDevice, ctx->stream));
+    HIPCHK(hipMemcpyAsync(s->d_order, order.data(), sizeof(int32_t) * order.size(), hipMemcpyHostToDevice, ctx->stream));
+    HIPCHK(hipMemcpyAsync(s->d_ksteps, steps.data(), sizeof(int32_t) * steps.size(), hipMemcpyHostToDevice,
+                          ctx->stream));
+    HIPCHK(hipMemcpyAsync(s->d_mtoff, mtoff.data(), sizeof(int64_t) * mtoff.size(), hipMemcpyHostToDevice, ctx->stream));
+    // the raw blocks, only until the transformed ones are built
+    struct Tmp {
+        void* p = nullptr;
+        ~Tmp() { if (p) (void)hipFree(p); }
+    } t_raw, t_jobs;
+    HIPCHK(hipMalloc(&t_raw.p, sizeof(double2) * (size_t)raw));
+    HIPCHK(hipMalloc(&t_jobs.p, sizeof(MtJob) * owners.size()));
+    double2* d = (double2*)t_raw.p;
+    std::vector<MtJob> jobs;
+    for (int a : owners) {
+        const int64_t n = s->atoms[a].nlm;
+        MtJob j{};
+        j.taa = d + traw[a];
+        j.tab = j.taa + n * n;
+        j.tbb = j.tab + n * n;
+        j.off = off[a];
+        j.nlm = (int32_t)n;
+        j.rows = (int32_t)roundup(2 * n, 4);
+        j.ldm = (int32_t)roundup(2 * n, 16);
+        const std::vector<std::complex<double>>* src[3] = {&s->h_taa[a], &s->h_tab[a], &s->h_tbb[a]};
+        for (int b = 0; b < 3; ++b)
+            HIPCHK(hipMemcpyAsync(d + traw[a] + b * n * n, src[b]->data(), sizeof(double2) * (size_t)(n * n),
+                                  hipMemcpyHostToDevice, ctx->stream));
+        jobs.push_back(j);
+    }
+    HIPCHK(hipMemcpyAsync(t_jobs.p, jobs.data(), sizeof(MtJob) * jobs.size(), hipMemcpyHostToDevice, ctx->stream));
+    // grid.y is at most 65535
+    for (size_t j0 = 0; j0 < jobs.size(); j0 += 32768)
+        HIPCHK(launch_build_mt((const MtJob*)t_jobs.p + j0, (int)std::min<size_t>(32768, jobs.size() - j0), most, s->d_mt,
+                               ctx->stream));
+    HIPCHK(hipStreamSynchronize(ctx->stream));
+    return HSGEN_OK;
+}
+
+// Operand layout of a call over k-points of ngs[] plane waves (each > 0).
+SphereLayout sphere_layout(const hsgen_ctx* ctx, const hsgen_sys* s, const std::vector<int>& ngs, bool do_h)
+{
+    SphereLayout l;
+    const int ncu = std::max(ctx->n_cu, 1);
+    int64_t t64 = 0, most = 1;
+    for (int ng : ngs) {
+        const int64_t nt = (ng + 63) / 64;
+        t64 += lower(nt);
+        most = std::max(most, nt);
+        l.gtot += nt * 64;
+    }
+    // H tiles of 64 x 64 once they give every CU a workgroup, else 32 x 32:
+    // four times the workgroups for a triangle that leaves CUs idle
+    l.htile = t64 >= ncu ? 64 : 32;
+    l.ttile = (int64_t)s->rt64 * (l.gtot / 64) >= ncu ? 64 : 32;
+    l.stile = overlap_tile(t64, ncu);
+    // patches: 8 x 8 tiles are what the 32 CUs of an XCD run at once; smaller
+    // ones where a triangle has few, so that the XCDs share it evenly
+    l.pside = most >= 128 ? 8 : most >= 24 ? 4 : 1;
+    for (int ng : ngs) {
+        const int64_t np = ((ng + l.htile - 1) / l.htile + l.pside - 1) / l.pside;
+        l.npatch += lower(np);
+        l.nstiles += lower((ng + l.stile - 1) / l.stile);
+        l.ngcols += ng;
+    }
+    const size_t g = (size_t)l.gtot;
+    l.b_ph = sizeof(double2) * g * (size_t)(s->natoms + 1);
+    l.b_rs = sizeof(double2) * g * (size_t)s->ldr;
+    l.b_y = do_h ? sizeof(double) * g * (size_t)s->ldy : 0;
+    l.b_w = do_h ? sizeof(double2) * g * (size_t)s->ldw : 0;
+    return l;
+}
+
+SphereArgs sphere_args(const hsgen_sys* s, const SphereLayout& l, void* ph, void* rs, void* y, void* w)
+{
+    SphereArgs p;
+    std::memset(&p, 0, sizeof p);
+    p.kinds = s->d_kinds;
+    p.atoms = s->d_atoms;
+    p.order = s->d_order;
+    p.rad = s->d_rad;
+    p.ynorm = s->d_ynorm;
+    std::memcpy(p.bmat, s->bmat, sizeof p.bmat);
+    p.vol_prefac = s->vol_prefac;
+    p.natoms = s->natoms;
+    p.nkinds = s->nkinds;
+    p.max_lmax = s->max_lmax;
+    p.nl = s->nl;
+    p.L = s->L;
+    p.chunk = sphere_chunk(s->nl, s->L);
+    p.nk = 1;
+    p.ngcols = (int32_t)l.ngcols;
+    p.gtot = l.gtot;
+    p.ph = (double2*)ph;
+    p.rs = (double2*)rs;
+    p.ldr = s->ldr;
+    p.y = (double*)y;
+    p.W = (double2*)w;
+    p.ldy = s->ldy;
+    p.ldw = s->ldw;
+    p.mt = s->d_mt;
+    p.mtoff = s->d_mtoff;
+    p.ksteps = s->d_ksteps;
+    p.nksteps = s->nksteps;
+    p.pside = l.pside;
+    p.npatch = (int32_t)l.npatch;
+    return p;
+}
+
+// The k-points of a call in layout order; gs, H, S device pointers.
+std::vector<SphereK> sphere_ks(const SphereLayout& l, const std::vector<const hsgen_kpoint*>& kps,
+                               const std::vector<const int32_t*>& gs, const std::vector<double2*>& H,
+                               const std::vector<double2*>& S, const std::vector<int64_t>& ldH,
+                               const std::vector<int64_t>& ldS)
+{
+    std::vector<SphereK> ks(kps.size());
+    int64_t col = 0, g = 0, st = 0, hp = 0;
+    for (size_t i = 0; i < kps.size(); ++i) {
+        SphereK& k = ks[i];
+        std::memset(&k, 0, sizeof k);
+        for (int q = 0; q < 3; ++q) k.k[q] = kps[i]->k[q];
+        k.g = gs[i];
+        k.H = H[i];
+        k.S = S[i];
+        k.ldH = ldH[i];
+        k.ldS = ldS[i];
+        k.col0 = col;
+        k.ng = kps[i]->ng;
+        k.gcol0 = (int32_t)g;
+        k.stile0 = (int32_t)st;
+        k.hpatch0 = (int32_t)hp;
+        col += roundup(k.ng, 64);
+        g += k.ng;
+        st += lower((k.ng + l.stile - 1) / l.stile);
+        hp += lower(((k.ng + l.htile - 1) / l.htile + l.pside - 1) / l.pside);
+    }
+    return ks;
+}
+
+// The launches of one call.  ev: events recorded after the generator and after
+// the T application, or null.
+hipError_t sphere_launch(const SphereArgs& p, const SphereLayout& l, const hsgen_sys* s, bool do_h, bool do_s,
+                         hipEvent_t ev_gen, hipEvent_t ev_tapp, hipStream_t st)
+{
+    hipError_t e = launch_sphere_gen(p, st);
+    if (e == hipSuccess && ev_gen) e = hipEventRecord(ev_gen, st);
+    if (e == hipSuccess && do_h) e = launch_sphere_tapp(p, l.ttile, l.ttile == 64 ? s->rt64 : s->rt32, st);
+    if (e == hipSuccess && ev_tapp) e = hipEventRecord(ev_tapp, st);
+    if (e == hipSuccess && do_h) e = launch_sphere_h(p, l.htile, st);
+    if (e == hipSuccess && do_s) e = launch_overlap(p, l.stile, l.nstiles, st);
+    return e;
+}
+
+}  // namespace hsgen

@@ -155,7 +155,10 @@ hsgen_status hsgen_autotune(hsgen_ctx* ctx, const hsgen_sys* sys, const hsgen_kp
         hsgen_report r{};
         double ms = 0.0;
         for (int rep = 0; rep < 2; ++rep) {   // warm-up, then the timed run
-            st = hsgen_create_hs(ctx, sys, kp, &o, dH, dS, ng, &r);
+            // FP64: the configurations are those of the general operands
+            st = precision == HSGEN_PREC_FP64
+                     ? create_hs_general(ctx, const_cast<hsgen_sys*>(sys), kp, o, dH, dS, ng, &r)
+                     : hsgen_create_hs(ctx, sys, kp, &o, dH, dS, ng, &r);
             if (st) return st;
             ms = precision == HSGEN_PREC_FP64 ? r.ms_contract : r.ms_igemm;
         }

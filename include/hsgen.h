@@ -103,7 +103,9 @@ typedef struct {
     int32_t flags;             /* HSGEN_FILL_UPPER | HSGEN_SKIP_H | HSGEN_SKIP_S */
     int32_t tile;              /* contraction tile config id (0 = the one hsgen_autotune chose
                                   for this size, else the built-in default for the size: smaller
-                                  tiles for calls too small to fill the GPU with the large ones) */
+                                  tiles for calls too small to fill the GPU with the large ones).
+                                  FP64 from a system picks its kernels by size alone: the id is
+                                  accepted and reported, every id gives the same bits */
 } hsgen_opts;
 
 typedef struct {
@@ -113,7 +115,8 @@ typedef struct {
     double ms_slice;           /* split precision: slicing */
     double ms_contract;        /* H and S contraction */
     double flops_alg;          /* 16 G^2 K + 32 G sum L_a^2 (K = sum L_a) */
-    double bytes_abgen;        /* algorithmic bytes written by A/B generation */
+    double bytes_abgen;        /* algorithmic bytes written by A/B generation (FP64 from a system:
+                                  phases, radial factors and real vectors) */
     int32_t ng;                /* G */
     int32_t kdim;              /* K = sum_a L_a */
     int32_t slices_used;       /* split precision: slices actually used */
@@ -209,18 +212,17 @@ hsgen_status hsgen_contract_hs(hsgen_ctx* ctx, int32_t L, int32_t a, int32_t G,
                                const hsgen_opts* opts, double* H, double* S,
                                int64_t ld, hsgen_report* report);
 
-/* Bytes of device scratch the allocation-free entry point below has per GPU. */
+/* Bytes of operands the allocation-free entry point below serves. */
 #define HSGEN_NOALLOC_SCRATCH_BYTES ((uint64_t)256 << 20)
 
 /* hsgen_create_hs in FP64 with no device allocation.  No counterpart in the
  * reference: for callers that cannot allocate device memory (code under HIP
  * graph capture, tight serving loops, harnesses that forbid hipMalloc).  The
- * call's workspaces (a host G list's device copy, the grouped-GEMM work
- * lists, the operands: 2 x 16 B x (2K + 32) x roundup(ng, 128) for the
- * default tile, 3 x for a system with a zero ||u_dot||^2) live in one device
- * array of HSGEN_NOALLOC_SCRATCH_BYTES
- * per GPU, held by the library until the process ends; a problem that needs
- * more is HSGEN_ERR_ARG.  H and S must be device memory (HSGEN_ERR_ARG
+ * call's workspaces live in one device array per GPU (513 MiB), held by the
+ * library until the process ends.  A problem whose general operands (a host G
+ * list's device copy, the grouped-GEMM work lists and 2 x 16 B x (2K + 32) x
+ * roundup(ng, 128) for the default tile, 3 x for a system with a zero
+ * ||u_dot||^2) pass HSGEN_NOALLOC_SCRATCH_BYTES is HSGEN_ERR_ARG.  H and S must be device memory (HSGEN_ERR_ARG
  * otherwise); kp->g may be host or device memory.  opts->precision must be
  * HSGEN_PREC_FP64 (HSGEN_ERR_UNSUPPORTED otherwise); flags and tile as for
  * hsgen_create_hs, with the tile's T-block padding already in place (the

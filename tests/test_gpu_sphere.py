@@ -1,0 +1,116 @@
+"""FP64 H and S from a system: coefficients as a phase times real vectors that
+atoms of one kind share, S by the addition theorem.  Against the oracle at the
+edges of its tiles (16, 32, 64 plane waves), of its k-step and stage depths
+(2 (lmax+1)^2 against multiples of 4 and 16) and of its atom chunks, and tile
+against tile: an element depends on its two plane waves alone, so every size
+gives the same bits.
+
+Tolerance as in test_gpu_parity.py: relative Frobenius error of the lower
+triangle <= 1e-13."""
+import numpy as np
+import pytest
+
+from hybridhsdla_amd import make_config, tiny_system
+from hybridhsdla_amd.system import KPoint
+from oracle import pyoracle as po
+from tests.helpers import rel_fro_lower
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-13
+
+
+def _subset(kp, idx):
+    return KPoint(k=kp.k, g=np.ascontiguousarray(kp.g[np.asarray(idx, dtype=np.int64)]), kmax=kp.kmax)
+
+
+def _check(ctx, s, kp):
+    h = ctx.upload(s)
+    H, S = ctx.create_HS2(h, kp)
+    Hr, Sr = po.reference_hs(s, kp)
+    # scaled by the largest element: the squares of the norm test's 1e200 overflow
+    eh, es = (rel_fro_lower(X / np.abs(R).max(), R / np.abs(R).max()) for X, R in ((H, Hr), (S, Sr)))
+    print(f"ng {kp.ng} lmax {list(s.lmax)[:6]}: H {eh:.2e} S {es:.2e}", flush=True)
+    assert eh <= TOL and es <= TOL
+    h.close()
+    return H, S
+
+
+@pytest.mark.parametrize("lmax", [(1,), (0, 1), (2, 1, 0), (3,), (5, 4), (8, 7)])
+@pytest.mark.parametrize("natoms", [1, 9, 17])
+def test_depths_and_atom_counts(ctx, lmax, natoms):
+    """Depths of one k-step (lmax 0) to many stages, one atom, and more atoms
+    of a kind than a chunk of phases holds."""
+    if max(lmax) < 1 or (natoms < len(lmax) and max(lmax[:natoms]) < 1):
+        pytest.skip("max_lmax 0 is refused")
+    s, kp = tiny_system(natoms=natoms, lmax=lmax, a_cell=9.0, ng_target=90, seed=31)
+    if s.lmax.max() < 1:
+        pytest.skip("max_lmax 0 is refused")
+    _check(ctx, s, kp)
+
+
+def test_every_size_gives_the_same_bits(ctx):
+    """Tiles of 16, 32 and 64 and the patch orders: principal submatrices of a
+    1500-plane-wave call equal calls on subsets bit for bit."""
+    s, kps = make_config(1, ng=1500, natoms=6)
+    kp = kps[0]
+    h = ctx.upload(s)
+    H, S = ctx.create_HS2(h, kp)
+    rng = np.random.default_rng(3)
+    for n in (1, 15, 17, 31, 33, 63, 65, 480, 1023, 1409):
+        idx = np.sort(rng.permutation(kp.ng)[:n])
+        Hs, Ss = ctx.create_HS2(h, _subset(kp, idx))
+        assert np.array_equal(Hs, H[np.ix_(idx, idx)]) and np.array_equal(Ss, S[np.ix_(idx, idx)]), n
+    idx = np.sort(rng.permutation(kp.ng)[:70])
+    Hr, Sr = po.reference_hs(s, _subset(kp, idx))
+    assert rel_fro_lower(H[np.ix_(idx, idx)], Hr) <= TOL and rel_fro_lower(S[np.ix_(idx, idx)], Sr) <= TOL
+    h.close()
+
+
+def test_larger_triangle_with_patches(ctx):
+    """Tiles of 64 in patches of 4 x 4 (25 tile rows and more)."""
+    s, kp = tiny_system(natoms=2, lmax=(3, 2), a_cell=14.0, ng_target=1700, seed=8)
+    _check(ctx, s, kp)
+
+
+def test_opposite_and_equal_directions(ctx):
+    """G and -G at the Gamma point: parallel, antiparallel and zero vectors."""
+    s, kp = tiny_system(natoms=3, lmax=(6, 5), kpt=(0.0, 0.0, 0.0), ng_target=120, seed=12)
+    assert np.any(np.all(kp.g == 0, axis=1))
+    _check(ctx, s, kp)
+
+
+@pytest.mark.parametrize("norm", [0.0, 1e-200, 1e200])
+def test_norms_outside_folding(ctx, norm):
+    """Norms that cannot be folded into the general operands need no other
+    form here (the overlap weights carry them)."""
+    s, kp = tiny_system(natoms=3, lmax=(3, 2, 4), ng_target=100, seed=9)
+    s.match[1, 1, 4] = norm
+    _check(ctx, s, kp)
+
+
+def test_one_of_the_two_matrices(ctx):
+    from hybridhsdla_amd.api import HSGEN_SKIP_H, HSGEN_SKIP_S
+    s, kp = tiny_system(natoms=3, lmax=(3, 2, 4), ng_target=150, seed=5)
+    h = ctx.upload(s)
+    H, S = ctx.create_HS2(h, kp)
+    H1, S1 = ctx.create_HS2(h, kp, flags=HSGEN_SKIP_S)
+    H2, S2 = ctx.create_HS2(h, kp, flags=HSGEN_SKIP_H)
+    assert np.array_equal(H, H1) and not S1.any() and np.array_equal(S, S2) and not H2.any()
+    h.close()
+
+
+@pytest.mark.parametrize("ng", [65, 129, 300])
+def test_general_contraction_tiles_give_the_same_bits(ctx, ng):
+    """The contraction of given coefficients keeps its tile configurations:
+    every one gives the bits of the default."""
+    s, kp = tiny_system(natoms=3, lmax=(3, 5, 2), ng_target=300, seed=6)
+    sub = _subset(kp, np.arange(min(ng, kp.ng)))
+    A, B = po.construct_ab(s, sub)
+    args = (s.L, s.natoms, sub.ng, A, B, s.taa, s.tab, s.tbb, s.lmax, s.max_lmax, s.sqrt_u_norms())
+    H0, S0 = ctx.create_HS2_stripped_v2(*args)
+    Hr, Sr = po.reference_hs(s, sub)
+    assert rel_fro_lower(H0, Hr) <= TOL and rel_fro_lower(S0, Sr) <= TOL
+    for tile in range(1, 15):
+        H, S = ctx.create_HS2_stripped_v2(*args, tile=tile)
+        assert np.array_equal(H, H0) and np.array_equal(S, S0), tile
