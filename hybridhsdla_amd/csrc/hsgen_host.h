@@ -148,9 +148,9 @@ struct hsgen_sys {
     double2* d_mt = nullptr;
     hsgen::KindDev* d_kinds = nullptr;
     int32_t* d_order = nullptr;
-    int32_t* d_ksteps = nullptr;
+    hsgen::SphereStage* d_stages = nullptr;
     int64_t* d_mtoff = nullptr;
-    int nkinds = 0, nksteps = 0, ldr = 0, rt64 = 0, rt32 = 0;
+    int nkinds = 0, nksteps = 0, ldr = 0, rt32 = 0;
     int64_t ldy = 0, ldw = 0;
     // first atom of each rotation class and of each rmt class (AtomDev::cls)
     std::vector<int32_t> rot_rep, rmt_rep;
@@ -235,8 +235,8 @@ hsgen_status create_hs_general(hsgen_ctx* ctx, hsgen_sys* s, const hsgen_kpoint*
 // ---- sphere_path.hip ----
 struct SphereLayout {
     int64_t gtot = 0;                       // operand columns, 64 per tile column of every k-point
-    int64_t ngcols = 0, npatch = 0, nstiles = 0;
-    int htile = 64, ttile = 64, stile = 64, pside = 1;
+    int64_t ngcols = 0, nsquares = 0, nstiles = 0;
+    int htile = 64, ttile = 64, stile = 64;
     size_t b_ph = 0, b_rs = 0, b_y = 0, b_w = 0;   // bytes of the operand arrays
 };
 hsgen_status sphere_setup(hsgen_ctx* ctx, hsgen_sys* s, const RadDev* rad);

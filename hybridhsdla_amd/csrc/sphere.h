@@ -19,6 +19,11 @@
 
 namespace hsgen {
 
+// Column padding of the operand arrays, and the squares of H tiles along a
+// patch that one XCD runs at a time (32 CUs, two 64 x 64 tiles each).
+constexpr int kSphereCols = 64;
+constexpr int kSpherePatch = 8;
+
 // Atoms of one kind share the real vector y and the radial factors.
 struct KindDev {
     int32_t lmax, nlm;
@@ -28,7 +33,7 @@ struct KindDev {
     int32_t rsoff;       // first row of the radial factors
     int32_t woff;        // first row of W
     int32_t ldm;         // leading dimension of Mt: 2 nlm rounded up to the stage depth of 16
-    int32_t rt64, rt32;  // T-application row tiles of the kinds before this one, for tiles of 64 and 32
+    int32_t rt32;        // T-application row tiles of 32 of the kinds before this one
     int32_t first, count;   // its atoms, in kind order
     double rmt;
     double rot[9];       // column-major R_atom * bmat
@@ -45,7 +50,7 @@ struct SphereK {
     int32_t ng;
     int32_t gcol0;       // plane waves of the k-points before this one
     int32_t stile0;      // S tiles before this one
-    int32_t hpatch0;     // H patches before this one
+    int32_t hsquare0;    // lower squares of H tiles before this one
 };
 
 // One T block to turn into real harmonics (device pointers).
@@ -56,6 +61,14 @@ struct MtJob {
     int64_t off;         // of its Mt (complex units)
     int32_t nlm, rows, ldm;
     int32_t pad;
+};
+
+// One stage of 16 rows of H's depth, four k-steps of 4.
+struct SphereStage {
+    int32_t step[4];     // row of y of the k-step (a multiple of 4); bit 0: an atom ends with it; bit 1: and
+                         // another one ended earlier in the stage
+    int32_t atom;        // first atom (kind order) that ends in the stage, or -1
+    int32_t pad[3];
 };
 
 // Everything the kernels read; one k-point travels in `one`, more in `many`.
@@ -73,7 +86,7 @@ struct SphereArgs {
     SphereK one;
     const SphereK* many;
     int64_t gtot;              // columns of the operand arrays
-    double2* ph;               // [natoms + 1][gtot] phases, kind order (the last row is not used)
+    double2* ph;               // [natoms][gtot] phases, kind order
     double2* rs;               // [gtot][ldr] radial factors (a_l, b_l)
     int32_t ldr;
     double* y;                 // [gtot][ldy] real vectors of all kinds, or null (S alone)
@@ -81,9 +94,9 @@ struct SphereArgs {
     int64_t ldy, ldw;
     const double2* mt;
     const int64_t* mtoff;      // [natoms] Mt of each atom, kind order
-    const int32_t* ksteps;     // per k-step of H: row of y (a multiple of 4), bit 0 set in an atom's last
+    const SphereStage* stages;
     int32_t nksteps;
-    int32_t pside, npatch;     // H patches
+    int32_t nsquares;          // lower squares of H tiles of all k-points
 };
 
 int sphere_chunk(int nl, int L);

@@ -1,6 +1,8 @@
 // FP64 kernels of the path from a system description to H and S that use the
 // form of the matching coefficients: a phase per atom times real numbers that
 // atoms of one kind share (sphere.h).
+#include <type_traits>
+
 #include "sphere.h"
 #include "sphere_dev.h"
 
@@ -401,10 +403,10 @@ __global__ __launch_bounds__(256 * M / MJ) void k_overlap(SphereArgs p)
 
 int overlap_tile(int64_t tiles64, int n_cu)
 {
-    // 64 x 64 tiles once they give every CU two workgroups, 32 x 32 once
-    // those do, else 16 x 16: a smaller tile reads its columns more often but
+    // 64 x 64 tiles once they give every CU four workgroups, 32 x 32 once
+    // those give two, else 16 x 16: a smaller tile reads its columns more often but
     // spreads a small triangle over more CUs
-    if (tiles64 >= 2 * (int64_t)n_cu) return 64;
+    if (tiles64 >= 4 * (int64_t)n_cu) return 64;
     return 4 * tiles64 >= 2 * (int64_t)n_cu ? 32 : 16;
 }
 
@@ -541,45 +543,68 @@ hipError_t launch_build_mt(const MtJob* jobs, int njobs, int64_t max_elems, doub
 // X's columns are 16 chunks of 16 bytes, chunk q stored at q ^ (column % 16),
 // y's 8 chunks, chunk q at q ^ (column / 2 % 8): 16 lanes that read one row
 // hit distinct banks.  The fragments of the next k-step are read before the
-// MFMAs of the current one, across the stage barrier too.
+// MFMAs of the current one, across the stage barrier too; a stage also brings
+// the phases of an atom that ends in it, so that no flush waits for memory;
+// LDS addresses are constants per lane and load bases scalar, which leaves the
+// vector pipe to the MFMAs.  Rings of 3 and 4 stages, 64 x 128 tiles and waves
+// of 32 x 32 measured no faster at any size from 235 to 25000 plane waves.
+// Rate of the H tiles: 0.87 of the FP64 peak at N_G 16000 and 25000, 0.85 at
+// 10000, 0.82 at 6002 (32 atoms, lmax 10).
 // Measured (whole call, complex-by-complex contraction of S and H before, now):
-// 713 -> 244 ms at N_G 12007 (128 atoms, lmax 12), 33.4 -> 12.3 ms at 6002 and
-// 5.42 -> 2.35 ms at 2003 (32 atoms, lmax 10).
+// 714 -> 208 ms at N_G 12007 (128 atoms, lmax 12), 33.5 -> 10.2 ms at 6002 and
+// 5.47 -> 1.46 ms at 2003 (32 atoms, lmax 10).
 // ---------------------------------------------------------------------------
 namespace {
 
 typedef double d4 __attribute__((ext_vector_type(4)));
 typedef double v2d __attribute__((ext_vector_type(2)));
-typedef int i4 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(4))) const i4* ctab;
+typedef int i8 __attribute__((ext_vector_type(8)));
+typedef __attribute__((address_space(4))) const i8* ctab;
 
 // s_waitcnt immediates (vmcnt bits [3:0] and [15:14], expcnt [6:4], lgkmcnt [11:8])
 constexpr int kWaitVm0 = (0 & 15) | (7 << 4) | (15 << 8);
 constexpr int kWaitVm0Lgkm0 = (0 & 15) | (7 << 4) | (0 << 8);
 
+// Atoms that end in a stage before its k-step ks.
+__device__ __forceinline__ int ends_before(i8 e, int ks)
+{
+    return (ks > 0 ? e[0] & 1 : 0) + (ks > 1 ? e[1] & 1 : 0) + (ks > 2 ? e[2] & 1 : 0);
+}
+
 }  // namespace
 
-template <int B>
+// BR x BC tile (rows: X columns, columns: y columns), waves of 16 RB x 16 CB.
+template <int BR, int BC, int RB, int CB>
 struct SphereTile {
-    static constexpr int kRB = 1;                 // 16-row blocks per wave
-    static constexpr int kCB = B == 64 ? 2 : 1;   // 16-column blocks per wave
-    static constexpr int kWR = B / (16 * kRB);    // waves along the rows
-    static constexpr int kWC = B / (16 * kCB);
+    static constexpr int kWR = BR / (16 * RB);    // waves along the rows
+    static constexpr int kWC = BC / (16 * CB);
     static constexpr int kWaves = kWR * kWC;
     static constexpr int kThreads = 64 * kWaves;
-    static constexpr int kXBytes = B * 256;       // one stage of X, of y
-    static constexpr int kYBytes = B * 128;
-    static constexpr int kStage = kXBytes + kYBytes;
-    static constexpr int kLoads = kStage / 1024 / kWaves;   // 1 KiB wave loads per wave and stage
-    static_assert(kStage / 1024 % kWaves == 0, "a stage splits evenly over the waves");
+    static constexpr int kXBytes = BR * 256;      // one stage of X, of y
+    static constexpr int kYBytes = BC * 128;
+    static constexpr int kPhBytes = 256 * CB;     // a wave's phases of an atom that ends in a stage
+    static constexpr int kStage = kXBytes + kYBytes + kWaves * kPhBytes;
+    static constexpr int kLds = 2 * kStage;
+    static constexpr int kXLoads = kXBytes / 1024 / kWaves;   // 1 KiB wave loads per wave and stage
+    static constexpr int kYLoads = kYBytes / 1024 / kWaves;
+    static_assert(kXLoads * kWaves * 1024 == kXBytes && kYLoads * kWaves * 1024 == kYBytes,
+                  "a stage splits evenly over the waves");
+    static_assert(BC % BR == 0, "patches are square in plane waves");
 };
 
-template <int B, bool kH>
-__global__ __launch_bounds__(SphereTile<B>::kThreads, B == 64 ? 4 : 2) void k_sphere_gemm(SphereArgs p)
+// Wave-uniform values the compiler is to keep in scalar registers.
+__device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ int64_t uni(int64_t v)
+{
+    return (int64_t)(((uint64_t)(uint32_t)uni((int)(v >> 32)) << 32) | (uint32_t)uni((int)v));
+}
+
+template <int BR, int BC, int RB, int CB, bool kH>
+__global__ __launch_bounds__((SphereTile<BR, BC, RB, CB>::kThreads), 4) void k_sphere_gemm(SphereArgs p)
 {
 #pragma clang fp contract(off)
-    using Tl = SphereTile<B>;
-    constexpr int RB = Tl::kRB, CB = Tl::kCB, LPW = Tl::kLoads;
+    using Tl = SphereTile<BR, BC, RB, CB>;
+    constexpr int NX = Tl::kXLoads, NY = Tl::kYLoads;
     extern __shared__ __attribute__((aligned(1024))) char lds[];
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -592,94 +617,132 @@ __global__ __launch_bounds__(SphereTile<B>::kThreads, B == 64 ? 4 : 2) void k_sp
     int R0, C0;             // first row (X column), first column (y column) of the tile
     int nsteps;             // k-steps of 4
     if constexpr (kH) {
-        // Workgroups go to the 8 XCDs in turn: XCD x takes the patches x,
-        // x + 8, ... of pside x pside tiles, so that the tiles in flight on
-        // one L2 share their panels.
-        const int pp = p.pside * p.pside;
-        const int slot = (int)blockIdx.x / 8;
-        const int patch = slot / pp * 8 + (int)blockIdx.x % 8;
-        if (patch >= p.npatch) return;
-        const int in = slot % pp;
-        if (p.nk > 1) kp = p.many + find_last(p.nk, patch, [&](int i) { return p.many[i].hpatch0; });
-        const int lp = patch - kp->hpatch0;
-        const int pi = tri_row(lp);
-        const int pj = lp - (int)((int64_t)pi * (pi + 1) / 2);
-        const int bi = pi * p.pside + in % p.pside, bj = pj * p.pside + in / p.pside;
-        if (bj > bi || bi * B >= kp->ng) return;
-        R0 = bj * B;
-        C0 = bi * B;
+        // Workgroups go to the 8 XCDs in turn.  The lower squares of BC of all
+        // k-points, in patches of P x P squares, are cut into 8 equal
+        // parts, one per XCD: the tiles in flight on one L2 share their
+        // panels, and every XCD has the same work.
+        constexpr int kRat = BC / BR;
+        constexpr int P = kSpherePatch;
+        const int n = p.nsquares * kRat;
+        const int x = (int)blockIdx.x % 8, at = (int)blockIdx.x / 8;
+        const int t0 = (int)((int64_t)n * x / 8), t1 = (int)((int64_t)n * (x + 1) / 8);
+        if (at >= t1 - t0) return;
+        const int sq = (t0 + at) / kRat;
+        if (p.nk > 1) kp = p.many + find_last(p.nk, sq, [&](int i) { return p.many[i].hsquare0; });
+        const int t = sq - kp->hsquare0;
+        const int nt = (kp->ng + BC - 1) / BC;
+        const int pi = tri_row(t) / P;                        // patch row
+        int u = t - (int)((int64_t)(pi * P) * (pi * P + 1) / 2);
+        const int h = min(P, nt - pi * P);                    // its rows
+        int bi, bj;
+        if (u < pi * P * h) {
+            const int pj = u / (P * h);
+            u -= pj * P * h;
+            bi = u % h;
+            bj = pj * P + u / h;
+        } else {
+            u -= pi * P * h;
+            bi = tri_row(u);
+            bj = pi * P + u - bi * (bi + 1) / 2;
+        }
+        C0 = uni((pi * P + bi) * BC);
+        R0 = uni(bj * BC + (t0 + at) % kRat * BR);
+        if (R0 >= kp->ng) return;
         nsteps = p.nksteps;
     } else {
         // kinds in turn; per kind its tiles of rows, per row tile all columns
-        const int ntc = (int)((p.gtot + B - 1) / B);
+        const int ntc = (int)(p.gtot / BC);
         const int tr = (int)blockIdx.x / ntc;
-        const int kk = find_last(p.nkinds, tr, [&](int i) { return B == 64 ? p.kinds[i].rt64 : p.kinds[i].rt32; });
+        const int kk = find_last(p.nkinds, tr, [&](int i) { return p.kinds[i].rt32; });
         kd = p.kinds + kk;
-        R0 = (tr - (B == 64 ? kd->rt64 : kd->rt32)) * B;
-        C0 = ((int)blockIdx.x - tr * ntc) * B;
-        nsteps = kd->r4 / 4;
+        R0 = uni((tr - kd->rt32) * BR);
+        C0 = uni(((int)blockIdx.x - tr * ntc) * BC);
+        nsteps = uni(kd->r4 / 4);
     }
-    const int nst = (nsteps + 3) / 4;
+    const int64_t col0 = kH ? uni(kp->col0) : 0;
+    const int nst = uni((nsteps + 3) / 4);
 
-    // ---- this lane's loads: X columns of 16 chunks, then y columns of 8 ----
-    const char* src[LPW];
-    bool isy[LPW];
-    int sel[LPW];
+    // ---- loads ----
+    // A wave load of X fills 4 columns of 16 chunks, one of y 8 columns of 8.
+    // Bases are wave-uniform, lanes add 32-bit offsets; only Mt, whose rows
+    // change blocks between atoms, takes a pointer per lane.
+    const char* xbase[NX];
+    uint32_t xoff[NX];
+    const char* xptr[NX];
 #pragma unroll
-    for (int r = 0; r < LPW; ++r) {
-        const int g = wave * LPW + r;
-        const int slot = g * 64 + lane;
-        isy[r] = g >= Tl::kXBytes / 1024;
-        if (!isy[r]) {
-            const int c = slot / 16;
-            const int q = (slot % 16) ^ (c & 15);
-            const double2* x;
-            if constexpr (kH) {
-                x = p.W + (kp->col0 + R0 + c) * p.ldw;
-            } else {
-                // row R0 + c of the kind's stacked Mt; past its last row the last one again
-                const int row = min(R0 + c, kd->count * kd->r4 - 1);
-                const int a = row / kd->r4;
-                x = p.mt + p.mtoff[kd->first + a] + (int64_t)(row - a * kd->r4) * kd->ldm;
-            }
-            src[r] = (const char*)(x + q);
-            sel[r] = 0;
+    for (int r = 0; r < NX; ++r) {
+        const int c0 = (wave * NX + r) * 4;
+        const int c = c0 + (lane >> 4);
+        const int q = (lane & 15) ^ (c & 15);
+        if constexpr (kH) {
+            xbase[r] = (const char*)(p.W + (col0 + R0 + c0) * p.ldw);
+            xoff[r] = (uint32_t)(((int64_t)(lane >> 4) * p.ldw + q) * 16);
         } else {
-            const int s2 = slot - B * 16;
-            const int c = s2 / 8;
-            const int q = (s2 % 8) ^ ((c >> 1) & 7);
-            const int64_t col = (kH ? kp->col0 : 0) + C0 + c;
-            const double* y = p.y + col * p.ldy + 2 * (q & 1);
-            if constexpr (!kH) y += kd->yoff;
-            src[r] = (const char*)y;
-            sel[r] = q >> 1;
+            // row R0 + c of the kind's stacked Mt; past its last row the last one again
+            const int row = min(R0 + c, kd->count * kd->r4 - 1);
+            const int a = row / kd->r4;
+            xptr[r] = (const char*)(p.mt + p.mtoff[kd->first + a] + (int64_t)(row - a * kd->r4) * kd->ldm + q);
         }
     }
+    const char* ybase[NY];
+    uint32_t yoff[NY];
+    int sel[NY];            // the lane's k-step within a stage
+#pragma unroll
+    for (int r = 0; r < NY; ++r) {
+        const int c0 = (wave * NY + r) * 8;
+        const int c = c0 + (lane >> 3);
+        const int q = (lane & 7) ^ ((c >> 1) & 7);
+        ybase[r] = (const char*)(p.y + (col0 + C0 + c0) * p.ldy);
+        yoff[r] = (uint32_t)(((int64_t)(lane >> 3) * p.ldy + 2 * (q & 1)) * 8);
+        if constexpr (!kH) yoff[r] += (uint32_t)(kd->yoff + 4 * (q >> 1)) * 8;
+        sel[r] = q >> 1;
+    }
+    // constant address space: the table's entries come by scalar loads
+    const ctab tab = (ctab)(const void*)p.stages;
+    // stage s (for T: nothing)
+    auto entry = [&](int s) -> i8 {
+        if constexpr (kH) return tab[uni(s)];
+        else return i8{0, 0, 0, 0, -1, 0, 0, 0};
+    };
+    typedef __attribute__((address_space(1))) const char gchar;
     typedef __attribute__((address_space(3))) char lchar;
     lchar* lbase = (lchar*)lds;
-    // constant address space: the table's entries come by scalar loads
-    const ctab tab = (ctab)(const void*)p.ksteps;
-    // the k-step entries of stage s (for T: none)
-    auto entries = [&](int s) -> i4 {
-        if constexpr (kH) return tab[__builtin_amdgcn_readfirstlane(s)];
-        else return i4{0, 0, 0, 0};
-    };
-    auto issue = [&](int s, int buf, i4 e) {
-#pragma unroll
-        for (int r = 0; r < LPW; ++r) {
-            const char* gb;
-            if (!isy[r]) {
-                gb = src[r] + (int64_t)s * 256;
-            } else if constexpr (kH) {
-                const int lo = sel[r] & 1 ? e.y : e.x, hi = sel[r] & 1 ? e.w : e.z;
-                const int row = sel[r] & 2 ? hi : lo;
-                gb = src[r] + (int64_t)(row & ~3) * 8;
-            } else {
-                gb = src[r] + (int64_t)(16 * s + 4 * sel[r]) * 8;
+    // one stage: the phases of the first atom that ends in it, X, y
+    auto issue = [&](int s, int buf, i8 e) {
+        if constexpr (kH) {
+            if (e[4] >= 0 && lane < 16 * CB) {
+                gchar* g = (gchar*)(p.ph + (int64_t)e[4] * p.gtot + (col0 + C0 + wc * 16 * CB)) + lane * 16;
+                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)g,
+                                                 (__attribute__((address_space(3))) void*)(lbase + buf * Tl::kStage +
+                                                                                           Tl::kXBytes + Tl::kYBytes +
+                                                                                           wave * Tl::kPhBytes),
+                                                 16, 0, 0);
             }
-            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)gb,
+        }
+#pragma unroll
+        for (int r = 0; r < NX; ++r) {
+            gchar* g;
+            if constexpr (kH) g = (gchar*)(xbase[r] + (int64_t)uni(s) * 256) + xoff[r];
+            else g = (gchar*)(xptr[r] + (int64_t)s * 256);
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)g,
                                              (__attribute__((address_space(3))) void*)(lbase + buf * Tl::kStage +
-                                                                                       (wave * LPW + r) * 1024),
+                                                                                       (wave * NX + r) * 1024),
+                                             16, 0, 0);
+        }
+#pragma unroll
+        for (int r = 0; r < NY; ++r) {
+            gchar* g;
+            if constexpr (kH) {
+                const int lo = sel[r] & 1 ? e[1] : e[0], hi = sel[r] & 1 ? e[3] : e[2];
+                const uint32_t row = (uint32_t)(sel[r] & 2 ? hi : lo) & ~3u;
+                g = (gchar*)ybase[r] + (yoff[r] + row * 8);
+            } else {
+                g = (gchar*)(ybase[r] + (int64_t)s * 128) + yoff[r];
+            }
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)g,
+                                             (__attribute__((address_space(3))) void*)(lbase + buf * Tl::kStage +
+                                                                                       Tl::kXBytes +
+                                                                                       (wave * NY + r) * 1024),
                                              16, 0, 0);
         }
     };
@@ -694,30 +757,36 @@ __global__ __launch_bounds__(SphereTile<B>::kThreads, B == 64 ? 4 : 2) void k_sp
             if constexpr (kH) cr[i][j] = ci[i][j] = d4{0.0, 0.0, 0.0, 0.0};
         }
 
-    int rowX[RB], colY[CB];
-#pragma unroll
-    for (int i = 0; i < RB; ++i) rowX[i] = wr * 16 * RB + i * 16 + (lane & 15);
-#pragma unroll
-    for (int j = 0; j < CB; ++j) colY[j] = wc * 16 * CB + j * 16 + (lane & 15);
+    // LDS offsets of the lane's fragments per k-step; further blocks of 16
+    // and the second stage are constant distances away
+    const int r0 = wr * 16 * RB + (lane & 15), c0 = wc * 16 * CB + (lane & 15);
     const int q0 = lane >> 4;
-    auto read_frags = [&](int buf, int ks, v2d* x, double* y) {
-        const char* lb = lds + buf * Tl::kStage;
+    int xat[4], yat[4];
 #pragma unroll
-        for (int i = 0; i < RB; ++i) x[i] = *(const v2d*)&lb[rowX[i] * 256 + 16 * ((q0 + 4 * ks) ^ (rowX[i] & 15))];
+    for (int ks = 0; ks < 4; ++ks) {
+        xat[ks] = r0 * 256 + 16 * ((q0 + 4 * ks) ^ (r0 & 15));
+        yat[ks] = Tl::kXBytes + c0 * 128 + 16 * (((q0 >> 1) + 2 * ks) ^ ((c0 >> 1) & 7)) + 8 * (q0 & 1);
+    }
+    auto read_frags = [&](int buf, int ks, v2d* x, double* y) {
+#pragma unroll
+        for (int i = 0; i < RB; ++i) x[i] = *(const v2d*)&lds[xat[ks] + (buf * Tl::kStage + i * 4096)];
+#pragma unroll
+        for (int j = 0; j < CB; ++j) y[j] = *(const double*)&lds[yat[ks] + (buf * Tl::kStage + j * 2048)];
+    };
+    // Phases at this lane's H rows: of the first atom that ends in a stage,
+    // from the stage; of further ones (atoms of few rows) from memory.
+    auto stage_phases = [&](int buf, double2* ph) {
 #pragma unroll
         for (int j = 0; j < CB; ++j)
-            y[j] = *(const double*)&lb[Tl::kXBytes + colY[j] * 128 +
-                                       16 * (((q0 >> 1) + 2 * ks) ^ ((colY[j] >> 1) & 7)) + 8 * (q0 & 1)];
+            ph[j] = *(const double2*)&lds[buf * Tl::kStage + Tl::kXBytes + Tl::kYBytes + wave * Tl::kPhBytes +
+                                          (lane & 15) * 16 + j * 256];
     };
-    // phases of the current atom at this lane's H rows
-    double2 ph[CB];
-    const double2* phsrc = nullptr;
-    if constexpr (kH) {
-        phsrc = p.ph + kp->col0 + C0;
+    auto far_phases = [&](int atom, double2* ph) {
 #pragma unroll
-        for (int j = 0; j < CB; ++j) ph[j] = phsrc[colY[j]];
-    }
-    auto flush = [&]() {
+        for (int j = 0; j < CB; ++j) ph[j] = p.ph[(int64_t)atom * p.gtot + (col0 + C0 + c0 + 16 * j)];
+    };
+    // C += conj(phase) T, T = 0
+    auto flush = [&](const double2* ph) {
 #pragma unroll
         for (int i = 0; i < RB; ++i)
 #pragma unroll
@@ -730,23 +799,24 @@ __global__ __launch_bounds__(SphereTile<B>::kThreads, B == 64 ? 4 : 2) void k_sp
                     tr_[i][j][q] = 0.0;
                     ti_[i][j][q] = 0.0;
                 }
-        // the next atom's (after the last: a spare row, unused)
-        phsrc += p.gtot;
-#pragma unroll
-        for (int j = 0; j < CB; ++j) ph[j] = phsrc[colY[j]];
     };
 
     // ---- main loop ----
-    i4 e0 = entries(0), e1 = entries(min(1, nst - 1));
-    issue(0, 0, e0);
+    // (at the end the last stage is loaded again: in bounds, unused)
+    const int last = nst - 1;
+    i8 en[2] = {entry(0), entry(min(1, last))};     // stage s's entries in en[s % 2]
+    issue(0, 0, en[0]);
     __builtin_amdgcn_s_waitcnt(kWaitVm0);
     asm volatile("s_barrier" ::: "memory");
-    issue(min(1, nst - 1), 1, e1);
+    issue(min(1, last), 1, en[1]);
     v2d fx[RB];
     double fy[CB];
     read_frags(0, 0, fx, fy);
-    for (int s = 0; s < nst; ++s) {
-        const i4 e2 = entries(min(s + 2, nst - 1));
+    // stage s from LDS buffer `buf`
+    auto stage = [&](auto bufc, int s) {
+        constexpr int buf = decltype(bufc)::value;
+        const i8 e = en[buf];
+        const i8 e2 = entry(min(s + 2, last));
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) {
             v2d x[RB];
@@ -755,38 +825,51 @@ __global__ __launch_bounds__(SphereTile<B>::kThreads, B == 64 ? 4 : 2) void k_sp
             for (int i = 0; i < RB; ++i) x[i] = fx[i];
 #pragma unroll
             for (int j = 0; j < CB; ++j) y[j] = fy[j];
+            double2 ph[CB];
             if (ks < 3) {
-                read_frags(s & 1, ks + 1, fx, fy);
-            } else if (s + 1 < nst) {
+                read_frags(buf, ks + 1, fx, fy);
+            } else if (s < last) {
+                // an atom that ends with the stage still needs its phases
+                if (kH && (e[3] & 3) == 1) stage_phases(buf, ph);
                 // this wave's loads of stage s+1 landed and its reads of stage
                 // s are done; after the barrier that holds for every wave, and
-                // stage s+2 (at the end the last again: in bounds, unused) may
-                // overwrite stage s
+                // stage s+2 may overwrite stage s
                 __builtin_amdgcn_s_waitcnt(kWaitVm0Lgkm0);
                 asm volatile("s_barrier" ::: "memory");
-                issue(min(s + 2, nst - 1), s & 1, e2);
-                read_frags((s + 1) & 1, 0, fx, fy);
+                issue(min(s + 2, last), buf, e2);
+                read_frags(buf ^ 1, 0, fx, fy);
             }
+            // reads ahead of the MFMAs, as written
+            __builtin_amdgcn_sched_barrier(0);
             // rows past the depth (in the last stage) are not multiplied
-            if (!kH && 4 * s + ks >= nsteps) break;
+            if (kH || 4 * s + ks < nsteps) {
 #pragma unroll
-            for (int i = 0; i < RB; ++i)
+                for (int i = 0; i < RB; ++i)
 #pragma unroll
-                for (int j = 0; j < CB; ++j)
-                    tr_[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[i].x, y[j], tr_[i][j], 0, 0, 0);
+                    for (int j = 0; j < CB; ++j)
+                        tr_[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[i].x, y[j], tr_[i][j], 0, 0, 0);
 #pragma unroll
-            for (int i = 0; i < RB; ++i)
+                for (int i = 0; i < RB; ++i)
 #pragma unroll
-                for (int j = 0; j < CB; ++j)
-                    ti_[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[i].y, y[j], ti_[i][j], 0, 0, 0);
+                    for (int j = 0; j < CB; ++j)
+                        ti_[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[i].y, y[j], ti_[i][j], 0, 0, 0);
+            }
             if constexpr (kH) {
-                const int f = ks == 0 ? e0.x : ks == 1 ? e0.y : ks == 2 ? e0.z : e0.w;
-                if (f & 1) flush();
+                if (e[ks] & 1) {
+                    if (e[ks] & 2) far_phases(e[4] + ends_before(e, ks), ph);
+                    else if (ks < 3 || s == last) stage_phases(buf, ph);
+                    flush(ph);
+                }
             }
         }
-        e0 = e1;
-        e1 = e2;
+        en[buf] = e2;
+    };
+    int s = 0;
+    for (; s < last; s += 2) {
+        stage(std::integral_constant<int, 0>{}, s);
+        stage(std::integral_constant<int, 1>{}, s + 1);
     }
+    if (s < nst) stage(std::integral_constant<int, 0>{}, s);
     __builtin_amdgcn_s_waitcnt(0);
 
     // ---- store: lane holds rows (lane >> 4) + 4 q of column lane & 15 ----
@@ -796,7 +879,7 @@ __global__ __launch_bounds__(SphereTile<B>::kThreads, B == 64 ? 4 : 2) void k_sp
         for (int i = 0; i < RB; ++i)
 #pragma unroll
             for (int j = 0; j < CB; ++j) {
-                const int gi = C0 + colY[j];
+                const int gi = C0 + c0 + 16 * j;
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
                     const int gj = R0 + wr * 16 * RB + i * 16 + q0 + 4 * q;
@@ -815,38 +898,47 @@ __global__ __launch_bounds__(SphereTile<B>::kThreads, B == 64 ? 4 : 2) void k_sp
                     const double2* phr = p.ph + (int64_t)(kd->first + row / kd->r4) * p.gtot;
 #pragma unroll
                     for (int j = 0; j < CB; ++j) {
-                        const int64_t col = C0 + colY[j];
-                        if (col < p.gtot) {
-                            const double2 f = phr[col];
-                            const double a = tr_[i][j][q], b = ti_[i][j][q];
-                            p.W[col * p.ldw + kd->woff + row] =
-                                make_double2(__builtin_fma(f.x, a, -(f.y * b)), __builtin_fma(f.x, b, f.y * a));
-                        }
+                        const int64_t col = C0 + c0 + 16 * j;
+                        const double2 f = phr[col];
+                        const double a = tr_[i][j][q], b = ti_[i][j][q];
+                        p.W[col * p.ldw + kd->woff + row] =
+                            make_double2(__builtin_fma(f.x, a, -(f.y * b)), __builtin_fma(f.x, b, f.y * a));
                     }
                 }
             }
     }
 }
 
-template <int B, bool kH>
+template <int BR, int BC, int RB, int CB, bool kH>
 static hipError_t launch_sphere_gemm(const SphereArgs& p, int64_t nblk, hipStream_t st)
 {
     if (nblk <= 0) return hipSuccess;
-    constexpr int lds = 2 * SphereTile<B>::kStage;
-    hipLaunchKernelGGL((k_sphere_gemm<B, kH>), dim3((unsigned)nblk), dim3(SphereTile<B>::kThreads), lds, st, p);
+    using Tl = SphereTile<BR, BC, RB, CB>;
+    constexpr int lds = Tl::kLds;
+    auto* k = k_sphere_gemm<BR, BC, RB, CB, kH>;
+    if (lds > 64 * 1024) {
+        /* per launch: the attribute is per device */
+        const hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        if (e != hipSuccess) return e;
+    }
+    hipLaunchKernelGGL(k, dim3((unsigned)nblk), dim3(Tl::kThreads), lds, st, p);
     return hipGetLastError();
 }
 
+// rtiles: row tiles of all kinds for the tile's rows (tile 64: 32 x 64)
 hipError_t launch_sphere_tapp(const SphereArgs& p, int tile, int rtiles, hipStream_t st)
 {
-    const int64_t n = (int64_t)rtiles * ((p.gtot + tile - 1) / tile);
-    return tile == 64 ? launch_sphere_gemm<64, false>(p, n, st) : launch_sphere_gemm<32, false>(p, n, st);
+    if (tile == 32) return launch_sphere_gemm<32, 32, 1, 1, false>(p, (int64_t)rtiles * (p.gtot / 32), st);
+    return launch_sphere_gemm<32, 64, 1, 2, false>(p, (int64_t)rtiles * (p.gtot / 64), st);
 }
 
+// tile: 64 (64 x 64), 48 (32 x 64) or 32 (32 x 32)
 hipError_t launch_sphere_h(const SphereArgs& p, int tile, hipStream_t st)
 {
-    const int64_t n = (int64_t)((p.npatch + 7) / 8) * 8 * p.pside * p.pside;
-    return tile == 64 ? launch_sphere_gemm<64, true>(p, n, st) : launch_sphere_gemm<32, true>(p, n, st);
+    const int64_t n = ((int64_t)p.nsquares * (tile == 48 ? 2 : 1) + 7) / 8 * 8;
+    if (tile == 32) return launch_sphere_gemm<32, 32, 1, 1, true>(p, n, st);
+    if (tile == 48) return launch_sphere_gemm<32, 64, 1, 2, true>(p, n, st);
+    return launch_sphere_gemm<64, 64, 1, 2, true>(p, n, st);
 }
 
 }  // namespace hsgen

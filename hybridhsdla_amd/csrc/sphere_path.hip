@@ -47,7 +47,7 @@ hsgen_status sphere_setup(hsgen_ctx* ctx, hsgen_sys* s, const RadDev* rad)
     std::vector<KindDev> kinds(members.size());
     std::vector<int32_t> order;
     std::vector<int32_t> steps;
-    int64_t ry = 0, rw = 0, rr = 0, rt64 = 0, rt32 = 0;
+    int64_t ry = 0, rw = 0, rr = 0, rt32 = 0;
     for (size_t i = 0; i < members.size(); ++i) {
         KindDev& k = kinds[i];
         const AtomDev& at = s->atoms[members[i][0]];
@@ -60,7 +60,6 @@ hsgen_status sphere_setup(hsgen_ctx* ctx, hsgen_sys* s, const RadDev* rad)
         k.rsoff = (int32_t)rr;
         k.woff = (int32_t)rw;
         k.ldm = (int32_t)roundup(2 * at.nlm, 16);
-        k.rt64 = (int32_t)rt64;
         k.rt32 = (int32_t)rt32;
         k.first = (int32_t)order.size();
         k.count = (int32_t)members[i].size();
@@ -73,15 +72,30 @@ hsgen_status sphere_setup(hsgen_ctx* ctx, hsgen_sys* s, const RadDev* rad)
         ry += k.r4;
         rr += at.lmax + 1;
         rw += (int64_t)k.count * k.r4;
-        rt64 += ((int64_t)k.count * k.r4 + 63) / 64;
         rt32 += ((int64_t)k.count * k.r4 + 31) / 32;
     }
     if (rw > INT32_MAX - 64) return fail(ctx, HSGEN_ERR_UNSUPPORTED, "contraction depth too large");
     s->nksteps = (int)steps.size();
-    while (steps.size() % 4) steps.push_back(0);    // the last stage reads four entries
+    std::vector<SphereStage> stages((steps.size() + 3) / 4);
+    int atoms = 0;
+    for (size_t i = 0; i < stages.size(); ++i) {
+        SphereStage& g = stages[i];
+        std::memset(&g, 0, sizeof g);
+        g.atom = -1;
+        for (int q = 0; q < 4; ++q) {
+            const size_t k = 4 * i + q;
+            // past the depth: any row, no end
+            int32_t e = k < steps.size() ? steps[k] : 0;
+            if (e & 1) {
+                if (g.atom >= 0) e |= 2;
+                else g.atom = atoms;
+                ++atoms;
+            }
+            g.step[q] = e;
+        }
+    }
     s->nkinds = (int)kinds.size();
     s->ldr = (int)rr;
-    s->rt64 = (int)rt64;
     s->rt32 = (int)rt32;
     // whole stages of 16 rows can be read at the end of a column, from any
     // kind's first row; the odd multiple of 16 spreads the columns over the
@@ -106,18 +120,18 @@ hsgen_status sphere_setup(hsgen_ctx* ctx, hsgen_sys* s, const RadDev* rad)
     for (int i = 0; i < na; ++i) mtoff[i] = off[s->h_owner[order[i]]];
     auto up = [](size_t b) { return (size_t)roundup((int64_t)b, 256); };
     const size_t b_mt = up(sizeof(double2) * (size_t)total), b_k = up(sizeof(KindDev) * kinds.size()),
-                 b_o = up(sizeof(int32_t) * order.size()), b_s = up(sizeof(int32_t) * steps.size()),
+                 b_o = up(sizeof(int32_t) * order.size()), b_s = up(sizeof(SphereStage) * stages.size()),
                  b_m = up(sizeof(int64_t) * mtoff.size());
     HIPCHK(hipMalloc(&s->d_sphere, b_mt + b_k + b_o + b_s + b_m));
     char* p = (char*)s->d_sphere;
     s->d_mt = (double2*)p;
     s->d_kinds = (KindDev*)(p += b_mt);
     s->d_order = (int32_t*)(p += b_k);
-    s->d_ksteps = (int32_t*)(p += b_o);
+    s->d_stages = (SphereStage*)(p += b_o);
     s->d_mtoff = (int64_t*)(p += b_s);
     HIPCHK(hipMemcpyAsync(s->d_kinds, kinds.data(), sizeof(KindDev) * kinds.size(), hipMemcpyHostToDevice, ctx->stream));
     HIPCHK(hipMemcpyAsync(s->d_order, order.data(), sizeof(int32_t) * order.size(), hipMemcpyHostToDevice, ctx->stream));
-    HIPCHK(hipMemcpyAsync(s->d_ksteps, steps.data(), sizeof(int32_t) * steps.size(), hipMemcpyHostToDevice,
+    HIPCHK(hipMemcpyAsync(s->d_stages, stages.data(), sizeof(SphereStage) * stages.size(), hipMemcpyHostToDevice,
                           ctx->stream));
     HIPCHK(hipMemcpyAsync(s->d_mtoff, mtoff.data(), sizeof(int64_t) * mtoff.size(), hipMemcpyHostToDevice, ctx->stream));
     // the raw blocks, only until the transformed ones are built
@@ -159,29 +173,29 @@ SphereLayout sphere_layout(const hsgen_ctx* ctx, const hsgen_sys* s, const std::
 {
     SphereLayout l;
     const int ncu = std::max(ctx->n_cu, 1);
-    int64_t t64 = 0, most = 1;
+    int64_t t64 = 0;
     for (int ng : ngs) {
-        const int64_t nt = (ng + 63) / 64;
-        t64 += lower(nt);
-        most = std::max(most, nt);
-        l.gtot += nt * 64;
+        t64 += lower((ng + 63) / 64);
+        l.gtot += roundup(ng, kSphereCols);
     }
-    // H tiles of 64 x 64 once they give every CU a workgroup, else 32 x 32:
-    // four times the workgroups for a triangle that leaves CUs idle
-    l.htile = t64 >= ncu ? 64 : 32;
-    l.ttile = (int64_t)s->rt64 * (l.gtot / 64) >= ncu ? 64 : 32;
+    // H tiles by the 64 x 64 ones per CU: smaller tiles share a small triangle
+    // more evenly, larger ones read less.  Measured, us (32 atoms, lmax 10; N_G,
+    // tiles of 32, 32 x 64, 64): 1000 410 / 534 / 541, 2003 1046 / 1265 / 1468,
+    // 3001 (24 atoms, lmax 8-12) 1846 / 1720 / 1864, 4000 4231 / 3946 / 3854,
+    // 6002 9583 / 8625 / 8566.
+    l.htile = t64 < 3 * (int64_t)ncu ? 32 : t64 < 6 * (int64_t)ncu ? 48 : 64;
+    // T-application tiles of 32 x 64 once they give every CU eight: us, 32 and
+    // 32 x 64: 235 12 / 15, 600 17 / 17, 1000 157 / 139, 6002 847 / 808
+    l.ttile = (int64_t)s->rt32 * (l.gtot / 64) >= 8 * (int64_t)ncu ? 64 : 32;
     l.stile = overlap_tile(t64, ncu);
-    // patches: 8 x 8 tiles are what the 32 CUs of an XCD run at once; smaller
-    // ones where a triangle has few, so that the XCDs share it evenly
-    l.pside = most >= 128 ? 8 : most >= 24 ? 4 : 1;
+    const int hc = l.htile == 32 ? 32 : 64;
     for (int ng : ngs) {
-        const int64_t np = ((ng + l.htile - 1) / l.htile + l.pside - 1) / l.pside;
-        l.npatch += lower(np);
+        l.nsquares += lower((ng + hc - 1) / hc);
         l.nstiles += lower((ng + l.stile - 1) / l.stile);
         l.ngcols += ng;
     }
     const size_t g = (size_t)l.gtot;
-    l.b_ph = sizeof(double2) * g * (size_t)(s->natoms + 1);
+    l.b_ph = sizeof(double2) * g * (size_t)s->natoms;
     l.b_rs = sizeof(double2) * g * (size_t)s->ldr;
     l.b_y = do_h ? sizeof(double) * g * (size_t)s->ldy : 0;
     l.b_w = do_h ? sizeof(double2) * g * (size_t)s->ldw : 0;
@@ -217,10 +231,9 @@ SphereArgs sphere_args(const hsgen_sys* s, const SphereLayout& l, void* ph, void
     p.ldw = s->ldw;
     p.mt = s->d_mt;
     p.mtoff = s->d_mtoff;
-    p.ksteps = s->d_ksteps;
+    p.stages = s->d_stages;
     p.nksteps = s->nksteps;
-    p.pside = l.pside;
-    p.npatch = (int32_t)l.npatch;
+    p.nsquares = (int32_t)l.nsquares;
     return p;
 }
 
@@ -231,6 +244,7 @@ std::vector<SphereK> sphere_ks(const SphereLayout& l, const std::vector<const hs
                                const std::vector<int64_t>& ldS)
 {
     std::vector<SphereK> ks(kps.size());
+    const int hc = l.htile == 32 ? 32 : 64;
     int64_t col = 0, g = 0, st = 0, hp = 0;
     for (size_t i = 0; i < kps.size(); ++i) {
         SphereK& k = ks[i];
@@ -245,11 +259,11 @@ std::vector<SphereK> sphere_ks(const SphereLayout& l, const std::vector<const hs
         k.ng = kps[i]->ng;
         k.gcol0 = (int32_t)g;
         k.stile0 = (int32_t)st;
-        k.hpatch0 = (int32_t)hp;
-        col += roundup(k.ng, 64);
+        k.hsquare0 = (int32_t)hp;
+        col += roundup(k.ng, kSphereCols);
         g += k.ng;
         st += lower((k.ng + l.stile - 1) / l.stile);
-        hp += lower(((k.ng + l.htile - 1) / l.htile + l.pside - 1) / l.pside);
+        hp += lower((k.ng + hc - 1) / hc);
     }
     return ks;
 }
@@ -261,7 +275,7 @@ hipError_t sphere_launch(const SphereArgs& p, const SphereLayout& l, const hsgen
 {
     hipError_t e = launch_sphere_gen(p, st);
     if (e == hipSuccess && ev_gen) e = hipEventRecord(ev_gen, st);
-    if (e == hipSuccess && do_h) e = launch_sphere_tapp(p, l.ttile, l.ttile == 64 ? s->rt64 : s->rt32, st);
+    if (e == hipSuccess && do_h) e = launch_sphere_tapp(p, l.ttile, s->rt32, st);
     if (e == hipSuccess && ev_tapp) e = hipEventRecord(ev_tapp, st);
     if (e == hipSuccess && do_h) e = launch_sphere_h(p, l.htile, st);
     if (e == hipSuccess && do_s) e = launch_overlap(p, l.stile, l.nstiles, st);
