@@ -147,10 +147,11 @@ struct hsgen_sys {
     void* d_sphere = nullptr;
     double2* d_mt = nullptr;
     hsgen::KindDev* d_kinds = nullptr;
+    hsgen::OverlapGroup* d_groups = nullptr;
     int32_t* d_order = nullptr;
     hsgen::SphereStage* d_stages = nullptr;
     int64_t* d_mtoff = nullptr;
-    int nkinds = 0, nksteps = 0, ldr = 0, rt32 = 0;
+    int nkinds = 0, ngroups = 0, nksteps = 0, ldr = 0, rt32 = 0;
     int64_t ldy = 0, ldw = 0;
     // first atom of each rotation class and of each rmt class (AtomDev::cls)
     std::vector<int32_t> rot_rep, rmt_rep;

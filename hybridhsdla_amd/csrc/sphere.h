@@ -9,8 +9,8 @@
 // for all atoms of one "kind" (equal l cutoff, radius, radial data and
 // rotation, bit for bit).  So
 //   H_ij = sum_a conj(ph_a(i)) [ y_a(i)^T W_a(j) ],   W_a = ph_a (D^H M_a D) y_a
-//   S_ij = sum_kind F(i, j) sum_l (2l+1)/4pi (a_l a_l' + N_l b_l b_l') P_l(cos),
-//          F(i, j) = sum_{a of the kind} conj(ph_a(i)) ph_a(j)
+//   S_ij = sum_group F(i, j) sum_l (2l+1)/4pi (a_l a_l' + N_l b_l b_l') P_l(cos),
+//          F(i, j) = sum_{a of the group} conj(ph_a(i)) ph_a(j)
 // (the addition theorem): H takes one real-by-complex product per depth, half
 // the operations of a complex one, and S next to none.
 #pragma once
@@ -30,13 +30,24 @@ struct KindDev {
     int32_t r4;          // rows of y and of one W_a: 2 nlm rounded up to the MFMA depth of 4
     int32_t rep;         // first atom of the kind (system order): RadDev row
     int32_t yoff;        // first row of y
-    int32_t rsoff;       // first row of the radial factors
+    int32_t rsoff;       // first row of its overlap group's radial factors, or -1 if another kind writes them
     int32_t woff;        // first row of W
     int32_t ldm;         // leading dimension of Mt: 2 nlm rounded up to the stage depth of 16
     int32_t rt32;        // T-application row tiles of 32 of the kinds before this one
     int32_t first, count;   // its atoms, in kind order
     double rmt;
     double rot[9];       // column-major R_atom * bmat
+};
+
+// Kinds that differ in their rotations only, all with the same cosines between
+// plane waves (equal R^T R): one Legendre sum of S for all their atoms.
+struct OverlapGroup {
+    int32_t lmax;
+    int32_t rep;         // an atom of it (system order): RadDev row
+    int32_t rsoff;       // first row of the radial factors
+    int32_t first, count;   // its atoms, in kind order
+    int32_t newdir;      // directions differ from the group before
+    double rot[9];       // the rotation that stands for the cosines
 };
 
 // One k-point of a launch.
@@ -74,13 +85,14 @@ struct SphereStage {
 // Everything the kernels read; one k-point travels in `one`, more in `many`.
 struct SphereArgs {
     const KindDev* kinds;
+    const OverlapGroup* groups;
     const AtomDev* atoms;      // system order
     const int32_t* order;      // [natoms] atoms in kind order
     const RadDev* rad;
     const double* ynorm;
     double bmat[9];
     double vol_prefac;
-    int32_t natoms, nkinds, max_lmax, nl, L;
+    int32_t natoms, nkinds, ngroups, max_lmax, nl, L;
     int32_t chunk;             // kinds per LDS chunk of the generator
     int32_t nk, ngcols;        // k-points; plane waves of all of them
     SphereK one;

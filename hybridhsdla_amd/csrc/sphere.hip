@@ -143,7 +143,7 @@ __global__ __launch_bounds__(256) void k_sphere_gen(SphereArgs p)
             const double bu = -m.u * Knorm * dfj[l] + m.u_dr * fj[l];
             const double2 ab = make_double2(pref * au, pref * bu);
             s_ab[t * nl + l] = ab;
-            p.rs[col * p.ldr + kd.rsoff + l] = ab;
+            if (kd.rsoff >= 0) p.rs[col * p.ldr + kd.rsoff + l] = ab;
         }
         if (p.y) {
             for (int q = tid; q < nk * nl; q += blockDim.x) {
@@ -191,12 +191,14 @@ hipError_t launch_sphere_gen(const SphereArgs& p, hipStream_t st)
 
 // ---------------------------------------------------------------------------
 // S by the addition theorem.  One workgroup per lower tile of 16 M x 16 M,
-// M x MJ elements per thread (rows tx + 16 m: stores of 16 consecutive rows).  Per kind, per element: the Legendre sum (7 FP64
-// operations per l) and 4 fused operations per atom of the kind, against
+// M x MJ elements per thread (rows tx + 16 m: stores of 16 consecutive rows).  Per group, per element: the Legendre sum (7
+// FP64 operations per l) and 4 fused operations per atom, against
 // 8 (2 L) per atom of the contraction S = Y^H Y it replaces; vector FP64 and
 // the LDS reads (M + MJ of 16 bytes per M MJ elements) bound it.  Measured:
 // 6.1 ms at N_G 12007 (128 atoms of 8 kinds, lmax 12), where the contraction
-// took about 350 ms; 0.10 ms at N_G 2003 (32 atoms, 4 kinds, lmax 10).
+// took about 350 ms; 0.10 ms at N_G 2003 (32 atoms, 4 kinds, lmax 10).  Atoms
+// whose rotations leave the cosines as they are share a group: at N_G 3001 24
+// atoms of 3 types and 22 rotations took 0.83 ms as 24 sums, 0.18 ms as 3.
 //
 // P_l comes from t = 1 - |cos| = |n -+ n'|^2 / 2, formed from the difference
 // (sum, where the cosine is negative) of the unit vectors, by
@@ -255,15 +257,11 @@ __global__ __launch_bounds__(256 * M / MJ) void k_overlap(SphereArgs p)
             sg[m][n] = 1.0;
         }
 
-    for (int kk = 0; kk < p.nkinds; ++kk) {
-        const KindDev& kd = p.kinds[kk];
+    for (int kk = 0; kk < p.ngroups; ++kk) {
+        const OverlapGroup& kd = p.groups[kk];
         const int nlk = kd.lmax + 1;
         const int count = kd.count;
-        // the direction of a column is kept while the rotation stays
-        bool newrot = kk == 0;
-        if (kk > 0)
-            for (int q = 0; q < 9; ++q)
-                newrot |= __double_as_longlong(kd.rot[q]) != __double_as_longlong(p.kinds[kk - 1].rot[q]);
+        const bool newdir = kd.newdir != 0;
         __syncthreads();
         for (int q = tid; q < nlk * T; q += NT) {
             const int c = q / nlk, l = q - c * nlk;
@@ -276,7 +274,7 @@ __global__ __launch_bounds__(256 * M / MJ) void k_overlap(SphereArgs p)
             const double wb = wl * p.rad[(int64_t)kd.rep * p.nl + l].dE_u_norm;
             s_rj[l * T + c] = make_double2(wl * r.x, wb * r.y);
         }
-        if (newrot && tid < 2 * T) {
+        if (newdir && tid < 2 * T) {
             const int side = tid / T, c = tid - side * T;
             const int gi = min((side ? J0 : I0) + c, ng - 1);
             const DirAngles d = dir_angles(kd.rot, kp->k[0] + kp->g[3 * gi], kp->k[1] + kp->g[3 * gi + 1],
@@ -294,7 +292,7 @@ __global__ __launch_bounds__(256 * M / MJ) void k_overlap(SphereArgs p)
             s_pj[q] = ph[cj + c];
         }
         __syncthreads();
-        if (newrot) {
+        if (newdir) {
 #pragma unroll
             for (int m = 0; m < M; ++m)
 #pragma unroll
@@ -348,7 +346,7 @@ __global__ __launch_bounds__(256 * M / MJ) void k_overlap(SphereArgs p)
 #pragma unroll
                 for (int n = 0; n < MJ; ++n) rad[m][n] = __builtin_fma(sg[m][n], od[m][n], ev[m][n]);
         }
-        // structure factor of the kind's atoms
+        // structure factor of the group's atoms
         double fr[M][MJ], fi[M][MJ];
 #pragma unroll
         for (int m = 0; m < M; ++m)

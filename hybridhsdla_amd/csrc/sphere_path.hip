@@ -4,6 +4,7 @@
 // shared by hsgen_create_hs, hsgen_create_hs_batched and
 // hsgen_create_hs_noalloc.
 #include <algorithm>
+#include <cmath>
 #include <cstring>
 #include <map>
 
@@ -13,15 +14,41 @@ namespace hsgen {
 
 namespace {
 
-// The bits that make two atoms one kind.
-std::string kind_key(const hsgen_sys* s, int a, const RadDev* rad)
+// The bits that make two atoms one kind, or, without the rotation, candidates
+// for one overlap group.
+std::string kind_key(const hsgen_sys* s, int a, const RadDev* rad, bool rot)
 {
     const AtomDev& at = s->atoms[a];
     std::string k((const char*)&at.lmax, sizeof at.lmax);
     k.append((const char*)&at.rmt, sizeof at.rmt);
-    k.append((const char*)at.rot, sizeof at.rot);
+    if (rot) k.append((const char*)at.rot, sizeof at.rot);
     k.append((const char*)(rad + (size_t)a * s->nl), sizeof(RadDev) * (size_t)(at.lmax + 1));
     return k;
+}
+
+// Two rotations give the same cosines between plane waves: their R R^T (of
+// kb = R^T K) agree to the rounding of the products, 4 units of the largest.
+bool same_cosines(const double* r, const double* q)
+{
+    double g[2][9], big = 0.0;
+    for (int w = 0; w < 2; ++w) {
+        const double* m = w ? q : r;
+        for (int i = 0; i < 3; ++i)
+            for (int j = 0; j < 3; ++j)
+                g[w][3 * i + j] = m[i] * m[j] + m[3 + i] * m[3 + j] + m[6 + i] * m[6 + j];
+    }
+    for (int i = 0; i < 9; ++i) big = std::max(big, std::fabs(g[0][i]));
+    for (int i = 0; i < 9; ++i)
+        if (!(std::fabs(g[0][i] - g[1][i]) <= 4.0 * 2.220446049250313e-16 * big)) return false;   // NaN too
+    return true;
+}
+
+// Rotation class of an atom (AtomDev::cls holds 16 bits of it).
+int rot_class(const hsgen_sys* s, int a)
+{
+    int c = s->atoms[a].cls & 0xffff;
+    while (std::memcmp(s->atoms[s->rot_rep[c]].rot, s->atoms[a].rot, sizeof s->atoms[a].rot)) c += 0x10000;
+    return c;
 }
 
 int64_t lower(int64_t n) { return n * (n + 1) / 2; }
@@ -33,44 +60,76 @@ int64_t lower(int64_t n) { return n * (n + 1) / 2; }
 hsgen_status sphere_setup(hsgen_ctx* ctx, hsgen_sys* s, const RadDev* rad)
 {
     const int na = s->natoms;
-    std::map<std::string, int> id;
-    std::vector<std::vector<int>> members;
-    for (int a = 0; a < na; ++a) {
-        const auto it = id.emplace(kind_key(s, a, rad), (int)members.size());
-        if (it.second) members.emplace_back();
-        members[it.first->second].push_back(a);
+    // classes of rotations with the same cosines
+    std::vector<int> cos_rep, cos_of_rot(s->rot_rep.size());
+    for (size_t c = 0; c < s->rot_rep.size(); ++c) {
+        const double* rot = s->atoms[s->rot_rep[c]].rot;
+        size_t k = 0;
+        while (k < cos_rep.size() && !same_cosines(s->atoms[cos_rep[k]].rot, rot)) ++k;
+        if (k == cos_rep.size()) cos_rep.push_back(s->rot_rep[c]);
+        cos_of_rot[c] = (int)k;
     }
-    // kinds of one rotation next to each other: S keeps its directions over them
-    std::stable_sort(members.begin(), members.end(), [&](const std::vector<int>& x, const std::vector<int>& y) {
-        return (s->atoms[x[0]].cls & 0xffff) < (s->atoms[y[0]].cls & 0xffff);
+    // kinds, sorted by cosine class, then by overlap group
+    struct Kind {
+        int cos, group;
+        std::vector<int> atoms;
+    };
+    std::map<std::string, int> id;
+    std::map<std::pair<int, std::string>, int> gid;
+    std::vector<Kind> members;
+    for (int a = 0; a < na; ++a) {
+        const auto it = id.emplace(kind_key(s, a, rad, true), (int)members.size());
+        if (it.second) {
+            const int c = cos_of_rot[rot_class(s, a)];
+            const auto g = gid.emplace(std::make_pair(c, kind_key(s, a, rad, false)), (int)gid.size());
+            members.push_back(Kind{c, g.first->second, {}});
+        }
+        members[it.first->second].atoms.push_back(a);
+    }
+    std::stable_sort(members.begin(), members.end(), [](const Kind& x, const Kind& y) {
+        return std::make_pair(x.cos, x.group) < std::make_pair(y.cos, y.group);
     });
+    std::vector<OverlapGroup> groups;
     std::vector<KindDev> kinds(members.size());
     std::vector<int32_t> order;
     std::vector<int32_t> steps;
     int64_t ry = 0, rw = 0, rr = 0, rt32 = 0;
     for (size_t i = 0; i < members.size(); ++i) {
         KindDev& k = kinds[i];
-        const AtomDev& at = s->atoms[members[i][0]];
+        const AtomDev& at = s->atoms[members[i].atoms[0]];
         std::memset(&k, 0, sizeof k);
         k.lmax = at.lmax;
         k.nlm = at.nlm;
         k.r4 = (int32_t)roundup(2 * at.nlm, 4);
-        k.rep = members[i][0];
+        k.rep = members[i].atoms[0];
         k.yoff = (int32_t)ry;
-        k.rsoff = (int32_t)rr;
         k.woff = (int32_t)rw;
         k.ldm = (int32_t)roundup(2 * at.nlm, 16);
         k.rt32 = (int32_t)rt32;
         k.first = (int32_t)order.size();
-        k.count = (int32_t)members[i].size();
+        k.count = (int32_t)members[i].atoms.size();
         k.rmt = at.rmt;
         std::memcpy(k.rot, at.rot, sizeof k.rot);
-        for (int a : members[i]) {
+        k.rsoff = -1;
+        if (i == 0 || members[i].group != members[i - 1].group) {
+            k.rsoff = (int32_t)rr;
+            OverlapGroup g;
+            std::memset(&g, 0, sizeof g);
+            g.lmax = at.lmax;
+            g.rep = k.rep;
+            g.rsoff = k.rsoff;
+            g.first = k.first;
+            g.newdir = i == 0 || members[i].cos != members[i - 1].cos;
+            std::memcpy(g.rot, s->atoms[cos_rep[members[i].cos]].rot, sizeof g.rot);
+            groups.push_back(g);
+            rr += at.lmax + 1;
+        }
+        groups.back().count += k.count;
+        for (int a : members[i].atoms) {
             order.push_back(a);
             for (int r = 0; r < k.r4; r += 4) steps.push_back(k.yoff + r + (r + 4 == k.r4));
         }
         ry += k.r4;
-        rr += at.lmax + 1;
         rw += (int64_t)k.count * k.r4;
         rt32 += ((int64_t)k.count * k.r4 + 31) / 32;
     }
@@ -95,6 +154,7 @@ hsgen_status sphere_setup(hsgen_ctx* ctx, hsgen_sys* s, const RadDev* rad)
         }
     }
     s->nkinds = (int)kinds.size();
+    s->ngroups = (int)groups.size();
     s->ldr = (int)rr;
     s->rt32 = (int)rt32;
     // whole stages of 16 rows can be read at the end of a column, from any
@@ -120,16 +180,20 @@ hsgen_status sphere_setup(hsgen_ctx* ctx, hsgen_sys* s, const RadDev* rad)
     for (int i = 0; i < na; ++i) mtoff[i] = off[s->h_owner[order[i]]];
     auto up = [](size_t b) { return (size_t)roundup((int64_t)b, 256); };
     const size_t b_mt = up(sizeof(double2) * (size_t)total), b_k = up(sizeof(KindDev) * kinds.size()),
+                 b_g = up(sizeof(OverlapGroup) * groups.size()),
                  b_o = up(sizeof(int32_t) * order.size()), b_s = up(sizeof(SphereStage) * stages.size()),
                  b_m = up(sizeof(int64_t) * mtoff.size());
-    HIPCHK(hipMalloc(&s->d_sphere, b_mt + b_k + b_o + b_s + b_m));
+    HIPCHK(hipMalloc(&s->d_sphere, b_mt + b_k + b_g + b_o + b_s + b_m));
     char* p = (char*)s->d_sphere;
     s->d_mt = (double2*)p;
     s->d_kinds = (KindDev*)(p += b_mt);
-    s->d_order = (int32_t*)(p += b_k);
+    s->d_groups = (OverlapGroup*)(p += b_k);
+    s->d_order = (int32_t*)(p += b_g);
     s->d_stages = (SphereStage*)(p += b_o);
     s->d_mtoff = (int64_t*)(p += b_s);
     HIPCHK(hipMemcpyAsync(s->d_kinds, kinds.data(), sizeof(KindDev) * kinds.size(), hipMemcpyHostToDevice, ctx->stream));
+    HIPCHK(hipMemcpyAsync(s->d_groups, groups.data(), sizeof(OverlapGroup) * groups.size(), hipMemcpyHostToDevice,
+                          ctx->stream));
     HIPCHK(hipMemcpyAsync(s->d_order, order.data(), sizeof(int32_t) * order.size(), hipMemcpyHostToDevice, ctx->stream));
     HIPCHK(hipMemcpyAsync(s->d_stages, stages.data(), sizeof(SphereStage) * stages.size(), hipMemcpyHostToDevice,
                           ctx->stream));
@@ -207,6 +271,7 @@ SphereArgs sphere_args(const hsgen_sys* s, const SphereLayout& l, void* ph, void
     SphereArgs p;
     std::memset(&p, 0, sizeof p);
     p.kinds = s->d_kinds;
+    p.groups = s->d_groups;
     p.atoms = s->d_atoms;
     p.order = s->d_order;
     p.rad = s->d_rad;
@@ -215,6 +280,7 @@ SphereArgs sphere_args(const hsgen_sys* s, const SphereLayout& l, void* ph, void
     p.vol_prefac = s->vol_prefac;
     p.natoms = s->natoms;
     p.nkinds = s->nkinds;
+    p.ngroups = s->ngroups;
     p.max_lmax = s->max_lmax;
     p.nl = s->nl;
     p.L = s->L;

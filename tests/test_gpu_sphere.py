@@ -114,3 +114,31 @@ def test_general_contraction_tiles_give_the_same_bits(ctx, ng):
     for tile in range(1, 15):
         H, S = ctx.create_HS2_stripped_v2(*args, tile=tile)
         assert np.array_equal(H, H0) and np.array_equal(S, S0), tile
+
+
+def _hexagonal(seed, natoms, turn):
+    """A hexagonal cell whose atoms, of two types, carry rotations by multiples
+    of 60 degrees (equal cosines up to rounding) or, with another kind of turn,
+    matrices that change the cosines."""
+    s, kp = tiny_system(natoms=natoms, lmax=(6, 4), a_cell=8.0, ng_target=150, seed=seed)
+    a1, a3 = 8.0, 9.0
+    amat = np.array([[a1, -a1 / 2, 0.0], [0.0, a1 * np.sqrt(3) / 2, 0.0], [0.0, 0.0, a3]])
+    b33 = 2 * np.pi * np.linalg.inv(amat).T
+    s.bmat = np.asfortranarray(b33).reshape(-1, order="F").copy()
+    s.omega = float(np.linalg.det(amat))
+    for a in range(natoms):
+        c, sn = np.cos(a * np.pi / 3), np.sin(a * np.pi / 3)
+        r = np.array([[c, -sn, 0.0], [sn, c, 0.0], [0.0, 0.0, 1.0]])
+        if turn == "sheared":
+            r = r + 0.05 * a * np.array([[0.0, 1.0, 0.0], [0.0, 0.0, 1.0], [0.0, 0.0, 0.0]])
+        s.rotmat[a] = (r @ b33).reshape(-1, order="F")
+    return s, kp
+
+
+@pytest.mark.parametrize("turn", ["rotated", "sheared"])
+@pytest.mark.parametrize("natoms", [3, 12])
+def test_rotations_with_equal_and_other_cosines(ctx, natoms, turn):
+    """Atoms that differ in their rotations alone share one Legendre sum where
+    the rotations leave the cosines between plane waves as they are."""
+    s, kp = _hexagonal(40, natoms, turn)
+    _check(ctx, s, kp)
