@@ -564,6 +564,7 @@ hsgen_status hsgen_system_destroy(hsgen_ctx* ctx, hsgen_sys* s)
     if (s->d_ynorm) (void)hipFree(s->d_ynorm);
     if (s->d_M) (void)hipFree(s->d_M);
     if (s->d_sphere) (void)hipFree(s->d_sphere);
+    if (s->d_split) (void)hipFree(s->d_split);
     delete s;
     return HSGEN_OK;
 }

@@ -225,8 +225,11 @@ hsgen_status run_grouped(hsgen_ctx* ctx, int cfg, std::vector<GemmProblem>& prob
 }
 
 // Common tail of create_hs / contract_hs: Y (or Z, Zs) resident -> tmul -> S, H.
+// With kp (split precision from a system, its G list in ctx->g) W comes from
+// the real vectors instead of Y: a real-by-complex T application, half the
+// operations.
 hsgen_status finish_hs(hsgen_ctx* ctx, hsgen_sys* s, const Geometry& geo, int ng, const hsgen_opts& o,
-                       double* H, double* S, int64_t ld, hsgen_report* rep, double ms_front)
+                       double* H, double* S, int64_t ld, hsgen_report* rep, double ms_front, const hsgen_kpoint* kp)
 {
     const int flags = o.flags;
     hsgen_status st;
@@ -256,16 +259,31 @@ hsgen_status finish_hs(hsgen_ctx* ctx, hsgen_sys* s, const Geometry& geo, int ng
         dS = (double2*)ctx->Stmp.p;
         ldS = ng;
     }
-    st = ensure_M(ctx, s, geo.t.bk, geo.t.bm);
-    if (st) return st;
+    if (kp) {
+        std::lock_guard<std::mutex> lk(s->m_mu);
+        s->pad_bk = geo.t.bk;
+        s->pad_bm = geo.t.bm;
+    } else {
+        st = ensure_M(ctx, s, geo.t.bk, geo.t.bm);
+        if (st) return st;
+    }
 
     std::vector<GemmProblem> probs;
     std::vector<TileWork> work;
     HIPCHK(hipEventRecord(ctx->ev[2], ctx->stream));
     if (need_h) {
-        const int tc = tapp_cfg(geo);
-        add_tmul_problems(probs, work, s, geo, zgemm_cfg(tc), ng, Z, W);
-        st = run_grouped(ctx, tc, probs, work);
+        if (kp) {
+            SphereK k;
+            std::memset(&k, 0, sizeof k);
+            for (int q = 0; q < 3; ++q) k.k[q] = kp->k[q];
+            k.g = (const int32_t*)ctx->g.p;
+            k.ng = ng;
+            st = sphere_split_w(ctx, s, {k}, nullptr, geo.gp, W, geo.ldz);
+        } else {
+            const int tc = tapp_cfg(geo);
+            add_tmul_problems(probs, work, s, geo, zgemm_cfg(tc), ng, Z, W);
+            st = run_grouped(ctx, tc, probs, work);
+        }
         if (st) return st;
         // rows 2K .. ldz-1 of W are not written by the T application; clear
         // them so that no earlier, larger system's values remain there (the
@@ -364,7 +382,7 @@ hsgen_status create_hs_general(hsgen_ctx* ctx, hsgen_sys* s, const hsgen_kpoint*
     HIPCHK(hipEventRecord(ctx->ev[0], ctx->stream));
     HIPCHK(launch_abgen(p, true, ctx->stream));
     HIPCHK(hipEventRecord(ctx->ev[1], ctx->stream));
-    st = finish_hs(ctx, s, geo, ng, o, H, S, ld, rep, 0.0);
+    st = finish_hs(ctx, s, geo, ng, o, H, S, ld, rep, 0.0, is_split(o.precision) ? kp : nullptr);
     if (st) return st;
     if (rep) {
         float t0 = 0;

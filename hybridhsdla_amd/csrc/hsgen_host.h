@@ -151,6 +151,12 @@ struct hsgen_sys {
     int32_t* d_order = nullptr;
     hsgen::SphereStage* d_stages = nullptr;
     int64_t* d_mtoff = nullptr;
+    std::vector<int32_t> h_order;      // atoms in kind order
+    // split precision (built by its first call): matrices, their offsets per
+    // atom in kind order, rows of W
+    void* d_split = nullptr;
+    int64_t* d_split_off = nullptr;
+    int32_t* d_split_rows = nullptr;
     int nkinds = 0, ngroups = 0, nksteps = 0, ldr = 0, rt32 = 0;
     int64_t ldy = 0, ldw = 0;
     // first atom of each rotation class and of each rmt class (AtomDev::cls)
@@ -227,7 +233,8 @@ void add_tmul_problems(std::vector<GemmProblem>& probs, std::vector<TileWork>& w
                        const Geometry& geo, const ZgemmLaunchCfg& tc, int64_t ncols, const double2* Z, double2* W);
 hsgen_status run_grouped(hsgen_ctx* ctx, int cfg, std::vector<GemmProblem>& probs, std::vector<TileWork>& work);
 hsgen_status finish_hs(hsgen_ctx* ctx, hsgen_sys* s, const Geometry& geo, int ng, const hsgen_opts& o, double* H,
-                       double* S, int64_t ld, hsgen_report* rep, double ms_front);
+                       double* S, int64_t ld, hsgen_report* rep, double ms_front,
+                       const hsgen_kpoint* kp = nullptr);
 
 // create_hs on the general operands (split precision; the autotuner's FP64 runs)
 hsgen_status create_hs_general(hsgen_ctx* ctx, hsgen_sys* s, const hsgen_kpoint* kp, const hsgen_opts& o, double* H,
@@ -249,6 +256,9 @@ std::vector<SphereK> sphere_ks(const SphereLayout& l, const std::vector<const hs
                                const std::vector<int64_t>& ldS);
 hipError_t sphere_launch(const SphereArgs& p, const SphereLayout& l, const hsgen_sys* s, bool do_h, bool do_s,
                          hipEvent_t ev_gen, hipEvent_t ev_tapp, hipStream_t st);
+hsgen_status sphere_split_setup(hsgen_ctx* ctx, hsgen_sys* s);
+hsgen_status sphere_split_w(hsgen_ctx* ctx, hsgen_sys* s, const std::vector<SphereK>& ks, const SphereK* ks_dev,
+                            int64_t ncols, double2* W, int64_t ldw);
 // Bytes of the operands per plane wave (reports).
 inline double sphere_gen_bytes(const hsgen_sys* s)
 {

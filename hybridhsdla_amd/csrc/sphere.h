@@ -74,6 +74,13 @@ struct MtJob {
     int32_t pad;
 };
 
+// One matrix of split precision's T application, from its Mt.
+struct SplitMtJob {
+    int64_t src, dst;    // offsets (complex units)
+    int32_t nlm, rows, ldm;
+    int32_t sq;          // first of the divisors of its B rows, per l
+};
+
 // One stage of 16 rows of H's depth, four k-steps of 4.
 struct SphereStage {
     int32_t step[4];     // row of y of the k-step (a multiple of 4); bit 0: an atom ends with it; bit 1: and
@@ -95,6 +102,11 @@ struct SphereArgs {
     int32_t natoms, nkinds, ngroups, max_lmax, nl, L;
     int32_t chunk;             // kinds per LDS chunk of the generator
     int32_t nk, ngcols;        // k-points; plane waves of all of them
+    // split precision: the arrays hold columns cbase .. cbase + gtot - 1 of the
+    // call, padding columns included (as zeros), and the T application stores
+    // row r of W where rowdst[r] says (-1: nowhere)
+    int64_t cbase;
+    const int32_t* rowdst;     // null: FP64
     SphereK one;
     const SphereK* many;
     int64_t gtot;              // columns of the operand arrays
@@ -112,6 +124,8 @@ struct SphereArgs {
 };
 
 int sphere_chunk(int nl, int L);
+hipError_t launch_split_mt(const SplitMtJob* jobs, int njobs, int64_t max_elems, const double* sq, const double2* mt,
+                           double2* out, hipStream_t st);
 hipError_t launch_build_mt(const MtJob* jobs, int njobs, int64_t max_elems, double2* mt, hipStream_t st);
 hipError_t launch_sphere_gen(const SphereArgs& p, hipStream_t st);
 // S tile side by the number of lower tiles; the bits do not depend on it

@@ -101,9 +101,24 @@ __global__ __launch_bounds__(256) void k_sphere_gen(SphereArgs p)
     unsigned char* s_l = (unsigned char*)(s_dir + p.chunk); // [L]       l of lm
     const int c = blockIdx.x;
     const SphereK* kp = &p.one;
-    if (p.nk > 1) kp = p.many + find_last(p.nk, c, [&](int i) { return p.many[i].gcol0; });
-    const int gi = c - kp->gcol0;
-    const int64_t col = kp->col0 + gi;
+    int gi;
+    int64_t col;
+    if (p.rowdst) {
+        // every column of the chunk, padding as zeros
+        const int at = (int)p.cbase + c;
+        if (p.nk > 1) kp = p.many + find_last(p.nk, at, [&](int i) { return (int)p.many[i].col0; });
+        gi = at - (int)kp->col0;
+        col = c;
+        if (gi >= kp->ng) {
+            for (int64_t r = tid; r < p.ldy; r += blockDim.x) p.y[col * p.ldy + r] = 0.0;
+            for (int a = tid; a < p.natoms; a += blockDim.x) p.ph[(int64_t)a * p.gtot + col] = make_double2(0.0, 0.0);
+            return;
+        }
+    } else {
+        if (p.nk > 1) kp = p.many + find_last(p.nk, c, [&](int i) { return p.many[i].gcol0; });
+        gi = c - kp->gcol0;
+        col = kp->col0 + gi;
+    }
     const double K0 = kp->k[0] + kp->g[3 * gi + 0];
     const double K1 = kp->k[1] + kp->g[3 * gi + 1];
     const double K2 = kp->k[2] + kp->g[3 * gi + 2];
@@ -143,7 +158,7 @@ __global__ __launch_bounds__(256) void k_sphere_gen(SphereArgs p)
             const double bu = -m.u * Knorm * dfj[l] + m.u_dr * fj[l];
             const double2 ab = make_double2(pref * au, pref * bu);
             s_ab[t * nl + l] = ab;
-            if (kd.rsoff >= 0) p.rs[col * p.ldr + kd.rsoff + l] = ab;
+            if (kd.rsoff >= 0 && p.rs) p.rs[col * p.ldr + kd.rsoff + l] = ab;
         }
         if (p.y) {
             for (int q = tid; q < nk * nl; q += blockDim.x) {
@@ -519,10 +534,55 @@ hipError_t launch_build_mt(const MtJob* jobs, int njobs, int64_t max_elems, doub
     return hipGetLastError();
 }
 
+// Split precision's W has complex rows: E M D = E D diag(1, 1/2) Mt, where
+// D^H D = diag(1 for m = 0, else 2) and E divides the B rows by sq (sqrt(N_l)
+// of folded operands, or 1).
+__global__ __launch_bounds__(256) void k_split_mt(const SplitMtJob* __restrict__ jobs, const double* __restrict__ sq,
+                                                  const double2* __restrict__ mt, double2* __restrict__ out)
+{
+#pragma clang fp contract(off)
+    const SplitMtJob jb = jobs[blockIdx.y];
+    const int n = jb.nlm;
+    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int r = (int)(e / jb.ldm), k = (int)(e - (int64_t)r * jb.ldm);
+    if (r >= jb.rows) return;
+    double2 v = make_double2(0.0, 0.0);
+    if (r < 2 * n) {
+        const int blk = r >= n ? n : 0;
+        const int l = l_of_lm(r - blk);
+        const int m = r - blk - l * (l + 1);
+        const int am = m < 0 ? -m : m;
+        const double2* src = mt + jb.src + (int64_t)(blk + l * (l + 1)) * jb.ldm + k;
+        const double2 c = src[(int64_t)am * jb.ldm];
+        v = c;
+        if (m != 0) {
+            const double2 s = src[-(int64_t)am * jb.ldm];
+            // (l, m): (c - i s) / 2; (l, -m): (-1)^m (c + i s) / 2
+            v = m > 0 ? make_double2(0.5 * (c.x + s.y), 0.5 * (c.y - s.x))
+                      : make_double2(0.5 * (c.x - s.y), 0.5 * (c.y + s.x));
+            if (m < 0 && (am & 1)) v = make_double2(-v.x, -v.y);
+        }
+        if (blk) {
+            const double d = sq[jb.sq + l];
+            v.x /= d;
+            v.y /= d;
+        }
+    }
+    out[jb.dst + e] = v;
+}
+
+hipError_t launch_split_mt(const SplitMtJob* jobs, int njobs, int64_t max_elems, const double* sq, const double2* mt,
+                           double2* out, hipStream_t st)
+{
+    if (njobs <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_split_mt, dim3((unsigned)((max_elems + 255) / 256), njobs), dim3(256), 0, st, jobs, sq, mt, out);
+    return hipGetLastError();
+}
+
 // ---------------------------------------------------------------------------
 // Complex-by-real products on v_mfma_f64_16x16x4.
 //
-// One tile is B x B: rows are columns of a complex operand X, columns are
+// One tile is BR x BC: rows are columns of a complex operand X, columns are
 // columns of a real operand y, both contiguous along the depth:
 //   T[r][c] = sum_k X[k, r] y[k, c]       two real MFMAs per 16 x 16 x 4.
 // kH: X = W of the tile's H columns j, y of the tile's H rows i.  The depth
@@ -892,14 +952,16 @@ __global__ __launch_bounds__((SphereTile<BR, BC, RB, CB>::kThreads), 4) void k_s
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 const int row = R0 + wr * 16 * RB + i * 16 + q0 + 4 * q;
-                if (row < nrow) {
+                int64_t dst = kd->woff + row;
+                if (row < nrow && p.rowdst) dst = p.rowdst[dst];
+                if (row < nrow && dst >= 0) {
                     const double2* phr = p.ph + (int64_t)(kd->first + row / kd->r4) * p.gtot;
 #pragma unroll
                     for (int j = 0; j < CB; ++j) {
                         const int64_t col = C0 + c0 + 16 * j;
                         const double2 f = phr[col];
                         const double a = tr_[i][j][q], b = ti_[i][j][q];
-                        p.W[col * p.ldw + kd->woff + row] =
+                        p.W[col * p.ldw + dst] =
                             make_double2(__builtin_fma(f.x, a, -(f.y * b)), __builtin_fma(f.x, b, f.y * a));
                     }
                 }

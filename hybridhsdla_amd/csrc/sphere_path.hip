@@ -5,6 +5,7 @@
 // hsgen_create_hs_noalloc.
 #include <algorithm>
 #include <cmath>
+#include <cstdlib>
 #include <cstring>
 #include <map>
 
@@ -52,6 +53,31 @@ int rot_class(const hsgen_sys* s, int a)
 }
 
 int64_t lower(int64_t n) { return n * (n + 1) / 2; }
+
+}  // namespace
+
+namespace {
+
+int64_t mt_size(int64_t nlm) { return roundup(2 * nlm, 4) * roundup(2 * nlm, 16); }
+
+// Device memory of a set-up step.
+struct Tmp {
+    void* p = nullptr;
+    ~Tmp() { if (p) (void)hipFree(p); }
+};
+
+// grid.y is at most 65535
+constexpr size_t kJobsPerLaunch = 32768;
+
+// T-application tiles of 32 x 64 once they give every CU eight: us, 32 and
+// 32 x 64: N_G 235 12 / 15, 600 17 / 17, 1000 157 / 139, 6002 847 / 808.
+int tapp_tile(const hsgen_ctx* ctx, const hsgen_sys* s, int64_t gtot)
+{
+    return (int64_t)s->rt32 * (gtot / 64) >= 8 * (int64_t)std::max(ctx->n_cu, 1) ? 64 : 32;
+}
+
+// Real vectors of split precision's T application at a time.
+constexpr int64_t kSplitChunkBytes = (int64_t)512 << 20;
 
 }  // namespace
 
@@ -154,6 +180,7 @@ hsgen_status sphere_setup(hsgen_ctx* ctx, hsgen_sys* s, const RadDev* rad)
         }
     }
     s->nkinds = (int)kinds.size();
+    s->h_order = order;
     s->ngroups = (int)groups.size();
     s->ldr = (int)rr;
     s->rt32 = (int)rt32;
@@ -163,17 +190,13 @@ hsgen_status sphere_setup(hsgen_ctx* ctx, hsgen_sys* s, const RadDev* rad)
     s->ldy = (roundup(ry, 16) + 16) | 16;
     s->ldw = roundup(rw, 16) | 16;
     // T blocks in real harmonics, one per distinct T (h_owner)
-    std::vector<int64_t> off(na, 0), traw(na, 0);
-    int64_t total = 0, raw = 0, most = 0;
+    std::vector<int64_t> off(na, 0);
+    int64_t total = 0;
     std::vector<int> owners;
     for (int a = 0; a < na; ++a) {
         if (s->h_owner[a] != a) continue;
-        const int64_t n = s->atoms[a].nlm;
         off[a] = total;
-        total += roundup(2 * n, 4) * roundup(2 * n, 16);
-        most = std::max(most, roundup(2 * n, 4) * roundup(2 * n, 16));
-        traw[a] = raw;
-        raw += 3 * n * n;
+        total += mt_size(s->atoms[a].nlm);
         owners.push_back(a);
     }
     std::vector<int64_t> mtoff(na);
@@ -198,37 +221,125 @@ hsgen_status sphere_setup(hsgen_ctx* ctx, hsgen_sys* s, const RadDev* rad)
     HIPCHK(hipMemcpyAsync(s->d_stages, stages.data(), sizeof(SphereStage) * stages.size(), hipMemcpyHostToDevice,
                           ctx->stream));
     HIPCHK(hipMemcpyAsync(s->d_mtoff, mtoff.data(), sizeof(int64_t) * mtoff.size(), hipMemcpyHostToDevice, ctx->stream));
-    // the raw blocks, only until the transformed ones are built
-    struct Tmp {
-        void* p = nullptr;
-        ~Tmp() { if (p) (void)hipFree(p); }
-    } t_raw, t_jobs;
+    // the raw blocks, only until the matrices are built
+    Tmp t_raw, t_jobs;
+    int64_t raw = 0, most = 0;
+    for (int a : owners) {
+        raw += 3 * (int64_t)s->atoms[a].nlm * s->atoms[a].nlm;
+        most = std::max(most, mt_size(s->atoms[a].nlm));
+    }
     HIPCHK(hipMalloc(&t_raw.p, sizeof(double2) * (size_t)raw));
     HIPCHK(hipMalloc(&t_jobs.p, sizeof(MtJob) * owners.size()));
     double2* d = (double2*)t_raw.p;
     std::vector<MtJob> jobs;
     for (int a : owners) {
-        const int64_t n = s->atoms[a].nlm;
-        MtJob j{};
-        j.taa = d + traw[a];
-        j.tab = j.taa + n * n;
-        j.tbb = j.tab + n * n;
-        j.off = off[a];
-        j.nlm = (int32_t)n;
-        j.rows = (int32_t)roundup(2 * n, 4);
-        j.ldm = (int32_t)roundup(2 * n, 16);
+        const int64_t n = s->atoms[a].nlm, n2 = n * n;
         const std::vector<std::complex<double>>* src[3] = {&s->h_taa[a], &s->h_tab[a], &s->h_tbb[a]};
         for (int b = 0; b < 3; ++b)
-            HIPCHK(hipMemcpyAsync(d + traw[a] + b * n * n, src[b]->data(), sizeof(double2) * (size_t)(n * n),
-                                  hipMemcpyHostToDevice, ctx->stream));
-        jobs.push_back(j);
+            HIPCHK(hipMemcpyAsync(d + b * n2, src[b]->data(), sizeof(double2) * (size_t)n2, hipMemcpyHostToDevice,
+                                  ctx->stream));
+        jobs.push_back(MtJob{d, d + n2, d + 2 * n2, off[a], (int32_t)n, (int32_t)roundup(2 * n, 4),
+                             (int32_t)roundup(2 * n, 16), 0});
+        d += 3 * n2;
     }
     HIPCHK(hipMemcpyAsync(t_jobs.p, jobs.data(), sizeof(MtJob) * jobs.size(), hipMemcpyHostToDevice, ctx->stream));
-    // grid.y is at most 65535
-    for (size_t j0 = 0; j0 < jobs.size(); j0 += 32768)
-        HIPCHK(launch_build_mt((const MtJob*)t_jobs.p + j0, (int)std::min<size_t>(32768, jobs.size() - j0), most, s->d_mt,
-                               ctx->stream));
+    for (size_t j0 = 0; j0 < jobs.size(); j0 += kJobsPerLaunch)
+        HIPCHK(launch_build_mt((const MtJob*)t_jobs.p + j0, (int)std::min(kJobsPerLaunch, jobs.size() - j0), most,
+                               s->d_mt, ctx->stream));
     HIPCHK(hipStreamSynchronize(ctx->stream));
+    return HSGEN_OK;
+}
+
+// The matrices of split precision's T application, one per distinct (T,
+// divisors of the B rows), and the rows of its W, in atom order without padding.
+hsgen_status sphere_split_setup(hsgen_ctx* ctx, hsgen_sys* s)
+{
+    std::lock_guard<std::mutex> lk(s->m_mu);
+    if (s->d_split) return HSGEN_OK;
+    const int na = s->natoms, nl = s->nl;
+    const std::vector<double> ones(nl, 1.0);
+    std::map<std::pair<int, std::vector<double>>, int64_t> seen;
+    std::vector<int64_t> src(na), off(na), mtoff;
+    std::vector<SplitMtJob> jobs;
+    std::vector<double> sq;
+    std::vector<int32_t> rows;
+    int64_t total = 0, most = 0, mt = 0;
+    for (int a = 0; a < na; ++a) {           // Mt in the order sphere_setup lays it out
+        if (s->h_owner[a] != a) continue;
+        src[a] = mt;
+        mt += mt_size(s->atoms[a].nlm);
+    }
+    for (int a = 0; a < na; ++a) {
+        const double* d = s->fold ? s->h_sqrtn.data() + (size_t)a * nl : ones.data();
+        const auto it = seen.emplace(std::make_pair(s->h_owner[a], std::vector<double>(d, d + nl)), total);
+        off[a] = it.first->second;
+        if (!it.second) continue;
+        const int n = s->atoms[a].nlm;
+        jobs.push_back(SplitMtJob{src[s->h_owner[a]], total, n, (int32_t)roundup(2 * n, 4), (int32_t)roundup(2 * n, 16),
+                                  (int32_t)sq.size()});
+        sq.insert(sq.end(), d, d + nl);
+        total += mt_size(n);
+        most = std::max(most, mt_size(n));
+    }
+    for (int a : s->h_order) {
+        const int n2 = 2 * s->atoms[a].nlm;
+        mtoff.push_back(off[a]);
+        for (int r = 0; r < (int)roundup(n2, 4); ++r) rows.push_back(r < n2 ? 2 * s->atoms[a].off + r : -1);
+    }
+    const size_t b_mt = (size_t)roundup((int64_t)(sizeof(double2) * (size_t)total), 256),
+                 b_m = (size_t)roundup((int64_t)(sizeof(int64_t) * mtoff.size()), 256);
+    Tmp keep, t_jobs, t_sq;
+    HIPCHK(hipMalloc(&keep.p, b_mt + b_m + sizeof(int32_t) * rows.size()));
+    HIPCHK(hipMalloc(&t_jobs.p, sizeof(SplitMtJob) * jobs.size()));
+    HIPCHK(hipMalloc(&t_sq.p, sizeof(double) * sq.size()));
+    char* p = (char*)keep.p;
+    HIPCHK(hipMemcpyAsync(p + b_mt, mtoff.data(), sizeof(int64_t) * mtoff.size(), hipMemcpyHostToDevice, ctx->stream));
+    HIPCHK(hipMemcpyAsync(p + b_mt + b_m, rows.data(), sizeof(int32_t) * rows.size(), hipMemcpyHostToDevice, ctx->stream));
+    HIPCHK(hipMemcpyAsync(t_jobs.p, jobs.data(), sizeof(SplitMtJob) * jobs.size(), hipMemcpyHostToDevice, ctx->stream));
+    HIPCHK(hipMemcpyAsync(t_sq.p, sq.data(), sizeof(double) * sq.size(), hipMemcpyHostToDevice, ctx->stream));
+    for (size_t j0 = 0; j0 < jobs.size(); j0 += kJobsPerLaunch)
+        HIPCHK(launch_split_mt((const SplitMtJob*)t_jobs.p + j0, (int)std::min(kJobsPerLaunch, jobs.size() - j0), most,
+                               (const double*)t_sq.p, s->d_mt, (double2*)p, ctx->stream));
+    HIPCHK(hipStreamSynchronize(ctx->stream));
+    s->d_split_off = (int64_t*)(p + b_mt);
+    s->d_split_rows = (int32_t*)(p + b_mt + b_m);
+    s->d_split = keep.p;
+    keep.p = nullptr;
+    return HSGEN_OK;
+}
+
+// W of split precision (rows 2 off_a .. of every column, leading dimension ldw)
+// over the ncols padded columns of the k-points ks (k, g, ng, col0 set;
+// ks_dev: their device copy).  Column chunks bound the real vectors' memory.
+hsgen_status sphere_split_w(hsgen_ctx* ctx, hsgen_sys* s, const std::vector<SphereK>& ks, const SphereK* ks_dev,
+                            int64_t ncols, double2* W, int64_t ldw)
+{
+    hsgen_status st = sphere_split_setup(ctx, s);
+    if (st) return st;
+    int64_t bytes = kSplitChunkBytes;
+    if (const char* e = std::getenv("HSGEN_BATCH_BYTES"))   // cap (tuning and tests)
+        if (std::strtoull(e, nullptr, 10) > 0) bytes = std::min<int64_t>(bytes, std::strtoll(e, nullptr, 10));
+    const int64_t per = 8 * s->ldy + 16 * (int64_t)s->natoms;
+    const int64_t chunk = std::min(ncols, std::max<int64_t>(kSphereCols, bytes / per / kSphereCols * kSphereCols));
+    if ((st = ensure(ctx, ctx->sph_ph, sizeof(double2) * (size_t)(chunk * s->natoms), false)) ||
+        (st = ensure(ctx, ctx->sph_y, sizeof(double) * (size_t)(chunk * s->ldy), false)))
+        return st;
+    for (int64_t c0 = 0; c0 < ncols; c0 += chunk) {
+        SphereLayout l;
+        l.gtot = std::min(chunk, ncols - c0);
+        l.ngcols = l.gtot;
+        SphereArgs p = sphere_args(s, l, ctx->sph_ph.p, nullptr, ctx->sph_y.p, W + c0 * ldw);
+        p.mt = (const double2*)s->d_split;
+        p.mtoff = s->d_split_off;
+        p.rowdst = s->d_split_rows;
+        p.cbase = c0;
+        p.ldw = ldw;
+        p.nk = (int32_t)ks.size();
+        p.one = ks[0];
+        p.many = ks_dev;
+        HIPCHK(launch_sphere_gen(p, ctx->stream));
+        HIPCHK(launch_sphere_tapp(p, tapp_tile(ctx, s, l.gtot), s->rt32, ctx->stream));
+    }
     return HSGEN_OK;
 }
 
@@ -248,9 +359,7 @@ SphereLayout sphere_layout(const hsgen_ctx* ctx, const hsgen_sys* s, const std::
     // 3001 (24 atoms, lmax 8-12) 1846 / 1720 / 1864, 4000 4231 / 3946 / 3854,
     // 6002 9583 / 8625 / 8566.
     l.htile = t64 < 3 * (int64_t)ncu ? 32 : t64 < 6 * (int64_t)ncu ? 48 : 64;
-    // T-application tiles of 32 x 64 once they give every CU eight: us, 32 and
-    // 32 x 64: 235 12 / 15, 600 17 / 17, 1000 157 / 139, 6002 847 / 808
-    l.ttile = (int64_t)s->rt32 * (l.gtot / 64) >= 8 * (int64_t)ncu ? 64 : 32;
+    l.ttile = tapp_tile(ctx, s, l.gtot);
     l.stile = overlap_tile(t64, ncu);
     const int hc = l.htile == 32 ? 32 : 64;
     for (int ng : ngs) {

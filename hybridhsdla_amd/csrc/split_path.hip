@@ -800,8 +800,12 @@ hsgen_status batched_split(hsgen_ctx* ctx, hsgen_sys* s, int nk, const hsgen_kpo
     const int64_t tm = std::max<int64_t>({(int64_t)g0.t.bm, (int64_t)g0.t.bn, align});
     const int64_t kd = roundup(g0.kpad, ic.bk);
     const int narr = oz_slots(ic, g0.fold).narr;
-    hsgen_status st = ensure_M(ctx, s, g0.t.bk, g0.t.bm);
-    if (st) return st;
+    hsgen_status st;
+    {
+        std::lock_guard<std::mutex> lk(s->m_mu);
+        s->pad_bk = g0.t.bk;
+        s->pad_bm = g0.t.bm;
+    }
     if (rep) std::memset(rep, 0, sizeof(hsgen_report) * nk);
     // largest k first; k-points without G-vectors have nothing to compute
     std::vector<int> order;
@@ -947,13 +951,22 @@ hsgen_status batched_split(hsgen_ctx* ctx, hsgen_sys* s, int nk, const hsgen_kpo
             HIPCHK(launch_abgen(p, true, ctx->stream));
         }
         if (do_h) {
-            // T application over every column of the batch in one grouped launch
-            std::vector<GemmProblem> probs;
-            std::vector<TileWork> work;
-            const int tc = tapp_cfg(geo);
-            add_tmul_problems(probs, work, s, geo, zgemm_cfg(tc), ncols, Z, W);
-            st = run_grouped(ctx, tc, probs, work);
+            // T application over every column of the batch from the real vectors
+            std::vector<SphereK> sk(bk.size());
+            for (size_t q = 0; q < bk.size(); ++q) {
+                std::memset(&sk[q], 0, sizeof sk[q]);
+                for (int c = 0; c < 3; ++c) sk[q].k[c] = kps[bk[q]].k[c];
+                sk[q].g = (const int32_t*)ctx->g.p + goff[q];
+                sk[q].ng = ks[q].ng;
+                sk[q].col0 = ks[q].col0;
+            }
+            st = ensure(ctx, ctx->probs, sizeof(SphereK) * sk.size(), false);
             if (st) return st;
+            HIPCHK(hipMemcpyAsync(ctx->probs.p, sk.data(), sizeof(SphereK) * sk.size(), hipMemcpyHostToDevice,
+                                  ctx->stream));
+            st = sphere_split_w(ctx, s, sk, (const SphereK*)ctx->probs.p, ncols, W, geo.ldz);
+            if (st) return st;
+            HIPCHK(hipStreamSynchronize(ctx->stream));   // sk must outlive its copy, ctx->probs its readers
             HIPCHK(launch_clear_rows(W, geo.ldz, 2 * (int64_t)s->kdim, geo.ldz, (int)ncols, ctx->stream));
         }
         std::vector<OzResult> ozr;

@@ -142,3 +142,28 @@ def test_rotations_with_equal_and_other_cosines(ctx, natoms, turn):
     the rotations leave the cosines between plane waves as they are."""
     s, kp = _hexagonal(40, natoms, turn)
     _check(ctx, s, kp)
+
+
+@pytest.mark.parametrize("norm", [None, 0.0])
+def test_split_precision_column_chunks(ctx, monkeypatch, norm):
+    """W of split precision comes from the real vectors in column chunks: 64
+    columns at a time give the bits of one chunk, folded or not, for one
+    k-point and for several (whose padding columns the chunks cut)."""
+    from hybridhsdla_amd.api import HSGEN_PREC_OZAKI_INT8
+    s, kp = tiny_system(natoms=5, lmax=(3, 2, 4), ng_target=300, seed=9, rotate=True)
+    if norm is not None:
+        s.match[1, 1, 4] = norm
+    h = ctx.upload(s)
+    H, S = ctx.create_HS2(h, kp, precision=HSGEN_PREC_OZAKI_INT8, slices=13)
+    Hr, Sr = po.reference_hs(s, kp)
+    assert rel_fro_lower(H, Hr) <= 1e-12 and rel_fro_lower(S, Sr) <= 1e-12
+    sub = _subset(kp, np.arange(0, kp.ng, 2))
+    Hs, Ss = ctx.create_HS2(h, sub, precision=HSGEN_PREC_OZAKI_INT8, slices=13)
+    monkeypatch.setenv("HSGEN_BATCH_BYTES", "1")
+    H1, S1 = ctx.create_HS2(h, kp, precision=HSGEN_PREC_OZAKI_INT8, slices=13)
+    assert np.array_equal(H, H1) and np.array_equal(S, S1)
+    monkeypatch.setenv("HSGEN_BATCH_BYTES", "60000000")
+    res, _ = ctx.create_HS2_batched(h, [kp, sub], precision=HSGEN_PREC_OZAKI_INT8, slices=13)
+    for (Hb, Sb), (Ha, Sa) in zip(res, ((H, S), (Hs, Ss))):
+        assert np.array_equal(Hb, Ha) and np.array_equal(Sb, Sa)
+    h.close()
