@@ -46,11 +46,11 @@ constexpr int kDefaultTile = 11;
 // quarter of the work and two of which a CU holds at once
 constexpr int kSmallTile = 12;
 constexpr int kSmallWaves = 6;
-// INT8 configuration for calls with few S and H lower tiles of 256 x 192 (all
-// k-points): 128 x 128 below kInt8FewTiles, 128 x 256 below kInt8SomeTiles;
-// BF16: 256 x 128 below kInt8SomeTiles
+// INT8 configurations of 128 x 128 and 128 x 256 tiles for smaller calls
+// (pick_tile), BF16: 256 x 128 below kBf16SomeTiles S and H lower tiles of 256 x 192
+// (all k-points)
 constexpr int kInt8SmallCfg = 14, kInt8MidCfg = 15, kBf16SmallCfg = 62;
-constexpr int kInt8FewTiles = 64, kInt8SomeTiles = 160;
+constexpr int kBf16SomeTiles = 160;
 constexpr int kFallbackTile = 8;   // register-staged, 64-bit addressing
 constexpr int kIgemmCfg = 51;      // default INT8 kernel configuration (256 x 192 tiles)
 constexpr int kBf16Cfg = 61;       // default BF16 kernel configuration (256 x 192 tiles)
@@ -305,7 +305,7 @@ std::vector<int> tune_key(int precision, int ng, int kdim);
 // this size, else 0 (the built-in default).
 // The tile of a call: opts.tile if set, else the autotuned one for the size,
 // else the default by size over the call's k-points (kps[0 .. nk-1], or one
-// k-point of ng when kps is null): see fp64_tile_by_size and int8_cfg_by_size.
+// k-point of ng when kps is null).
 int pick_tile(const hsgen_ctx* ctx, const hsgen_opts& o, int ng, int kdim, const hsgen_kpoint* kps = nullptr,
               int nk = 0);
 // FP64 tile by size: kSmallTile when the S and H lower tiles of 128 x 128 of

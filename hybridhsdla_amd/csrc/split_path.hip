@@ -563,11 +563,11 @@ hsgen_status run_ozaki(hsgen_ctx* ctx, const Geometry& geo, const std::vector<Oz
     // (the right operand's sampled columns are gathered first: the GEMM reads
     // contiguous columns, whole tiles of bn of them)
     // The sample GEMM of one k-point has only ng / 64 tiles per product: at
-    // large depth it is split into nsplit depth chunks (one per 16384 rows, at
+    // large depth it is split into nsplit depth chunks (one per 2048 rows, at
     // most 8), so that the launch fills the chip; the chunks' products are
     // summed in chunk order afterwards.  nsplit depends on the depth only, so
     // a k-point's sample is the same in single and batched calls.
-    const int nsplit = (int)std::max<int64_t>(1, std::min<int64_t>(8, geo.kpad / 16384));
+    const int nsplit = (int)std::max<int64_t>(1, std::min<int64_t>(8, geo.kpad / 2048));
     const int64_t kchunk = roundup((geo.kpad + nsplit - 1) / nsplit, sc.bk);
     st = ensure(ctx, ctx->oz_smp, sizeof(double2) * std::max<size_t>(2 * (smpt + gatht) + 2 * smpt * (nsplit - 1), 1),
                 false);

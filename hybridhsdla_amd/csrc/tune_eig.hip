@@ -106,9 +106,23 @@ int pick_tile(const hsgen_ctx* ctx, const hsgen_opts& o, int ng, int kdim, const
     if (it != ctx->tuned.end()) return it->second;
     if (o.precision == HSGEN_PREC_FP64) return fp64_tile_by_size(ctx, ng, kps, nk);
     const int64_t t = call_tiles(ng, kps, nk, 256, 192);
-    if (o.precision == HSGEN_PREC_OZAKI_INT8)
-        return t < kInt8FewTiles ? kInt8SmallCfg : t < kInt8SomeTiles ? kInt8MidCfg : 0;
-    return t < kInt8SomeTiles ? kBf16SmallCfg : 0;
+    if (o.precision == HSGEN_PREC_OZAKI_INT8) {
+        // A CU holds one workgroup of the larger tiles, so a launch takes whole
+        // rounds of n_cu tiles; a 128 x 256 round takes about 0.72 of a 256 x 192
+        // one.  128 x 128 tiles where they make one round; else, up to three
+        // rounds of 256 x 192 (where the rounding counts), the fewer.  INT8 GEMM
+        // ms of a call, 256 x 192 / 128 x 256 / 128 x 128 tiles (12 moduli; k-points
+        // of 48 atoms): 2 of 1200 plane waves 2.15 / 1.60 / 1.09, 2 of 1900 4.48 /
+        // 3.63 / 4.23, 4 of 1900 8.94 / 6.75 / 6.97, 8 of 1900 13.77 / 11.77 / 13.44;
+        // (32 atoms, N_G) 2500 3.02 / 2.34 / 2.95, 3000 3.38 / 4.33 / 4.30, 3500 6.47 /
+        // 4.95 / 6.18, 4000 6.53 / 7.25 / 7.70, 5000 9.94 / 9.88 / 11.23.
+        const int64_t ncu = std::max(ctx->n_cu, 1);
+        auto rounds = [&](int64_t n) { return (n + ncu - 1) / ncu; };
+        if (call_tiles(ng, kps, nk, 128, 128) <= ncu) return kInt8SmallCfg;
+        const int64_t big = rounds(t), mid = rounds(call_tiles(ng, kps, nk, 128, 256));
+        return big <= 3 && 72 * mid < 100 * big ? kInt8MidCfg : 0;
+    }
+    return t < kBf16SomeTiles ? kBf16SmallCfg : 0;
 }
 
 }  // namespace hsgen

@@ -167,3 +167,20 @@ def test_split_precision_column_chunks(ctx, monkeypatch, norm):
     for (Hb, Sb), (Ha, Sa) in zip(res, ((H, S), (Hs, Ss))):
         assert np.array_equal(Hb, Ha) and np.array_equal(Sb, Sa)
     h.close()
+
+
+@pytest.mark.parametrize("ng,nk,tile", [(1900, 1, 14), (1200, 2, 14), (1900, 2, 15), (3000, 1, 51), (3500, 1, 15)])
+def test_int8_tiles_by_rounds(ctx, ng, nk, tile):
+    """INT8 tiles by whole rounds of one per CU: 128 x 128 where they make one,
+    128 x 256 where they save rounds; the bits of the 256 x 192 tiles."""
+    from hybridhsdla_amd.api import HSGEN_PREC_OZAKI_INT8
+    s, kps = make_config(1, ng=ng, natoms=2)
+    kps = [kps[0], _subset(kps[0], np.arange(kps[0].ng - 5))][:nk]
+    h = ctx.upload(s)
+    res, reps = ctx.create_HS2_batched(h, kps, precision=HSGEN_PREC_OZAKI_INT8, slices=12)
+    ref, _ = ctx.create_HS2_batched(h, kps, precision=HSGEN_PREC_OZAKI_INT8, slices=12, tile=51)
+    print(f"ng {kps[0].ng} x {nk}: tile {reps[0]['tile_used']}", flush=True)
+    assert reps[0]["tile_used"] == tile
+    for (Ha, Sa), (Hb, Sb) in zip(res, ref):
+        assert np.array_equal(Ha, Hb) and np.array_equal(Sa, Sb)
+    h.close()
