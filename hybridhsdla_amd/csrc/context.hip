@@ -348,6 +348,11 @@ hsgen_status init_stream(hsgen_ctx* ctx)
     HIPCHK(hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking));
     for (auto& ev : ctx->ev) HIPCHK(hipEventCreate(&ev));
     for (auto& ev : ctx->oz_ev) HIPCHK(hipEventCreate(&ev));
+    HIPCHK(hipHostMalloc(&ctx->pin, kPinStamps + sizeof(int32_t) * 3 * kPinnedG, hipHostMallocDefault));
+    HIPCHK(hipHostGetDevicePointer(&ctx->pin_dev, ctx->pin, 0));
+    int khz = 0;
+    HIPCHK(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, ctx->device));
+    if (khz > 0) ctx->ms_per_tick = 1.0 / khz;
     return HSGEN_OK;
 }
 
@@ -416,6 +421,7 @@ hsgen_status hsgen_finalize(hsgen_ctx* ctx)
     if (ctx->blas) (void)rocblas_destroy_handle(ctx->blas);
     for (void*& p : ctx->stage)
         if (p) (void)hipHostFree(p);
+    if (ctx->pin) (void)hipHostFree(ctx->pin);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;
     return HSGEN_OK;

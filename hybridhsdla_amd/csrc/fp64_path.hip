@@ -409,8 +409,7 @@ hsgen_status create_hs_sphere(hsgen_ctx* ctx, hsgen_sys* s, const hsgen_kpoint* 
         s->pad_bk = geo.t.bk;
         s->pad_bm = geo.t.bm;
     }
-    hsgen_status st = upload_g(ctx, kp);
-    if (st) return st;
+    hsgen_status st;
     const SphereLayout l = sphere_layout(ctx, s, {ng}, do_h);
     if ((st = ensure(ctx, ctx->sph_ph, l.b_ph, false)) || (st = ensure(ctx, ctx->sph_rs, l.b_rs, false))) return st;
     if (do_h && ((st = ensure(ctx, ctx->sph_y, l.b_y, false)) || (st = ensure(ctx, ctx->sph_w, l.b_w, false)))) return st;
@@ -432,15 +431,11 @@ hsgen_status create_hs_sphere(hsgen_ctx* ctx, hsgen_sys* s, const hsgen_kpoint* 
     }
     SphereArgs p = sphere_args(s, l, ctx->sph_ph.p, ctx->sph_rs.p, do_h ? ctx->sph_y.p : nullptr,
                                do_h ? ctx->sph_w.p : nullptr);
-    p.one = sphere_ks(l, {kp}, {(const int32_t*)ctx->g.p}, {dH}, {dS}, {ldH}, {ldS})[0];
-    HIPCHK(hipEventRecord(ctx->ev[0], ctx->stream));
-    HIPCHK(sphere_launch(p, l, s, do_h, do_s, rep ? ctx->ev[1] : nullptr, rep ? ctx->ev[3] : nullptr, ctx->stream));
-    if (o.flags & HSGEN_FILL_UPPER) {
-        if (do_h) HIPCHK(launch_fill_upper(dH, ldH, ng, ctx->stream));
-        if (do_s) HIPCHK(launch_fill_upper(dS, ldS, ng, ctx->stream));
-    }
-    HIPCHK(hipEventRecord(ctx->ev[4], ctx->stream));
-    HIPCHK(hipEventSynchronize(ctx->ev[4]));
+    p.one = sphere_ks(l, {kp}, {nullptr}, {dH}, {dS}, {ldH}, {ldS})[0];
+    st = sphere_g(ctx, kp, nullptr, p.one);
+    if (st) return st;
+    st = sphere_run(ctx, s, l, p, o.flags, geo.cfg, rep);
+    if (st) return st;
     const bool full = (o.flags & HSGEN_FILL_UPPER) != 0;
     if (!hdev) {
         st = copy_lower_to_host(ctx, dH, ng, H, ld, full);
@@ -449,21 +444,6 @@ hsgen_status create_hs_sphere(hsgen_ctx* ctx, hsgen_sys* s, const hsgen_kpoint* 
     if (!sdev) {
         st = copy_lower_to_host(ctx, dS, ng, S, ld, full);
         if (st) return st;
-    }
-    if (rep) {
-        float t0 = 0, t1 = 0, t2 = 0;
-        HIPCHK(hipEventElapsedTime(&t0, ctx->ev[0], ctx->ev[1]));
-        HIPCHK(hipEventElapsedTime(&t1, ctx->ev[1], ctx->ev[3]));
-        HIPCHK(hipEventElapsedTime(&t2, ctx->ev[3], ctx->ev[4]));
-        rep->ms_abgen = t0;
-        rep->ms_tmul = t1;
-        rep->ms_contract = t2;
-        rep->ms_total = t0 + t1 + t2;
-        rep->ng = ng;
-        rep->kdim = s->kdim;
-        rep->flops_alg = 16.0 * (double)ng * ng * s->kdim + 32.0 * (double)ng * (double)s->sum_nlm2;
-        rep->bytes_abgen = sphere_gen_bytes(s) * ng;
-        rep->tile_used = geo.cfg;
     }
     return HSGEN_OK;
 }
@@ -616,7 +596,7 @@ hsgen_status batched_fp64(hsgen_ctx* ctx, hsgen_sys* s, int nk, const hsgen_kpoi
             p.many = (const SphereK*)bg.ks.p;
             // capture the launch sequence
             HIPCHK(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
-            hipError_t ce = sphere_launch(p, l, s, do_h, do_s, nullptr, nullptr, ctx->stream);
+            hipError_t ce = sphere_launch(p, l, s, do_h, do_s, nullptr, ctx->stream);
             for (size_t q = 0; q < ks.size() && ce == hipSuccess && (flags & HSGEN_FILL_UPPER); ++q) {
                 if (do_h) ce = launch_fill_upper(dH[q], ldH[q], kps[ks[q]].ng, ctx->stream);
                 if (ce == hipSuccess && do_s) ce = launch_fill_upper(dS[q], ldS[q], kps[ks[q]].ng, ctx->stream);

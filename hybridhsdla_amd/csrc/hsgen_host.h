@@ -55,6 +55,8 @@ constexpr int kFallbackTile = 8;   // register-staged, 64-bit addressing
 constexpr int kIgemmCfg = 51;      // default INT8 kernel configuration (256 x 192 tiles)
 constexpr int kBf16Cfg = 61;       // default BF16 kernel configuration (256 x 192 tiles)
 constexpr int kSampleTile = 12;    // FP64 tile of the split-precision sample: 64 x 64, so 64 columns
+constexpr int kPinnedG = 4096;     // plane waves of a G list that is read from pinned host memory
+constexpr size_t kPinStamps = 64;
 constexpr size_t kMaxOzGraphs = 16; // cached split-precision launch-segment sets per context
 
 struct DevBuf {
@@ -108,6 +110,11 @@ struct hsgen_ctx {
     // generalized eigensolver
     rocblas_handle blas = nullptr;
     hsgen::DevBuf eig_a, eig_b, eig_d;
+    // pinned buffer and its device address: kernel starts (kPinStamps bytes), then
+    // a short G list (kPinnedG plane waves)
+    void* pin = nullptr;
+    void* pin_dev = nullptr;
+    double ms_per_tick = 1e-5;                       // of the GPU's wall clock
     // pinned staging for device -> host copies of H and S
     void* stage[2] = {nullptr, nullptr};
     size_t stage_bytes = 0;
@@ -254,8 +261,11 @@ std::vector<SphereK> sphere_ks(const SphereLayout& l, const std::vector<const hs
                                const std::vector<const int32_t*>& gs, const std::vector<double2*>& H,
                                const std::vector<double2*>& S, const std::vector<int64_t>& ldH,
                                const std::vector<int64_t>& ldS);
+hsgen_status sphere_g(hsgen_ctx* ctx, const hsgen_kpoint* kp, int32_t* dev, SphereK& k);
 hipError_t sphere_launch(const SphereArgs& p, const SphereLayout& l, const hsgen_sys* s, bool do_h, bool do_s,
-                         hipEvent_t ev_gen, hipEvent_t ev_tapp, hipStream_t st);
+                         hipEvent_t stop, hipStream_t st);
+hsgen_status sphere_run(hsgen_ctx* ctx, const hsgen_sys* s, const SphereLayout& l, SphereArgs& p, int flags, int tile,
+                        hsgen_report* rep);
 hsgen_status sphere_split_setup(hsgen_ctx* ctx, hsgen_sys* s);
 hsgen_status sphere_split_w(hsgen_ctx* ctx, hsgen_sys* s, const std::vector<SphereK>& ks, const SphereK* ks_dev,
                             int64_t ncols, double2* W, int64_t ldw);

@@ -153,36 +153,9 @@ extern "C" hsgen_status hsgen_create_hs_noalloc(hsgen_ctx* ctx, const hsgen_sys*
     if (off > kScratchBytes)
         return fail(ctx, HSGEN_ERR_ARG, "N_G %d with K %d needs %zu bytes of scratch; the array has %zu", ng, s->kdim, off,
                     kScratchBytes);
-    const int32_t* dg = kp->g;
-    if (!gdev) {
-        HIPCHK(hipMemcpyAsync(base + o_g, kp->g, sizeof(int32_t) * 3 * (size_t)ng, hipMemcpyHostToDevice,
-                              ctx->stream));
-        dg = (const int32_t*)(base + o_g);
-    }
     SphereArgs p = sphere_args(s, l, base + o_ph, base + o_rs, do_h ? base + o_y : nullptr, do_h ? base + o_w : nullptr);
-    p.one = sphere_ks(l, {kp}, {dg}, {(double2*)H}, {(double2*)S}, {ld}, {ld})[0];
-    HIPCHK(hipEventRecord(ctx->ev[0], ctx->stream));
-    HIPCHK(sphere_launch(p, l, s, do_h, do_s, ctx->ev[1], ctx->ev[3], ctx->stream));
-    if (o.flags & HSGEN_FILL_UPPER) {
-        if (do_h) HIPCHK(launch_fill_upper((double2*)H, ld, ng, ctx->stream));
-        if (do_s) HIPCHK(launch_fill_upper((double2*)S, ld, ng, ctx->stream));
-    }
-    HIPCHK(hipEventRecord(ctx->ev[4], ctx->stream));
-    HIPCHK(hipEventSynchronize(ctx->ev[4]));
-    if (rep) {
-        float t0 = 0, t1 = 0, t2 = 0;
-        HIPCHK(hipEventElapsedTime(&t0, ctx->ev[0], ctx->ev[1]));
-        HIPCHK(hipEventElapsedTime(&t1, ctx->ev[1], ctx->ev[3]));
-        HIPCHK(hipEventElapsedTime(&t2, ctx->ev[3], ctx->ev[4]));
-        rep->ms_abgen = t0;
-        rep->ms_tmul = t1;
-        rep->ms_contract = t2;
-        rep->ms_total = t0 + t1 + t2;
-        rep->ng = ng;
-        rep->kdim = s->kdim;
-        rep->flops_alg = 16.0 * (double)ng * ng * s->kdim + 32.0 * (double)ng * (double)s->sum_nlm2;
-        rep->bytes_abgen = sphere_gen_bytes(s) * ng;
-        rep->tile_used = geo.cfg;
-    }
-    return HSGEN_OK;
+    p.one = sphere_ks(l, {kp}, {nullptr}, {(double2*)H}, {(double2*)S}, {ld}, {ld})[0];
+    st = sphere_g(ctx, kp, gdev ? nullptr : (int32_t*)(base + o_g), p.one);
+    if (st) return st;
+    return sphere_run(ctx, s, l, p, o.flags, geo.cfg, rep);
 }

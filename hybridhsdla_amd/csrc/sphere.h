@@ -53,7 +53,8 @@ struct OverlapGroup {
 // One k-point of a launch.
 struct SphereK {
     double k[3];
-    const int32_t* g;    // [ng][3], device memory
+    const int32_t* g;    // [ng][3], device or pinned host memory: read by the generator
+    int32_t* gd;         // device copy of g that the generator makes, or g itself: read by S
     double2* H;
     double2* S;
     int64_t ldH, ldS;
@@ -121,17 +122,21 @@ struct SphereArgs {
     const SphereStage* stages;
     int32_t nksteps;
     int32_t nsquares;          // lower squares of H tiles of all k-points
+    uint64_t* stamp;           // starts of the generator, T application, H and S kernels (wall clock), or null
 };
 
+// Launchers; stop: null, or an event that takes the kernel's end.
 int sphere_chunk(int nl, int L);
 hipError_t launch_split_mt(const SplitMtJob* jobs, int njobs, int64_t max_elems, const double* sq, const double2* mt,
                            double2* out, hipStream_t st);
 hipError_t launch_build_mt(const MtJob* jobs, int njobs, int64_t max_elems, double2* mt, hipStream_t st);
-hipError_t launch_sphere_gen(const SphereArgs& p, hipStream_t st);
+hipError_t launch_sphere_gen(const SphereArgs& p, hipEvent_t stop, hipStream_t st);
+hipError_t launch_sphere_tapp(const SphereArgs& p, int tile, int rtiles, hipEvent_t stop, hipStream_t st);
+hipError_t launch_sphere_h(const SphereArgs& p, int tile, hipEvent_t stop, hipStream_t st);
 // S tile side by the number of lower tiles; the bits do not depend on it
-int overlap_tile(int64_t tiles64, int n_cu);
-hipError_t launch_sphere_tapp(const SphereArgs& p, int tile, int rtiles, hipStream_t st);
-hipError_t launch_sphere_h(const SphereArgs& p, int tile, hipStream_t st);
-hipError_t launch_overlap(const SphereArgs& p, int tile, int64_t ntiles, hipStream_t st);
+int overlap_tile_size(int64_t tiles64, int n_cu);
+hipError_t launch_overlap(const SphereArgs& p, int tile, int64_t ntiles, hipEvent_t stop, hipStream_t st);
+// H tiles of 32 x 32 and S tiles of 16 or 32 in one launch
+hipError_t launch_sphere_hs(const SphereArgs& p, int stile, int64_t nstiles, hipEvent_t stop, hipStream_t st);
 
 }  // namespace hsgen

@@ -1,7 +1,10 @@
 // FP64 kernels of the path from a system description to H and S that use the
 // form of the matching coefficients: a phase per atom times real numbers that
 // atoms of one kind share (sphere.h).
+#include <algorithm>
 #include <type_traits>
+
+#include <hip/hip_ext.h>
 
 #include "sphere.h"
 #include "sphere_dev.h"
@@ -9,6 +12,30 @@
 namespace hsgen {
 
 namespace {
+
+// Launch, with the event that the call waits for attached to the kernel itself.
+template <class... A>
+hipError_t launch(void (*k)(A...), dim3 grid, int threads, size_t lds, hipEvent_t stop, hipStream_t st, A... args)
+{
+    if (grid.x == 0) return hipSuccess;
+    if (lds > 64 * 1024) {
+        // per launch: the attribute is per device
+        const hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) return e;
+    }
+    if (stop)
+        hipExtLaunchKernelGGL(k, grid, dim3(threads), lds, st, nullptr, stop, 0, args...);
+    else
+        hipLaunchKernelGGL(k, grid, dim3(threads), lds, st, args...);
+    return hipGetLastError();
+}
+
+// The kernel's start, by its first workgroup, for the report: events between
+// the kernels of a call cost 5 us each.
+__device__ __forceinline__ void stamp(const SphereArgs& p, int which)
+{
+    if (p.stamp && blockIdx.x == 0 && threadIdx.x == 0) p.stamp[which] = (uint64_t)wall_clock64();
+}
 
 // Largest i in [0, n) with key(i) <= v; key ascending, key(0) <= v.
 template <class Key>
@@ -31,6 +58,17 @@ __device__ __forceinline__ int tri_row(int t)
     while ((int64_t)r * (r + 1) / 2 > t) --r;
     return r;
 }
+
+struct Reciprocals {
+    double v[kMaxLmax + 1];
+};
+constexpr Reciprocals reciprocals()
+{
+    Reciprocals r{};
+    for (int i = 1; i <= kMaxLmax; ++i) r.v[i] = 1.0 / i;
+    return r;
+}
+__constant__ const Reciprocals kReciprocal = reciprocals();
 
 // Real harmonics of one m >= 0 by the ylm4 recurrences (ylm4.f:194-217):
 // Y_l0, and for m > 0 Re and Im of Y_lm at l(l+1)+m and l(l+1)-m, so that
@@ -63,7 +101,13 @@ __device__ inline void ylm_real(int m, int lmax, const DirAngles& dir, const dou
         double pv;
         if (l == m) pv = fac;
         else if (l == m + 1) pv = (m + m + 1) * dir.cth * fac;
-        else pv = ((l + l - 1) * dir.cth * pl1 - (l + m - 1) * pl2) / (l - m);
+        else {
+            // divided by l - m: the product with its reciprocal, corrected
+            const double num = (l + l - 1) * dir.cth * pl1 - (l + m - 1) * pl2;
+            const double rec = kReciprocal.v[l - m];
+            pv = num * rec;
+            pv = __builtin_fma(__builtin_fma(-(double)(l - m), pv, num), rec, pv);
+        }
         if (l > m) {
             pl2 = pl1;
             pl1 = pv;
@@ -88,9 +132,11 @@ __device__ inline void ylm_real(int m, int lmax, const DirAngles& dir, const dou
 // harmonics (one lane per kind and m) and, with y, the real vectors
 // [a_l Y_lm; b_l Y_lm].
 // ---------------------------------------------------------------------------
+template <bool kSplit>
 __global__ __launch_bounds__(256) void k_sphere_gen(SphereArgs p)
 {
     extern __shared__ double smem[];
+    stamp(p, 0);
     const int tid = threadIdx.x;
     const int nl = p.nl;
     const int L = p.L;
@@ -99,29 +145,25 @@ __global__ __launch_bounds__(256) void k_sphere_gen(SphereArgs p)
     double* s_y = (double*)(s_ab + p.chunk * nl);      // [chunk][L]     real harmonics
     DirAngles* s_dir = (DirAngles*)(s_y + p.chunk * L);     // [chunk]
     unsigned char* s_l = (unsigned char*)(s_dir + p.chunk); // [L]       l of lm
-    const int c = blockIdx.x;
-    const SphereK* kp = &p.one;
-    int gi;
-    int64_t col;
-    if (p.rowdst) {
-        // every column of the chunk, padding as zeros
-        const int at = (int)p.cbase + c;
-        if (p.nk > 1) kp = p.many + find_last(p.nk, at, [&](int i) { return (int)p.many[i].col0; });
-        gi = at - (int)kp->col0;
-        col = c;
-        if (gi >= kp->ng) {
-            for (int64_t r = tid; r < p.ldy; r += blockDim.x) p.y[col * p.ldy + r] = 0.0;
-            for (int a = tid; a < p.natoms; a += blockDim.x) p.ph[(int64_t)a * p.gtot + col] = make_double2(0.0, 0.0);
-            return;
-        }
-    } else {
-        if (p.nk > 1) kp = p.many + find_last(p.nk, c, [&](int i) { return p.many[i].gcol0; });
-        gi = c - kp->gcol0;
-        col = kp->col0 + gi;
+    // the k-point and the plane wave: every column of the chunk, padding as
+    // zeros (kSplit), or the plane waves of all k-points
+    const int c = kSplit ? (int)p.cbase + (int)blockIdx.x : (int)blockIdx.x;
+    int ki = 0;
+    if (p.nk > 1)
+        ki = find_last(p.nk, c, [&](int i) { return kSplit ? (int)p.many[i].col0 : p.many[i].gcol0; });
+    const SphereK k = p.nk > 1 ? p.many[ki] : p.one;
+    const int gi = c - (kSplit ? (int)k.col0 : k.gcol0);
+    const int64_t col = kSplit ? blockIdx.x : k.col0 + gi;
+    if (kSplit && gi >= k.ng) {
+        for (int64_t r = tid; r < p.ldy; r += blockDim.x) p.y[col * p.ldy + r] = 0.0;
+        for (int a = tid; a < p.natoms; a += blockDim.x) p.ph[(int64_t)a * p.gtot + col] = make_double2(0.0, 0.0);
+        return;
     }
-    const double K0 = kp->k[0] + kp->g[3 * gi + 0];
-    const double K1 = kp->k[1] + kp->g[3 * gi + 1];
-    const double K2 = kp->k[2] + kp->g[3 * gi + 2];
+    const int g0 = k.g[3 * gi + 0], g1 = k.g[3 * gi + 1], g2 = k.g[3 * gi + 2];
+    if (!kSplit && k.gd != k.g && tid < 3) k.gd[3 * gi + tid] = tid == 0 ? g0 : tid == 1 ? g1 : g2;
+    const double K0 = k.k[0] + g0;
+    const double K1 = k.k[1] + g1;
+    const double K2 = k.k[2] + g2;
     const double c0 = p.bmat[0] * K0 + p.bmat[3] * K1 + p.bmat[6] * K2;
     const double c1 = p.bmat[1] * K0 + p.bmat[4] * K1 + p.bmat[7] * K2;
     const double c2 = p.bmat[2] * K0 + p.bmat[5] * K1 + p.bmat[8] * K2;
@@ -158,10 +200,11 @@ __global__ __launch_bounds__(256) void k_sphere_gen(SphereArgs p)
             const double bu = -m.u * Knorm * dfj[l] + m.u_dr * fj[l];
             const double2 ab = make_double2(pref * au, pref * bu);
             s_ab[t * nl + l] = ab;
-            if (kd.rsoff >= 0 && p.rs) p.rs[col * p.ldr + kd.rsoff + l] = ab;
+            if (!kSplit && kd.rsoff >= 0) p.rs[col * p.ldr + kd.rsoff + l] = ab;
         }
         if (p.y) {
-            for (int q = tid; q < nk * nl; q += blockDim.x) {
+            // from the other end: the first waves have the radial factors
+            for (int q = blockDim.x - 1 - tid; q < nk * nl; q += blockDim.x) {
                 const int t = q / nl;
                 const int m = q - t * nl;
                 if (m <= p.kinds[k0 + t].lmax) ylm_real(m, p.kinds[k0 + t].lmax, s_dir[t], p.ynorm, s_y + t * L);
@@ -196,12 +239,10 @@ int sphere_chunk(int nl, int L)
     return chunk;
 }
 
-hipError_t launch_sphere_gen(const SphereArgs& p, hipStream_t st)
+hipError_t launch_sphere_gen(const SphereArgs& p, hipEvent_t stop, hipStream_t st)
 {
-    if (p.ngcols <= 0) return hipSuccess;
     const size_t lds = sphere_gen_lds(p.chunk, p.nl, p.L);
-    hipLaunchKernelGGL(k_sphere_gen, dim3(p.ngcols), dim3(256), lds, st, p);
-    return hipGetLastError();
+    return launch(p.rowdst ? k_sphere_gen<true> : k_sphere_gen<false>, dim3(p.ngcols), 256, lds, stop, st, p);
 }
 
 // ---------------------------------------------------------------------------
@@ -238,12 +279,11 @@ constexpr LegendreCoef legendre_coef()
 __constant__ const LegendreCoef kLegendre = legendre_coef();
 
 template <int M, int MJ>
-__global__ __launch_bounds__(256 * M / MJ) void k_overlap(SphereArgs p)
+__device__ __forceinline__ void overlap_tile(const SphereArgs& p, int blk, double* smem)
 {
     // one rounding per written operation: every tile gives the same bits
 #pragma clang fp contract(off)
     constexpr int T = 16 * M, TY = T / MJ, NT = 16 * TY;
-    extern __shared__ double smem[];
     double2* s_ri = (double2*)smem;               // [nl][T] (a_l, b_l) of the rows
     double2* s_rj = s_ri + p.nl * T;              // [nl][T] weighted, of the columns
     double2* s_pi = s_rj + p.nl * T;              // [kOvAtoms][T] phases
@@ -253,8 +293,8 @@ __global__ __launch_bounds__(256 * M / MJ) void k_overlap(SphereArgs p)
     const int tid = threadIdx.x;
     const int tx = tid & 15, ty = tid >> 4;
     const SphereK* kp = &p.one;
-    if (p.nk > 1) kp = p.many + find_last(p.nk, (int)blockIdx.x, [&](int i) { return p.many[i].stile0; });
-    const int tile = (int)blockIdx.x - kp->stile0;
+    if (p.nk > 1) kp = p.many + find_last(p.nk, blk, [&](int i) { return p.many[i].stile0; });
+    const int tile = blk - kp->stile0;
     const int bi = tri_row(tile);
     const int bj = tile - (int)((int64_t)bi * (bi + 1) / 2);
     const int I0 = bi * T, J0 = bj * T;
@@ -292,8 +332,8 @@ __global__ __launch_bounds__(256 * M / MJ) void k_overlap(SphereArgs p)
         if (newdir && tid < 2 * T) {
             const int side = tid / T, c = tid - side * T;
             const int gi = min((side ? J0 : I0) + c, ng - 1);
-            const DirAngles d = dir_angles(kd.rot, kp->k[0] + kp->g[3 * gi], kp->k[1] + kp->g[3 * gi + 1],
-                                           kp->k[2] + kp->g[3 * gi + 2]);
+            const DirAngles d = dir_angles(kd.rot, kp->k[0] + kp->gd[3 * gi], kp->k[1] + kp->gd[3 * gi + 1],
+                                           kp->k[2] + kp->gd[3 * gi + 2]);
             double* s = s_n + side * 3 * T + c;
             s[0] = d.sth * d.cph;
             s[T] = d.sth * d.sph;
@@ -414,7 +454,15 @@ __global__ __launch_bounds__(256 * M / MJ) void k_overlap(SphereArgs p)
         }
 }
 
-int overlap_tile(int64_t tiles64, int n_cu)
+template <int M, int MJ>
+__global__ __launch_bounds__(256 * M / MJ) void k_overlap(SphereArgs p)
+{
+    extern __shared__ double smem[];
+    stamp(p, 3);
+    overlap_tile<M, MJ>(p, (int)blockIdx.x, smem);
+}
+
+int overlap_tile_size(int64_t tiles64, int n_cu)
 {
     // 64 x 64 tiles once they give every CU four workgroups, 32 x 32 once
     // those give two, else 16 x 16: a smaller tile reads its columns more often but
@@ -423,22 +471,19 @@ int overlap_tile(int64_t tiles64, int n_cu)
     return 4 * tiles64 >= 2 * (int64_t)n_cu ? 32 : 16;
 }
 
-hipError_t launch_overlap(const SphereArgs& p, int tile, int64_t ntiles, hipStream_t st)
+static size_t overlap_lds(int tile, int nl)
+{
+    return sizeof(double2) * (size_t)tile * 2 * (nl + kOvAtoms) + sizeof(double) * 6 * tile;
+}
+
+hipError_t launch_overlap(const SphereArgs& p, int tile, int64_t ntiles, hipEvent_t stop, hipStream_t st)
 {
     if (ntiles <= 0) return hipSuccess;
-    const size_t lds = sizeof(double2) * (size_t)tile * 2 * (p.nl + kOvAtoms) + sizeof(double) * 6 * tile;
-    const dim3 grid((unsigned)ntiles), block(tile == 64 ? 512 : 256);
-    if (tile == 64) {
-        const hipError_t e =
-            hipFuncSetAttribute((const void*)(k_overlap<4, 2>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return e;
-        hipLaunchKernelGGL((k_overlap<4, 2>), grid, block, lds, st, p);
-    } else if (tile == 32) {
-        hipLaunchKernelGGL((k_overlap<2, 2>), grid, block, lds, st, p);
-    } else {
-        hipLaunchKernelGGL((k_overlap<1, 1>), grid, block, lds, st, p);
-    }
-    return hipGetLastError();
+    const size_t lds = overlap_lds(tile, p.nl);
+    const dim3 grid((unsigned)ntiles);
+    if (tile == 64) return launch(k_overlap<4, 2>, grid, 512, lds, stop, st, p);
+    if (tile == 32) return launch(k_overlap<2, 2>, grid, 256, lds, stop, st, p);
+    return launch(k_overlap<1, 1>, grid, 256, lds, stop, st, p);
 }
 
 // ---------------------------------------------------------------------------
@@ -605,7 +650,14 @@ hipError_t launch_split_mt(const SplitMtJob* jobs, int njobs, int64_t max_elems,
 // the phases of an atom that ends in it, so that no flush waits for memory;
 // LDS addresses are constants per lane and load bases scalar, which leaves the
 // vector pipe to the MFMAs.  Rings of 3 and 4 stages, 64 x 128 tiles and waves
-// of 32 x 32 measured no faster at any size from 235 to 25000 plane waves.
+// of 32 x 32 measured no faster for these tiles at any size from 235 to 25000
+// plane waves.
+// The 32 x 32 tiles of H serve triangles that leave CUs idle, with two or three
+// waves per SIMD: there the latency of a stage counts.  Four stages in LDS, the
+// fragments of a whole stage read while the one before is multiplied, table
+// entries two barriers ahead: H and S together 21.3 us (two stages 26.9) at
+// N_G 600, 12.5 (13.7) at 235, 1105 (1121) at 2003; the T application, with
+// depths of 10 to 20 stages, gained nothing.
 // Rate of the H tiles: 0.87 of the FP64 peak at N_G 16000 and 25000, 0.85 at
 // 10000, 0.82 at 6002 (32 atoms, lmax 10).
 // Measured (whole call, complex-by-complex contraction of S and H before, now):
@@ -619,9 +671,13 @@ typedef double v2d __attribute__((ext_vector_type(2)));
 typedef int i8 __attribute__((ext_vector_type(8)));
 typedef __attribute__((address_space(4))) const i8* ctab;
 
-// s_waitcnt immediates (vmcnt bits [3:0] and [15:14], expcnt [6:4], lgkmcnt [11:8])
-constexpr int kWaitVm0 = (0 & 15) | (7 << 4) | (15 << 8);
-constexpr int kWaitVm0Lgkm0 = (0 & 15) | (7 << 4) | (0 << 8);
+// s_waitcnt immediate: at most n vector-memory operations outstanding and, with
+// lgkm, no LDS or scalar ones (vmcnt bits [3:0] and [15:14], expcnt [6:4],
+// lgkmcnt [11:8]).
+constexpr int wait_vm(int n, bool lgkm)
+{
+    return (n & 15) | (7 << 4) | ((lgkm ? 0 : 15) << 8) | ((n >> 4) << 14);
+}
 
 // Atoms that end in a stage before its k-step ks.
 __device__ __forceinline__ int ends_before(i8 e, int ks)
@@ -631,8 +687,9 @@ __device__ __forceinline__ int ends_before(i8 e, int ks)
 
 }  // namespace
 
-// BR x BC tile (rows: X columns, columns: y columns), waves of 16 RB x 16 CB.
-template <int BR, int BC, int RB, int CB>
+// BR x BC tile (rows: X columns, columns: y columns), waves of 16 RB x 16 CB,
+// NS stages in LDS.
+template <int BR, int BC, int RB, int CB, int NS>
 struct SphereTile {
     static constexpr int kWR = BR / (16 * RB);    // waves along the rows
     static constexpr int kWC = BC / (16 * CB);
@@ -642,7 +699,7 @@ struct SphereTile {
     static constexpr int kYBytes = BC * 128;
     static constexpr int kPhBytes = 256 * CB;     // a wave's phases of an atom that ends in a stage
     static constexpr int kStage = kXBytes + kYBytes + kWaves * kPhBytes;
-    static constexpr int kLds = 2 * kStage;
+    static constexpr int kLds = NS * kStage;
     static constexpr int kXLoads = kXBytes / 1024 / kWaves;   // 1 KiB wave loads per wave and stage
     static constexpr int kYLoads = kYBytes / 1024 / kWaves;
     static_assert(kXLoads * kWaves * 1024 == kXBytes && kYLoads * kWaves * 1024 == kYBytes,
@@ -657,13 +714,12 @@ __device__ __forceinline__ int64_t uni(int64_t v)
     return (int64_t)(((uint64_t)(uint32_t)uni((int)(v >> 32)) << 32) | (uint32_t)uni((int)v));
 }
 
-template <int BR, int BC, int RB, int CB, bool kH>
-__global__ __launch_bounds__((SphereTile<BR, BC, RB, CB>::kThreads), 4) void k_sphere_gemm(SphereArgs p)
+template <int BR, int BC, int RB, int CB, int NS, bool kH>
+__device__ __forceinline__ void sphere_gemm_tile(const SphereArgs& p, int blk, char* lds)
 {
 #pragma clang fp contract(off)
-    using Tl = SphereTile<BR, BC, RB, CB>;
+    using Tl = SphereTile<BR, BC, RB, CB, NS>;
     constexpr int NX = Tl::kXLoads, NY = Tl::kYLoads;
-    extern __shared__ __attribute__((aligned(1024))) char lds[];
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -682,7 +738,7 @@ __global__ __launch_bounds__((SphereTile<BR, BC, RB, CB>::kThreads), 4) void k_s
         constexpr int kRat = BC / BR;
         constexpr int P = kSpherePatch;
         const int n = p.nsquares * kRat;
-        const int x = (int)blockIdx.x % 8, at = (int)blockIdx.x / 8;
+        const int x = blk % 8, at = blk / 8;
         const int t0 = (int)((int64_t)n * x / 8), t1 = (int)((int64_t)n * (x + 1) / 8);
         if (at >= t1 - t0) return;
         const int sq = (t0 + at) / kRat;
@@ -710,11 +766,11 @@ __global__ __launch_bounds__((SphereTile<BR, BC, RB, CB>::kThreads), 4) void k_s
     } else {
         // kinds in turn; per kind its tiles of rows, per row tile all columns
         const int ntc = (int)(p.gtot / BC);
-        const int tr = (int)blockIdx.x / ntc;
+        const int tr = blk / ntc;
         const int kk = find_last(p.nkinds, tr, [&](int i) { return p.kinds[i].rt32; });
         kd = p.kinds + kk;
         R0 = uni((tr - kd->rt32) * BR);
-        C0 = uni(((int)blockIdx.x - tr * ntc) * BC);
+        C0 = uni((blk - tr * ntc) * BC);
         nsteps = uni(kd->r4 / 4);
     }
     const int64_t col0 = kH ? uni(kp->col0) : 0;
@@ -765,7 +821,8 @@ __global__ __launch_bounds__((SphereTile<BR, BC, RB, CB>::kThreads), 4) void k_s
     typedef __attribute__((address_space(1))) const char gchar;
     typedef __attribute__((address_space(3))) char lchar;
     lchar* lbase = (lchar*)lds;
-    // one stage: the phases of the first atom that ends in it, X, y
+    // one stage: the phases of the first atom that ends in it, X, y (the wait
+    // for a stage counts the X and y loads of the stages after it)
     auto issue = [&](int s, int buf, i8 e) {
         if constexpr (kH) {
             if (e[4] >= 0 && lane < 16 * CB) {
@@ -831,20 +888,20 @@ __global__ __launch_bounds__((SphereTile<BR, BC, RB, CB>::kThreads), 4) void k_s
 #pragma unroll
         for (int j = 0; j < CB; ++j) y[j] = *(const double*)&lds[yat[ks] + (buf * Tl::kStage + j * 2048)];
     };
+    const int phat = Tl::kXBytes + Tl::kYBytes + wave * Tl::kPhBytes + (lane & 15) * 16;
     // Phases at this lane's H rows: of the first atom that ends in a stage,
     // from the stage; of further ones (atoms of few rows) from memory.
-    auto stage_phases = [&](int buf, double2* ph) {
+    auto stage_phases = [&](int buf, v2d* ph) {
 #pragma unroll
         for (int j = 0; j < CB; ++j)
-            ph[j] = *(const double2*)&lds[buf * Tl::kStage + Tl::kXBytes + Tl::kYBytes + wave * Tl::kPhBytes +
-                                          (lane & 15) * 16 + j * 256];
+            ph[j] = *(const v2d*)&lds[phat + (buf * Tl::kStage + j * 256)];
     };
-    auto far_phases = [&](int atom, double2* ph) {
+    auto far_phases = [&](int atom, v2d* ph) {
 #pragma unroll
-        for (int j = 0; j < CB; ++j) ph[j] = p.ph[(int64_t)atom * p.gtot + (col0 + C0 + c0 + 16 * j)];
+        for (int j = 0; j < CB; ++j) ph[j] = *(const v2d*)&p.ph[(int64_t)atom * p.gtot + (col0 + C0 + c0 + 16 * j)];
     };
     // C += conj(phase) T, T = 0
-    auto flush = [&](const double2* ph) {
+    auto flush = [&](const v2d* ph) {
 #pragma unroll
         for (int i = 0; i < RB; ++i)
 #pragma unroll
@@ -862,72 +919,136 @@ __global__ __launch_bounds__((SphereTile<BR, BC, RB, CB>::kThreads), 4) void k_s
     // ---- main loop ----
     // (at the end the last stage is loaded again: in bounds, unused)
     const int last = nst - 1;
-    i8 en[2] = {entry(0), entry(min(1, last))};     // stage s's entries in en[s % 2]
-    issue(0, 0, en[0]);
-    __builtin_amdgcn_s_waitcnt(kWaitVm0);
+    // one k-step: T += X y; rows past the depth (in the last stage) are not
+    // multiplied
+    auto mfmas = [&](int s, int ks, const v2d* x, const double* y) {
+        if (kH || 4 * s + ks < nsteps) {
+#pragma unroll
+            for (int i = 0; i < RB; ++i)
+#pragma unroll
+                for (int j = 0; j < CB; ++j)
+                    tr_[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[i].x, y[j], tr_[i][j], 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < RB; ++i)
+#pragma unroll
+                for (int j = 0; j < CB; ++j)
+                    ti_[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[i].y, y[j], ti_[i][j], 0, 0, 0);
+        }
+    };
+    i8 en[NS];              // stage s's entries in en[s % NS]
+#pragma unroll
+    for (int i = 0; i < NS; ++i) en[i] = entry(min(i, last));
+#pragma unroll
+    for (int i = 0; i + 1 < NS; ++i) issue(min(i, last), i, en[i]);
+    __builtin_amdgcn_s_waitcnt(wait_vm((NS - 2) * (NX + NY), false));
     asm volatile("s_barrier" ::: "memory");
-    issue(min(1, last), 1, en[1]);
-    v2d fx[RB];
-    double fy[CB];
-    read_frags(0, 0, fx, fy);
-    // stage s from LDS buffer `buf`
-    auto stage = [&](auto bufc, int s) {
-        constexpr int buf = decltype(bufc)::value;
-        const i8 e = en[buf];
-        const i8 e2 = entry(min(s + 2, last));
+    issue(min(NS - 1, last), NS - 1, en[NS - 1]);
+    if constexpr (NS > 2) {
+        // Few waves per SIMD: the fragments (and phases) of a whole stage are
+        // read while the one before is multiplied, three stages of loads in
+        // flight behind it.
+        v2d fx[2][4][RB];
+        double fy[2][4][CB];
+        v2d fp[2][CB];
+        auto read_stage = [&](int buf, int set) {
 #pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-            v2d x[RB];
-            double y[CB];
-#pragma unroll
-            for (int i = 0; i < RB; ++i) x[i] = fx[i];
-#pragma unroll
-            for (int j = 0; j < CB; ++j) y[j] = fy[j];
-            double2 ph[CB];
-            if (ks < 3) {
-                read_frags(buf, ks + 1, fx, fy);
-            } else if (s < last) {
-                // an atom that ends with the stage still needs its phases
-                if (kH && (e[3] & 3) == 1) stage_phases(buf, ph);
+            for (int ks = 0; ks < 4; ++ks) read_frags(buf, ks, fx[set][ks], fy[set][ks]);
+            if constexpr (kH) stage_phases(buf, fp[set]);
+        };
+        read_stage(0, 0);
+        i8 next = entry(min(NS, last));     // the entry of the stage issued next
+        auto stage = [&](auto bufc, int s) {
+            constexpr int buf = decltype(bufc)::value, set = buf & 1;
+            const i8 e = en[buf];
+            __builtin_amdgcn_s_waitcnt(wait_vm(63, true));
+            if (s < last) {
                 // this wave's loads of stage s+1 landed and its reads of stage
                 // s are done; after the barrier that holds for every wave, and
-                // stage s+2 may overwrite stage s
-                __builtin_amdgcn_s_waitcnt(kWaitVm0Lgkm0);
+                // stage s+NS may overwrite stage s
+                __builtin_amdgcn_s_waitcnt(wait_vm((NS - 2) * (NX + NY), false));
                 asm volatile("s_barrier" ::: "memory");
-                issue(min(s + 2, last), buf, e2);
-                read_frags(buf ^ 1, 0, fx, fy);
+                issue(min(s + NS, last), buf, next);
+                en[buf] = next;
+                next = entry(min(s + NS + 1, last));
+                read_stage((buf + 1) % NS, set ^ 1);
             }
-            // reads ahead of the MFMAs, as written
             __builtin_amdgcn_sched_barrier(0);
-            // rows past the depth (in the last stage) are not multiplied
-            if (kH || 4 * s + ks < nsteps) {
 #pragma unroll
-                for (int i = 0; i < RB; ++i)
+            for (int ks = 0; ks < 4; ++ks) {
+                mfmas(s, ks, fx[set][ks], fy[set][ks]);
+                if constexpr (kH) {
+                    if (e[ks] & 1) {
+                        v2d ph[CB];
+                        if (e[ks] & 2) {
+                            far_phases(e[4] + ends_before(e, ks), ph);
+                        } else {
 #pragma unroll
-                    for (int j = 0; j < CB; ++j)
-                        tr_[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[i].x, y[j], tr_[i][j], 0, 0, 0);
-#pragma unroll
-                for (int i = 0; i < RB; ++i)
-#pragma unroll
-                    for (int j = 0; j < CB; ++j)
-                        ti_[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[i].y, y[j], ti_[i][j], 0, 0, 0);
-            }
-            if constexpr (kH) {
-                if (e[ks] & 1) {
-                    if (e[ks] & 2) far_phases(e[4] + ends_before(e, ks), ph);
-                    else if (ks < 3 || s == last) stage_phases(buf, ph);
-                    flush(ph);
+                            for (int j = 0; j < CB; ++j) ph[j] = fp[set][j];
+                        }
+                        flush(ph);
+                    }
                 }
             }
+        };
+        int s = 0;
+        for (; s + NS <= nst; s += NS) {
+            stage(std::integral_constant<int, 0>{}, s);
+            stage(std::integral_constant<int, 1>{}, s + 1);
+            stage(std::integral_constant<int, 2>{}, s + 2);
+            stage(std::integral_constant<int, 3>{}, s + 3);
         }
-        en[buf] = e2;
-    };
-    int s = 0;
-    for (; s < last; s += 2) {
-        stage(std::integral_constant<int, 0>{}, s);
-        stage(std::integral_constant<int, 1>{}, s + 1);
+        if (s < nst) stage(std::integral_constant<int, 0>{}, s);
+        if (s + 1 < nst) stage(std::integral_constant<int, 1>{}, s + 1);
+        if (s + 2 < nst) stage(std::integral_constant<int, 2>{}, s + 2);
+    } else {
+        v2d fx[RB];
+        double fy[CB];
+        read_frags(0, 0, fx, fy);
+        // stage s from LDS buffer `buf`
+        auto stage = [&](auto bufc, int s) {
+            constexpr int buf = decltype(bufc)::value;
+            const i8 e = en[buf];
+            const i8 e2 = entry(min(s + 2, last));
+#pragma unroll
+            for (int ks = 0; ks < 4; ++ks) {
+                v2d x[RB];
+                double y[CB];
+#pragma unroll
+                for (int i = 0; i < RB; ++i) x[i] = fx[i];
+#pragma unroll
+                for (int j = 0; j < CB; ++j) y[j] = fy[j];
+                v2d ph[CB];
+                if (ks < 3) {
+                    read_frags(buf, ks + 1, fx, fy);
+                } else if (s < last) {
+                    // an atom that ends with the stage still needs its phases
+                    if (kH && (e[3] & 3) == 1) stage_phases(buf, ph);
+                    // as above, with two stages
+                    __builtin_amdgcn_s_waitcnt(wait_vm(0, true));
+                    asm volatile("s_barrier" ::: "memory");
+                    issue(min(s + 2, last), buf, e2);
+                    read_frags(buf ^ 1, 0, fx, fy);
+                }
+                // reads ahead of the MFMAs, as written
+                __builtin_amdgcn_sched_barrier(0);
+                mfmas(s, ks, x, y);
+                if constexpr (kH) {
+                    if (e[ks] & 1) {
+                        if (e[ks] & 2) far_phases(e[4] + ends_before(e, ks), ph);
+                        else if (ks < 3 || s == last) stage_phases(buf, ph);
+                        flush(ph);
+                    }
+                }
+            }
+            en[buf] = e2;
+        };
+        int s = 0;
+        for (; s < last; s += 2) {
+            stage(std::integral_constant<int, 0>{}, s);
+            stage(std::integral_constant<int, 1>{}, s + 1);
+        }
+        if (s < nst) stage(std::integral_constant<int, 0>{}, s);
     }
-    if (s < nst) stage(std::integral_constant<int, 0>{}, s);
     __builtin_amdgcn_s_waitcnt(0);
 
     // ---- store: lane holds rows (lane >> 4) + 4 q of column lane & 15 ----
@@ -969,36 +1090,61 @@ __global__ __launch_bounds__((SphereTile<BR, BC, RB, CB>::kThreads), 4) void k_s
     }
 }
 
-template <int BR, int BC, int RB, int CB, bool kH>
-static hipError_t launch_sphere_gemm(const SphereArgs& p, int64_t nblk, hipStream_t st)
+template <int BR, int BC, int RB, int CB, int NS, bool kH>
+__global__ __launch_bounds__((SphereTile<BR, BC, RB, CB, NS>::kThreads), 4) void k_sphere_gemm(SphereArgs p)
 {
-    if (nblk <= 0) return hipSuccess;
-    using Tl = SphereTile<BR, BC, RB, CB>;
-    constexpr int lds = Tl::kLds;
-    auto* k = k_sphere_gemm<BR, BC, RB, CB, kH>;
-    if (lds > 64 * 1024) {
-        /* per launch: the attribute is per device */
-        const hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-        if (e != hipSuccess) return e;
-    }
-    hipLaunchKernelGGL(k, dim3((unsigned)nblk), dim3(Tl::kThreads), lds, st, p);
-    return hipGetLastError();
+    extern __shared__ __attribute__((aligned(1024))) char lds[];
+    stamp(p, kH ? 2 : 1);
+    sphere_gemm_tile<BR, BC, RB, CB, NS, kH>(p, (int)blockIdx.x, lds);
+}
+
+// H tiles of 32 x 32 and S tiles of 16 M x 16 M in one launch, for triangles
+// whose H tiles leave CUs or the vector pipe idle: S costs no time of its own.
+template <int M>
+__global__ __launch_bounds__(256, 2) void k_sphere_hs(SphereArgs p, int hblocks)
+{
+    extern __shared__ __attribute__((aligned(1024))) char lds[];
+    stamp(p, 2);
+    if ((int)blockIdx.x < hblocks) sphere_gemm_tile<32, 32, 1, 1, 4, true>(p, (int)blockIdx.x, lds);
+    else overlap_tile<M, M>(p, (int)blockIdx.x - hblocks, (double*)lds);
+}
+
+template <int BR, int BC, int RB, int CB, int NS, bool kH>
+static hipError_t launch_sphere_gemm(const SphereArgs& p, int64_t nblk, hipEvent_t stop, hipStream_t st)
+{
+    using Tl = SphereTile<BR, BC, RB, CB, NS>;
+    return launch(k_sphere_gemm<BR, BC, RB, CB, NS, kH>, dim3((unsigned)nblk), Tl::kThreads, Tl::kLds, stop, st, p);
 }
 
 // rtiles: row tiles of all kinds for the tile's rows (tile 64: 32 x 64)
-hipError_t launch_sphere_tapp(const SphereArgs& p, int tile, int rtiles, hipStream_t st)
+hipError_t launch_sphere_tapp(const SphereArgs& p, int tile, int rtiles, hipEvent_t stop, hipStream_t st)
 {
-    if (tile == 32) return launch_sphere_gemm<32, 32, 1, 1, false>(p, (int64_t)rtiles * (p.gtot / 32), st);
-    return launch_sphere_gemm<32, 64, 1, 2, false>(p, (int64_t)rtiles * (p.gtot / 64), st);
+    if (tile == 32) return launch_sphere_gemm<32, 32, 1, 1, 2, false>(p, (int64_t)rtiles * (p.gtot / 32), stop, st);
+    return launch_sphere_gemm<32, 64, 1, 2, 2, false>(p, (int64_t)rtiles * (p.gtot / 64), stop, st);
 }
 
+static int64_t hblocks(const SphereArgs& p, int tile) { return ((int64_t)p.nsquares * (tile == 48 ? 2 : 1) + 7) / 8 * 8; }
+
 // tile: 64 (64 x 64), 48 (32 x 64) or 32 (32 x 32)
-hipError_t launch_sphere_h(const SphereArgs& p, int tile, hipStream_t st)
+hipError_t launch_sphere_h(const SphereArgs& p, int tile, hipEvent_t stop, hipStream_t st)
 {
-    const int64_t n = ((int64_t)p.nsquares * (tile == 48 ? 2 : 1) + 7) / 8 * 8;
-    if (tile == 32) return launch_sphere_gemm<32, 32, 1, 1, true>(p, n, st);
-    if (tile == 48) return launch_sphere_gemm<32, 64, 1, 2, true>(p, n, st);
-    return launch_sphere_gemm<64, 64, 1, 2, true>(p, n, st);
+    const int64_t n = hblocks(p, tile);
+    if (tile == 32) return launch_sphere_gemm<32, 32, 1, 1, 4, true>(p, n, stop, st);
+    if (tile == 48) return launch_sphere_gemm<32, 64, 1, 2, 2, true>(p, n, stop, st);
+    return launch_sphere_gemm<64, 64, 1, 2, 2, true>(p, n, stop, st);
+}
+
+template <int M>
+static hipError_t launch_hs(const SphereArgs& p, int64_t nstiles, hipEvent_t stop, hipStream_t st)
+{
+    const int64_t n = hblocks(p, 32);
+    const size_t lds = std::max<size_t>(SphereTile<32, 32, 1, 1, 4>::kLds, overlap_lds(16 * M, p.nl));
+    return launch(k_sphere_hs<M>, dim3((unsigned)(n + nstiles)), 256, lds, stop, st, p, (int)n);
+}
+
+hipError_t launch_sphere_hs(const SphereArgs& p, int stile, int64_t nstiles, hipEvent_t stop, hipStream_t st)
+{
+    return stile == 32 ? launch_hs<2>(p, nstiles, stop, st) : launch_hs<1>(p, nstiles, stop, st);
 }
 
 }  // namespace hsgen

@@ -337,8 +337,8 @@ hsgen_status sphere_split_w(hsgen_ctx* ctx, hsgen_sys* s, const std::vector<Sphe
         p.nk = (int32_t)ks.size();
         p.one = ks[0];
         p.many = ks_dev;
-        HIPCHK(launch_sphere_gen(p, ctx->stream));
-        HIPCHK(launch_sphere_tapp(p, tapp_tile(ctx, s, l.gtot), s->rt32, ctx->stream));
+        HIPCHK(launch_sphere_gen(p, nullptr, ctx->stream));
+        HIPCHK(launch_sphere_tapp(p, tapp_tile(ctx, s, l.gtot), s->rt32, nullptr, ctx->stream));
     }
     return HSGEN_OK;
 }
@@ -360,7 +360,7 @@ SphereLayout sphere_layout(const hsgen_ctx* ctx, const hsgen_sys* s, const std::
     // 6002 9583 / 8625 / 8566.
     l.htile = t64 < 3 * (int64_t)ncu ? 32 : t64 < 6 * (int64_t)ncu ? 48 : 64;
     l.ttile = tapp_tile(ctx, s, l.gtot);
-    l.stile = overlap_tile(t64, ncu);
+    l.stile = overlap_tile_size(t64, ncu);
     const int hc = l.htile == 32 ? 32 : 64;
     for (int ng : ngs) {
         l.nsquares += lower((ng + hc - 1) / hc);
@@ -426,6 +426,7 @@ std::vector<SphereK> sphere_ks(const SphereLayout& l, const std::vector<const hs
         std::memset(&k, 0, sizeof k);
         for (int q = 0; q < 3; ++q) k.k[q] = kps[i]->k[q];
         k.g = gs[i];
+        k.gd = const_cast<int32_t*>(gs[i]);
         k.H = H[i];
         k.S = S[i];
         k.ldH = ldH[i];
@@ -443,18 +444,87 @@ std::vector<SphereK> sphere_ks(const SphereLayout& l, const std::vector<const hs
     return ks;
 }
 
-// The launches of one call.  ev: events recorded after the generator and after
-// the T application, or null.
-hipError_t sphere_launch(const SphereArgs& p, const SphereLayout& l, const hsgen_sys* s, bool do_h, bool do_s,
-                         hipEvent_t ev_gen, hipEvent_t ev_tapp, hipStream_t st)
+// The G list of a one-k-point call: device memory as it is; a short host list
+// goes into the context's pinned buffer, which the generator reads and copies
+// to dev (a copy on the stream costs 12 us); a longer one is copied to dev.
+// dev: room for the list in device memory, or null to take ctx->g.
+hsgen_status sphere_g(hsgen_ctx* ctx, const hsgen_kpoint* kp, int32_t* dev, SphereK& k)
 {
-    hipError_t e = launch_sphere_gen(p, st);
-    if (e == hipSuccess && ev_gen) e = hipEventRecord(ev_gen, st);
-    if (e == hipSuccess && do_h) e = launch_sphere_tapp(p, l.ttile, s->rt32, st);
-    if (e == hipSuccess && ev_tapp) e = hipEventRecord(ev_tapp, st);
-    if (e == hipSuccess && do_h) e = launch_sphere_h(p, l.htile, st);
-    if (e == hipSuccess && do_s) e = launch_overlap(p, l.stile, l.nstiles, st);
+    if (is_device_ptr(kp->g)) {
+        k.g = kp->g;
+        k.gd = const_cast<int32_t*>(kp->g);
+        return HSGEN_OK;
+    }
+    const size_t bytes = sizeof(int32_t) * 3 * (size_t)kp->ng;
+    if (!dev) {
+        const hsgen_status st = ensure(ctx, ctx->g, bytes, false);
+        if (st) return st;
+        dev = (int32_t*)ctx->g.p;
+    }
+    k.gd = dev;
+    if (kp->ng <= kPinnedG) {
+        std::memcpy((char*)ctx->pin + kPinStamps, kp->g, bytes);
+        k.g = (const int32_t*)((char*)ctx->pin_dev + kPinStamps);
+    } else {
+        HIPCHK(hipMemcpyAsync(dev, kp->g, bytes, hipMemcpyHostToDevice, ctx->stream));
+        k.g = dev;
+    }
+    return HSGEN_OK;
+}
+
+// The launches of one call.  stop: null, or an event that takes the end of the
+// last of them.
+hipError_t sphere_launch(const SphereArgs& p, const SphereLayout& l, const hsgen_sys* s, bool do_h, bool do_s,
+                         hipEvent_t stop, hipStream_t st)
+{
+    const hipEvent_t none = nullptr, last = stop;
+    hipError_t e = launch_sphere_gen(p, do_h || do_s ? none : last, st);
+    if (e == hipSuccess && do_h) e = launch_sphere_tapp(p, l.ttile, s->rt32, none, st);
+    if (e != hipSuccess) return e;
+    if (do_h && do_s && l.htile == 32 && l.stile <= 32) return launch_sphere_hs(p, l.stile, l.nstiles, last, st);
+    if (do_h) e = launch_sphere_h(p, l.htile, do_s ? none : last, st);
+    if (e == hipSuccess && do_s) e = launch_overlap(p, l.stile, l.nstiles, last, st);
     return e;
+}
+
+// A one-k-point call on device matrices: launches, wait, report.
+hsgen_status sphere_run(hsgen_ctx* ctx, const hsgen_sys* s, const SphereLayout& l, SphereArgs& p, int flags, int tile,
+                        hsgen_report* rep)
+{
+    const bool do_h = !(flags & HSGEN_SKIP_H), do_s = !(flags & HSGEN_SKIP_S);
+    const SphereK& k = p.one;
+    p.stamp = rep ? (uint64_t*)ctx->pin_dev : nullptr;
+    if (rep) HIPCHK(hipEventRecord(ctx->ev[0], ctx->stream));
+    const hipError_t le = sphere_launch(p, l, s, do_h, do_s, ctx->ev[1], ctx->stream);
+    if (le != hipSuccess) {
+        (void)hipStreamSynchronize(ctx->stream);    // nothing reads the pinned buffer after the call
+        HIPCHK(le);
+    }
+    hipEvent_t end = ctx->ev[1];
+    if (flags & HSGEN_FILL_UPPER) {
+        if (do_h) HIPCHK(launch_fill_upper(k.H, k.ldH, k.ng, ctx->stream));
+        if (do_s) HIPCHK(launch_fill_upper(k.S, k.ldS, k.ng, ctx->stream));
+        end = ctx->ev[2];
+        HIPCHK(hipEventRecord(end, ctx->stream));
+    }
+    HIPCHK(hipEventSynchronize(end));
+    if (!rep) return HSGEN_OK;
+    // the whole by events, the kernels' starts by the wall clock: a call of 50 us
+    // took 14 us more with events around each kernel
+    float total = 0;
+    HIPCHK(hipEventElapsedTime(&total, ctx->ev[0], end));
+    const volatile uint64_t* t = (const volatile uint64_t*)ctx->pin;
+    auto ms = [&](int from, int to) { return (double)(int64_t)(t[to] - t[from]) * ctx->ms_per_tick; };
+    rep->ms_total = total;
+    rep->ms_abgen = do_h ? ms(0, 1) : do_s ? ms(0, 3) : total;
+    rep->ms_tmul = do_h ? ms(1, 2) : 0.0;
+    rep->ms_contract = do_h || do_s ? std::max(0.0, total - rep->ms_abgen - rep->ms_tmul) : 0.0;
+    rep->ng = k.ng;
+    rep->kdim = s->kdim;
+    rep->flops_alg = 16.0 * (double)k.ng * k.ng * s->kdim + 32.0 * (double)k.ng * (double)s->sum_nlm2;
+    rep->bytes_abgen = sphere_gen_bytes(s) * k.ng;
+    rep->tile_used = tile;
+    return HSGEN_OK;
 }
 
 }  // namespace hsgen

@@ -184,3 +184,45 @@ def test_int8_tiles_by_rounds(ctx, ng, nk, tile):
     for (Ha, Sa), (Hb, Sb) in zip(res, ref):
         assert np.array_equal(Ha, Hb) and np.array_equal(Sa, Sb)
     h.close()
+
+
+@pytest.mark.parametrize("ng", [4095, 4096, 4097])
+def test_short_and_long_g_lists(ctx, ng):
+    """G lists of up to 4096 plane waves are read from pinned memory, longer
+    ones copied: both end in the bits of a small call."""
+    s, kp = tiny_system(natoms=1, lmax=(2,), a_cell=19.0, ng_target=4600, seed=14)
+    assert kp.ng > ng
+    h = ctx.upload(s)
+    H, S = ctx.create_HS2(h, _subset(kp, np.arange(ng)))
+    idx = np.r_[0:20, ng // 2:ng // 2 + 20, ng - 20:ng]
+    Hs, Ss = ctx.create_HS2(h, _subset(kp, idx))
+    assert np.array_equal(Hs, H[np.ix_(idx, idx)]) and np.array_equal(Ss, S[np.ix_(idx, idx)])
+    h.close()
+
+
+@pytest.mark.parametrize("lmax", [(1,), (2,), (4,), (9, 3)])
+@pytest.mark.parametrize("ng", [33, 300, 1100])
+def test_h_and_s_in_one_launch(ctx, ng, lmax):
+    """H and S tiles of one launch equal those of two, and the parts of the
+    reported time are there for every choice of matrices."""
+    from hybridhsdla_amd.api import HSGEN_FILL_UPPER, HSGEN_SKIP_H, HSGEN_SKIP_S
+    torch = pytest.importorskip("torch")
+    s, kp = tiny_system(natoms=5, lmax=lmax, a_cell=13.0, ng_target=1300, seed=4)
+    sub = _subset(kp, np.arange(min(ng, kp.ng)))
+    h = ctx.upload(s)
+    n = sub.ng
+    out = {}
+    for flags in (0, HSGEN_SKIP_H, HSGEN_SKIP_S, HSGEN_FILL_UPPER, HSGEN_SKIP_H | HSGEN_SKIP_S):
+        H, S = (torch.zeros(n, n, dtype=torch.complex128, device="cuda") for _ in range(2))
+        torch.cuda.synchronize()
+        r = ctx.create_hs_device(h, sub, H.data_ptr(), S.data_ptr(), n, flags=flags)
+        out[flags] = [X.cpu().numpy().T for X in (H, S)]
+        assert r["ms_total"] > 0 and r["ms_abgen"] >= 0 and r["ms_tmul"] >= 0 and r["ms_contract"] >= 0
+        assert r["ms_abgen"] + r["ms_tmul"] + r["ms_contract"] <= r["ms_total"] * (1 + 1e-6) + 1e-2
+        assert (r["ms_tmul"] > 0) == (not flags & HSGEN_SKIP_H)
+    H, S = out[0]
+    assert np.array_equal(out[HSGEN_SKIP_S][0], H) and np.array_equal(out[HSGEN_SKIP_H][1], S)
+    for X, F in zip((H, S), out[HSGEN_FILL_UPPER]):
+        assert np.array_equal(np.tril(F), np.tril(X)) and np.array_equal(F, np.tril(F) + np.tril(F, -1).conj().T)
+    assert rel_fro_lower(H, po.reference_hs(s, sub)[0]) <= TOL
+    h.close()
