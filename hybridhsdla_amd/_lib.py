@@ -18,6 +18,7 @@ HSGEN_PREC_OZAKI_BF16 = 2
 HSGEN_FILL_UPPER = 1
 HSGEN_SKIP_H = 2
 HSGEN_SKIP_S = 4
+HSGEN_CLEAR_UPPER = 8
 
 _p = C.c_void_p
 

@@ -18,7 +18,7 @@ from typing import Optional, Sequence, Tuple
 import numpy as np
 
 from . import _lib
-from ._lib import (HSGEN_FILL_UPPER, HSGEN_PREC_FP64, HSGEN_PREC_OZAKI_BF16, HSGEN_PREC_OZAKI_INT8, HSGEN_SKIP_H,
+from ._lib import (HSGEN_CLEAR_UPPER, HSGEN_FILL_UPPER, HSGEN_PREC_FP64, HSGEN_PREC_OZAKI_BF16, HSGEN_PREC_OZAKI_INT8, HSGEN_SKIP_H,
                    HSGEN_SKIP_S, HsgenError, HsgenKpoint, HsgenOpts, HsgenReport, HsgenSystem)
 from .system import KPoint, System
 
@@ -38,6 +38,24 @@ def _kpoint(kp: KPoint) -> Tuple[HsgenKpoint, np.ndarray]:
     s.ng = int(g.shape[0])
     s.g = g.ctypes.data if g.size else None
     return s, g
+
+
+def _results(ng: int, H, S, flags: int):
+    """H and S, allocated where the caller gave none, and the call's flags.
+    Memory that the library writes as a whole is left uninitialised: clearing
+    it here would be a pass of one thread over memory that the copy of the
+    results writes anyway.  Beyond 32 MiB the C library maps fresh pages, which
+    are zero by themselves."""
+    shape = dict(shape=(ng, ng), dtype=np.complex128, order="F")
+    whole = flags & HSGEN_FILL_UPPER
+    if not whole and H is None and S is None and 16 * ng * ng <= 32 << 20:
+        flags |= HSGEN_CLEAR_UPPER
+        whole = True
+    if H is None:
+        H = (np.empty if whole and not flags & HSGEN_SKIP_H else np.zeros)(**shape)
+    if S is None:
+        S = (np.empty if whole and not flags & HSGEN_SKIP_S else np.zeros)(**shape)
+    return H, S, flags
 
 
 def _opts(precision=HSGEN_PREC_FP64, slices=0, target_rel_err=0.0, flags=0, tile=0) -> HsgenOpts:
@@ -141,8 +159,9 @@ class Context:
         arma::cx_cube layout (lm fastest)."""
         s = sysh.system
         L = s.L
-        A = np.zeros((L, s.natoms, kp.ng), dtype=np.complex128, order="F")
-        B = np.zeros_like(A)
+        # every element is written
+        A = np.empty((L, s.natoms, kp.ng), dtype=np.complex128, order="F")
+        B = np.empty((L, s.natoms, kp.ng), dtype=np.complex128, order="F")
         ks, g = _kpoint(kp)
         _lib.check(self.lib.hsgen_construct_ab(self.handle, sysh.handle, C.byref(ks), _ptr(A), _ptr(B)),
                    self.handle)
@@ -155,10 +174,7 @@ class Context:
         preallocated arrays (numpy, or ints = device pointers with ld = ng)
         the library writes into them and leaves their upper triangles alone."""
         ng = kp.ng
-        if H is None:
-            H = np.zeros((ng, ng), dtype=np.complex128, order="F")
-        if S is None:
-            S = np.zeros((ng, ng), dtype=np.complex128, order="F")
+        H, S, flags = _results(ng, H, S, flags)
         hp = H if isinstance(H, int) else _ptr(H)
         sp = S if isinstance(S, int) else _ptr(S)
         ks, g = _kpoint(kp)
@@ -242,9 +258,10 @@ class Context:
             keep.append(g)
         res = []
         if outputs is None:
+            asked = flags
             for kp in kps:
-                res.append((np.zeros((kp.ng, kp.ng), np.complex128, order="F"),
-                            np.zeros((kp.ng, kp.ng), np.complex128, order="F")))
+                H, S, flags = _results(kp.ng, None, None, asked)
+                res.append((H, S))
             hp = (C.c_void_p * nk)(*[_ptr(h) for h, _ in res])
             sp = (C.c_void_p * nk)(*[_ptr(s) for _, s in res])
             lds = (C.c_int64 * nk)(*[max(kp.ng, 1) for kp in kps])
@@ -278,10 +295,7 @@ class Context:
         pc = (C.c_void_p * a)(*[t.ctypes.data for t in fc])
         lm = np.ascontiguousarray(l_maxs, dtype=np.int32)
         un = np.ascontiguousarray(u_norms, dtype=np.float64).reshape(-1)
-        if H is None:
-            H = np.zeros((G, G), dtype=np.complex128, order="F")
-        if S is None:
-            S = np.zeros((G, G), dtype=np.complex128, order="F")
+        H, S, flags = _results(G, H, S, flags)
         o = _opts(precision, slices, target_rel_err, flags, tile)
         rep = HsgenReport()
         _lib.check(self.lib.hsgen_contract_hs(self.handle, L, a, G, _ptr(A), _ptr(B), _ptr(tsz), pa, pb,

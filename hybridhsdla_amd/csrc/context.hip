@@ -15,7 +15,6 @@
 #include <map>
 #include <numeric>
 #include <string>
-#include <thread>
 #include <vector>
 
 #include "hsgen_host.h"
@@ -242,74 +241,6 @@ hsgen_status upload_g(hsgen_ctx* ctx, const hsgen_kpoint* kp)
     return HSGEN_OK;
 }
 
-// Copy the lower triangle (and optionally everything) of a device matrix with
-// ld = n into a host matrix with leading dimension ld: blocks of columns go
-// through two pinned staging buffers (the DMA of one block overlaps the
-// host-side copy of the previous one, which several threads share), so that
-// only the requested triangle of the caller's matrix is written.
-hsgen_status copy_lower_to_host(hsgen_ctx* ctx, const double2* dsrc, int n, double* H, int64_t ld,
-                                bool full)
-{
-    if (n <= 0) return HSGEN_OK;
-    const size_t kStage = (size_t)64 << 20;
-    if (!ctx->stage[0]) {
-        for (int b = 0; b < 2; ++b) {
-            hipError_t e = hipHostMalloc(&ctx->stage[b], kStage, hipHostMallocDefault);
-            if (e != hipSuccess) {
-                (void)hipGetLastError();
-                ctx->stage[b] = nullptr;
-                return fail(ctx, HSGEN_ERR_NOMEM, "hipHostMalloc(%zu bytes) failed: %s", kStage, hipGetErrorString(e));
-            }
-        }
-        ctx->stage_bytes = kStage;
-    }
-    const size_t colb = sizeof(double2) * (size_t)n;
-    const int cpb = (int)std::max<size_t>(1, ctx->stage_bytes / colb);     // columns per block
-    if ((size_t)cpb * colb > ctx->stage_bytes) {
-        // one column exceeds a staging buffer: copy column pieces directly
-        std::vector<double2> tmp((size_t)n);
-        for (int j = 0; j < n; ++j) {
-            const int i0 = full ? 0 : j;
-            HIPCHK(hipMemcpy(tmp.data() + i0, dsrc + (int64_t)j * n + i0, sizeof(double2) * (n - i0),
-                             hipMemcpyDeviceToHost));
-            std::memcpy((double2*)H + (int64_t)j * ld + i0, tmp.data() + i0, sizeof(double2) * (n - i0));
-        }
-        return HSGEN_OK;
-    }
-    const int nblk = (n + cpb - 1) / cpb;
-    auto issue = [&](int b) -> hipError_t {
-        const int j0 = b * cpb, j1 = std::min(n, j0 + cpb);
-        hipError_t e = hipMemcpyAsync(ctx->stage[b & 1], dsrc + (int64_t)j0 * n, colb * (size_t)(j1 - j0),
-                                      hipMemcpyDeviceToHost, ctx->stream);
-        if (e == hipSuccess) e = hipEventRecord(ctx->ev[5 + (b & 1)], ctx->stream);
-        return e;
-    };
-    const int nthr = (int)std::max(1u, std::min(8u, std::thread::hardware_concurrency()));
-    HIPCHK(issue(0));
-    for (int b = 0; b < nblk; ++b) {
-        HIPCHK(hipEventSynchronize(ctx->ev[5 + (b & 1)]));
-        if (b + 1 < nblk) HIPCHK(issue(b + 1));
-        const int j0 = b * cpb, j1 = std::min(n, j0 + cpb);
-        const double2* src = (const double2*)ctx->stage[b & 1];
-        auto work = [&](int t) {
-            for (int j = j0 + t; j < j1; j += nthr) {
-                const int i0 = full ? 0 : j;
-                std::memcpy((double2*)H + (int64_t)j * ld + i0, src + (size_t)(j - j0) * n + i0,
-                            sizeof(double2) * (size_t)(n - i0));
-            }
-        };
-        if (nthr > 1 && (size_t)(j1 - j0) * colb >= ((size_t)4 << 20)) {
-            std::vector<std::thread> th;
-            for (int t2 = 1; t2 < nthr; ++t2) th.emplace_back(work, t2);
-            work(0);
-            for (auto& x : th) x.join();
-        } else {
-            for (int t2 = 0; t2 < nthr; ++t2) work(t2);
-        }
-    }
-    return HSGEN_OK;
-}
-
 }  // namespace hsgen
 
 using namespace hsgen;
@@ -394,8 +325,8 @@ hsgen_status hsgen_release_workspace(hsgen_ctx* ctx)
     HIPCHK(hipStreamSynchronize(ctx->stream));
     for (DevBuf* b : {&ctx->Z, &ctx->Zs, &ctx->W, &ctx->Htmp, &ctx->Stmp, &ctx->A, &ctx->B, &ctx->g,
                       &ctx->probs, &ctx->work, &ctx->unorm2, &ctx->atoms_tmp, &ctx->oz_e, &ctx->oz_res,
-                      &ctx->oz_out, &ctx->oz_fprob, &ctx->oz_probs, &ctx->oz_work, &ctx->oz_smp, &ctx->btmp, &ctx->eig_a,
-                      &ctx->eig_b, &ctx->eig_d, &ctx->sph_ph, &ctx->sph_rs, &ctx->sph_y, &ctx->sph_w})
+                      &ctx->oz_out, &ctx->oz_fprob, &ctx->oz_probs, &ctx->oz_work, &ctx->oz_smp, &ctx->btmp,
+                      &ctx->ring_left, &ctx->eig_a, &ctx->eig_b, &ctx->eig_d, &ctx->sph_ph, &ctx->sph_rs, &ctx->sph_y, &ctx->sph_w})
         release(*b);
     for (auto& bg : ctx->bgraphs) {
         if (bg.exec) (void)hipGraphExecDestroy(bg.exec);
@@ -419,8 +350,7 @@ hsgen_status hsgen_finalize(hsgen_ctx* ctx)
     for (auto& ev : ctx->oz_ev)
         if (ev) (void)hipEventDestroy(ev);
     if (ctx->blas) (void)rocblas_destroy_handle(ctx->blas);
-    for (void*& p : ctx->stage)
-        if (p) (void)hipHostFree(p);
+    if (ctx->ring) (void)hipHostFree(ctx->ring);
     if (ctx->pin) (void)hipHostFree(ctx->pin);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;

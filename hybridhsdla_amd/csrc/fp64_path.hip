@@ -268,6 +268,10 @@ hsgen_status finish_hs(hsgen_ctx* ctx, hsgen_sys* s, const Geometry& geo, int ng
         if (st) return st;
     }
 
+    std::vector<HostCopy> out;
+    if (need_h && !hdev) out.push_back(copy_matrix(dH, ng, H, ld, o.flags));
+    if (!(flags & HSGEN_SKIP_S) && !sdev) out.push_back(copy_matrix(dS, ng, S, ld, o.flags));
+    Prefault pages(ctx, out);
     std::vector<GemmProblem> probs;
     std::vector<TileWork> work;
     HIPCHK(hipEventRecord(ctx->ev[2], ctx->stream));
@@ -326,14 +330,8 @@ hsgen_status finish_hs(hsgen_ctx* ctx, hsgen_sys* s, const Geometry& geo, int ng
     }
     HIPCHK(hipEventRecord(ctx->ev[4], ctx->stream));
     HIPCHK(hipEventSynchronize(ctx->ev[4]));
-    if (need_h && !hdev) {
-        st = copy_lower_to_host(ctx, dH, ng, H, ld, (flags & HSGEN_FILL_UPPER) != 0);
-        if (st) return st;
-    }
-    if (!(flags & HSGEN_SKIP_S) && !sdev) {
-        st = copy_lower_to_host(ctx, dS, ng, S, ld, (flags & HSGEN_FILL_UPPER) != 0);
-        if (st) return st;
-    }
+    st = host_copy(ctx, out, true);
+    if (st) return st;
     if (rep) {
         float t1 = 0, t2 = 0;
         HIPCHK(hipEventElapsedTime(&t1, ctx->ev[2], ctx->ev[3]));
@@ -434,18 +432,13 @@ hsgen_status create_hs_sphere(hsgen_ctx* ctx, hsgen_sys* s, const hsgen_kpoint* 
     p.one = sphere_ks(l, {kp}, {nullptr}, {dH}, {dS}, {ldH}, {ldS})[0];
     st = sphere_g(ctx, kp, nullptr, p.one);
     if (st) return st;
+    std::vector<HostCopy> out;
+    if (!hdev) out.push_back(copy_matrix(dH, ng, H, ld, o.flags));
+    if (!sdev) out.push_back(copy_matrix(dS, ng, S, ld, o.flags));
+    Prefault pages(ctx, out);
     st = sphere_run(ctx, s, l, p, o.flags, geo.cfg, rep);
     if (st) return st;
-    const bool full = (o.flags & HSGEN_FILL_UPPER) != 0;
-    if (!hdev) {
-        st = copy_lower_to_host(ctx, dH, ng, H, ld, full);
-        if (st) return st;
-    }
-    if (!sdev) {
-        st = copy_lower_to_host(ctx, dS, ng, S, ld, full);
-        if (st) return st;
-    }
-    return HSGEN_OK;
+    return host_copy(ctx, out, true);
 }
 
 // ---------------------------------------------------------------------------
@@ -616,6 +609,13 @@ hsgen_status batched_fp64(hsgen_ctx* ctx, hsgen_sys* s, int nk, const hsgen_kpoi
             }
             bg.sig = sig;
         }
+        std::vector<HostCopy> out;
+        for (size_t q = 0; q < ks.size(); ++q) {
+            const int i = ks[q];
+            if (do_h && !hdev[i]) out.push_back(copy_matrix(dH[q], kps[i].ng, H[i], ld[i], flags));
+            if (do_s && !sdev[i]) out.push_back(copy_matrix(dS[q], kps[i].ng, S[i], ld[i], flags));
+        }
+        Prefault pages(ctx, out);
         HIPCHK(hipEventRecord(ctx->ev[0], ctx->stream));
         HIPCHK(hipGraphLaunch(bg.exec, ctx->stream));
         HIPCHK(hipEventRecord(ctx->ev[1], ctx->stream));
@@ -623,18 +623,8 @@ hsgen_status batched_fp64(hsgen_ctx* ctx, hsgen_sys* s, int nk, const hsgen_kpoi
         float ms = 0.0f;
         HIPCHK(hipEventElapsedTime(&ms, ctx->ev[0], ctx->ev[1]));
         ms_all += ms;
-        for (size_t q = 0; q < ks.size(); ++q) {
-            const int i = ks[q];
-            const bool full = (flags & HSGEN_FILL_UPPER) != 0;
-            if (do_h && !hdev[i]) {
-                st = copy_lower_to_host(ctx, dH[q], kps[i].ng, H[i], ld[i], full);
-                if (st) return st;
-            }
-            if (do_s && !sdev[i]) {
-                st = copy_lower_to_host(ctx, dS[q], kps[i].ng, S[i], ld[i], full);
-                if (st) return st;
-            }
-        }
+        st = host_copy(ctx, out, true);
+        if (st) return st;
     }
     if (rep) {
         for (int i = 0; i < nk; ++i) {
@@ -687,9 +677,13 @@ hsgen_status hsgen_construct_ab(hsgen_ctx* ctx, const hsgen_sys* s, const hsgen_
     p.ncols = kp->ng;
     p.A = dA;
     p.B = dB;
+    std::vector<HostCopy> out;
+    if (!adev) out.push_back(copy_run(dA, A, sizeof(double2) * n));
+    if (!bdev) out.push_back(copy_run(dB, B, sizeof(double2) * n));
+    Prefault pages(ctx, out);
     HIPCHK(launch_abgen(p, false, ctx->stream));
-    if (!adev) HIPCHK(hipMemcpyAsync(A, dA, sizeof(double2) * n, hipMemcpyDeviceToHost, ctx->stream));
-    if (!bdev) HIPCHK(hipMemcpyAsync(B, dB, sizeof(double2) * n, hipMemcpyDeviceToHost, ctx->stream));
+    st = host_copy(ctx, out, true);
+    if (st) return st;
     HIPCHK(hipStreamSynchronize(ctx->stream));
     return HSGEN_OK;
 }
@@ -826,18 +820,24 @@ hsgen_status hsgen_contract_hs(hsgen_ctx* ctx, int32_t L, int32_t a, int32_t G, 
     const size_t nab = (size_t)L * a * G;
     const double2* dA = (const double2*)A;
     const double2* dB = (const double2*)B;
+    std::vector<HostCopy> in, out;
+    if (!(o.flags & HSGEN_SKIP_H) && H && !is_device_ptr(H)) out.push_back(copy_matrix(nullptr, G, H, ld, o.flags));
+    if (!(o.flags & HSGEN_SKIP_S) && S && !is_device_ptr(S)) out.push_back(copy_matrix(nullptr, G, S, ld, o.flags));
+    Prefault pages(ctx, out);
     if (!is_device_ptr(A)) {
         st = ensure(ctx, ctx->A, sizeof(double2) * nab, false);
         if (st) return st;
-        HIPCHK(hipMemcpyAsync(ctx->A.p, A, sizeof(double2) * nab, hipMemcpyHostToDevice, ctx->stream));
+        in.push_back(copy_run(ctx->A.p, A, sizeof(double2) * nab));
         dA = (const double2*)ctx->A.p;
     }
     if (!is_device_ptr(B)) {
         st = ensure(ctx, ctx->B, sizeof(double2) * nab, false);
         if (st) return st;
-        HIPCHK(hipMemcpyAsync(ctx->B.p, B, sizeof(double2) * nab, hipMemcpyHostToDevice, ctx->stream));
+        in.push_back(copy_run(ctx->B.p, B, sizeof(double2) * nab));
         dB = (const double2*)ctx->B.p;
     }
+    st = host_copy(ctx, in, false);
+    if (st) return st;
     st = ensure(ctx, ctx->atoms_tmp, sizeof(AtomDev) * a, false);
     if (st) return st;
     st = ensure(ctx, ctx->unorm2, sizeof(double) * un2.size(), false);

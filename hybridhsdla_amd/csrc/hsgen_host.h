@@ -23,12 +23,18 @@
 // element is zero so the kernels need no bounds checks along k.
 #pragma once
 
+#include <atomic>
 #include <complex>
+#include <condition_variable>
 #include <cstdarg>
+#include <functional>
 #include <list>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <string>
+#include <thread>
+#include <utility>
 #include <vector>
 
 #include <rocblas/rocblas.h>
@@ -57,6 +63,7 @@ constexpr int kBf16Cfg = 61;       // default BF16 kernel configuration (256 x 1
 constexpr int kSampleTile = 12;    // FP64 tile of the split-precision sample: 64 x 64, so 64 columns
 constexpr int kPinnedG = 4096;     // plane waves of a G list that is read from pinned host memory
 constexpr size_t kPinStamps = 64;
+constexpr int kRingSlots = 6;       // pinned slots of a host copy
 constexpr size_t kMaxOzGraphs = 16; // cached split-precision launch-segment sets per context
 
 struct DevBuf {
@@ -69,6 +76,71 @@ struct MLoc {
     int64_t off;       // offset of M_a (complex units)
     int32_t ld;        // leading dimension (2 nlm_a rounded up to the tile's BK)
     int32_t cols;      // padded column count (2 nlm_a rounded up to the tile's BM)
+};
+
+// Columns to copy between device and host memory; sizes and strides in bytes.
+// Device addresses and strides are multiples of 16, so are sizes of several
+// columns; a run's size is a multiple of 8.
+struct HostCopy {
+    char* dev;
+    char* host;
+    size_t rows, cols, ldd, ldh;
+    bool lower;        // of column j only the 16-byte rows from j on
+    bool clear;        // and zeros into the host's rows above them
+};
+inline HostCopy copy_run(void* dev, const void* host, size_t bytes)
+{
+    return {(char*)dev, (char*)host, bytes, 1, bytes, bytes, false, false};
+}
+// an n x n matrix, its lower triangle or (HSGEN_FILL_UPPER) all of it
+inline HostCopy copy_matrix(const double2* dev, int n, double* host, int64_t ld, int flags)
+{
+    const size_t e = sizeof(double2);
+    return {(char*)dev, (char*)host, e * n, (size_t)n, e * n, e * ld, !(flags & HSGEN_FILL_UPPER),
+            (flags & HSGEN_CLEAR_UPPER) != 0};
+}
+
+// Threads of a context that copy host memory: started with its first large
+// copy, at most 8, joined with the context.  Tasks run in the order they are
+// posted; finish() withdraws a group's waiting tasks and waits for its running
+// ones.
+class HostPool {
+public:
+    HostPool();
+    ~HostPool();
+    size_t size() const { return threads_.size(); }
+    void post(const void* group, const std::function<void()>& run, size_t n);
+    void finish(const void* group);
+
+private:
+    struct Task {
+        const void* group;
+        std::function<void()> run;
+    };
+    void loop(int me);
+    std::mutex mu_;
+    std::condition_variable wake_, done_;
+    std::list<Task> tasks_;
+    std::vector<const void*> current_;     // per thread: the group it works for
+    std::vector<std::thread> threads_;
+    bool quit_ = false;
+    int pid_;
+};
+
+// Maps the pages of a call's host results in the background until they are
+// copied or the object goes.
+class Prefault {
+public:
+    Prefault(hsgen_ctx* ctx, const std::vector<HostCopy>& list);
+    ~Prefault();
+    void stop() { stop_.store(true, std::memory_order_relaxed); }
+
+private:
+    hsgen_ctx* ctx_;
+    HostPool* pool_ = nullptr;
+    std::vector<std::pair<char*, size_t>> ranges_;
+    std::atomic<size_t> next_{0};
+    std::atomic<bool> stop_{false};
 };
 
 }  // namespace hsgen
@@ -115,9 +187,13 @@ struct hsgen_ctx {
     void* pin = nullptr;
     void* pin_dev = nullptr;
     double ms_per_tick = 1e-5;                       // of the GPU's wall clock
-    // pinned staging for device -> host copies of H and S
-    void* stage[2] = {nullptr, nullptr};
-    size_t stage_bytes = 0;
+    // pinned slots of copies from and to pageable memory
+    char* ring = nullptr;
+    void* ring_dev = nullptr;
+    uint64_t ring_seq = 0;
+    hsgen::DevBuf ring_left;
+    std::unique_ptr<hsgen::HostPool> pool;
+    hsgen::Prefault* prefault = nullptr;
 };
 
 struct hsgen_sys {
@@ -201,7 +277,7 @@ bool fold_ok(double n);
 hsgen_status ensure_M(hsgen_ctx* ctx, hsgen_sys* s, int bk, int bm);
 hsgen_status check_kpoint(hsgen_ctx* ctx, const hsgen_kpoint* kp);
 hsgen_status upload_g(hsgen_ctx* ctx, const hsgen_kpoint* kp);
-hsgen_status copy_lower_to_host(hsgen_ctx* ctx, const double2* dsrc, int n, double* H, int64_t ld, bool full);
+hsgen_status host_copy(hsgen_ctx* ctx, const std::vector<HostCopy>& list, bool to_host);
 
 // ---- fp64_path.hip ----
 struct Geometry {

@@ -969,6 +969,13 @@ hsgen_status batched_split(hsgen_ctx* ctx, hsgen_sys* s, int nk, const hsgen_kpo
             HIPCHK(hipStreamSynchronize(ctx->stream));   // sk must outlive its copy, ctx->probs its readers
             HIPCHK(launch_clear_rows(W, geo.ldz, 2 * (int64_t)s->kdim, geo.ldz, (int)ncols, ctx->stream));
         }
+        std::vector<HostCopy> out;
+        for (size_t q = 0; q < bk.size(); ++q) {
+            const int i = bk[q];
+            if (do_h && !hdev[i]) out.push_back(copy_matrix(ks[q].dH, kps[i].ng, H[i], ld[i], flags));
+            if (do_s && !sdev[i]) out.push_back(copy_matrix(ks[q].dS, kps[i].ng, S[i], ld[i], flags));
+        }
+        Prefault pages(ctx, out);
         std::vector<OzResult> ozr;
         st = run_ozaki(ctx, geo, ks, flags, icfg, o.slices, o.target_rel_err, ozr, true);
         if (st) return st;
@@ -983,15 +990,6 @@ hsgen_status batched_split(hsgen_ctx* ctx, hsgen_sys* s, int nk, const hsgen_kpo
         ms_all += ms;
         for (size_t q = 0; q < bk.size(); ++q) {
             const int i = bk[q];
-            const bool full = (flags & HSGEN_FILL_UPPER) != 0;
-            if (do_h && !hdev[i]) {
-                st = copy_lower_to_host(ctx, ks[q].dH, kps[i].ng, H[i], ld[i], full);
-                if (st) return st;
-            }
-            if (do_s && !sdev[i]) {
-                st = copy_lower_to_host(ctx, ks[q].dS, kps[i].ng, S[i], ld[i], full);
-                if (st) return st;
-            }
             if (rep) {
                 hsgen_report& r = rep[i];
                 r.slices_used = ozr[q].nmod;
@@ -1002,6 +1000,8 @@ hsgen_status batched_split(hsgen_ctx* ctx, hsgen_sys* s, int nk, const hsgen_kpo
                 r.err_smp_s = ozr[q].smp_s;
             }
         }
+        st = host_copy(ctx, out, true);
+        if (st) return st;
     }
     if (rep) {
         for (int i = 0; i < nk; ++i) {

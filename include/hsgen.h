@@ -56,7 +56,10 @@ typedef enum {
 enum {
     HSGEN_FILL_UPPER = 1,     /* also write the upper triangle (Hermitian mirror) */
     HSGEN_SKIP_H = 2,         /* compute S only */
-    HSGEN_SKIP_S = 4          /* compute H only */
+    HSGEN_SKIP_S = 4,         /* compute H only */
+    HSGEN_CLEAR_UPPER = 8     /* host matrices: zeros above the diagonal (memory that the
+                                 caller has not cleared); device matrices and
+                                 HSGEN_FILL_UPPER: no effect */
 };
 
 typedef struct hsgen_ctx hsgen_ctx;   /* one GPU, one stream */
@@ -100,7 +103,7 @@ typedef struct {
                                   model and an FP64 sample of columns of H and S, then checked
                                   against the model with the exact norms, with a retry) */
     double target_rel_err;     /* split precision: target relative Frobenius error (0 = 1e-12) */
-    int32_t flags;             /* HSGEN_FILL_UPPER | HSGEN_SKIP_H | HSGEN_SKIP_S */
+    int32_t flags;             /* HSGEN_FILL_UPPER | HSGEN_SKIP_H | HSGEN_SKIP_S | HSGEN_CLEAR_UPPER */
     int32_t tile;              /* contraction tile config id (0 = the one hsgen_autotune chose
                                   for this size, else the built-in default for the size: smaller
                                   tiles for calls too small to fill the GPU with the large ones).
