@@ -116,21 +116,18 @@ bool fold_ok(double n)
 // M'_a = D^-1/2 M_a D^-1/2, D = diag(1 on A rows, N_l on B rows), so that
 // Z^H M Z = Y^H M' Y with Y = D^1/2 Z.
 hsgen_status upload_M(hsgen_ctx* ctx, hsgen_sys* s, const int32_t* nlm, const double* const* taa,
-                      const double* const* tab, const double* const* tbb, const double* rsc, int bk, int bm)
+                      const double* const* tab, const double* const* tbb, const double* rsc, int bk, int bm, DevBuf* into,
+                      std::vector<HostCopy> in)
 {
-    if (s->d_M) {
-        (void)hipFree(s->d_M);
-        s->d_M = nullptr;
-        s->d_mloc = nullptr;
-    }
     const int na = s->natoms;
     const int nl = s->nl;
     s->m_off.assign(na, 0);
     s->m_ld.assign(na, 0);
     s->m_cols.assign(na, 0);
     std::map<std::pair<std::vector<const void*>, std::vector<double>>, int> seen;
-    std::vector<int> owner(na, -1);
-    int64_t total = 0;
+    std::vector<MJob> jobs;
+    std::vector<int> owners;
+    int64_t total = 0, most = 0, raw = 0;
     for (int a = 0; a < na; ++a) {
         std::pair<std::vector<const void*>, std::vector<double>> key{
             {taa[a], tab[a], tbb[a], (const void*)(intptr_t)nlm[a]},
@@ -140,63 +137,50 @@ hsgen_status upload_M(hsgen_ctx* ctx, hsgen_sys* s, const int32_t* nlm, const do
         s->m_ld[a] = (int32_t)roundup(n2, bk);
         s->m_cols[a] = (int32_t)roundup(n2, bm);
         if (it != seen.end()) {
-            owner[a] = it->second;
             s->m_off[a] = s->m_off[it->second];
             continue;
         }
         seen[key] = a;
-        owner[a] = a;
         s->m_off[a] = total;
-        total += (int64_t)s->m_ld[a] * s->m_cols[a];
+        owners.push_back(a);
+        const int64_t e = (int64_t)s->m_ld[a] * s->m_cols[a];
+        total += e;
+        most = std::max(most, e);
+        raw += 3 * (int64_t)nlm[a] * nlm[a];
     }
-    std::vector<std::complex<double>> hM((size_t)std::max<int64_t>(total, 1), 0.0);
-    std::vector<double> sq;
-    for (int a = 0; a < na; ++a) {
-        if (owner[a] != a) continue;
-        const int n = nlm[a];
-        const int64_t ld = s->m_ld[a];
-        std::complex<double>* M = hM.data() + s->m_off[a];
-        const std::complex<double>* Taa = (const std::complex<double>*)taa[a];
-        const std::complex<double>* Tab = (const std::complex<double>*)tab[a];
-        const std::complex<double>* Tbb = (const std::complex<double>*)tbb[a];
-        // B-row scale per lm (1 without folding)
-        sq.assign(n, 1.0);
-        if (rsc)
-            for (int lm = 0; lm < n; ++lm) {
-                int l = (int)std::sqrt((double)lm + 0.5);
-                while ((l + 1) * (l + 1) <= lm) ++l;
-                while (l * l > lm) --l;
-                sq[lm] = rsc[(size_t)a * nl + l];
-            }
-        for (int c = 0; c < n; ++c)
-            for (int r = 0; r < n; ++r) {
-                // Hermitian expansion from the lower triangle
-                std::complex<double> aa = r >= c ? Taa[r + (int64_t)n * c] : std::conj(Taa[c + (int64_t)n * r]);
-                std::complex<double> bb = r >= c ? Tbb[r + (int64_t)n * c] : std::conj(Tbb[c + (int64_t)n * r]);
-                if (r == c) { aa = aa.real(); bb = bb.real(); }
-                std::complex<double> ab = Tab[r + (int64_t)n * c];              // T_ab block
-                std::complex<double> ba = std::conj(Tab[c + (int64_t)n * r]);   // T_ab^H block
-                if (rsc) {
-                    ab /= sq[c];
-                    ba /= sq[r];
-                    bb /= sq[r] * sq[c];
-                }
-                M[r + ld * c] = aa;
-                M[(n + r) + ld * (n + c)] = bb;
-                M[r + ld * (n + c)] = ab;
-                M[(n + r) + ld * c] = ba;
-            }
+    // raw blocks, divisors and jobs, only until M is built
+    const size_t b_raw = sizeof(double2) * (size_t)raw, b_rsc = rsc ? sizeof(double) * (size_t)na * nl : 0;
+    hsgen_status st = ensure(ctx, ctx->m_in, b_raw + b_rsc + sizeof(MJob) * owners.size(), false);
+    if (st) return st;
+    double2* d = (double2*)ctx->m_in.p;
+    const double* d_rsc = (const double*)((char*)ctx->m_in.p + b_raw);
+    for (int a : owners) {
+        const int64_t n2 = (int64_t)nlm[a] * nlm[a];
+        const double* src[3] = {taa[a], tab[a], tbb[a]};
+        for (int b = 0; b < 3; ++b) in.push_back(copy_run(d + b * n2, src[b], sizeof(double2) * (size_t)n2));
+        jobs.push_back(MJob{d, d + n2, d + 2 * n2, rsc ? d_rsc + (size_t)a * nl : nullptr, s->m_off[a], nlm[a], s->m_ld[a],
+                            s->m_cols[a], 0});
+        d += 3 * n2;
     }
-    // the per-atom layout table (offset, leading dimension) follows the
-    // blocks in the same allocation, for kernels that build their own work
-    // lists
-    const size_t mbytes = (size_t)roundup((int64_t)(sizeof(double2) * hM.size()), 256);
-    std::vector<MLoc> loc(na);
-    for (int a = 0; a < na; ++a) loc[a] = MLoc{s->m_off[a], s->m_ld[a], s->m_cols[a]};
-    HIPCHK(hipMalloc(&s->d_M, mbytes + sizeof(MLoc) * na));
-    HIPCHK(hipMemcpy(s->d_M, hM.data(), sizeof(double2) * hM.size(), hipMemcpyHostToDevice));
-    s->d_mloc = (MLoc*)((char*)s->d_M + mbytes);
-    HIPCHK(hipMemcpy(s->d_mloc, loc.data(), sizeof(MLoc) * na, hipMemcpyHostToDevice));
+    std::vector<char> tail(b_rsc + sizeof(MJob) * jobs.size());
+    if (rsc) std::memcpy(tail.data(), rsc, b_rsc);
+    std::memcpy(tail.data() + b_rsc, jobs.data(), sizeof(MJob) * jobs.size());
+    in.push_back(copy_run((char*)ctx->m_in.p + b_raw, tail.data(), tail.size()));
+    const size_t b_m = sizeof(double2) * (size_t)std::max<int64_t>(total, 1);
+    if (into) {
+        if ((st = ensure(ctx, *into, b_m, false))) return st;
+        s->d_M = (double2*)into->p;
+    } else {
+        if (s->d_M) (void)hipFree(s->d_M);
+        s->d_M = nullptr;
+        HIPCHK(hipMalloc(&s->d_M, b_m));
+    }
+    if ((st = host_copy(ctx, in, false))) return st;
+    const MJob* dj = (const MJob*)((char*)ctx->m_in.p + b_raw + b_rsc);
+    constexpr size_t kJobs = 32768;      // of one launch's y extent
+    for (size_t j0 = 0; j0 < jobs.size(); j0 += kJobs)
+        HIPCHK(launch_build_m(dj + j0, (int)std::min(kJobs, jobs.size() - j0), most, s->d_M, ctx->stream));
+    if (!into) HIPCHK(hipStreamSynchronize(ctx->stream));    // other contexts may read it
     s->m_bk = bk;
     s->m_bm = bm;
     return HSGEN_OK;
@@ -219,7 +203,7 @@ hsgen_status ensure_M(hsgen_ctx* ctx, hsgen_sys* s, int bk, int bm)
         nlm[a] = s->atoms[a].nlm;
     }
     return upload_M(ctx, s, nlm.data(), pa.data(), pb.data(), pc.data(), s->fold ? s->h_sqrtn.data() : nullptr,
-                    bk, bm);
+                    bk, bm, nullptr, {});
 }
 
 hsgen_status check_kpoint(hsgen_ctx* ctx, const hsgen_kpoint* kp)
@@ -324,9 +308,9 @@ hsgen_status hsgen_release_workspace(hsgen_ctx* ctx)
     HIPCHK(hipSetDevice(ctx->device));
     HIPCHK(hipStreamSynchronize(ctx->stream));
     for (DevBuf* b : {&ctx->Z, &ctx->Zs, &ctx->W, &ctx->Htmp, &ctx->Stmp, &ctx->A, &ctx->B, &ctx->g,
-                      &ctx->probs, &ctx->work, &ctx->unorm2, &ctx->atoms_tmp, &ctx->oz_e, &ctx->oz_res,
+                      &ctx->probs, &ctx->work, &ctx->pack, &ctx->oz_e, &ctx->oz_res,
                       &ctx->oz_out, &ctx->oz_fprob, &ctx->oz_probs, &ctx->oz_work, &ctx->oz_smp, &ctx->btmp,
-                      &ctx->ring_left, &ctx->eig_a, &ctx->eig_b, &ctx->eig_d, &ctx->sph_ph, &ctx->sph_rs, &ctx->sph_y, &ctx->sph_w})
+                      &ctx->ring_left, &ctx->m_in, &ctx->M, &ctx->eig_a, &ctx->eig_b, &ctx->eig_d, &ctx->sph_ph, &ctx->sph_rs, &ctx->sph_y, &ctx->sph_w})
         release(*b);
     for (auto& bg : ctx->bgraphs) {
         if (bg.exec) (void)hipGraphExecDestroy(bg.exec);

@@ -809,14 +809,9 @@ hsgen_status hsgen_contract_hs(hsgen_ctx* ctx, int32_t L, int32_t a, int32_t G, 
     Geometry geo = geometry(o.precision == HSGEN_PREC_FP64 ? o.tile : fp64_tile_by_size(ctx, G), s.kdim, G,
                             o.precision == HSGEN_PREC_FP64 ? 1 : split_col_align(o.precision, o.tile));
     geo.fold = s.fold;
-    hsgen_status st = upload_M(ctx, &s, t_size, t_aa, t_ab, t_bb, s.fold ? s.h_sqrtn.data() : nullptr, geo.t.bk,
-                               geo.t.bm);
-    if (st) return st;
-    struct Guard {
-        hsgen_sys* s;
-        ~Guard() { if (s->d_M) (void)hipFree(s->d_M); s->d_M = nullptr; s->d_mloc = nullptr; }
-    } guard{&s};
-    // device copies of A, B if they are host memory
+    hsgen_status st;
+    // device copies of A, B if they are host memory, with the T blocks and the
+    // packing kernel's tables in one go
     const size_t nab = (size_t)L * a * G;
     const double2* dA = (const double2*)A;
     const double2* dB = (const double2*)B;
@@ -836,16 +831,15 @@ hsgen_status hsgen_contract_hs(hsgen_ctx* ctx, int32_t L, int32_t a, int32_t G, 
         in.push_back(copy_run(ctx->B.p, B, sizeof(double2) * nab));
         dB = (const double2*)ctx->B.p;
     }
-    st = host_copy(ctx, in, false);
+    const size_t b_scale = sizeof(double) * un2.size();
+    std::vector<char> tables(b_scale + sizeof(AtomDev) * a);
+    std::memcpy(tables.data(), s.fold ? s.h_sqrtn.data() : un2.data(), b_scale);
+    std::memcpy(tables.data() + b_scale, s.atoms.data(), sizeof(AtomDev) * a);
+    st = ensure(ctx, ctx->pack, tables.size(), false);
     if (st) return st;
-    st = ensure(ctx, ctx->atoms_tmp, sizeof(AtomDev) * a, false);
+    in.push_back(copy_run(ctx->pack.p, tables.data(), tables.size()));
+    st = upload_M(ctx, &s, t_size, t_aa, t_ab, t_bb, s.fold ? s.h_sqrtn.data() : nullptr, geo.t.bk, geo.t.bm, &ctx->M, in);
     if (st) return st;
-    st = ensure(ctx, ctx->unorm2, sizeof(double) * un2.size(), false);
-    if (st) return st;
-    HIPCHK(hipMemcpyAsync(ctx->atoms_tmp.p, s.atoms.data(), sizeof(AtomDev) * a, hipMemcpyHostToDevice,
-                          ctx->stream));
-    HIPCHK(hipMemcpyAsync(ctx->unorm2.p, s.fold ? s.h_sqrtn.data() : un2.data(), sizeof(double) * un2.size(),
-                          hipMemcpyHostToDevice, ctx->stream));
     const size_t zbytes = sizeof(double2) * (size_t)geo.ldz * geo.gp;
     st = ensure(ctx, ctx->Z, zbytes, false);
     if (st) return st;
@@ -856,8 +850,8 @@ hsgen_status hsgen_contract_hs(hsgen_ctx* ctx, int32_t L, int32_t a, int32_t G, 
     PackParams pp;
     pp.A = dA;
     pp.B = dB;
-    pp.atoms = (const AtomDev*)ctx->atoms_tmp.p;
-    pp.scale = (const double*)ctx->unorm2.p;
+    pp.atoms = (const AtomDev*)((char*)ctx->pack.p + b_scale);
+    pp.scale = (const double*)ctx->pack.p;
     pp.natoms = a;
     pp.L = L;
     pp.nl = s.nl;

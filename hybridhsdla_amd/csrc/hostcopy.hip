@@ -42,6 +42,9 @@ constexpr size_t kSlotBytes = (size_t)4 << 20;
 constexpr size_t kPieceBytes = (size_t)256 << 10;    // what a thread copies at a time
 constexpr size_t kThreadBytes = (size_t)1 << 20;     // one more thread per so many bytes
 constexpr size_t kFlagBytes = 64 * kRingSlots;       // one line per slot, after the slots
+#ifndef GRIDN
+#define GRIDN 24
+#endif
 constexpr int kGroup = kRingSlots / 2;               // slots of one launch
 constexpr size_t kRange = (size_t)2 << 20;           // memory that Prefault maps at a time
 
@@ -73,42 +76,42 @@ struct SlotGroup {
     int32_t n;
 };
 
+// units of 16 bytes [first, n) of one column, `stride` lanes side by side
+__device__ __forceinline__ void copy_units(const char* src, char* dst, uint32_t first, uint32_t n, uint32_t stride)
+{
+    const v2d* s = (const v2d*)src;
+    v2d* d = (v2d*)dst;
+    for (uint32_t u0 = first; u0 < n; u0 += 4 * stride) {
+        v2d v[4];
+#pragma unroll
+        for (uint32_t i = 0; i < 4; ++i)
+            if (u0 + i * stride < n) v[i] = s[u0 + i * stride];
+#pragma unroll
+        for (uint32_t i = 0; i < 4; ++i)
+            if (u0 + i * stride < n) d[u0 + i * stride] = v[i];
+    }
+}
+
 template <bool kToHost>
 __global__ __launch_bounds__(256) void k_slot_copy(SlotGroup g)
 {
     for (int b = 0; b < g.n; ++b) {
         const SlotCopy& p = g.c[b];
-        const size_t w = p.width / 16, total = w * p.height, step = (size_t)gridDim.x * 256;
-        const uint32_t w32 = (uint32_t)w;
-        // addresses of unit u, or nothing above the diagonal
-        auto at = [&](size_t u, char*& d, char*& s) {
-            uint32_t c = 0, r = (uint32_t)u;
-            if (p.height > 1) {
-                c = (uint32_t)u / w32;
-                r = (uint32_t)u - c * w32;
+        const uint32_t w = (uint32_t)(p.width / 16);
+        if (p.height == 1) {             // a run: all workgroups side by side
+            copy_units(kToHost ? p.dev : p.slot, kToHost ? p.slot : p.dev, blockIdx.x * 256 + threadIdx.x, w,
+                       gridDim.x * 256);
+            if (p.width % 16 && blockIdx.x == 0 && threadIdx.x == 0) {     // a multiple of 8 bytes
+                const size_t o = p.width - 8;
+                if (kToHost) *(double*)(p.slot + o) = *(const double*)(p.dev + o);
+                else *(double*)(p.dev + o) = *(const double*)(p.slot + o);
             }
-            d = p.dev + c * p.dpitch + (size_t)r * 16;
-            s = p.slot + u * 16;
-            return !p.lower || r >= c;
-        };
-        for (size_t u0 = (size_t)blockIdx.x * 256 + threadIdx.x; u0 < total; u0 += 4 * step) {
-            v2d v[4];
-            char *d[4], *s[4];
-            bool on[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const size_t u = u0 + i * step;
-                on[i] = u < total && at(u, d[i], s[i]);
-                if (on[i]) v[i] = *(const v2d*)(kToHost ? d[i] : s[i]);
+        } else {
+            for (int c = blockIdx.x; c < p.height; c += gridDim.x) {
+                char* d = p.dev + c * p.dpitch;
+                char* s = p.slot + c * p.width;
+                copy_units(kToHost ? d : s, kToHost ? s : d, (p.lower ? c : 0) + threadIdx.x, w, 256);
             }
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                if (on[i]) *(v2d*)(kToHost ? s[i] : d[i]) = v[i];
-        }
-        if (p.width % 16 && blockIdx.x == 0 && threadIdx.x == 0) {    // one column, a multiple of 8 bytes
-            const size_t o = p.width - 8;
-            if (kToHost) *(double*)(p.slot + o) = *(const double*)(p.dev + o);
-            else *(double*)(p.dev + o) = *(const double*)(p.slot + o);
         }
         __threadfence_system();
         __syncthreads();
@@ -391,7 +394,8 @@ hsgen_status host_copy(hsgen_ctx* ctx, const std::vector<HostCopy>& list, bool t
                                 (uint64_t*)((char*)ctx->ring_dev + kSlotBytes * kN + 64 * i), seq0 + b + g.n};
             most = std::max(most, k.width * k.height);
         }
-        const dim3 grid((unsigned)std::min<size_t>(to_host ? 128 : 64, most / 16384 + 1));
+        const dim3 grid((unsigned)std::min<size_t>(GRIDN, most / 16384 + 1));
+
         if (to_host) hipLaunchKernelGGL(k_slot_copy<true>, grid, dim3(256), 0, ctx->stream, g);
         else hipLaunchKernelGGL(k_slot_copy<false>, grid, dim3(256), 0, ctx->stream, g);
         return hipGetLastError();

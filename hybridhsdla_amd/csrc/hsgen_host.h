@@ -71,13 +71,6 @@ struct DevBuf {
     size_t bytes = 0;
 };
 
-// Where atom a's M_a block lives in the system's device allocation.
-struct MLoc {
-    int64_t off;       // offset of M_a (complex units)
-    int32_t ld;        // leading dimension (2 nlm_a rounded up to the tile's BK)
-    int32_t cols;      // padded column count (2 nlm_a rounded up to the tile's BM)
-};
-
 // Columns to copy between device and host memory; sizes and strides in bytes.
 // Device addresses and strides are multiples of 16, so are sizes of several
 // columns; a run's size is a multiple of 8.
@@ -151,7 +144,7 @@ struct hsgen_ctx {
     hipEvent_t ev[8] = {};
     std::string err;
     // workspace
-    hsgen::DevBuf Z, Zs, W, Htmp, Stmp, A, B, g, probs, work, unorm2, atoms_tmp;
+    hsgen::DevBuf Z, Zs, W, Htmp, Stmp, A, B, g, probs, work, pack, m_in, M;
     // FP64 from a system: phases, radial factors, real vectors (W, host-output copies above)
     hsgen::DevBuf sph_ph, sph_rs, sph_y, sph_w;
     // split precision
@@ -221,7 +214,6 @@ struct hsgen_sys {
     hsgen::RadDev* d_rad = nullptr;
     double* d_ynorm = nullptr;
     double2* d_M = nullptr;
-    hsgen::MLoc* d_mloc = nullptr;     // [natoms] M_a layout, in the same allocation as d_M
     // host copies of the T blocks, so that M can be rebuilt for another tile
     // geometry
     std::vector<std::vector<std::complex<double>>> h_taa, h_tab, h_tbb;
@@ -267,9 +259,11 @@ hsgen_status ensure(hsgen_ctx* ctx, DevBuf& b, size_t bytes, bool zero_new);
 void release(DevBuf& b);
 bool is_device_ptr(const void* p);
 // M_a blocks of every atom padded for tile geometry (bk, bm), deduplicated by
-// T pointer triple, uploaded to s->d_M.
+// T pointer triple, built at s->d_M: in `into`, or (null) in an allocation of
+// the system's own.  in: further copies to the device that the call needs.
 hsgen_status upload_M(hsgen_ctx* ctx, hsgen_sys* s, const int32_t* nlm, const double* const* taa,
-                      const double* const* tab, const double* const* tbb, const double* rsc, int bk, int bm);
+                      const double* const* tab, const double* const* tbb, const double* rsc, int bk, int bm, DevBuf* into,
+                      std::vector<HostCopy> in);
 // Folded operands unless HSGEN_FOLD=0 (environment; tests and comparisons).
 bool fold_enabled();
 // N_l usable for folding (positive, 1/sqrt(N) far from overflow).

@@ -75,6 +75,18 @@ struct MtJob {
     int32_t pad;
 };
 
+// One M_a of the general T application: [T_aa T_ab; T_ab^H T_bb] with the B rows
+// and columns divided by rsc (null: by 1), zero beyond 2 nlm.
+struct MJob {
+    const double2* taa;
+    const double2* tab;
+    const double2* tbb;
+    const double* rsc;   // per l
+    int64_t off;         // of its M (complex units)
+    int32_t nlm, ld, cols;
+    int32_t pad;
+};
+
 // One matrix of split precision's T application, from its Mt.
 struct SplitMtJob {
     int64_t src, dst;    // offsets (complex units)
@@ -129,6 +141,7 @@ struct SphereArgs {
 int sphere_chunk(int nl, int L);
 hipError_t launch_split_mt(const SplitMtJob* jobs, int njobs, int64_t max_elems, const double* sq, const double2* mt,
                            double2* out, hipStream_t st);
+hipError_t launch_build_m(const MJob* jobs, int njobs, int64_t max_elems, double2* m, hipStream_t st);
 hipError_t launch_build_mt(const MtJob* jobs, int njobs, int64_t max_elems, double2* mt, hipStream_t st);
 hipError_t launch_sphere_gen(const SphereArgs& p, hipEvent_t stop, hipStream_t st);
 hipError_t launch_sphere_tapp(const SphereArgs& p, int tile, int rtiles, hipEvent_t stop, hipStream_t st);

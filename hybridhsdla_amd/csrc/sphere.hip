@@ -521,6 +521,35 @@ __device__ __forceinline__ double2 t_elem(const double2* taa, const double2* tab
 
 }  // namespace
 
+// Bound by latency: 7 MB of M for 16 atoms of lmax 8 take 12 us, where a loop on
+// the host with the copy of its result took 1.9 ms.
+__global__ __launch_bounds__(256) void k_build_m(const MJob* __restrict__ jobs, double2* __restrict__ m)
+{
+#pragma clang fp contract(off)
+    const MJob jb = jobs[blockIdx.y];
+    const int n = jb.nlm;
+    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int c = (int)(e / jb.ld), r = (int)(e - (int64_t)c * jb.ld);
+    if (c >= jb.cols) return;
+    double2 v = make_double2(0.0, 0.0);
+    if (r < 2 * n && c < 2 * n) {
+        v = t_elem(jb.taa, jb.tab, jb.tbb, n, r, c);
+        if (jb.rsc && (r >= n || c >= n)) {
+            const double d = (r >= n ? jb.rsc[l_of_lm(r - n)] : 1.0) * (c >= n ? jb.rsc[l_of_lm(c - n)] : 1.0);
+            v.x /= d;
+            v.y /= d;
+        }
+    }
+    m[jb.off + e] = v;
+}
+
+hipError_t launch_build_m(const MJob* jobs, int njobs, int64_t max_elems, double2* m, hipStream_t st)
+{
+    if (njobs <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_build_m, dim3((unsigned)((max_elems + 255) / 256), njobs), dim3(256), 0, st, jobs, m);
+    return hipGetLastError();
+}
+
 __global__ __launch_bounds__(256) void k_build_mt(const MtJob* __restrict__ jobs, double2* __restrict__ mt)
 {
 #pragma clang fp contract(off)
