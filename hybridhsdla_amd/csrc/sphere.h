@@ -133,6 +133,7 @@ struct SphereArgs {
     const int64_t* mtoff;      // [natoms] Mt of each atom, kind order
     const SphereStage* stages;
     int32_t nksteps;
+    int32_t rtiles;            // T application: tiles of rows of all kinds
     int32_t nsquares;          // lower squares of H tiles of all k-points
     uint64_t* stamp;           // starts of the generator, T application, H and S kernels (wall clock), or null
 };

@@ -681,12 +681,13 @@ hipError_t launch_split_mt(const SplitMtJob* jobs, int njobs, int64_t max_elems,
 // vector pipe to the MFMAs.  Rings of 3 and 4 stages, 64 x 128 tiles and waves
 // of 32 x 32 measured no faster for these tiles at any size from 235 to 25000
 // plane waves.
-// The 32 x 32 tiles of H serve triangles that leave CUs idle, with two or three
-// waves per SIMD: there the latency of a stage counts.  Four stages in LDS, the
+// The 32 x 32 tiles of H serve triangles that leave CUs idle, with two to four
+// waves per SIMD: there the latency of a stage counts.  A deeper ring, the
 // fragments of a whole stage read while the one before is multiplied, table
-// entries two barriers ahead: H and S together 21.3 us (two stages 26.9) at
-// N_G 600, 12.5 (13.7) at 235, 1105 (1121) at 2003; the T application, with
-// depths of 10 to 20 stages, gained nothing.
+// entries two barriers ahead: H and S together 20.8 us (two stages without:
+// 26.9) at N_G 600, 12.5 (13.7) at 235, 1075 (1121) at 2003; four stages and
+// three workgroups per CU 21.3, 12.7 and 1112.  The T application, with depths of
+// 10 to 20 stages, loses with a third stage what it loses in workgroups.
 // Rate of the H tiles: 0.87 of the FP64 peak at N_G 16000 and 25000, 0.85 at
 // 10000, 0.82 at 6002 (32 atoms, lmax 10).
 // Measured (whole call, complex-by-complex contraction of S and H before, now):
@@ -699,6 +700,18 @@ typedef double d4 __attribute__((ext_vector_type(4)));
 typedef double v2d __attribute__((ext_vector_type(2)));
 typedef int i8 __attribute__((ext_vector_type(8)));
 typedef __attribute__((address_space(4))) const i8* ctab;
+
+// Columns of a group in the T application's order: an XCD's eighth of a
+// group's y (340 rows at lmax 12) is 1.4 MB of its 4 MB L2.  T application in
+// one group, in groups of 8192, 4096, 2048: 13.2, 12.7, 12.4, 12.4 ms at N_G 12007;
+// a batch of 22800 columns (whole) 17.00, 16.87, 16.75, 16.83 ms; nothing
+// changes up to 4096 columns.  An eighth of the tiles of contiguous columns per
+// XCD instead: 351 -> 370 us at N_G 3001.
+constexpr int kSphereColumns = 4096;
+
+// Stages in LDS of the 32 x 32 tiles of H: three of 13 KB let four workgroups
+// share a CU, as 128 VGPRs do.
+constexpr int kSphereSmall = 3;
 
 // s_waitcnt immediate: at most n vector-memory operations outstanding and, with
 // lgkm, no LDS or scalar ones (vmcnt bits [3:0] and [15:14], expcnt [6:4],
@@ -735,6 +748,12 @@ struct SphereTile {
                   "a stage splits evenly over the waves");
     static_assert(BC % BR == 0, "patches are square in plane waves");
 };
+
+template <class F, int... I>
+__device__ __forceinline__ void stages(const F& f, int s, std::integer_sequence<int, I...>)
+{
+    f(s, std::integral_constant<int, I>{}...);
+}
 
 // Wave-uniform values the compiler is to keep in scalar registers.
 __device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
@@ -793,13 +812,20 @@ __device__ __forceinline__ void sphere_gemm_tile(const SphereArgs& p, int blk, c
         if (R0 >= kp->ng) return;
         nsteps = p.nksteps;
     } else {
-        // kinds in turn; per kind its tiles of rows, per row tile all columns
+        // Columns in groups of P tiles; per group the tiles of rows of all
+        // kinds in turn, per row tile the group's columns, which go to the XCDs
+        // in turn: what an XCD reads of the group's y stays in its L2 while the
+        // rows pass.
+        constexpr int P = kSphereColumns / BC;
         const int ntc = (int)(p.gtot / BC);
-        const int tr = blk / ntc;
+        const int cg = (int)(blk / ((int64_t)P * p.rtiles));
+        const int u = (int)(blk - (int64_t)cg * P * p.rtiles);
+        const int h = min(P, ntc - cg * P);                   // the group's columns
+        const int tr = u / h;
         const int kk = find_last(p.nkinds, tr, [&](int i) { return p.kinds[i].rt32; });
         kd = p.kinds + kk;
         R0 = uni((tr - kd->rt32) * BR);
-        C0 = uni((blk - tr * ntc) * BC);
+        C0 = uni((cg * P + u - tr * h) * BC);
         nsteps = uni(kd->r4 / 4);
     }
     const int64_t col0 = kH ? uni(kp->col0) : 0;
@@ -986,8 +1012,8 @@ __device__ __forceinline__ void sphere_gemm_tile(const SphereArgs& p, int blk, c
         };
         read_stage(0, 0);
         i8 next = entry(min(NS, last));     // the entry of the stage issued next
-        auto stage = [&](auto bufc, int s) {
-            constexpr int buf = decltype(bufc)::value, set = buf & 1;
+        auto stage = [&](auto at, int s) {
+            constexpr int buf = decltype(at)::value % NS, set = decltype(at)::value & 1;
             const i8 e = en[buf];
             __builtin_amdgcn_s_waitcnt(wait_vm(63, true));
             if (s < last) {
@@ -1019,16 +1045,9 @@ __device__ __forceinline__ void sphere_gemm_tile(const SphereArgs& p, int blk, c
                 }
             }
         };
-        int s = 0;
-        for (; s + NS <= nst; s += NS) {
-            stage(std::integral_constant<int, 0>{}, s);
-            stage(std::integral_constant<int, 1>{}, s + 1);
-            stage(std::integral_constant<int, 2>{}, s + 2);
-            stage(std::integral_constant<int, 3>{}, s + 3);
-        }
-        if (s < nst) stage(std::integral_constant<int, 0>{}, s);
-        if (s + 1 < nst) stage(std::integral_constant<int, 1>{}, s + 1);
-        if (s + 2 < nst) stage(std::integral_constant<int, 2>{}, s + 2);
+        constexpr int U = NS % 2 ? 2 * NS : NS;     // buffers and register sets in step
+        auto round = [&](int s, auto... i) { (((int)i + s < nst ? stage(i, s + (int)i) : (void)0), ...); };
+        for (int s = 0; s < nst; s += U) stages(round, s, std::make_integer_sequence<int, U>{});
     } else {
         v2d fx[RB];
         double fy[CB];
@@ -1130,11 +1149,11 @@ __global__ __launch_bounds__((SphereTile<BR, BC, RB, CB, NS>::kThreads), 4) void
 // H tiles of 32 x 32 and S tiles of 16 M x 16 M in one launch, for triangles
 // whose H tiles leave CUs or the vector pipe idle: S costs no time of its own.
 template <int M>
-__global__ __launch_bounds__(256, 2) void k_sphere_hs(SphereArgs p, int hblocks)
+__global__ __launch_bounds__(256, 4) void k_sphere_hs(SphereArgs p, int hblocks)
 {
     extern __shared__ __attribute__((aligned(1024))) char lds[];
     stamp(p, 2);
-    if ((int)blockIdx.x < hblocks) sphere_gemm_tile<32, 32, 1, 1, 4, true>(p, (int)blockIdx.x, lds);
+    if ((int)blockIdx.x < hblocks) sphere_gemm_tile<32, 32, 1, 1, kSphereSmall, true>(p, (int)blockIdx.x, lds);
     else overlap_tile<M, M>(p, (int)blockIdx.x - hblocks, (double*)lds);
 }
 
@@ -1148,8 +1167,11 @@ static hipError_t launch_sphere_gemm(const SphereArgs& p, int64_t nblk, hipEvent
 // rtiles: row tiles of all kinds for the tile's rows (tile 64: 32 x 64)
 hipError_t launch_sphere_tapp(const SphereArgs& p, int tile, int rtiles, hipEvent_t stop, hipStream_t st)
 {
-    if (tile == 32) return launch_sphere_gemm<32, 32, 1, 1, 2, false>(p, (int64_t)rtiles * (p.gtot / 32), stop, st);
-    return launch_sphere_gemm<32, 64, 1, 2, 2, false>(p, (int64_t)rtiles * (p.gtot / 64), stop, st);
+    SphereArgs q = p;
+    q.rtiles = rtiles;
+    const int64_t nblk = (int64_t)rtiles * (p.gtot / (tile == 32 ? 32 : 64));
+    if (tile == 32) return launch_sphere_gemm<32, 32, 1, 1, 2, false>(q, nblk, stop, st);
+    return launch_sphere_gemm<32, 64, 1, 2, 2, false>(q, nblk, stop, st);
 }
 
 static int64_t hblocks(const SphereArgs& p, int tile) { return ((int64_t)p.nsquares * (tile == 48 ? 2 : 1) + 7) / 8 * 8; }
@@ -1158,7 +1180,7 @@ static int64_t hblocks(const SphereArgs& p, int tile) { return ((int64_t)p.nsqua
 hipError_t launch_sphere_h(const SphereArgs& p, int tile, hipEvent_t stop, hipStream_t st)
 {
     const int64_t n = hblocks(p, tile);
-    if (tile == 32) return launch_sphere_gemm<32, 32, 1, 1, 4, true>(p, n, stop, st);
+    if (tile == 32) return launch_sphere_gemm<32, 32, 1, 1, kSphereSmall, true>(p, n, stop, st);
     if (tile == 48) return launch_sphere_gemm<32, 64, 1, 2, 2, true>(p, n, stop, st);
     return launch_sphere_gemm<64, 64, 1, 2, 2, true>(p, n, stop, st);
 }
@@ -1167,7 +1189,7 @@ template <int M>
 static hipError_t launch_hs(const SphereArgs& p, int64_t nstiles, hipEvent_t stop, hipStream_t st)
 {
     const int64_t n = hblocks(p, 32);
-    const size_t lds = std::max<size_t>(SphereTile<32, 32, 1, 1, 4>::kLds, overlap_lds(16 * M, p.nl));
+    const size_t lds = std::max<size_t>(SphereTile<32, 32, 1, 1, kSphereSmall>::kLds, overlap_lds(16 * M, p.nl));
     return launch(k_sphere_hs<M>, dim3((unsigned)(n + nstiles)), 256, lds, stop, st, p, (int)n);
 }
 
