@@ -175,7 +175,7 @@ hsgen_status upload_M(hsgen_ctx* ctx, hsgen_sys* s, const int32_t* nlm, const do
         s->d_M = nullptr;
         HIPCHK(hipMalloc(&s->d_M, b_m));
     }
-    if ((st = host_copy(ctx, in, false))) return st;
+    if ((st = host_copy(ctx, in, false, ctx->stream))) return st;
     const MJob* dj = (const MJob*)((char*)ctx->m_in.p + b_raw + b_rsc);
     constexpr size_t kJobs = 32768;      // of one launch's y extent
     for (size_t j0 = 0; j0 < jobs.size(); j0 += kJobs)
@@ -308,7 +308,7 @@ hsgen_status hsgen_release_workspace(hsgen_ctx* ctx)
     HIPCHK(hipSetDevice(ctx->device));
     HIPCHK(hipStreamSynchronize(ctx->stream));
     for (DevBuf* b : {&ctx->Z, &ctx->Zs, &ctx->W, &ctx->Htmp, &ctx->Stmp, &ctx->A, &ctx->B, &ctx->g,
-                      &ctx->probs, &ctx->work, &ctx->pack, &ctx->oz_e, &ctx->oz_res,
+                      &ctx->probs, &ctx->work, &ctx->probs2, &ctx->work2, &ctx->tprobs, &ctx->twork, &ctx->pack, &ctx->oz_e, &ctx->oz_res,
                       &ctx->oz_out, &ctx->oz_fprob, &ctx->oz_probs, &ctx->oz_work, &ctx->oz_smp, &ctx->btmp,
                       &ctx->ring_left, &ctx->m_in, &ctx->M, &ctx->eig_a, &ctx->eig_b, &ctx->eig_d, &ctx->sph_ph, &ctx->sph_rs, &ctx->sph_y, &ctx->sph_w})
         release(*b);
@@ -337,6 +337,7 @@ hsgen_status hsgen_finalize(hsgen_ctx* ctx)
     if (ctx->ring) (void)hipHostFree(ctx->ring);
     if (ctx->pin) (void)hipHostFree(ctx->pin);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
+    if (ctx->stream2) (void)hipStreamDestroy(ctx->stream2);
     delete ctx;
     return HSGEN_OK;
 }

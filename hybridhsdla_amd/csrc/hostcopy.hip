@@ -329,7 +329,7 @@ Prefault::~Prefault()
     ctx_->prefault = nullptr;
 }
 
-hsgen_status host_copy(hsgen_ctx* ctx, const std::vector<HostCopy>& list, bool to_host)
+hsgen_status host_copy(hsgen_ctx* ctx, const std::vector<HostCopy>& list, bool to_host, hipStream_t stream)
 {
     constexpr int kN = kRingSlots;
     Plan plan;
@@ -351,10 +351,13 @@ hsgen_status host_copy(hsgen_ctx* ctx, const std::vector<HostCopy>& list, bool t
         std::memset((char*)p + kSlotBytes * kN, 0, kFlagBytes);
         ctx->ring = (char*)p;
     }
-    const hsgen_status st = ensure(ctx, ctx->ring_left, sizeof(uint32_t) * kN, true);
-    if (st) return st;
+    if (!ctx->ring_left.p) {
+        const hsgen_status st = ensure(ctx, ctx->ring_left, sizeof(uint32_t) * kN, true);
+        if (st) return st;
+        HIPCHK(hipStreamSynchronize(ctx->stream));
+    }
     // an earlier copy to the device may still read the slots
-    if (!to_host) HIPCHK(hipStreamSynchronize(ctx->stream));
+    if (!to_host) HIPCHK(hipStreamSynchronize(stream));
 
     auto slot = [&](int b) { return ctx->ring + kSlotBytes * (size_t)(b % kN); };
     std::unique_ptr<std::atomic<int>[]> done(new std::atomic<int>[n]);    // pieces of a block that are copied
@@ -396,8 +399,8 @@ hsgen_status host_copy(hsgen_ctx* ctx, const std::vector<HostCopy>& list, bool t
         }
         const dim3 grid((unsigned)std::min<size_t>(GRIDN, most / 16384 + 1));
 
-        if (to_host) hipLaunchKernelGGL(k_slot_copy<true>, grid, dim3(256), 0, ctx->stream, g);
-        else hipLaunchKernelGGL(k_slot_copy<false>, grid, dim3(256), 0, ctx->stream, g);
+        if (to_host) hipLaunchKernelGGL(k_slot_copy<true>, grid, dim3(256), 0, stream, g);
+        else hipLaunchKernelGGL(k_slot_copy<false>, grid, dim3(256), 0, stream, g);
         return hipGetLastError();
     };
     auto landed = [&](int b) {
@@ -441,7 +444,7 @@ hsgen_status host_copy(hsgen_ctx* ctx, const std::vector<HostCopy>& list, bool t
                 idle = 0;
             } else if (++idle % 4096 == 0) {
                 // a stream that failed, or is done without the flag, ends the wait
-                const hipError_t q = hipStreamQuery(ctx->stream);
+                const hipError_t q = hipStreamQuery(stream);
                 if (q == hipErrorNotReady) (void)hipGetLastError();
                 else if (q != hipSuccess) e = q;
                 else if (!landed(oldest)) e = hipErrorUnknown;
@@ -456,7 +459,7 @@ hsgen_status host_copy(hsgen_ctx* ctx, const std::vector<HostCopy>& list, bool t
     }
     stop.store(true);
     if (threads) threads->finish(&plan);
-    if (e != hipSuccess) (void)hipStreamSynchronize(ctx->stream);
+    if (e != hipSuccess) (void)hipStreamSynchronize(stream);
     HIPCHK(e);
     return HSGEN_OK;
 }

@@ -141,10 +141,11 @@ private:
 struct hsgen_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
+    hipStream_t stream2 = nullptr;                   // S beside the T application and H
     hipEvent_t ev[8] = {};
     std::string err;
     // workspace
-    hsgen::DevBuf Z, Zs, W, Htmp, Stmp, A, B, g, probs, work, pack, m_in, M;
+    hsgen::DevBuf Z, Zs, W, Htmp, Stmp, A, B, g, probs, work, pack, m_in, M, probs2, work2, tprobs, twork;
     // FP64 from a system: phases, radial factors, real vectors (W, host-output copies above)
     hsgen::DevBuf sph_ph, sph_rs, sph_y, sph_w;
     // split precision
@@ -271,7 +272,9 @@ bool fold_ok(double n);
 hsgen_status ensure_M(hsgen_ctx* ctx, hsgen_sys* s, int bk, int bm);
 hsgen_status check_kpoint(hsgen_ctx* ctx, const hsgen_kpoint* kp);
 hsgen_status upload_g(hsgen_ctx* ctx, const hsgen_kpoint* kp);
-hsgen_status host_copy(hsgen_ctx* ctx, const std::vector<HostCopy>& list, bool to_host);
+// Copies of a call, started on `stream` and complete on return (to the device:
+// the host side is; calls with different streams order their slots' use).
+hsgen_status host_copy(hsgen_ctx* ctx, const std::vector<HostCopy>& list, bool to_host, hipStream_t stream);
 
 // ---- fp64_path.hip ----
 struct Geometry {

@@ -1000,7 +1000,7 @@ hsgen_status batched_split(hsgen_ctx* ctx, hsgen_sys* s, int nk, const hsgen_kpo
                 r.err_smp_s = ozr[q].smp_s;
             }
         }
-        st = host_copy(ctx, out, true);
+        st = host_copy(ctx, out, true, ctx->stream);
         if (st) return st;
     }
     if (rep) {
