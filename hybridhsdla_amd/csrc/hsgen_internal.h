@@ -143,16 +143,28 @@ struct IgemmProblem {
     int32_t m, n, kdepth, lower;
 };
 
-// One modulus of an INT8 launch.  The kernel writes C mod p, as (re, im)
-// byte pairs in [0, p), into out: tile slot s owns bytes [2 s BM BN,
+// The moduli of an INT8 launch: its blocks are the tiles of the work list, for
+// every modulus in turn.  The kernel writes C mod p, as (re, im) byte pairs in
+// [0, p), into the modulus's part of out: tile slot s owns bytes [2 s BM BN,
 // 2 (s+1) BM BN), in the order the MFMA fragments hold them (element
 // (wave, i, j, q, lane) at (((wave RB + i) CB + j) 4 + q) 64 + lane, see
 // igemm_frag_pos).  Launches after the first depth chunk add to what is there.
+struct IgemmModuli {
+    int32_t n;
+    int32_t first_chunk;
+    int32_t chunk_stages;
+    int32_t prob_stride;        // problems of a modulus's set, to the next one's
+    int64_t mod_stride;         // bytes of out per modulus
+    uint8_t* out;
+    int32_t p[16];
+    double invp[16];
+};
+
+// One of them, as a block sees it.
 struct IgemmModulus {
     int32_t p;
     int32_t first_chunk;
     int32_t chunk_stages;
-    int32_t pad;
     double invp;
     uint8_t* out;
 };
@@ -198,7 +210,7 @@ hipError_t launch_gather_cols(const double2* X, int64_t ld, const int32_t* cols,
 hipError_t launch_residues(const OzResParams& p, int ncols, hipStream_t st);
 IgemmLaunchCfg igemm_cfg(int id);
 hipError_t launch_igemm(int id, const IgemmProblem* probs, const TileWork* work, int nwork,
-                        const IgemmModulus& md, hipStream_t st);
+                        const IgemmModuli& md, hipStream_t st);
 hipError_t launch_crt_final(const OzFinalParams& p, const TileWork* work, int nwork, hipStream_t st);
 
 }  // namespace hsgen

@@ -335,6 +335,12 @@ __device__ __forceinline__ int igemm_frag_pos(int wave, int i, int j, int q, int
 // lane holds D[4*(lane>>4) + q][lane & 15] of MFMA block (i, j) in register q.
 // Every element of the tile is written, padding included: the recombination
 // reads only the lower-triangle elements inside the matrix.
+__device__ __forceinline__ IgemmModulus block_modulus(const IgemmModuli& m)
+{
+    const int i = blockIdx.y;
+    return IgemmModulus{m.p[i], m.first_chunk, m.chunk_stages, m.invp[i], m.out + (int64_t)i * m.mod_stride};
+}
+
 template <int RB, int CB, int TILE>
 __device__ __forceinline__ void store_residues(const IgemmModulus& md, int slot, int wave, int lane,
                                                const i4v (&are)[RB][CB], const i4v (&aim)[RB][CB])
@@ -384,7 +390,7 @@ struct IgemmCfg {
 template <int BM, int BN, int BK, int WGM, int WGN>
 __global__ __launch_bounds__(WGM * WGN * 64) void k_igemm_crt(const IgemmProblem* __restrict__ probs,
                                                               const TileWork* __restrict__ work, int nwork,
-                                                              IgemmModulus md)
+                                                              IgemmModuli mds)
 {
     using Cfg = IgemmCfg<BM, BN, BK, WGM, WGN>;
     constexpr int NT = Cfg::kThreads;
@@ -396,6 +402,8 @@ __global__ __launch_bounds__(WGM * WGN * 64) void k_igemm_crt(const IgemmProblem
 
     const int wid = blockIdx.x;
     if (wid >= nwork) return;
+    const IgemmModulus md = block_modulus(mds);
+    probs += (int64_t)blockIdx.y * mds.prob_stride;
     const TileWork tw = work[wid];
     const IgemmProblem pb = probs[tw.prob];
     const int I0 = tw.bi * BM;
@@ -585,7 +593,7 @@ __device__ inline int rot_bf16(int x)
 template <int BM, int BN, int KS, int WGM, int WGN, int NS, int ROTR, int ES = 1>
 __global__ __launch_bounds__(WGM * WGN * 64) void k_igemm2_crt(const IgemmProblem* __restrict__ probs,
                                                                const TileWork* __restrict__ work, int nwork,
-                                                               IgemmModulus md)
+                                                               IgemmModuli mds)
 {
     using Cfg = Igemm2Cfg<BM, BN, KS, WGM, WGN, NS, ROTR, ES>;
     using AccT = typename std::conditional<ES == 1, i4v, f4v>::type;
@@ -597,6 +605,8 @@ __global__ __launch_bounds__(WGM * WGN * 64) void k_igemm2_crt(const IgemmProble
 
     const int wid = blockIdx.x;
     if (wid >= nwork) return;
+    const IgemmModulus md = block_modulus(mds);
+    probs += (int64_t)blockIdx.y * mds.prob_stride;
     const TileWork tw = work[wid];
     const IgemmProblem pb = probs[tw.prob];
     const int I0 = tw.bi * BM;
@@ -909,9 +919,9 @@ IgemmLaunchCfg igemm_cfg(int id)
 }
 
 hipError_t launch_igemm(int id, const IgemmProblem* probs, const TileWork* work, int nwork,
-                        const IgemmModulus& md, hipStream_t st)
+                        const IgemmModuli& md, hipStream_t st)
 {
-    if (nwork <= 0) return hipSuccess;
+    if (nwork <= 0 || md.n <= 0) return hipSuccess;
 #define X(ID, BM, BN, BK, WGM, WGN)                                                            \
     if (id == ID) {                                                                            \
         constexpr int lds = IgemmCfg<BM, BN, BK, WGM, WGN>::kStageBytes * 2;                  \
@@ -919,7 +929,7 @@ hipError_t launch_igemm(int id, const IgemmProblem* probs, const TileWork* work,
         hipError_t e = hipFuncSetAttribute((const void*)k_igemm_crt<BM, BN, BK, WGM, WGN>,      \
                                            hipFuncAttributeMaxDynamicSharedMemorySize, lds);     \
         if (e != hipSuccess) return e;                                                         \
-        hipLaunchKernelGGL((k_igemm_crt<BM, BN, BK, WGM, WGN>), dim3(nwork), dim3(WGM * WGN * 64), \
+        hipLaunchKernelGGL((k_igemm_crt<BM, BN, BK, WGM, WGN>), dim3(nwork, md.n), dim3(WGM * WGN * 64), \
                            lds, st, probs, work, nwork, md);                                   \
         return hipGetLastError();                                                              \
     }
@@ -932,7 +942,7 @@ hipError_t launch_igemm(int id, const IgemmProblem* probs, const TileWork* work,
         hipError_t e = hipFuncSetAttribute((const void*)k_igemm2_crt<BM, BN, KS, WGM, WGN, NS, ROTR>, \
                                            hipFuncAttributeMaxDynamicSharedMemorySize, lds);       \
         if (e != hipSuccess) return e;                                                           \
-        hipLaunchKernelGGL((k_igemm2_crt<BM, BN, KS, WGM, WGN, NS, ROTR>), dim3(nwork),           \
+        hipLaunchKernelGGL((k_igemm2_crt<BM, BN, KS, WGM, WGN, NS, ROTR>), dim3(nwork, md.n),           \
                            dim3(WGM * WGN * 64), lds, st, probs, work, nwork, md);               \
         return hipGetLastError();                                                                \
     }
@@ -944,7 +954,7 @@ hipError_t launch_igemm(int id, const IgemmProblem* probs, const TileWork* work,
         hipError_t e = hipFuncSetAttribute((const void*)k_igemm2_crt<BM, BN, KS, WGM, WGN, NS, 0, 2>, \
                                            hipFuncAttributeMaxDynamicSharedMemorySize, lds);       \
         if (e != hipSuccess) return e;                                                           \
-        hipLaunchKernelGGL((k_igemm2_crt<BM, BN, KS, WGM, WGN, NS, 0, 2>), dim3(nwork),           \
+        hipLaunchKernelGGL((k_igemm2_crt<BM, BN, KS, WGM, WGN, NS, 0, 2>), dim3(nwork, md.n),           \
                            dim3(WGM * WGN * 64), lds, st, probs, work, nwork, md);               \
         return hipGetLastError();                                                                \
     }

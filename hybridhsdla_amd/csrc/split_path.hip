@@ -187,8 +187,8 @@ OzSlotLayout oz_slots(const IgemmLaunchCfg& ic, bool fold)
 }
 
 // One split-precision evaluation of every k-point with nmod moduli: residues,
-// INT8 GEMMs that store C mod p (one launch per modulus over the tiles of all
-// k-points), final recombination into the outputs.  With capture the launch
+// INT8 GEMMs that store C mod p (one launch per residue group over the tiles of
+// all k-points and moduli), final recombination into the outputs.  With capture the launch
 // segments (per residue group: its residue pass, then its INT8 launches; then
 // the recombination) are captured into hipGraphs on the first call with a
 // given key (modulus count, k-points, outputs, workspace addresses) and
@@ -427,24 +427,30 @@ hsgen_status oz_execute(hsgen_ctx* ctx, const Geometry& geo, const std::vector<O
         if (st) return st;
         HIPCHK(hipEventRecord(ctx->oz_ev[2 * ngroups], ctx->stream));
         st = segment([&]() -> hipError_t {
+            // all moduli of the group in one launch per depth chunk: the tiles of
+            // the next one fill what a modulus's last round leaves idle.  INT8 GEMMs
+            // of 12 moduli, one launch each before: 4 k-points of 1900 plane waves
+            // 6.97 -> 6.02 ms, 2 of 1200 1.09 -> 0.94; at N_G 6002, 3.2 rounds per
+            // modulus at the board's power limit, 12.4 ms both.
+            IgemmModuli md;
+            std::memset(&md, 0, sizeof md);
+            md.n = gn;
+            // INT8: 2048 MFMA k-steps <= 2080 (|acc| < 2^31); BF16: 32 k-steps of
+            // 32 x 127^2 each, exact in FP32 (|acc| < 2^24); a stage holds bk / 32
+            // (INT8) or bk / 16 (BF16) k-steps
+            md.chunk_stages = ic.esize == 1 ? 2048 / (ic.bk / 32) : 32 / (ic.bk / 16);
+            md.prob_stride = (int32_t)(nchunk * nprob);
+            md.mod_stride = (int64_t)mod_stride;
+            md.out = rout + (size_t)m0 * mod_stride;
             for (int i = 0; i < gn; ++i) {
-                const int m = m0 + i;
-                for (int c = 0; c < nchunk; ++c) {
-                    IgemmModulus md;
-                    md.p = kModuli[m];
-                    md.first_chunk = c == 0;
-                    // INT8: 2048 MFMA k-steps <= 2080 (|acc| < 2^31); BF16: 32 k-steps of
-                    // 32 x 127^2 each, exact in FP32 (|acc| < 2^24); a stage holds bk / 32
-                    // (INT8) or bk / 16 (BF16) k-steps
-                    md.chunk_stages = ic.esize == 1 ? 2048 / (ic.bk / 32) : 32 / (ic.bk / 16);
-                    md.pad = 0;
-                    md.invp = 1.0 / kModuli[m];
-                    md.out = rout + (size_t)m * mod_stride;
-                    const hipError_t e =
-                        launch_igemm(icfg, (const IgemmProblem*)b_probs.p + (i * nchunk + c) * nprob,
-                                     (const TileWork*)b_work.p, (int)work.size(), md, ctx->stream);
-                    if (e != hipSuccess) return e;
-                }
+                md.p[i] = kModuli[m0 + i];
+                md.invp[i] = 1.0 / kModuli[m0 + i];
+            }
+            for (int c = 0; c < nchunk; ++c) {
+                md.first_chunk = c == 0;
+                const hipError_t e = launch_igemm(icfg, (const IgemmProblem*)b_probs.p + c * nprob,
+                                                  (const TileWork*)b_work.p, (int)work.size(), md, ctx->stream);
+                if (e != hipSuccess) return e;
             }
             return hipSuccess;
         });
@@ -781,7 +787,7 @@ hsgen_status run_ozaki(hsgen_ctx* ctx, const Geometry& geo, const std::vector<Oz
 // columns padded to a multiple of both INT8 tile sides), ONE grouped launch
 // for the T application of all their columns, then one split-precision
 // evaluation of the whole batch: per modulus count that its k-points need,
-// one INT8 launch per modulus over the tiles of all of them.  Each k-point
+// one INT8 launch over the tiles of all of them and all moduli.  Each k-point
 // gets the modulus count its own error model asks for, so its H and S are
 // those of a single-k call, bit for bit.
 // ---------------------------------------------------------------------------
