@@ -44,7 +44,7 @@ struct KindDev {
 struct OverlapGroup {
     int32_t lmax;
     int32_t rep;         // an atom of it (system order): RadDev row
-    int32_t rsoff;       // first row of the radial factors
+    int32_t rsoff;       // first row of the radial factors (a_l, b_l), then of the weighted ones
     int32_t first, count;   // its atoms, in kind order
     int32_t newdir;      // directions differ from the group before
     double rot[9];       // the rotation that stands for the cosines
@@ -124,7 +124,7 @@ struct SphereArgs {
     const SphereK* many;
     int64_t gtot;              // columns of the operand arrays
     double2* ph;               // [natoms][gtot] phases, kind order
-    double2* rs;               // [gtot][ldr] radial factors (a_l, b_l)
+    double2* rs;               // [gtot][ldr] radial factors per overlap group: (a_l, b_l), then with S's weights
     int32_t ldr;
     double* y;                 // [gtot][ldy] real vectors of all kinds, or null (S alone)
     double2* W;                // [gtot][ldw]

@@ -200,7 +200,14 @@ __global__ __launch_bounds__(256) void k_sphere_gen(SphereArgs p)
             const double bu = -m.u * Knorm * dfj[l] + m.u_dr * fj[l];
             const double2 ab = make_double2(pref * au, pref * bu);
             s_ab[t * nl + l] = ab;
-            if (!kSplit && kd.rsoff >= 0) p.rs[col * p.ldr + kd.rsoff + l] = ab;
+            if (!kSplit && kd.rsoff >= 0) {
+                // as they are, and with the weights of S
+                double2* r = p.rs + col * p.ldr + kd.rsoff + l;
+                const double wl = (2 * l + 1) / (4.0 * kPi);
+                const double wb = wl * m.dE_u_norm;
+                r[0] = ab;
+                r[kd.lmax + 1] = make_double2(wl * ab.x, wb * ab.y);
+            }
         }
         if (p.y) {
             // from the other end: the first waves have the radial factors
@@ -247,50 +254,79 @@ hipError_t launch_sphere_gen(const SphereArgs& p, hipEvent_t stop, hipStream_t s
 
 // ---------------------------------------------------------------------------
 // S by the addition theorem.  One workgroup per lower tile of 16 M x 16 M,
-// M x MJ elements per thread (rows tx + 16 m: stores of 16 consecutive rows).  Per group, per element: the Legendre sum (7
-// FP64 operations per l) and 4 fused operations per atom, against
-// 8 (2 L) per atom of the contraction S = Y^H Y it replaces; vector FP64 and
-// the LDS reads (M + MJ of 16 bytes per M MJ elements) bound it.  Measured:
-// 6.1 ms at N_G 12007 (128 atoms of 8 kinds, lmax 12), where the contraction
-// took about 350 ms; 0.10 ms at N_G 2003 (32 atoms, 4 kinds, lmax 10).  Atoms
-// whose rotations leave the cosines as they are share a group: at N_G 3001 24
-// atoms of 3 types and 22 rotations took 0.83 ms as 24 sums, 0.18 ms as 3.
+// M x MJ elements per thread (rows tx + 16 m: stores of 16 consecutive rows).
+// Per group, per element: the Legendre sum (6 FP64 operations per l) and 4 fused
+// operations per atom, against 8 (2 L) per atom of the contraction S = Y^H Y it
+// replaces.  Vector FP64 takes a third of its time, the start and end of a tile
+// (one workgroup of 64 x 64 per CU) most of the rest: a group's radial factors
+// and phases go straight into LDS while the group before is summed, and the
+// factors of the next l are read ahead.  Measured: 5.5 ms at N_G 12007 (128
+// atoms of 8 kinds, lmax 12; 6.0 with the loads in front of each group), where
+// the contraction took about 350 ms; 0.52 (0.59) ms at 6002 (32 atoms, 4 kinds,
+// lmax 10).  Atoms whose rotations leave the cosines as they are share a group:
+// at N_G 3001 24 atoms of 3 types and 22 rotations took 0.83 ms as 24 sums, 0.12
+// ms as 3.
 //
 // P_l comes from t = 1 - |cos| = |n -+ n'|^2 / 2, formed from the difference
 // (sum, where the cosine is negative) of the unit vectors, by
-//   P_l+1 - P_l = (l (P_l - P_l-1) - (2l+1) t P_l) / (l+1):
+//   D_l+1 = D_l - (2l+1) t P_l,  P_l+1 = P_l + D_l+1 / (l+1):
 // near parallel and antiparallel vectors, where P_l varies fastest, t keeps
 // its relative accuracy, which a cosine would lose.  Odd l carry the sign.
 // ---------------------------------------------------------------------------
-constexpr int kOvAtoms = 8;     // atoms whose phases are staged at a time
+namespace {
+
+typedef double v2d __attribute__((ext_vector_type(2)));
+
+// s_waitcnt immediate: at most n vector-memory operations outstanding and, with
+// lgkm, no LDS or scalar ones (vmcnt bits [3:0] and [15:14], expcnt [6:4],
+// lgkmcnt [11:8]).
+constexpr int wait_vm(int n, bool lgkm)
+{
+    return (n & 15) | (7 << 4) | ((lgkm ? 0 : 15) << 8) | ((n >> 4) << 14);
+}
 
 struct LegendreCoef {
-    double a[kMaxLmax + 1], b[kMaxLmax + 1];
+    double v[kMaxLmax + 1];
 };
 constexpr LegendreCoef legendre_coef()
 {
     LegendreCoef c{};
-    for (int l = 0; l <= kMaxLmax; ++l) {
-        c.a[l] = (double)l / (double)(l + 1);
-        c.b[l] = (double)(2 * l + 1) / (double)(l + 1);
-    }
+    for (int l = 0; l <= kMaxLmax; ++l) c.v[l] = 1.0 / (double)(l + 1);
     return c;
 }
 __constant__ const LegendreCoef kLegendre = legendre_coef();
 
+// 1 KiB into LDS: lane i's 16 bytes at dst + 16 i
+__device__ __forceinline__ void load_lds(const void* src, char* dst)
+{
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                     (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
+}
+
+}  // namespace
+
+// Wave-uniform values the compiler is to keep in scalar registers.
+__device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
+
 template <int M, int MJ>
-__device__ __forceinline__ void overlap_tile(const SphereArgs& p, int blk, double* smem)
+struct OverlapTile {
+    static constexpr int T = 16 * M, TY = T / MJ, NT = 16 * TY, NW = NT / 64;
+    static constexpr int kAtoms = M == 2 ? 4 : 8;        // whose phases are staged at a time
+    static constexpr int kPlane = T * 256;               // 16 values of l of T columns
+    static constexpr int kPhases = 2 * kAtoms * T * 16;  // of the rows, of the columns
+    // two buffers of each; planes: of 16 values of l
+    static constexpr int lds(int planes) { return 4 * planes * kPlane + 2 * kPhases; }
+};
+
+template <int M, int MJ, bool kAhead>
+__device__ __forceinline__ void overlap_tile(const SphereArgs& p, int blk, char* lds)
 {
     // one rounding per written operation: every tile gives the same bits
 #pragma clang fp contract(off)
-    constexpr int T = 16 * M, TY = T / MJ, NT = 16 * TY;
-    double2* s_ri = (double2*)smem;               // [nl][T] (a_l, b_l) of the rows
-    double2* s_rj = s_ri + p.nl * T;              // [nl][T] weighted, of the columns
-    double2* s_pi = s_rj + p.nl * T;              // [kOvAtoms][T] phases
-    double2* s_pj = s_pi + kOvAtoms * T;
-    double* s_n = (double*)(s_pj + kOvAtoms * T); // [2][3][T] unit vectors
-
-    const int tid = threadIdx.x;
+    using Ov = OverlapTile<M, MJ>;
+    constexpr int T = Ov::T, TY = Ov::TY, NW = Ov::NW, kAtoms = Ov::kAtoms;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = uni(tid >> 6);
     const int tx = tid & 15, ty = tid >> 4;
     const SphereK* kp = &p.one;
     if (p.nk > 1) kp = p.many + find_last(p.nk, blk, [&](int i) { return p.many[i].stile0; });
@@ -300,8 +336,37 @@ __device__ __forceinline__ void overlap_tile(const SphereArgs& p, int blk, doubl
     const int I0 = bi * T, J0 = bj * T;
     const int ng = kp->ng;
     const int64_t ci = kp->col0 + I0, cj = kp->col0 + J0;
+    const int planes = (p.nl + 15) / 16;
+    char* const ph0 = lds + 4 * planes * Ov::kPlane;
+    // constant address space: the groups come by scalar loads
+    typedef __attribute__((address_space(4))) const OverlapGroup* cgroups;
+    const cgroups groups = (cgroups)(const void*)p.groups;
 
-    double sr[M][MJ], si[M][MJ], t[M][MJ], sg[M][MJ];
+    // Radial factors of group kk (rows: as they are, columns: weighted):
+    // [buffer][side][plane][T][16], value l of column c at l ^ (c % 16) so that
+    // 16 columns hit distinct banks; past the last l that one again.
+    auto load_radial = [&](int kk, int buf) {
+        const auto& kd = groups[kk];
+        const int nlk = kd.lmax + 1;
+        for (int w = wave; w < 2 * planes * (T / 4); w += NW) {
+            const int part = w / (T / 4), c0 = 4 * (w % (T / 4));
+            const int side = part >= planes, plane = part - side * planes;
+            const int c = c0 + (lane >> 4), l = plane * 16 + ((lane & 15) ^ (c & 15));
+            const double2* src = p.rs + ((side ? cj : ci) + c) * p.ldr + kd.rsoff + side * nlk + min(l, nlk - 1);
+            load_lds(src, lds + (buf * 2 * planes + part) * Ov::kPlane + c0 * 256);
+        }
+    };
+    // Phases of kAtoms atoms from `first` on, n of them: [buffer][side][atom][T]
+    auto load_phases = [&](int first, int n, int buf) {
+        for (int w = wave; w < 2 * kAtoms * T / 64; w += NW) {
+            const int e = w * 64 + lane;
+            const int side = w * 64 >= kAtoms * T;
+            const int a = min(e / T % kAtoms, n - 1), c = e % T;
+            load_lds(p.ph + (int64_t)(first + a) * p.gtot + (side ? cj : ci) + c, ph0 + buf * Ov::kPhases + w * 1024);
+        }
+    };
+
+    double sr[M][MJ], si[M][MJ], t[M][MJ], sg[M][MJ], rad[M][MJ], fr[M][MJ], fi[M][MJ];
 #pragma unroll
     for (int m = 0; m < M; ++m)
 #pragma unroll
@@ -311,43 +376,36 @@ __device__ __forceinline__ void overlap_tile(const SphereArgs& p, int blk, doubl
             t[m][n] = 0.0;
             sg[m][n] = 1.0;
         }
-
+    // 1 / (l + 1) in lane l: read from there, not by a load that a step would wait for
+    const double inv_l = kLegendre.v[min(lane, kMaxLmax)];
+    const int inv_lo = __double2loint(inv_l), inv_hi = __double2hiint(inv_l);
+    // Steps: per group its atoms, kAtoms at a time.  The loads of the next step
+    // are in flight during a step; its buffers were last read before the
+    // barrier that begins this one.
+    load_radial(0, 0);
+    load_phases(groups[0].first, min(kAtoms, groups[0].count), 0);
+    int pb = 0;                           // buffer of the step's phases
     for (int kk = 0; kk < p.ngroups; ++kk) {
-        const OverlapGroup& kd = p.groups[kk];
-        const int nlk = kd.lmax + 1;
-        const int count = kd.count;
-        const bool newdir = kd.newdir != 0;
-        __syncthreads();
-        for (int q = tid; q < nlk * T; q += NT) {
-            const int c = q / nlk, l = q - c * nlk;
-            s_ri[l * T + c] = p.rs[(ci + c) * p.ldr + kd.rsoff + l];
-        }
-        for (int q = tid; q < nlk * T; q += NT) {
-            const int c = q / nlk, l = q - c * nlk;
-            const double wl = (2 * l + 1) / (4.0 * kPi);
-            const double2 r = p.rs[(cj + c) * p.ldr + kd.rsoff + l];
-            const double wb = wl * p.rad[(int64_t)kd.rep * p.nl + l].dE_u_norm;
-            s_rj[l * T + c] = make_double2(wl * r.x, wb * r.y);
-        }
-        if (newdir && tid < 2 * T) {
-            const int side = tid / T, c = tid - side * T;
-            const int gi = min((side ? J0 : I0) + c, ng - 1);
-            const DirAngles d = dir_angles(kd.rot, kp->k[0] + kp->gd[3 * gi], kp->k[1] + kp->gd[3 * gi + 1],
-                                           kp->k[2] + kp->gd[3 * gi + 2]);
-            double* s = s_n + side * 3 * T + c;
-            s[0] = d.sth * d.cph;
-            s[T] = d.sth * d.sph;
-            s[2 * T] = d.cth;
-        }
-        const int n0 = min(kOvAtoms, count);
-        for (int q = tid; q < n0 * T; q += NT) {
-            const int a = q / T, c = q - a * T;
-            const double2* ph = p.ph + (int64_t)(kd.first + a) * p.gtot;
-            s_pi[q] = ph[ci + c];
-            s_pj[q] = ph[cj + c];
-        }
-        __syncthreads();
-        if (newdir) {
+        const auto& kd = groups[kk];
+        const int nlk = kd.lmax + 1, count = kd.count, rb = kk & 1;
+        if (kd.newdir) {
+            // unit vectors [side][3][T] where the next group's radial factors will be
+            double* s_n = (double*)(lds + (rb ^ 1) * 2 * planes * Ov::kPlane);
+            __syncthreads();
+            if (tid < 2 * T) {
+                const int side = tid / T, c = tid - side * T;
+                const int gi = min((side ? J0 : I0) + c, ng - 1);
+                double rot[9];
+#pragma unroll
+                for (int q = 0; q < 9; ++q) rot[q] = kd.rot[q];
+                const DirAngles d = dir_angles(rot, kp->k[0] + kp->gd[3 * gi], kp->k[1] + kp->gd[3 * gi + 1],
+                                               kp->k[2] + kp->gd[3 * gi + 2]);
+                double* s = s_n + side * 3 * T + c;
+                s[0] = d.sth * d.cph;
+                s[T] = d.sth * d.sph;
+                s[2 * T] = d.cth;
+            }
+            __syncthreads();
 #pragma unroll
             for (int m = 0; m < M; ++m)
 #pragma unroll
@@ -362,72 +420,86 @@ __device__ __forceinline__ void overlap_tile(const SphereArgs& p, int blk, doubl
                     t[m][n] = 0.5 * __builtin_fma(z, z, __builtin_fma(y, y, x * x));
                 }
         }
-        // sum over l, even and odd apart
-        double rad[M][MJ];
-        {
-            double P[M][MJ], d[M][MJ], ev[M][MJ], od[M][MJ];
-#pragma unroll
-            for (int m = 0; m < M; ++m)
-#pragma unroll
-                for (int n = 0; n < MJ; ++n) {
-                    P[m][n] = 1.0;
-                    d[m][n] = 0.0;
-                    ev[m][n] = 0.0;
-                    od[m][n] = 0.0;
-                }
-            auto step = [&](int l, double(&acc)[M][MJ]) {
-                double2 ri[M], rj[MJ];
-#pragma unroll
-                for (int m = 0; m < M; ++m) ri[m] = s_ri[l * T + tx + 16 * m];
-#pragma unroll
-                for (int n = 0; n < MJ; ++n) rj[n] = s_rj[l * T + ty + TY * n];
-                const double ca = kLegendre.a[l], cb = kLegendre.b[l];
+        for (int a0 = 0; a0 < count; a0 += kAtoms, pb ^= 1) {
+            // this wave's loads of the step landed and its reads of the last
+            // one are done; after the barrier every wave's
+            __builtin_amdgcn_s_waitcnt(wait_vm(0, true));
+            asm volatile("s_barrier" ::: "memory");
+            if (a0 + kAtoms < count) {
+                load_phases(kd.first + a0 + kAtoms, min(kAtoms, count - a0 - kAtoms), pb ^ 1);
+            } else if (kk + 1 < p.ngroups) {
+                load_radial(kk + 1, rb ^ 1);
+                load_phases(groups[kk + 1].first, min(kAtoms, groups[kk + 1].count), pb ^ 1);
+            }
+            if (a0 == 0) {
+                // sum over l, even and odd apart
+                double P[M][MJ], d[M][MJ], od[M][MJ];
 #pragma unroll
                 for (int m = 0; m < M; ++m)
 #pragma unroll
                     for (int n = 0; n < MJ; ++n) {
-                        const double w = __builtin_fma(ri[m].y, rj[n].y, ri[m].x * rj[n].x);
-                        acc[m][n] = __builtin_fma(w, P[m][n], acc[m][n]);
-                        d[m][n] = __builtin_fma(-cb, t[m][n] * P[m][n], ca * d[m][n]);
-                        P[m][n] += d[m][n];
+                        P[m][n] = 1.0;
+                        d[m][n] = 0.0;
+                        rad[m][n] = 0.0;
+                        od[m][n] = 0.0;
+                        fr[m][n] = 0.0;
+                        fi[m][n] = 0.0;
                     }
-            };
-            for (int l = 0; l < nlk; l += 2) {
-                step(l, ev);
-                if (l + 1 < nlk) step(l + 1, od);
-            }
+                const char* ri0 = lds + rb * 2 * planes * Ov::kPlane;
+                struct Factors {
+                    v2d ri[M], rj[MJ];
+                };
+                auto read = [&](int l, Factors& f) {
+                    const char* base = ri0 + (l >> 4) * Ov::kPlane;
 #pragma unroll
-            for (int m = 0; m < M; ++m)
+                    for (int m = 0; m < M; ++m)
+                        f.ri[m] = *(const v2d*)&base[(tx + 16 * m) * 256 + ((l & 15) ^ tx) * 16];
 #pragma unroll
-                for (int n = 0; n < MJ; ++n) rad[m][n] = __builtin_fma(sg[m][n], od[m][n], ev[m][n]);
-        }
-        // structure factor of the group's atoms
-        double fr[M][MJ], fi[M][MJ];
+                    for (int n = 0; n < MJ; ++n)
+                        f.rj[n] = *(const v2d*)&base[planes * Ov::kPlane + (ty + TY * n) * 256 + ((l & 15) ^ (ty & 15)) * 16];
+                };
+                auto step = [&](int l, const Factors& f, double(&acc)[M][MJ]) {
+                    const double cb = -(double)(2 * l + 1);
+                    const double inv = __hiloint2double(__builtin_amdgcn_readlane(inv_hi, l), __builtin_amdgcn_readlane(inv_lo, l));
 #pragma unroll
-        for (int m = 0; m < M; ++m)
+                    for (int m = 0; m < M; ++m)
 #pragma unroll
-            for (int n = 0; n < MJ; ++n) {
-                fr[m][n] = 0.0;
-                fi[m][n] = 0.0;
-            }
-        for (int a0 = 0; a0 < count; a0 += kOvAtoms) {
-            const int na = min(kOvAtoms, count - a0);
-            if (a0 > 0) {
-                __syncthreads();
-                for (int q = tid; q < na * T; q += NT) {
-                    const int a = q / T, c = q - a * T;
-                    const double2* ph = p.ph + (int64_t)(kd.first + a0 + a) * p.gtot;
-                    s_pi[q] = ph[ci + c];
-                    s_pj[q] = ph[cj + c];
+                        for (int n = 0; n < MJ; ++n) {
+                            const double w = __builtin_fma(f.ri[m].y, f.rj[n].y, f.ri[m].x * f.rj[n].x);
+                            acc[m][n] = __builtin_fma(w, P[m][n], acc[m][n]);
+                            d[m][n] = __builtin_fma(cb, t[m][n] * P[m][n], d[m][n]);
+                            P[m][n] = __builtin_fma(d[m][n], inv, P[m][n]);
+                        }
+                };
+                // kAhead: the factors of the next l are read ahead of a step
+                Factors even, odd;
+                if (kAhead) read(0, even);
+                for (int l = 0; l < nlk; l += 2) {
+                    if (kAhead) read(min(l + 1, nlk - 1), odd);
+                    else read(l, even);
+                    if (kAhead) __builtin_amdgcn_sched_barrier(0);
+                    step(l, even, rad);
+                    if (l + 1 >= nlk) break;
+                    if (kAhead) read(min(l + 2, nlk - 1), even);
+                    else read(l + 1, odd);
+                    if (kAhead) __builtin_amdgcn_sched_barrier(0);
+                    step(l + 1, odd, od);
                 }
-                __syncthreads();
+#pragma unroll
+                for (int m = 0; m < M; ++m)
+#pragma unroll
+                    for (int n = 0; n < MJ; ++n) rad[m][n] = __builtin_fma(sg[m][n], od[m][n], rad[m][n]);
             }
-            for (int a = 0; a < na; ++a) {
-                double2 u[M], v[MJ];
+            // structure factor of the group's atoms
+            const int na = min(kAtoms, count - a0);
+            const char* pi0 = ph0 + pb * Ov::kPhases;
+            auto read_phases = [&](int a, v2d* u, v2d* v) {
 #pragma unroll
-                for (int m = 0; m < M; ++m) u[m] = s_pi[a * T + tx + 16 * m];
+                for (int m = 0; m < M; ++m) u[m] = *(const v2d*)&pi0[(a * T + tx + 16 * m) * 16];
 #pragma unroll
-                for (int n = 0; n < MJ; ++n) v[n] = s_pj[a * T + ty + TY * n];
+                for (int n = 0; n < MJ; ++n) v[n] = *(const v2d*)&pi0[((kAtoms + a) * T + ty + TY * n) * 16];
+            };
+            auto add_atom = [&](const v2d* u, const v2d* v) {
 #pragma unroll
                 for (int m = 0; m < M; ++m)
 #pragma unroll
@@ -435,6 +507,19 @@ __device__ __forceinline__ void overlap_tile(const SphereArgs& p, int blk, doubl
                         fr[m][n] = __builtin_fma(u[m].y, v[n].y, __builtin_fma(u[m].x, v[n].x, fr[m][n]));
                         fi[m][n] = __builtin_fma(-u[m].y, v[n].x, __builtin_fma(u[m].x, v[n].y, fi[m][n]));
                     }
+            };
+            v2d u0[M], v0[MJ], u1[M], v1[MJ];
+            if (kAhead) read_phases(0, u0, v0);
+            for (int a = 0; a < na; a += 2) {
+                if (kAhead) read_phases(min(a + 1, na - 1), u1, v1);
+                else read_phases(a, u0, v0);
+                if (kAhead) __builtin_amdgcn_sched_barrier(0);
+                add_atom(u0, v0);
+                if (a + 1 >= na) break;
+                if (kAhead) read_phases(min(a + 2, na - 1), u0, v0);
+                else read_phases(a + 1, u1, v1);
+                if (kAhead) __builtin_amdgcn_sched_barrier(0);
+                add_atom(u1, v1);
             }
         }
 #pragma unroll
@@ -457,33 +542,36 @@ __device__ __forceinline__ void overlap_tile(const SphereArgs& p, int blk, doubl
 template <int M, int MJ>
 __global__ __launch_bounds__(256 * M / MJ) void k_overlap(SphereArgs p)
 {
-    extern __shared__ double smem[];
+    extern __shared__ __attribute__((aligned(1024))) char lds[];
     stamp(p, 3);
-    overlap_tile<M, MJ>(p, (int)blockIdx.x, smem);
+    overlap_tile<M, MJ, true>(p, (int)blockIdx.x, lds);
 }
 
 int overlap_tile_size(int64_t tiles64, int n_cu)
 {
-    // 64 x 64 tiles once they give every CU four workgroups, 32 x 32 once
+    // 64 x 64 tiles, one workgroup per CU, once every CU has eight; 32 x 32 once
     // those give two, else 16 x 16: a smaller tile reads its columns more often but
-    // spreads a small triangle over more CUs
-    if (tiles64 >= 4 * (int64_t)n_cu) return 64;
+    // spreads a small triangle over more CUs.  H and S at N_G 3001 with S in tiles
+    // of 64 and 32: 1846, 1824 us; 6002: 9126, 9110; 12007: 190.4, 191.2 ms; a batch
+    // of 12 of 1900 plane waves 16.38, 16.39 ms.
+    if (tiles64 >= 8 * (int64_t)n_cu) return 64;
     return 4 * tiles64 >= 2 * (int64_t)n_cu ? 32 : 16;
 }
 
-static size_t overlap_lds(int tile, int nl)
+template <int M, int MJ>
+static hipError_t launch_overlap_tile(const SphereArgs& p, int64_t ntiles, hipEvent_t stop, hipStream_t st)
 {
-    return sizeof(double2) * (size_t)tile * 2 * (nl + kOvAtoms) + sizeof(double) * 6 * tile;
+    using Ov = OverlapTile<M, MJ>;
+    const size_t lds = Ov::lds((p.nl + 15) / 16);
+    return launch(k_overlap<M, MJ>, dim3((unsigned)ntiles), Ov::NT, lds, stop, st, p);
 }
 
 hipError_t launch_overlap(const SphereArgs& p, int tile, int64_t ntiles, hipEvent_t stop, hipStream_t st)
 {
     if (ntiles <= 0) return hipSuccess;
-    const size_t lds = overlap_lds(tile, p.nl);
-    const dim3 grid((unsigned)ntiles);
-    if (tile == 64) return launch(k_overlap<4, 2>, grid, 512, lds, stop, st, p);
-    if (tile == 32) return launch(k_overlap<2, 2>, grid, 256, lds, stop, st, p);
-    return launch(k_overlap<1, 1>, grid, 256, lds, stop, st, p);
+    if (tile == 64) return launch_overlap_tile<4, 2>(p, ntiles, stop, st);
+    if (tile == 32) return launch_overlap_tile<2, 2>(p, ntiles, stop, st);
+    return launch_overlap_tile<1, 1>(p, ntiles, stop, st);
 }
 
 // ---------------------------------------------------------------------------
@@ -697,7 +785,6 @@ hipError_t launch_split_mt(const SplitMtJob* jobs, int njobs, int64_t max_elems,
 namespace {
 
 typedef double d4 __attribute__((ext_vector_type(4)));
-typedef double v2d __attribute__((ext_vector_type(2)));
 typedef int i8 __attribute__((ext_vector_type(8)));
 typedef __attribute__((address_space(4))) const i8* ctab;
 
@@ -712,14 +799,6 @@ constexpr int kSphereColumns = 4096;
 // Stages in LDS of the 32 x 32 tiles of H: three of 13 KB let four workgroups
 // share a CU, as 128 VGPRs do.
 constexpr int kSphereSmall = 3;
-
-// s_waitcnt immediate: at most n vector-memory operations outstanding and, with
-// lgkm, no LDS or scalar ones (vmcnt bits [3:0] and [15:14], expcnt [6:4],
-// lgkmcnt [11:8]).
-constexpr int wait_vm(int n, bool lgkm)
-{
-    return (n & 15) | (7 << 4) | ((lgkm ? 0 : 15) << 8) | ((n >> 4) << 14);
-}
 
 // Atoms that end in a stage before its k-step ks.
 __device__ __forceinline__ int ends_before(i8 e, int ks)
@@ -755,8 +834,6 @@ __device__ __forceinline__ void stages(const F& f, int s, std::integer_sequence<
     f(s, std::integral_constant<int, I>{}...);
 }
 
-// Wave-uniform values the compiler is to keep in scalar registers.
-__device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
 __device__ __forceinline__ int64_t uni(int64_t v)
 {
     return (int64_t)(((uint64_t)(uint32_t)uni((int)(v >> 32)) << 32) | (uint32_t)uni((int)v));
@@ -1154,7 +1231,7 @@ __global__ __launch_bounds__(256, 4) void k_sphere_hs(SphereArgs p, int hblocks)
     extern __shared__ __attribute__((aligned(1024))) char lds[];
     stamp(p, 2);
     if ((int)blockIdx.x < hblocks) sphere_gemm_tile<32, 32, 1, 1, kSphereSmall, true>(p, (int)blockIdx.x, lds);
-    else overlap_tile<M, M>(p, (int)blockIdx.x - hblocks, (double*)lds);
+    else overlap_tile<M, M, false>(p, (int)blockIdx.x - hblocks, lds);
 }
 
 template <int BR, int BC, int RB, int CB, int NS, bool kH>
@@ -1189,7 +1266,7 @@ template <int M>
 static hipError_t launch_hs(const SphereArgs& p, int64_t nstiles, hipEvent_t stop, hipStream_t st)
 {
     const int64_t n = hblocks(p, 32);
-    const size_t lds = std::max<size_t>(SphereTile<32, 32, 1, 1, kSphereSmall>::kLds, overlap_lds(16 * M, p.nl));
+    const size_t lds = std::max<size_t>(SphereTile<32, 32, 1, 1, kSphereSmall>::kLds, OverlapTile<M, M>::lds((p.nl + 15) / 16));
     return launch(k_sphere_hs<M>, dim3((unsigned)(n + nstiles)), 256, lds, stop, st, p, (int)n);
 }
 

@@ -148,7 +148,7 @@ hsgen_status sphere_setup(hsgen_ctx* ctx, hsgen_sys* s, const RadDev* rad)
             g.newdir = i == 0 || members[i].cos != members[i - 1].cos;
             std::memcpy(g.rot, s->atoms[cos_rep[members[i].cos]].rot, sizeof g.rot);
             groups.push_back(g);
-            rr += at.lmax + 1;
+            rr += 2 * (at.lmax + 1);
         }
         groups.back().count += k.count;
         for (int a : members[i].atoms) {

@@ -226,3 +226,21 @@ def test_h_and_s_in_one_launch(ctx, ng, lmax):
         assert np.array_equal(np.tril(F), np.tril(X)) and np.array_equal(F, np.tril(F) + np.tril(F, -1).conj().T)
     assert rel_fro_lower(H, po.reference_hs(s, sub)[0]) <= TOL
     h.close()
+
+
+@pytest.mark.parametrize("lmax,natoms", [((16, 3), 10), ((24,), 1), ((15, 16), 9)])
+def test_more_than_sixteen_l_and_all_s_tiles(ctx, lmax, natoms):
+    """Radial factors in two planes of 16 values of l, groups of more atoms than
+    are staged at a time, S tiles of 16, 32 and 64."""
+    s, kp = tiny_system(natoms=natoms, lmax=lmax, a_cell=19.0, ng_target=4300, seed=3)
+    h = ctx.upload(s)
+    n = 4200
+    H, S = ctx.create_HS2(h, _subset(kp, np.arange(n)))
+    for m in (40, 900):
+        idx = np.sort(np.random.default_rng(m).permutation(n)[:m])
+        Hs, Ss = ctx.create_HS2(h, _subset(kp, idx))
+        assert np.array_equal(Hs, H[np.ix_(idx, idx)]) and np.array_equal(Ss, S[np.ix_(idx, idx)]), m
+        if m == 40:
+            Hr, Sr = po.reference_hs(s, _subset(kp, idx))
+            assert rel_fro_lower(Hs, Hr) <= TOL and rel_fro_lower(Ss, Sr) <= TOL
+    h.close()
