@@ -1,7 +1,9 @@
-// FP64 path of the hsgen C ABI: tile geometry and grouped-GEMM work lists,
-// one k-point (hsgen_create_hs, hsgen_construct_ab, hsgen_contract_hs) and many
-// k-points in one captured launch sequence (hsgen_create_hs_batched).
-//   abgen (A/B generator) -> tmul (W_a = M_a Z_a) -> lower-triangle S and H.
+// FP64 path of the hsgen C ABI.  H and S from a system (hsgen_create_hs,
+// hsgen_create_hs_batched in one captured launch sequence): phases and real
+// vectors, sphere_path.hip.  Given coefficients (hsgen_contract_hs), and the
+// autotuner: tile geometry and grouped-GEMM work lists of
+//   operands Z -> tmul (W_a = M_a Z_a) -> lower-triangle S and H.
+// hsgen_construct_ab: the coefficients themselves.
 #include <algorithm>
 #include <array>
 #include <atomic>

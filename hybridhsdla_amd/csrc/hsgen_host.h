@@ -151,7 +151,7 @@ struct hsgen_ctx {
     // split precision
     hsgen::DevBuf oz_e, oz_res, oz_out, oz_probs, oz_work, oz_smp, oz_fprob;
     hipEvent_t oz_ev[2 * hsgen::kMaxModuli] = {};   // INT8 GEMM start/stop per residue group
-    int n_cu = 0;                                    // compute units (persistent grids)
+    int n_cu = 0;                                    // compute units
     // batched k-points: one captured graph per batch, replayed while the
     // call signature is unchanged
     struct BatchGraph {

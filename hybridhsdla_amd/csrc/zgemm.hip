@@ -380,17 +380,10 @@ __global__ __launch_bounds__(WGM * WGN * 64) void k_zgemm2_lh(const GemmProblem*
                                                               const TileWork* __restrict__ work, int nwork)
 {
     extern __shared__ __attribute__((aligned(1024))) char zlds[];
-    for (int wid = blockIdx.x; wid < nwork; wid += gridDim.x) {
-        zgemm2_tile<BM, BN, BK, WGM, WGN>(probs, work, wid, zlds);
-        __syncthreads();   // the next tile's first stage overwrites LDS
-    }
+    if ((int)blockIdx.x < nwork) zgemm2_tile<BM, BN, BK, WGM, WGN>(probs, work, blockIdx.x, zlds);
 }
 
-// Workgroups take tiles wid = blockIdx.x, blockIdx.x + gridDim.x, ...: with
-// one workgroup per tile (grid = nwork) that is a single tile; with a grid of
-// one workgroup per CU slot the launch is persistent and every workgroup
-// walks the list, keeping the dispatch order (and so the XCD a tile runs on)
-// of the one-per-tile launch.
+// One workgroup per tile of the list.
 template <int BM, int BN, int BK, int WGM, int WGN>
 __global__ __launch_bounds__(WGM * WGN * 64) void k_zgemm_lh(const GemmProblem* __restrict__ probs,
                                                              const TileWork* __restrict__ work,
@@ -398,10 +391,7 @@ __global__ __launch_bounds__(WGM * WGN * 64) void k_zgemm_lh(const GemmProblem* 
 {
     using Cfg = ZgemmCfg<BM, BN, BK, WGM, WGN>;
     __shared__ double lds[2 * Cfg::kStageDoubles];
-    for (int wid = blockIdx.x; wid < nwork; wid += gridDim.x) {
-        zgemm_tile<BM, BN, BK, WGM, WGN>(probs, work, wid, lds);
-        __syncthreads();   // the next tile's first stage overwrites LDS
-    }
+    if ((int)blockIdx.x < nwork) zgemm_tile<BM, BN, BK, WGM, WGN>(probs, work, blockIdx.x, lds);
 }
 
 // Tile configurations (id -> template instance).
@@ -445,39 +435,13 @@ ZgemmLaunchCfg zgemm_cfg(int id)
     return ZgemmLaunchCfg{0, 0, 0, 0};
 }
 
-// Workgroups of configuration id that one CU holds at once (registers, LDS
-// and waves permitting): a persistent launch sizes its grid by it.
-int zgemm_blocks_per_cu(int id)
-{
-    int n = 0;
-    hipError_t e = hipErrorInvalidValue;
-#define X(ID, BM, BN, BK, WGM, WGN)                                                                   \
-    if (id == ID)                                                                                     \
-        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, (const void*)k_zgemm_lh<BM, BN, BK, WGM, WGN>, \
-                                                         WGM * WGN * 64, 0);
-    HSGEN_ZGEMM_CFGS(X)
-#undef X
-#define Y(ID, BM, BN, BK, WGM, WGN)                                                                     \
-    if (id == ID)                                                                                       \
-        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, (const void*)k_zgemm2_lh<BM, BN, BK, WGM, WGN>, \
-                                                         WGM * WGN * 64, Zgemm2Cfg<BM, BN, BK, WGM, WGN>::kLdsBytes);
-    HSGEN_ZGEMM2_CFGS(Y)
-#undef Y
-    if (e != hipSuccess) {
-        (void)hipGetLastError();
-        return 1;
-    }
-    return n > 0 ? n : 1;
-}
-
 hipError_t launch_zgemm(int id, const GemmProblem* probs, const TileWork* work, int nwork,
-                        hipStream_t st, int max_grid)
+                        hipStream_t st)
 {
     if (nwork <= 0) return hipSuccess;
-    const int grid = max_grid > 0 ? std::min(nwork, max_grid) : nwork;
 #define X(ID, BM, BN, BK, WGM, WGN)                                                      \
     if (id == ID) {                                                                      \
-        hipLaunchKernelGGL((k_zgemm_lh<BM, BN, BK, WGM, WGN>), dim3(grid),              \
+        hipLaunchKernelGGL((k_zgemm_lh<BM, BN, BK, WGM, WGN>), dim3(nwork),              \
                            dim3(WGM * WGN * 64), 0, st, probs, work, nwork);             \
         return hipGetLastError();                                                        \
     }
@@ -490,7 +454,7 @@ hipError_t launch_zgemm(int id, const GemmProblem* probs, const TileWork* work, 
         hipError_t e = hipFuncSetAttribute((const void*)k_zgemm2_lh<BM, BN, BK, WGM, WGN>,             \
                                            hipFuncAttributeMaxDynamicSharedMemorySize, lds);            \
         if (e != hipSuccess) return e;                                                                \
-        hipLaunchKernelGGL((k_zgemm2_lh<BM, BN, BK, WGM, WGN>), dim3(grid), dim3(WGM * WGN * 64), lds, \
+        hipLaunchKernelGGL((k_zgemm2_lh<BM, BN, BK, WGM, WGN>), dim3(nwork), dim3(WGM * WGN * 64), lds, \
                            st, probs, work, nwork);                                                   \
         return hipGetLastError();                                                                     \
     }
