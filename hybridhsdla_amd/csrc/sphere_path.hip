@@ -214,38 +214,51 @@ hsgen_status sphere_setup(hsgen_ctx* ctx, hsgen_sys* s, const RadDev* rad)
     s->d_order = (int32_t*)(p += b_g);
     s->d_stages = (SphereStage*)(p += b_o);
     s->d_mtoff = (int64_t*)(p += b_s);
-    HIPCHK(hipMemcpyAsync(s->d_kinds, kinds.data(), sizeof(KindDev) * kinds.size(), hipMemcpyHostToDevice, ctx->stream));
-    HIPCHK(hipMemcpyAsync(s->d_groups, groups.data(), sizeof(OverlapGroup) * groups.size(), hipMemcpyHostToDevice,
-                          ctx->stream));
-    HIPCHK(hipMemcpyAsync(s->d_order, order.data(), sizeof(int32_t) * order.size(), hipMemcpyHostToDevice, ctx->stream));
-    HIPCHK(hipMemcpyAsync(s->d_stages, stages.data(), sizeof(SphereStage) * stages.size(), hipMemcpyHostToDevice,
-                          ctx->stream));
-    HIPCHK(hipMemcpyAsync(s->d_mtoff, mtoff.data(), sizeof(int64_t) * mtoff.size(), hipMemcpyHostToDevice, ctx->stream));
-    // the raw blocks, only until the matrices are built
-    Tmp t_raw, t_jobs;
+    // the tables in one copy
+    std::vector<char> tables(b_k + b_g + b_o + b_s + b_m);
+    auto put = [&](const void* dev, const void* src, size_t n) {
+        std::memcpy(tables.data() + ((const char*)dev - (const char*)s->d_kinds), src, n);
+    };
+    put(s->d_kinds, kinds.data(), sizeof(KindDev) * kinds.size());
+    put(s->d_groups, groups.data(), sizeof(OverlapGroup) * groups.size());
+    put(s->d_order, order.data(), sizeof(int32_t) * order.size());
+    put(s->d_stages, stages.data(), sizeof(SphereStage) * stages.size());
+    put(s->d_mtoff, mtoff.data(), sizeof(int64_t) * mtoff.size());
+    HIPCHK(hipMemcpyAsync(s->d_kinds, tables.data(), tables.size(), hipMemcpyHostToDevice, ctx->stream));
+    // the raw blocks and the jobs, only until the matrices are built: in one
+    // copy, large ones through the pinned slots
     int64_t raw = 0, most = 0;
     for (int a : owners) {
         raw += 3 * (int64_t)s->atoms[a].nlm * s->atoms[a].nlm;
         most = std::max(most, mt_size(s->atoms[a].nlm));
     }
-    HIPCHK(hipMalloc(&t_raw.p, sizeof(double2) * (size_t)raw));
-    HIPCHK(hipMalloc(&t_jobs.p, sizeof(MtJob) * owners.size()));
+    const size_t b_raw = sizeof(double2) * (size_t)raw, b_jobs = sizeof(MtJob) * owners.size();
+    Tmp t_raw;
+    HIPCHK(hipMalloc(&t_raw.p, b_raw + b_jobs));
     double2* d = (double2*)t_raw.p;
     std::vector<MtJob> jobs;
+    std::vector<HostCopy> in;
     for (int a : owners) {
         const int64_t n = s->atoms[a].nlm, n2 = n * n;
         const std::vector<std::complex<double>>* src[3] = {&s->h_taa[a], &s->h_tab[a], &s->h_tbb[a]};
-        for (int b = 0; b < 3; ++b)
-            HIPCHK(hipMemcpyAsync(d + b * n2, src[b]->data(), sizeof(double2) * (size_t)n2, hipMemcpyHostToDevice,
-                                  ctx->stream));
+        for (int b = 0; b < 3; ++b) in.push_back(copy_run(d + b * n2, src[b]->data(), sizeof(double2) * (size_t)n2));
         jobs.push_back(MtJob{d, d + n2, d + 2 * n2, off[a], (int32_t)n, (int32_t)roundup(2 * n, 4),
                              (int32_t)roundup(2 * n, 16), 0});
         d += 3 * n2;
     }
-    HIPCHK(hipMemcpyAsync(t_jobs.p, jobs.data(), sizeof(MtJob) * jobs.size(), hipMemcpyHostToDevice, ctx->stream));
+    in.push_back(copy_run(d, jobs.data(), b_jobs));
+    std::vector<char> small;
+    if (b_raw + b_jobs < ((size_t)4 << 20)) {
+        small.resize(b_raw + b_jobs);
+        for (const HostCopy& c : in) std::memcpy(small.data() + (c.dev - (char*)t_raw.p), c.host, c.rows);
+        HIPCHK(hipMemcpyAsync(t_raw.p, small.data(), small.size(), hipMemcpyHostToDevice, ctx->stream));
+    } else {
+        const hsgen_status st = host_copy(ctx, in, false, ctx->stream);
+        if (st) return st;
+    }
     for (size_t j0 = 0; j0 < jobs.size(); j0 += kJobsPerLaunch)
-        HIPCHK(launch_build_mt((const MtJob*)t_jobs.p + j0, (int)std::min(kJobsPerLaunch, jobs.size() - j0), most,
-                               s->d_mt, ctx->stream));
+        HIPCHK(launch_build_mt((const MtJob*)d + j0, (int)std::min(kJobsPerLaunch, jobs.size() - j0), most, s->d_mt,
+                               ctx->stream));
     HIPCHK(hipStreamSynchronize(ctx->stream));
     return HSGEN_OK;
 }
