@@ -13,11 +13,13 @@
 //
 // What is served is set by the size of the general operands (Y and W, or Z,
 // Zs and W, and their work lists) against HSGEN_NOALLOC_SCRATCH_BYTES.  The
-// call's own operands need less for the l cutoffs in use, but up to twice as
-// much where every atom has lmax 0 and is of a kind of its own (two rows
-// padded to the MFMA depth of four), hence the array's size.
+// call's own operands need less for the l cutoffs in use, but up to 9/4 as
+// much where atoms have lmax 0 and each is of a kind of its own (144 bytes per
+// plane wave: phase 16, radial factors 32, y and W of two rows padded to the
+// MFMA depth of four 32 and 64; general operands 64), hence the array's size.
 //
-// The call copies nothing from host memory except a host G list.  Every value
+// The call copies nothing from host memory except a host G list (a short one is
+// read from pinned memory).  Every value
 // that reaches H or S is written earlier in the same call, so nothing needs
 // clearing between calls.  Calls on one GPU share its array and the last
 // call's contents stay there: calls that overlap on one GPU, from any
@@ -31,7 +33,7 @@
 namespace hsgen {
 
 constexpr size_t kScratchLimit = HSGEN_NOALLOC_SCRATCH_BYTES;      // of the general operands
-constexpr size_t kScratchBytes = 2 * kScratchLimit + ((size_t)1 << 20);   // the array
+constexpr size_t kScratchBytes = kScratchLimit / 4 * 9 + ((size_t)1 << 20);   // the array
 constexpr int kScratchDevices = 64;
 
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
