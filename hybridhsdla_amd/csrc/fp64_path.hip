@@ -288,6 +288,7 @@ hsgen_status finish_hs(hsgen_ctx* ctx, hsgen_sys* s, const Geometry& geo, int ng
     const bool apart = !is_split(o.precision) && need_h && !out_h.empty() && !out_s.empty();
     // problem and tile lists, until the streams are waited for
     std::vector<GemmProblem> tprobs, probs, sprobs;
+    OzSample smp;
     std::vector<TileWork> twork, work, swork;
     auto products = [&](std::vector<GemmProblem>& pr, std::vector<TileWork>& wk, int skip) {
         add_hs_problems(pr, wk, geo, ng, Z, Zs, W, dH, dS, 0, flags | skip);
@@ -324,7 +325,14 @@ hsgen_status finish_hs(hsgen_ctx* ctx, hsgen_sys* s, const Geometry& geo, int ng
             for (int q = 0; q < 3; ++q) k.k[q] = kp->k[q];
             k.g = (const int32_t*)ctx->g.p;
             k.ng = ng;
-            st = sphere_split_w(ctx, s, {k}, nullptr, geo.gp, W, geo.ldz);
+            std::vector<OzK> ks(1);
+            ks[0].ng = ng;
+            if ((st = oz_sample(ctx, geo, ks, smp))) return st;
+            k.H = smp.H;
+            k.S = smp.S;
+            k.ldH = k.ldS = ng;
+            const std::vector<int32_t> cols = smp.padded();
+            st = sphere_split_w(ctx, s, {k}, nullptr, geo.gp, W, geo.ldz, &cols, do_s);
         } else {
             const int tc = tapp_cfg(geo);
             add_tmul_problems(tprobs, twork, s, geo, zgemm_cfg(tc), ng, Z, W);
@@ -349,7 +357,7 @@ hsgen_status finish_hs(hsgen_ctx* ctx, hsgen_sys* s, const Geometry& geo, int ng
         ks[0].dS = dS;
         ks[0].ldS = ldS;
         std::vector<OzResult> ozr;
-        st = run_ozaki(ctx, geo, ks, flags, icfg, o.slices, o.target_rel_err, ozr, false);
+        st = run_ozaki(ctx, geo, ks, flags, icfg, o.slices, o.target_rel_err, ozr, false, kp && need_h ? &smp : nullptr);
         if (st) return st;
         oz = ozr[0];
     } else {

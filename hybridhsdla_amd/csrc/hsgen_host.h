@@ -147,7 +147,7 @@ struct hsgen_ctx {
     // workspace
     hsgen::DevBuf Z, Zs, W, Htmp, Stmp, A, B, g, probs, work, pack, m_in, M, probs2, work2, tprobs, twork;
     // FP64 from a system: phases, radial factors, real vectors (W, host-output copies above)
-    hsgen::DevBuf sph_ph, sph_rs, sph_y, sph_w;
+    hsgen::DevBuf sph_ph, sph_rs, sph_y, sph_w, sph_smp;
     // split precision
     hsgen::DevBuf oz_e, oz_res, oz_out, oz_probs, oz_work, oz_smp, oz_fprob;
     hipEvent_t oz_ev[2 * hsgen::kMaxModuli] = {};   // INT8 GEMM start/stop per residue group
@@ -341,7 +341,7 @@ hsgen_status sphere_run(hsgen_ctx* ctx, const hsgen_sys* s, const SphereLayout& 
                         hsgen_report* rep);
 hsgen_status sphere_split_setup(hsgen_ctx* ctx, hsgen_sys* s);
 hsgen_status sphere_split_w(hsgen_ctx* ctx, hsgen_sys* s, const std::vector<SphereK>& ks, const SphereK* ks_dev,
-                            int64_t ncols, double2* W, int64_t ldw);
+                            int64_t ncols, double2* W, int64_t ldw, const std::vector<int32_t>* cols, bool do_s);
 // Bytes of the operands per plane wave (reports).
 inline double sphere_gen_bytes(const hsgen_sys* s)
 {
@@ -369,10 +369,29 @@ struct OzK {
     int64_t ldS = 0;
 };
 
+// The FP64 sample of a call: nb evenly spaced columns of S and H of every
+// k-point, all rows, leading dimension ng, in the context's sample buffer.
+struct OzSample {
+    std::vector<int> nb;
+    std::vector<int32_t> cols;                 // the columns, relative to their k-point
+    std::vector<size_t> soff, off, gath;       // per k-point: first of cols, of S and H, of the gathered operands
+    size_t nbt = 0, total = 0, gath_total = 0;
+    int nsplit = 1;
+    double2* S = nullptr;
+    double2* H = nullptr;
+    double2* gath_s = nullptr;
+    double2* gath_h = nullptr;
+    double2* parts = nullptr;
+    // kSampleCols columns per k-point, the last again past nb
+    std::vector<int32_t> padded() const;
+};
+hsgen_status oz_sample(hsgen_ctx* ctx, const Geometry& geo, const std::vector<OzK>& ks, OzSample& smp);
+
 // capture: the INT8 launch sequence of each modulus count runs as cached
-// hipGraphs (the batched path), else eagerly.
+// hipGraphs (the batched path), else eagerly.  sample: null, or the call's
+// sample, computed already.
 hsgen_status run_ozaki(hsgen_ctx* ctx, const Geometry& geo, const std::vector<OzK>& ks, int flags, int icfg,
-                       int nmod_req, double target, std::vector<OzResult>& res, bool capture);
+                       int nmod_req, double target, std::vector<OzResult>& res, bool capture, const OzSample* sample);
 void destroy_oz_graph(hsgen_ctx::OzGraph& g);
 hsgen_status batched_split(hsgen_ctx* ctx, hsgen_sys* s, int nk, const hsgen_kpoint* kps, const hsgen_opts& o,
                            double* const* H, double* const* S, const int64_t* ld, hsgen_report* rep);

@@ -135,9 +135,19 @@ struct SphereArgs {
     int32_t nksteps;
     int32_t rtiles;            // T application: tiles of rows of all kinds
     int32_t nsquares;          // lower squares of H tiles of all k-points
+    // split precision's FP64 sample: kSampleCols columns per k-point of their own
+    // operands, read beside the chunk's; H and S of a k-point are its samples
+    const double2* smp_W;
+    const double2* smp_ph;     // [natoms][smp_gtot]
+    const double2* smp_rs;
+    const int32_t* smp_g;      // [smp_gtot][3]
+    int64_t smp_ldw, smp_gtot;
     uint64_t* stamp;           // starts of the generator, T application, H and S kernels (wall clock), or null
 };
 
+constexpr int kSampleCols = 64;
+hipError_t launch_sample_g(const SphereArgs& p, const int32_t* cols, int32_t* out, hipStream_t st);
+hipError_t launch_sample(const SphereArgs& p, bool do_h, bool do_s, hipStream_t st);
 // Launchers; stop: null, or an event that takes the kernel's end.
 int sphere_chunk(int nl, int L);
 hipError_t launch_split_mt(const SplitMtJob* jobs, int njobs, int64_t max_elems, const double* sq, const double2* mt,

@@ -200,7 +200,7 @@ __global__ __launch_bounds__(256) void k_sphere_gen(SphereArgs p)
             const double bu = -m.u * Knorm * dfj[l] + m.u_dr * fj[l];
             const double2 ab = make_double2(pref * au, pref * bu);
             s_ab[t * nl + l] = ab;
-            if (!kSplit && kd.rsoff >= 0) {
+            if (p.rs && kd.rsoff >= 0) {
                 // as they are, and with the weights of S
                 double2* r = p.rs + col * p.ldr + kd.rsoff + l;
                 const double wl = (2 * l + 1) / (4.0 * kPi);
@@ -318,7 +318,8 @@ struct OverlapTile {
     static constexpr int lds(int planes) { return 4 * planes * kPlane + 2 * kPhases; }
 };
 
-template <int M, int MJ, bool kAhead>
+// kSample: the sampled columns of S, all rows of a chunk's columns.
+template <int M, int MJ, bool kAhead, bool kSample>
 __device__ __forceinline__ void overlap_tile(const SphereArgs& p, int blk, char* lds)
 {
     // one rounding per written operation: every tile gives the same bits
@@ -329,13 +330,34 @@ __device__ __forceinline__ void overlap_tile(const SphereArgs& p, int blk, char*
     const int wave = uni(tid >> 6);
     const int tx = tid & 15, ty = tid >> 4;
     const SphereK* kp = &p.one;
-    if (p.nk > 1) kp = p.many + find_last(p.nk, blk, [&](int i) { return p.many[i].stile0; });
-    const int tile = blk - kp->stile0;
-    const int bi = tri_row(tile);
-    const int bj = tile - (int)((int64_t)bi * (bi + 1) / 2);
-    const int I0 = bi * T, J0 = bj * T;
+    int I0, J0;                           // first row, first column (sampled: among the samples)
+    int64_t ci, cj;                       // their columns of the operands
+    if constexpr (kSample) {
+        constexpr int kRow = kSampleCols / T;
+        const int tc = blk / kRow;
+        const int c = (int)p.cbase + tc * T;
+        const int ki = p.nk > 1 ? find_last(p.nk, c, [&](int i) { return (int)p.many[i].col0; }) : 0;
+        if (p.nk > 1) kp = p.many + ki;
+        I0 = c - (int)kp->col0;
+        J0 = (blk - tc * kRow) * T;
+        if (I0 >= kp->ng || J0 >= min(kp->ng, kSampleCols)) return;
+        ci = tc * T;
+        cj = ki * kSampleCols + J0;
+    } else {
+        if (p.nk > 1) kp = p.many + find_last(p.nk, blk, [&](int i) { return p.many[i].stile0; });
+        const int tile = blk - kp->stile0;
+        const int bi = tri_row(tile);
+        const int bj = tile - (int)((int64_t)bi * (bi + 1) / 2);
+        I0 = bi * T;
+        J0 = bj * T;
+        ci = kp->col0 + I0;
+        cj = kp->col0 + J0;
+    }
     const int ng = kp->ng;
-    const int64_t ci = kp->col0 + I0, cj = kp->col0 + J0;
+    // the columns' operands
+    const double2* const rs_j = kSample ? p.smp_rs : p.rs;
+    const double2* const ph_j = kSample ? p.smp_ph : p.ph;
+    const int64_t gtot_j = kSample ? p.smp_gtot : p.gtot;
     const int planes = (p.nl + 15) / 16;
     char* const ph0 = lds + 4 * planes * Ov::kPlane;
     // constant address space: the groups come by scalar loads
@@ -352,7 +374,8 @@ __device__ __forceinline__ void overlap_tile(const SphereArgs& p, int blk, char*
             const int part = w / (T / 4), c0 = 4 * (w % (T / 4));
             const int side = part >= planes, plane = part - side * planes;
             const int c = c0 + (lane >> 4), l = plane * 16 + ((lane & 15) ^ (c & 15));
-            const double2* src = p.rs + ((side ? cj : ci) + c) * p.ldr + kd.rsoff + side * nlk + min(l, nlk - 1);
+            const double2* src = (side ? rs_j + (cj + c) * p.ldr : p.rs + (ci + c) * p.ldr) + kd.rsoff + side * nlk +
+                                 min(l, nlk - 1);
             load_lds(src, lds + (buf * 2 * planes + part) * Ov::kPlane + c0 * 256);
         }
     };
@@ -362,7 +385,7 @@ __device__ __forceinline__ void overlap_tile(const SphereArgs& p, int blk, char*
             const int e = w * 64 + lane;
             const int side = w * 64 >= kAtoms * T;
             const int a = min(e / T % kAtoms, n - 1), c = e % T;
-            load_lds(p.ph + (int64_t)(first + a) * p.gtot + (side ? cj : ci) + c, ph0 + buf * Ov::kPhases + w * 1024);
+            load_lds((side ? ph_j + (int64_t)(first + a) * gtot_j + cj : p.ph + (int64_t)(first + a) * p.gtot + ci) + c, ph0 + buf * Ov::kPhases + w * 1024);
         }
     };
 
@@ -394,12 +417,13 @@ __device__ __forceinline__ void overlap_tile(const SphereArgs& p, int blk, char*
             __syncthreads();
             if (tid < 2 * T) {
                 const int side = tid / T, c = tid - side * T;
-                const int gi = min((side ? J0 : I0) + c, ng - 1);
+                const int32_t* g = kSample ? kp->g : kp->gd;
+                if (kSample && side) g = p.smp_g + 3 * (cj - J0 + min(J0 + c, min(ng, kSampleCols) - 1));
+                else g += 3 * min((side ? J0 : I0) + c, ng - 1);
                 double rot[9];
 #pragma unroll
                 for (int q = 0; q < 9; ++q) rot[q] = kd.rot[q];
-                const DirAngles d = dir_angles(rot, kp->k[0] + kp->gd[3 * gi], kp->k[1] + kp->gd[3 * gi + 1],
-                                               kp->k[2] + kp->gd[3 * gi + 2]);
+                const DirAngles d = dir_angles(rot, kp->k[0] + g[0], kp->k[1] + g[1], kp->k[2] + g[2]);
                 double* s = s_n + side * 3 * T + c;
                 s[0] = d.sth * d.cph;
                 s[T] = d.sth * d.sph;
@@ -535,7 +559,11 @@ __device__ __forceinline__ void overlap_tile(const SphereArgs& p, int blk, char*
 #pragma unroll
         for (int m = 0; m < M; ++m) {
             const int i = I0 + tx + 16 * m, j = J0 + ty + TY * n;
-            if (i < ng && i >= j) kp->S[(int64_t)j * kp->ldS + i] = make_double2(sr[m][n], i == j ? 0.0 : si[m][n]);
+            if constexpr (kSample) {
+                if (i < ng && j < min(ng, kSampleCols)) kp->S[(int64_t)j * kp->ldS + i] = make_double2(sr[m][n], si[m][n]);
+            } else {
+                if (i < ng && i >= j) kp->S[(int64_t)j * kp->ldS + i] = make_double2(sr[m][n], i == j ? 0.0 : si[m][n]);
+            }
         }
 }
 
@@ -544,7 +572,13 @@ __global__ __launch_bounds__(256 * M / MJ) void k_overlap(SphereArgs p)
 {
     extern __shared__ __attribute__((aligned(1024))) char lds[];
     stamp(p, 3);
-    overlap_tile<M, MJ, true>(p, (int)blockIdx.x, lds);
+    overlap_tile<M, MJ, true, false>(p, (int)blockIdx.x, lds);
+}
+
+__global__ __launch_bounds__(256) void k_overlap_sample(SphereArgs p)
+{
+    extern __shared__ __attribute__((aligned(1024))) char lds[];
+    overlap_tile<2, 2, true, true>(p, (int)blockIdx.x, lds);
 }
 
 int overlap_tile_size(int64_t tiles64, int n_cu)
@@ -839,10 +873,15 @@ __device__ __forceinline__ int64_t uni(int64_t v)
     return (int64_t)(((uint64_t)(uint32_t)uni((int)(v >> 32)) << 32) | (uint32_t)uni((int)v));
 }
 
-template <int BR, int BC, int RB, int CB, int NS, bool kH>
+// What a product computes: W (T application), the lower triangle of H, or the
+// sampled columns of H.
+enum SphereMode { kTApp, kLowerH, kSampleH };
+
+template <int BR, int BC, int RB, int CB, int NS, int kMode>
 __device__ __forceinline__ void sphere_gemm_tile(const SphereArgs& p, int blk, char* lds)
 {
 #pragma clang fp contract(off)
+    constexpr bool kH = kMode != kTApp;
     using Tl = SphereTile<BR, BC, RB, CB, NS>;
     constexpr int NX = Tl::kXLoads, NY = Tl::kYLoads;
     const int tid = threadIdx.x;
@@ -855,7 +894,21 @@ __device__ __forceinline__ void sphere_gemm_tile(const SphereArgs& p, int blk, c
     const KindDev* kd = nullptr;
     int R0, C0;             // first row (X column), first column (y column) of the tile
     int nsteps;             // k-steps of 4
-    if constexpr (kH) {
+    int i0 = 0, xcol = 0;   // samples: H row of the tile's first y column, first of the k-point's X columns
+    if constexpr (kMode == kSampleH) {
+        // tiles of the chunk's columns in turn, per tile the sampled ones
+        constexpr int kRow = kSampleCols / BR;
+        const int tc = blk / kRow;
+        C0 = uni(tc * BC);
+        R0 = uni((blk - tc * kRow) * BR);
+        const int c = (int)p.cbase + C0;
+        const int ki = p.nk > 1 ? find_last(p.nk, c, [&](int i) { return (int)p.many[i].col0; }) : 0;
+        if (p.nk > 1) kp = p.many + ki;
+        i0 = uni(c - (int)kp->col0);
+        xcol = uni(ki * kSampleCols);
+        if (i0 >= kp->ng || R0 >= min(kp->ng, kSampleCols)) return;
+        nsteps = p.nksteps;
+    } else if constexpr (kH) {
         // Workgroups go to the 8 XCDs in turn.  The lower squares of BC of all
         // k-points, in patches of P x P squares, are cut into 8 equal
         // parts, one per XCD: the tiles in flight on one L2 share their
@@ -905,7 +958,9 @@ __device__ __forceinline__ void sphere_gemm_tile(const SphereArgs& p, int blk, c
         C0 = uni((cg * P + u - tr * h) * BC);
         nsteps = uni(kd->r4 / 4);
     }
-    const int64_t col0 = kH ? uni(kp->col0) : 0;
+    const int64_t col0 = kMode == kLowerH ? uni(kp->col0) : 0;
+    const double2* const X = kMode == kSampleH ? p.smp_W + (int64_t)xcol * p.smp_ldw : p.W + col0 * p.ldw;
+    const int64_t ldx = kMode == kSampleH ? p.smp_ldw : p.ldw;
     const int nst = uni((nsteps + 3) / 4);
 
     // ---- loads ----
@@ -921,8 +976,8 @@ __device__ __forceinline__ void sphere_gemm_tile(const SphereArgs& p, int blk, c
         const int c = c0 + (lane >> 4);
         const int q = (lane & 15) ^ (c & 15);
         if constexpr (kH) {
-            xbase[r] = (const char*)(p.W + (col0 + R0 + c0) * p.ldw);
-            xoff[r] = (uint32_t)(((int64_t)(lane >> 4) * p.ldw + q) * 16);
+            xbase[r] = (const char*)(X + (R0 + c0) * ldx);
+            xoff[r] = (uint32_t)(((int64_t)(lane >> 4) * ldx + q) * 16);
         } else {
             // row R0 + c of the kind's stacked Mt; past its last row the last one again
             const int row = min(R0 + c, kd->count * kd->r4 - 1);
@@ -1177,7 +1232,20 @@ __device__ __forceinline__ void sphere_gemm_tile(const SphereArgs& p, int blk, c
     __builtin_amdgcn_s_waitcnt(0);
 
     // ---- store: lane holds rows (lane >> 4) + 4 q of column lane & 15 ----
-    if constexpr (kH) {
+    if constexpr (kMode == kSampleH) {
+        const int ng = kp->ng, nb = min(ng, kSampleCols);
+#pragma unroll
+        for (int i = 0; i < RB; ++i)
+#pragma unroll
+            for (int j = 0; j < CB; ++j) {
+                const int gi = i0 + c0 + 16 * j;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const int gj = R0 + wr * 16 * RB + i * 16 + q0 + 4 * q;
+                    if (gi < ng && gj < nb) kp->H[(int64_t)gj * kp->ldH + gi] = make_double2(cr[i][j][q], ci[i][j][q]);
+                }
+            }
+    } else if constexpr (kH) {
         const int ng = kp->ng;
 #pragma unroll
         for (int i = 0; i < RB; ++i)
@@ -1215,12 +1283,12 @@ __device__ __forceinline__ void sphere_gemm_tile(const SphereArgs& p, int blk, c
     }
 }
 
-template <int BR, int BC, int RB, int CB, int NS, bool kH>
+template <int BR, int BC, int RB, int CB, int NS, int kMode>
 __global__ __launch_bounds__((SphereTile<BR, BC, RB, CB, NS>::kThreads), 4) void k_sphere_gemm(SphereArgs p)
 {
     extern __shared__ __attribute__((aligned(1024))) char lds[];
-    stamp(p, kH ? 2 : 1);
-    sphere_gemm_tile<BR, BC, RB, CB, NS, kH>(p, (int)blockIdx.x, lds);
+    stamp(p, kMode == kTApp ? 1 : 2);
+    sphere_gemm_tile<BR, BC, RB, CB, NS, kMode>(p, (int)blockIdx.x, lds);
 }
 
 // H tiles of 32 x 32 and S tiles of 16 M x 16 M in one launch, for triangles
@@ -1230,15 +1298,15 @@ __global__ __launch_bounds__(256, 4) void k_sphere_hs(SphereArgs p, int hblocks)
 {
     extern __shared__ __attribute__((aligned(1024))) char lds[];
     stamp(p, 2);
-    if ((int)blockIdx.x < hblocks) sphere_gemm_tile<32, 32, 1, 1, kSphereSmall, true>(p, (int)blockIdx.x, lds);
-    else overlap_tile<M, M, false>(p, (int)blockIdx.x - hblocks, lds);
+    if ((int)blockIdx.x < hblocks) sphere_gemm_tile<32, 32, 1, 1, kSphereSmall, kLowerH>(p, (int)blockIdx.x, lds);
+    else overlap_tile<M, M, false, false>(p, (int)blockIdx.x - hblocks, lds);
 }
 
-template <int BR, int BC, int RB, int CB, int NS, bool kH>
+template <int BR, int BC, int RB, int CB, int NS, int kMode>
 static hipError_t launch_sphere_gemm(const SphereArgs& p, int64_t nblk, hipEvent_t stop, hipStream_t st)
 {
     using Tl = SphereTile<BR, BC, RB, CB, NS>;
-    return launch(k_sphere_gemm<BR, BC, RB, CB, NS, kH>, dim3((unsigned)nblk), Tl::kThreads, Tl::kLds, stop, st, p);
+    return launch(k_sphere_gemm<BR, BC, RB, CB, NS, kMode>, dim3((unsigned)nblk), Tl::kThreads, Tl::kLds, stop, st, p);
 }
 
 // rtiles: row tiles of all kinds for the tile's rows (tile 64: 32 x 64)
@@ -1247,8 +1315,8 @@ hipError_t launch_sphere_tapp(const SphereArgs& p, int tile, int rtiles, hipEven
     SphereArgs q = p;
     q.rtiles = rtiles;
     const int64_t nblk = (int64_t)rtiles * (p.gtot / (tile == 32 ? 32 : 64));
-    if (tile == 32) return launch_sphere_gemm<32, 32, 1, 1, 2, false>(q, nblk, stop, st);
-    return launch_sphere_gemm<32, 64, 1, 2, 2, false>(q, nblk, stop, st);
+    if (tile == 32) return launch_sphere_gemm<32, 32, 1, 1, 2, kTApp>(q, nblk, stop, st);
+    return launch_sphere_gemm<32, 64, 1, 2, 2, kTApp>(q, nblk, stop, st);
 }
 
 static int64_t hblocks(const SphereArgs& p, int tile) { return ((int64_t)p.nsquares * (tile == 48 ? 2 : 1) + 7) / 8 * 8; }
@@ -1257,9 +1325,9 @@ static int64_t hblocks(const SphereArgs& p, int tile) { return ((int64_t)p.nsqua
 hipError_t launch_sphere_h(const SphereArgs& p, int tile, hipEvent_t stop, hipStream_t st)
 {
     const int64_t n = hblocks(p, tile);
-    if (tile == 32) return launch_sphere_gemm<32, 32, 1, 1, kSphereSmall, true>(p, n, stop, st);
-    if (tile == 48) return launch_sphere_gemm<32, 64, 1, 2, 2, true>(p, n, stop, st);
-    return launch_sphere_gemm<64, 64, 1, 2, 2, true>(p, n, stop, st);
+    if (tile == 32) return launch_sphere_gemm<32, 32, 1, 1, kSphereSmall, kLowerH>(p, n, stop, st);
+    if (tile == 48) return launch_sphere_gemm<32, 64, 1, 2, 2, kLowerH>(p, n, stop, st);
+    return launch_sphere_gemm<64, 64, 1, 2, 2, kLowerH>(p, n, stop, st);
 }
 
 template <int M>
@@ -1273,6 +1341,31 @@ static hipError_t launch_hs(const SphereArgs& p, int64_t nstiles, hipEvent_t sto
 hipError_t launch_sphere_hs(const SphereArgs& p, int stile, int64_t nstiles, hipEvent_t stop, hipStream_t st)
 {
     return stile == 32 ? launch_hs<2>(p, nstiles, stop, st) : launch_hs<1>(p, nstiles, stop, st);
+}
+
+// G of the sampled columns: block ki, lane j.
+__global__ __launch_bounds__(kSampleCols) void k_sample_g(SphereArgs p, const int32_t* __restrict__ cols, int32_t* __restrict__ out)
+{
+    const SphereK* kp = p.nk > 1 ? p.many + blockIdx.x : &p.one;
+    const int at = blockIdx.x * kSampleCols + threadIdx.x;
+    for (int q = 0; q < 3; ++q) out[3 * at + q] = kp->g[3 * cols[at] + q];
+}
+
+hipError_t launch_sample_g(const SphereArgs& p, const int32_t* cols, int32_t* out, hipStream_t st)
+{
+    hipLaunchKernelGGL(k_sample_g, dim3(p.nk), dim3(kSampleCols), 0, st, p, cols, out);
+    return hipGetLastError();
+}
+
+hipError_t launch_sample(const SphereArgs& p, bool do_h, bool do_s, hipStream_t st)
+{
+    hipError_t e = hipSuccess;
+    if (do_h)
+        e = launch_sphere_gemm<32, 32, 1, 1, kSphereSmall, kSampleH>(p, p.gtot / 32 * (kSampleCols / 32), nullptr, st);
+    if (e == hipSuccess && do_s)
+        e = launch(k_overlap_sample, dim3((unsigned)(p.gtot / 32 * (kSampleCols / 32))), 256,
+                   (size_t)OverlapTile<2, 2>::lds((p.nl + 15) / 16), nullptr, st, p);
+    return e;
 }
 
 }  // namespace hsgen

@@ -491,15 +491,56 @@ hsgen_status oz_execute(hsgen_ctx* ctx, const Geometry& geo, const std::vector<O
 }  // namespace
 
 
+hsgen_status oz_sample(hsgen_ctx* ctx, const Geometry& geo, const std::vector<OzK>& ks, OzSample& smp)
+{
+    const ZgemmLaunchCfg sc = zgemm_cfg(kSampleTile);
+    smp = OzSample{};
+    for (const OzK& k : ks) {
+        const int nb = std::min(k.ng, sc.bn);
+        smp.nb.push_back(nb);
+        smp.soff.push_back(smp.nbt);
+        smp.nbt += nb;
+        smp.off.push_back(smp.total);
+        smp.total += (size_t)k.ng * nb;
+        smp.gath.push_back(smp.gath_total);
+        smp.gath_total += (size_t)geo.ldz * roundup(nb, sc.bn);
+        for (int j = 0; j < nb; ++j) smp.cols.push_back((int32_t)(((2 * (int64_t)j + 1) * k.ng) / (2 * (int64_t)nb)));
+    }
+    // The sample GEMM of one k-point has only ng / 64 tiles per product: at
+    // large depth it is split into nsplit depth chunks (one per 2048 rows, at
+    // most 8), so that the launch fills the chip; the chunks' products are
+    // summed in chunk order afterwards.  nsplit depends on the depth only, so
+    // a k-point's sample is the same in single and batched calls.
+    smp.nsplit = (int)std::max<int64_t>(1, std::min<int64_t>(8, geo.kpad / 2048));
+    const hsgen_status st =
+        ensure(ctx, ctx->oz_smp, sizeof(double2) * std::max<size_t>(2 * (smp.total + smp.gath_total) + 2 * smp.total * (smp.nsplit - 1), 1),
+               false);
+    if (st) return st;
+    smp.S = (double2*)ctx->oz_smp.p;
+    smp.H = smp.S + smp.total;
+    smp.gath_s = smp.H + smp.total;
+    smp.gath_h = smp.gath_s + smp.gath_total;
+    smp.parts = smp.gath_h + smp.gath_total;     // chunks 1 .. nsplit-1 of S and H, 2 total each
+    return HSGEN_OK;
+}
+
+std::vector<int32_t> OzSample::padded() const
+{
+    std::vector<int32_t> out;
+    for (size_t k = 0; k < nb.size(); ++k)
+        for (int j = 0; j < kSampleCols; ++j) out.push_back(cols[soff[k] + std::min(j, nb[k] - 1)]);
+    return out;
+}
+
 // S = Z^H Zs and H = Z^H W of every k-point from the resident FP64 operands,
 // on INT8 MFMA.  With nmod_req == 0 the modulus count is chosen for `target`:
-// per k-point, 64 evenly spaced columns of S and H computed in FP64 (all rows)
-// give |tril C|_F for the error model before any INT8 work, and the largest
+// per k-point, 64 evenly spaced columns of S and H computed in FP64 (all rows:
+// from a system by sphere_split_w, else from the operands) give |tril C|_F for the error model before any INT8 work, and the largest
 // count any k-point needs is used for all; after the run the model is
 // evaluated with the exact norms and the run repeated with more moduli if a
 // k-point misses the target.  The same samples measure the actual errors.
 hsgen_status run_ozaki(hsgen_ctx* ctx, const Geometry& geo, const std::vector<OzK>& ks, int flags, int icfg,
-                       int nmod_req, double target, std::vector<OzResult>& res, bool capture)
+                       int nmod_req, double target, std::vector<OzResult>& res, bool capture, const OzSample* sample)
 {
     const IgemmLaunchCfg ic = igemm_cfg(icfg);
     const int64_t kd = roundup(geo.kpad, ic.bk);           // INT8 contraction depth (complex)
@@ -522,19 +563,17 @@ hsgen_status run_ozaki(hsgen_ctx* ctx, const Geometry& geo, const std::vector<Oz
     // sample statistics over as many columns as the sample tile is wide
     const ZgemmLaunchCfg sc = zgemm_cfg(kSampleTile);
     const int kNblk = 1024;
-    std::vector<int> nb(nk);
-    std::vector<size_t> soff(nk), smp_off(nk), gath_off(nk);
-    size_t nbt = 0, smpt = 0, gatht = 0;
-    for (int k = 0; k < nk; ++k) {
-        nb[k] = std::min(ks[k].ng, sc.bn);
-        soff[k] = nbt;
-        nbt += nb[k];
-        smp_off[k] = smpt;
-        smpt += (size_t)ks[k].ng * nb[k];
-        gath_off[k] = gatht;
-        gatht += (size_t)geo.ldz * roundup(nb[k], sc.bn);
+    hsgen_status st = HSGEN_OK;
+    OzSample own;
+    if (!sample) {
+        if ((st = oz_sample(ctx, geo, ks, own))) return st;
+        sample = &own;
     }
-    hsgen_status st = ensure(ctx, ctx->oz_e, (sizeof(int32_t) + sizeof(double)) * 3 * (size_t)gp +
+    const std::vector<int>& nb = sample->nb;
+    const std::vector<size_t>&soff = sample->soff, &smp_off = sample->off, &gath_off = sample->gath;
+    const std::vector<int32_t>& cols = sample->cols;
+    const size_t nbt = sample->nbt, smpt = sample->total;
+    st = ensure(ctx, ctx->oz_e, (sizeof(int32_t) + sizeof(double)) * 3 * (size_t)gp +
                                                  sizeof(double) * (2 * (size_t)kNblk * nk + 2 * 3 * nbt) +
                                                  sizeof(int32_t) * std::max<size_t>(nbt, 1), false);
     if (st) return st;
@@ -547,10 +586,6 @@ hsgen_status run_ozaki(hsgen_ctx* ctx, const Geometry& geo, const std::vector<Oz
     int32_t* eZs = eZ + gp;
     int32_t* eW = eZs + gp;
     int32_t* dcols = eW + gp;                      // the sampled columns, relative to their k-point
-    std::vector<int32_t> cols(std::max<size_t>(nbt, 1));
-    for (int k = 0; k < nk; ++k)
-        for (int j = 0; j < nb[k]; ++j)
-            cols[soff[k] + j] = (int32_t)(((2 * (int64_t)j + 1) * ks[k].ng) / (2 * (int64_t)nb[k]));
     if (nbt > 0)
         HIPCHK(hipMemcpyAsync(dcols, cols.data(), sizeof(int32_t) * nbt, hipMemcpyHostToDevice, ctx->stream));
     const double2* Z = (const double2*)ctx->Z.p;
@@ -568,22 +603,15 @@ hsgen_status run_ozaki(hsgen_ctx* ctx, const Geometry& geo, const std::vector<Oz
     // FP64 samples: columns cols[] of S and H of each k-point, all rows, ld = ng
     // (the right operand's sampled columns are gathered first: the GEMM reads
     // contiguous columns, whole tiles of bn of them)
-    // The sample GEMM of one k-point has only ng / 64 tiles per product: at
-    // large depth it is split into nsplit depth chunks (one per 2048 rows, at
-    // most 8), so that the launch fills the chip; the chunks' products are
-    // summed in chunk order afterwards.  nsplit depends on the depth only, so
-    // a k-point's sample is the same in single and batched calls.
-    const int nsplit = (int)std::max<int64_t>(1, std::min<int64_t>(8, geo.kpad / 2048));
+    // A sample from a system's real vectors is there already.
+    const int nsplit = sample->nsplit;
     const int64_t kchunk = roundup((geo.kpad + nsplit - 1) / nsplit, sc.bk);
-    st = ensure(ctx, ctx->oz_smp, sizeof(double2) * std::max<size_t>(2 * (smpt + gatht) + 2 * smpt * (nsplit - 1), 1),
-                false);
-    if (st) return st;
-    double2* smpS = (double2*)ctx->oz_smp.p;
-    double2* smpH = smpS + smpt;
-    double2* gathS = smpH + smpt;
-    double2* gathH = gathS + gatht;
-    double2* smp_part = gathH + gatht;             // chunks 1 .. nsplit-1 of smpS and smpH, 2 smpt each
-    {
+    double2* smpS = sample->S;
+    double2* smpH = sample->H;
+    double2* gathS = sample->gath_s;
+    double2* gathH = sample->gath_h;
+    double2* smp_part = sample->parts;
+    if (sample == &own) {
         std::vector<GemmProblem> probs;
         std::vector<TileWork> work;
         auto add = [&](const OzK& k, const double2* R, double2* C, int n) {
@@ -956,8 +984,10 @@ hsgen_status batched_split(hsgen_ctx* ctx, hsgen_sys* s, int nk, const hsgen_kpo
             p.fold = geo.fold;
             HIPCHK(launch_abgen(p, true, ctx->stream));
         }
+        OzSample smp;
         if (do_h) {
             // T application over every column of the batch from the real vectors
+            if ((st = oz_sample(ctx, geo, ks, smp))) return st;
             std::vector<SphereK> sk(bk.size());
             for (size_t q = 0; q < bk.size(); ++q) {
                 std::memset(&sk[q], 0, sizeof sk[q]);
@@ -965,12 +995,16 @@ hsgen_status batched_split(hsgen_ctx* ctx, hsgen_sys* s, int nk, const hsgen_kpo
                 sk[q].g = (const int32_t*)ctx->g.p + goff[q];
                 sk[q].ng = ks[q].ng;
                 sk[q].col0 = ks[q].col0;
+                sk[q].H = smp.H + smp.off[q];
+                sk[q].S = smp.S + smp.off[q];
+                sk[q].ldH = sk[q].ldS = ks[q].ng;
             }
             st = ensure(ctx, ctx->probs, sizeof(SphereK) * sk.size(), false);
             if (st) return st;
             HIPCHK(hipMemcpyAsync(ctx->probs.p, sk.data(), sizeof(SphereK) * sk.size(), hipMemcpyHostToDevice,
                                   ctx->stream));
-            st = sphere_split_w(ctx, s, sk, (const SphereK*)ctx->probs.p, ncols, W, geo.ldz);
+            const std::vector<int32_t> cols = smp.padded();
+            st = sphere_split_w(ctx, s, sk, (const SphereK*)ctx->probs.p, ncols, W, geo.ldz, &cols, do_s);
             if (st) return st;
             HIPCHK(hipStreamSynchronize(ctx->stream));   // sk must outlive its copy, ctx->probs its readers
             HIPCHK(launch_clear_rows(W, geo.ldz, 2 * (int64_t)s->kdim, geo.ldz, (int)ncols, ctx->stream));
@@ -983,7 +1017,7 @@ hsgen_status batched_split(hsgen_ctx* ctx, hsgen_sys* s, int nk, const hsgen_kpo
         }
         Prefault pages(ctx, out);
         std::vector<OzResult> ozr;
-        st = run_ozaki(ctx, geo, ks, flags, icfg, o.slices, o.target_rel_err, ozr, true);
+        st = run_ozaki(ctx, geo, ks, flags, icfg, o.slices, o.target_rel_err, ozr, true, do_h ? &smp : nullptr);
         if (st) return st;
         for (size_t q = 0; q < bk.size() && (flags & HSGEN_FILL_UPPER); ++q) {
             if (do_h) HIPCHK(launch_fill_upper(ks[q].dH, ks[q].ldH, ks[q].ng, ctx->stream));

@@ -244,3 +244,30 @@ def test_more_than_sixteen_l_and_all_s_tiles(ctx, lmax, natoms):
             Hr, Sr = po.reference_hs(s, _subset(kp, idx))
             assert rel_fro_lower(Hs, Hr) <= TOL and rel_fro_lower(Ss, Sr) <= TOL
     h.close()
+
+
+@pytest.mark.parametrize("ng,cap", [(50, None), (64, None), (700, None), (700, 200000)])
+@pytest.mark.parametrize("norm", [None, 0.0])
+def test_split_sample_from_real_vectors(ctx, monkeypatch, ng, cap, norm):
+    """The FP64 sample of split precision, over one and several column chunks:
+    the error it reports is the split result's distance from FP64 on the sampled
+    columns.  FP64's own rounding, 1e-14 at most, is 1e-3 of the 1e-11 that 9
+    moduli leave."""
+    from hybridhsdla_amd.api import HSGEN_PREC_OZAKI_INT8
+    s, kp = tiny_system(natoms=10, lmax=(3, 5), a_cell=11.0, ng_target=720, seed=17)
+    if norm is not None:
+        s.match[1, 1, 4] = norm
+    sub = _subset(kp, np.arange(ng))
+    h = ctx.upload(s)
+    H0, S0 = ctx.create_HS2(h, sub)
+    if cap:
+        monkeypatch.setenv("HSGEN_BATCH_BYTES", str(cap))
+    H, S, rep = ctx.create_HS2(h, sub, precision=HSGEN_PREC_OZAKI_INT8, slices=9, report=True)
+    nb = min(ng, 64)
+    cols = [(2 * j + 1) * ng // (2 * nb) for j in range(nb)]
+    for X, X0, e in ((H, H0, rep["err_smp_h"]), (S, S0, rep["err_smp_s"])):
+        d = np.sqrt(sum(np.sum(np.abs(X[j:, j] - X0[j:, j]) ** 2) for j in cols) /
+                    sum(np.sum(np.abs(X0[j:, j]) ** 2) for j in cols))
+        print(f"sample {e:.4e} direct {d:.4e}", flush=True)
+        assert d > 1e-12 and abs(e - d) <= 1e-2 * d
+    h.close()
