@@ -123,6 +123,13 @@ __device__ inline void ylm_real(int m, int lmax, const DirAngles& dir, const dou
     }
 }
 
+// a b - c d without the rounding of c d, which counts where they cancel.
+__device__ __forceinline__ double product_difference(double a, double b, double c, double d)
+{
+    const double cd = c * d;
+    return __builtin_fma(a, b, -cd) - __builtin_fma(c, d, -cd);
+}
+
 }  // namespace
 
 // ---------------------------------------------------------------------------
@@ -173,9 +180,18 @@ __global__ __launch_bounds__(256) void k_sphere_gen(SphereArgs p)
     // phases e^{i 2 pi K.tau}; the lanes with the Bessel recurrences come last
     for (int a = blockDim.x - 1 - tid; a < p.natoms; a += blockDim.x) {
         const AtomDev& at = p.atoms[p.order[a]];
-        const double kt = K0 * at.pos[0] + K1 * at.pos[1] + K2 * at.pos[2];
+        // the fraction of K.tau, term by term: its rounding, not that of the whole
+        const double kq[6] = {(double)g0, (double)g1, (double)g2, k.k[0], k.k[1], k.k[2]};
+        double f = 0.0, rest = 0.0;
+#pragma unroll
+        for (int q = 0; q < 6; ++q) {
+            const double v = kq[q] * at.pos[q % 3];
+            rest += __builtin_fma(kq[q], at.pos[q % 3], -v);
+            f += v - rint(v);
+        }
+        f += rest;
         double ps, pc;
-        sincos(2.0 * kPi * kt, &ps, &pc);
+        sincospi(2.0 * (f - rint(f)), &ps, &pc);
         p.ph[(int64_t)a * p.gtot + col] = make_double2(pc, ps);
     }
     for (int k0 = 0; k0 < p.nkinds; k0 += p.chunk) {
@@ -196,8 +212,8 @@ __global__ __launch_bounds__(256) void k_sphere_gen(SphereArgs p)
             const double* dfj = fj + nl;
             const RadDev m = p.rad[(int64_t)kd.rep * nl + l];
             const double pref = p.vol_prefac * m.inv_wronk;
-            const double au = m.dE_u * Knorm * dfj[l] - m.dE_u_dr * fj[l];
-            const double bu = -m.u * Knorm * dfj[l] + m.u_dr * fj[l];
+            const double au = product_difference(m.dE_u * Knorm, dfj[l], m.dE_u_dr, fj[l]);
+            const double bu = product_difference(m.u_dr, fj[l], m.u * Knorm, dfj[l]);
             const double2 ab = make_double2(pref * au, pref * bu);
             s_ab[t * nl + l] = ab;
             if (p.rs && kd.rsoff >= 0) {
