@@ -10,16 +10,17 @@
 // bytes (43 GB/s in slots of 2 MiB, 48 in 4, 51 in 8), and a lower triangle is a
 // rectangle to it; the kernel takes each column from its diagonal on and says
 // itself, in pinned memory, when a slot has landed.  To the host three slots per
-// launch (62 MB in 1230 us; one: 1370), 128 workgroups (64: 1260, 256: 1320);
-// from it a slot as soon as it is filled, 64 workgroups (62 MB in 970 us; 16:
-// 1160, 256: 1240).
+// launch (62 MB in 1230 us; one: 1370); from it a slot as soon as it is filled.
+// Few workgroups: the link takes slots of 4 MiB at 52 GB/s to the host and 53 from
+// it with 24, 51 and 48 with 64, 44 and 34 with 256.
 // Threads matter most where the host pages are fresh: one thread writes them at
 // 15 GB/s, eight at 65, more not faster.  The last slot's host side overlaps
 // nothing, so slots are small.
 // Measured, whole calls, the runtime's copies before: A and B of 16 atoms at
 // N_G 1500 (62 MB) 5.0 -> 1.3 ms; H and S at N_G 1201 (46 MB, both triangles)
 // 2.87 -> 1.45 ms; the contraction of given coefficients at N_G 1500 (62 MB in,
-// two lower triangles out) 7.7 -> 4.9 ms.
+// two lower triangles out) 7.7 -> 4.9 ms, 3.4 with M built on the GPU and S's copy
+// beside H.
 #include <sys/mman.h>
 #include <unistd.h>
 
@@ -42,9 +43,7 @@ constexpr size_t kSlotBytes = (size_t)4 << 20;
 constexpr size_t kPieceBytes = (size_t)256 << 10;    // what a thread copies at a time
 constexpr size_t kThreadBytes = (size_t)1 << 20;     // one more thread per so many bytes
 constexpr size_t kFlagBytes = 64 * kRingSlots;       // one line per slot, after the slots
-#ifndef GRIDN
-#define GRIDN 24
-#endif
+constexpr size_t kGrid = 24;                         // workgroups of a copy kernel
 constexpr int kGroup = kRingSlots / 2;               // slots of one launch
 constexpr size_t kRange = (size_t)2 << 20;           // memory that Prefault maps at a time
 
@@ -397,7 +396,7 @@ hsgen_status host_copy(hsgen_ctx* ctx, const std::vector<HostCopy>& list, bool t
                                 (uint64_t*)((char*)ctx->ring_dev + kSlotBytes * kN + 64 * i), seq0 + b + g.n};
             most = std::max(most, k.width * k.height);
         }
-        const dim3 grid((unsigned)std::min<size_t>(GRIDN, most / 16384 + 1));
+        const dim3 grid((unsigned)std::min<size_t>(kGrid, most / 16384 + 1));
 
         if (to_host) hipLaunchKernelGGL(k_slot_copy<true>, grid, dim3(256), 0, stream, g);
         else hipLaunchKernelGGL(k_slot_copy<false>, grid, dim3(256), 0, stream, g);

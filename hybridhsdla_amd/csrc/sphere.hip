@@ -829,8 +829,8 @@ hipError_t launch_split_mt(const SplitMtJob* jobs, int njobs, int64_t max_elems,
 // Rate of the H tiles: 0.87 of the FP64 peak at N_G 16000 and 25000, 0.85 at
 // 10000, 0.82 at 6002 (32 atoms, lmax 10).
 // Measured (whole call, complex-by-complex contraction of S and H before, now):
-// 714 -> 208 ms at N_G 12007 (128 atoms, lmax 12), 33.5 -> 10.2 ms at 6002 and
-// 5.47 -> 1.46 ms at 2003 (32 atoms, lmax 10).
+// 714 -> 202 ms at N_G 12007 (128 atoms, lmax 12), 33.5 -> 10.0 ms at 6002 and
+// 5.41 -> 1.37 ms at 2003 (32 atoms, lmax 10), with S and all else since.
 // ---------------------------------------------------------------------------
 namespace {
 
