@@ -207,29 +207,69 @@ void add_tmul_problems(std::vector<GemmProblem>& probs, std::vector<TileWork>& w
     }
 }
 
-// The vectors must outlive the copies: until the stream is waited for.
-static hsgen_status launch_grouped(hsgen_ctx* ctx, int cfg, const std::vector<GemmProblem>& probs,
-                                   const std::vector<TileWork>& work, DevBuf& dprobs, DevBuf& dwork, hipStream_t stream)
-{
-    if (work.empty()) return HSGEN_OK;
-    hsgen_status st = ensure(ctx, dprobs, sizeof(GemmProblem) * probs.size(), false);
-    if (st) return st;
-    st = ensure(ctx, dwork, sizeof(TileWork) * work.size(), false);
-    if (st) return st;
-    HIPCHK(hipMemcpyAsync(dprobs.p, probs.data(), sizeof(GemmProblem) * probs.size(), hipMemcpyHostToDevice, stream));
-    HIPCHK(hipMemcpyAsync(dwork.p, work.data(), sizeof(TileWork) * work.size(), hipMemcpyHostToDevice, stream));
-    HIPCHK(launch_zgemm(cfg, (const GemmProblem*)dprobs.p, (const TileWork*)dwork.p, (int)work.size(), stream));
-    return HSGEN_OK;
-}
-
 hsgen_status run_grouped(hsgen_ctx* ctx, int cfg, std::vector<GemmProblem>& probs,
                          std::vector<TileWork>& work)
 {
-    hsgen_status st = launch_grouped(ctx, cfg, probs, work, ctx->probs, ctx->work, ctx->stream);
+    if (work.empty()) return HSGEN_OK;
+    hsgen_status st = ensure(ctx, ctx->probs, sizeof(GemmProblem) * probs.size(), false);
     if (st) return st;
+    st = ensure(ctx, ctx->work, sizeof(TileWork) * work.size(), false);
+    if (st) return st;
+    HIPCHK(hipMemcpyAsync(ctx->probs.p, probs.data(), sizeof(GemmProblem) * probs.size(),
+                          hipMemcpyHostToDevice, ctx->stream));
+    HIPCHK(hipMemcpyAsync(ctx->work.p, work.data(), sizeof(TileWork) * work.size(),
+                          hipMemcpyHostToDevice, ctx->stream));
+    HIPCHK(launch_zgemm(cfg, (const GemmProblem*)ctx->probs.p, (const TileWork*)ctx->work.p,
+                        (int)work.size(), ctx->stream));
+    // the host vectors must outlive the async copies
     HIPCHK(hipStreamSynchronize(ctx->stream));
     return HSGEN_OK;
 }
+
+namespace {
+
+// Problem and tile lists of several launches, sent in one copy (10 us each
+// otherwise).
+struct GroupedLists {
+    struct List {
+        std::vector<GemmProblem> probs;
+        std::vector<TileWork> work;
+        size_t at = 0;
+    };
+    List list[3];
+    std::vector<char> host;
+    const char* dev = nullptr;
+
+    hsgen_status send(hsgen_ctx* ctx)
+    {
+        for (List& l : list) {
+            l.at = host.size();
+            host.resize(host.size() + sizeof(GemmProblem) * l.probs.size() + roundup(sizeof(TileWork) * l.work.size(), 16));
+            if (l.work.empty()) continue;
+            std::memcpy(host.data() + l.at, l.probs.data(), sizeof(GemmProblem) * l.probs.size());
+            std::memcpy(host.data() + l.at + sizeof(GemmProblem) * l.probs.size(), l.work.data(),
+                        sizeof(TileWork) * l.work.size());
+        }
+        if (host.empty()) return HSGEN_OK;
+        const hsgen_status st = ensure(ctx, ctx->lists, host.size(), false);
+        if (st) return st;
+        dev = (const char*)ctx->lists.p;
+        HIPCHK(hipMemcpyAsync(ctx->lists.p, host.data(), host.size(), hipMemcpyHostToDevice, ctx->stream));
+        return HSGEN_OK;
+    }
+
+    hipError_t launch(int i, int cfg, hipStream_t stream) const
+    {
+        const List& l = list[i];
+        if (l.work.empty()) return hipSuccess;
+        return launch_zgemm(cfg, (const GemmProblem*)(dev + l.at),
+                            (const TileWork*)(dev + l.at + sizeof(GemmProblem) * l.probs.size()), (int)l.work.size(),
+                            stream);
+    }
+};
+static_assert(sizeof(GemmProblem) % 8 == 0 && sizeof(TileWork) % 4 == 0, "lists follow each other");
+
+}  // namespace
 
 // Common tail of create_hs / contract_hs: Y (or Z, Zs) resident -> tmul -> S, H.
 // With kp (split precision from a system, its G list in ctx->g) W comes from
@@ -286,35 +326,38 @@ hsgen_status finish_hs(hsgen_ctx* ctx, hsgen_sys* s, const Geometry& geo, int ng
     // to the second stream, and its copy to the host runs while H is computed
     // (3.72 -> 3.39 ms at N_G 1500 from given coefficients).
     const bool apart = !is_split(o.precision) && need_h && !out_h.empty() && !out_s.empty();
-    // problem and tile lists, until the streams are waited for
-    std::vector<GemmProblem> tprobs, probs, sprobs;
     OzSample smp;
-    std::vector<TileWork> twork, work, swork;
-    auto products = [&](std::vector<GemmProblem>& pr, std::vector<TileWork>& wk, int skip) {
-        add_hs_problems(pr, wk, geo, ng, Z, Zs, W, dH, dS, 0, flags | skip);
-        xcd_permute(wk);
-        for (auto& p : pr) {
+    // T application, S apart, and the rest; kept until the streams are waited for
+    GroupedLists lists;
+    const int tc = tapp_cfg(geo);
+    auto products = [&](GroupedLists::List& l, int skip) {
+        add_hs_problems(l.probs, l.work, geo, ng, Z, Zs, W, dH, dS, 0, flags | skip);
+        xcd_permute(l.work);
+        for (auto& p : l.probs) {
             p.ldl = geo.ldz;
             p.ldr = geo.ldz;
             p.kdepth = (int32_t)geo.kpad;
             p.ldc = (p.C == dH) ? ldH : ldS;
         }
     };
+    if (need_h && !kp) add_tmul_problems(lists.list[0].probs, lists.list[0].work, s, geo, zgemm_cfg(tc), ng, Z, W);
+    if (apart) products(lists.list[1], HSGEN_SKIP_H);
+    if (!is_split(o.precision)) products(lists.list[2], apart ? HSGEN_SKIP_S : 0);
     if (apart && !ctx->stream2) HIPCHK(hipStreamCreateWithFlags(&ctx->stream2, hipStreamNonBlocking));
     struct Wait {
         hsgen_ctx* ctx;
         ~Wait()
         {
+            if (!ctx) return;
             (void)hipStreamSynchronize(ctx->stream);
             if (ctx->stream2) (void)hipStreamSynchronize(ctx->stream2);
         }
     } wait{ctx};
+    if ((st = lists.send(ctx))) return st;
     HIPCHK(hipEventRecord(ctx->ev[2], ctx->stream));
     if (apart) {
         HIPCHK(hipStreamWaitEvent(ctx->stream2, ctx->ev[2], 0));
-        products(sprobs, swork, HSGEN_SKIP_H);
-        st = launch_grouped(ctx, geo.cfg, sprobs, swork, ctx->probs2, ctx->work2, ctx->stream2);
-        if (st) return st;
+        HIPCHK(lists.launch(1, geo.cfg, ctx->stream2));
         if (flags & HSGEN_FILL_UPPER) HIPCHK(launch_fill_upper(dS, ldS, ng, ctx->stream2));
         HIPCHK(hipEventRecord(ctx->ev[5], ctx->stream2));
     }
@@ -334,9 +377,7 @@ hsgen_status finish_hs(hsgen_ctx* ctx, hsgen_sys* s, const Geometry& geo, int ng
             const std::vector<int32_t> cols = smp.padded();
             st = sphere_split_w(ctx, s, {k}, nullptr, geo.gp, W, geo.ldz, &cols, do_s);
         } else {
-            const int tc = tapp_cfg(geo);
-            add_tmul_problems(tprobs, twork, s, geo, zgemm_cfg(tc), ng, Z, W);
-            st = launch_grouped(ctx, tc, tprobs, twork, ctx->tprobs, ctx->twork, ctx->stream);
+            HIPCHK(lists.launch(0, tc, ctx->stream));
         }
         if (st) return st;
         // rows 2K .. ldz-1 of W are not written by the T application; clear
@@ -361,9 +402,7 @@ hsgen_status finish_hs(hsgen_ctx* ctx, hsgen_sys* s, const Geometry& geo, int ng
         if (st) return st;
         oz = ozr[0];
     } else {
-        products(probs, work, apart ? HSGEN_SKIP_S : 0);
-        st = launch_grouped(ctx, geo.cfg, probs, work, ctx->probs, ctx->work, ctx->stream);
-        if (st) return st;
+        HIPCHK(lists.launch(2, geo.cfg, ctx->stream));
     }
     if (flags & HSGEN_FILL_UPPER) {
         if (need_h) HIPCHK(launch_fill_upper(dH, ldH, ng, ctx->stream));
@@ -377,7 +416,8 @@ hsgen_status finish_hs(hsgen_ctx* ctx, hsgen_sys* s, const Geometry& geo, int ng
         HIPCHK(hipEventSynchronize(ctx->ev[4]));
         if ((st = host_copy(ctx, out, true, ctx->stream))) return st;
     }
-    HIPCHK(hipEventSynchronize(ctx->ev[4]));
+    HIPCHK(hipEventSynchronize(ctx->ev[4]));    // of both streams
+    wait.ctx = nullptr;
     if (rep) {
         float t1 = 0, t2 = 0;
         HIPCHK(hipEventElapsedTime(&t1, ctx->ev[2], ctx->ev[3]));
@@ -911,9 +951,11 @@ hsgen_status hsgen_contract_hs(hsgen_ctx* ctx, int32_t L, int32_t a, int32_t G, 
     HIPCHK(hipEventRecord(ctx->ev[0], ctx->stream));
     HIPCHK(launch_pack_ref(pp, (int)geo.gp, ctx->stream));
     HIPCHK(hipEventRecord(ctx->ev[1], ctx->stream));
-    st = finish_hs(ctx, &s, geo, G, o, H, S, ld, rep, 0.0);
-    HIPCHK(hipStreamSynchronize(ctx->stream));
-    if (st) return st;
+    st = finish_hs(ctx, &s, geo, G, o, H, S, ld, rep, 0.0, nullptr);
+    if (st) {
+        (void)hipStreamSynchronize(ctx->stream);
+        return st;
+    }
     if (rep) {
         float t0 = 0;
         HIPCHK(hipEventElapsedTime(&t0, ctx->ev[0], ctx->ev[1]));

@@ -145,7 +145,7 @@ struct hsgen_ctx {
     hipEvent_t ev[8] = {};
     std::string err;
     // workspace
-    hsgen::DevBuf Z, Zs, W, Htmp, Stmp, A, B, g, probs, work, pack, m_in, M, probs2, work2, tprobs, twork;
+    hsgen::DevBuf Z, Zs, W, Htmp, Stmp, A, B, g, probs, work, pack, m_in, M, lists;
     // FP64 from a system: phases, radial factors, real vectors (W, host-output copies above)
     hsgen::DevBuf sph_ph, sph_rs, sph_y, sph_w, sph_smp;
     // split precision
