@@ -160,7 +160,7 @@ hipError_t launch_sphere_h(const SphereArgs& p, int tile, hipEvent_t stop, hipSt
 // S tile side by the number of lower tiles; the bits do not depend on it
 int overlap_tile_size(int64_t tiles64, int n_cu);
 hipError_t launch_overlap(const SphereArgs& p, int tile, int64_t ntiles, hipEvent_t stop, hipStream_t st);
-// H tiles of 32 x 32 and S tiles of 16 or 32 in one launch
-hipError_t launch_sphere_hs(const SphereArgs& p, int stile, int64_t nstiles, hipEvent_t stop, hipStream_t st);
+// H tiles of 32 x 32 (or 16 x 32: tile 16, S tile 16) and S tiles of 16 or 32 in one launch
+hipError_t launch_sphere_hs(const SphereArgs& p, int tile, int stile, int64_t nstiles, hipEvent_t stop, hipStream_t st);
 
 }  // namespace hsgen

@@ -859,18 +859,19 @@ __device__ __forceinline__ int ends_before(i8 e, int ks)
 }  // namespace
 
 // BR x BC tile (rows: X columns, columns: y columns), waves of 16 RB x 16 CB,
-// NS stages in LDS.
-template <int BR, int BC, int RB, int CB, int NS>
+// NS stages in LDS.  PARTS 2: one wave the real, one the imaginary part.
+template <int BR, int BC, int RB, int CB, int NS, int PARTS = 1>
 struct SphereTile {
     static constexpr int kWR = BR / (16 * RB);    // waves along the rows
     static constexpr int kWC = BC / (16 * CB);
-    static constexpr int kWaves = kWR * kWC;
+    static constexpr int kWaves = kWR * kWC * PARTS;
     static constexpr int kThreads = 64 * kWaves;
     static constexpr int kXBytes = BR * 256;      // one stage of X, of y
     static constexpr int kYBytes = BC * 128;
     static constexpr int kPhBytes = 256 * CB;     // a wave's phases of an atom that ends in a stage
     static constexpr int kStage = kXBytes + kYBytes + kWaves * kPhBytes;
-    static constexpr int kLds = NS * kStage;
+    static constexpr int kSwap = PARTS == 2 ? 2 * kWaves * RB * CB * 2048 : 0;   // T that the parts exchange
+    static constexpr int kLds = NS * kStage + kSwap;
     static constexpr int kXLoads = kXBytes / 1024 / kWaves;   // 1 KiB wave loads per wave and stage
     static constexpr int kYLoads = kYBytes / 1024 / kWaves;
     static_assert(kXLoads * kWaves * 1024 == kXBytes && kYLoads * kWaves * 1024 == kYBytes,
@@ -893,17 +894,18 @@ __device__ __forceinline__ int64_t uni(int64_t v)
 // sampled columns of H.
 enum SphereMode { kTApp, kLowerH, kSampleH };
 
-template <int BR, int BC, int RB, int CB, int NS, int kMode>
+template <int BR, int BC, int RB, int CB, int NS, int kMode, int PARTS = 1>
 __device__ __forceinline__ void sphere_gemm_tile(const SphereArgs& p, int blk, char* lds)
 {
 #pragma clang fp contract(off)
     constexpr bool kH = kMode != kTApp;
-    using Tl = SphereTile<BR, BC, RB, CB, NS>;
+    using Tl = SphereTile<BR, BC, RB, CB, NS, PARTS>;
     constexpr int NX = Tl::kXLoads, NY = Tl::kYLoads;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wr = wave % Tl::kWR, wc = wave / Tl::kWR;
+    const int wr = wave % Tl::kWR, wc = wave / Tl::kWR % Tl::kWC;
+    const int part = PARTS == 2 ? wave / (Tl::kWR * Tl::kWC) : 0;
 
     // ---- the tile ----
     const SphereK* kp = &p.one;
@@ -1087,7 +1089,10 @@ __device__ __forceinline__ void sphere_gemm_tile(const SphereArgs& p, int blk, c
     }
     auto read_frags = [&](int buf, int ks, v2d* x, double* y) {
 #pragma unroll
-        for (int i = 0; i < RB; ++i) x[i] = *(const v2d*)&lds[xat[ks] + (buf * Tl::kStage + i * 4096)];
+        for (int i = 0; i < RB; ++i) {
+            if constexpr (PARTS == 2) x[i].x = *(const double*)&lds[xat[ks] + 8 * part + (buf * Tl::kStage + i * 4096)];
+            else x[i] = *(const v2d*)&lds[xat[ks] + (buf * Tl::kStage + i * 4096)];
+        }
 #pragma unroll
         for (int j = 0; j < CB; ++j) y[j] = *(const double*)&lds[yat[ks] + (buf * Tl::kStage + j * 2048)];
     };
@@ -1104,7 +1109,41 @@ __device__ __forceinline__ void sphere_gemm_tile(const SphereArgs& p, int blk, c
         for (int j = 0; j < CB; ++j) ph[j] = *(const v2d*)&p.ph[(int64_t)atom * p.gtot + (col0 + C0 + c0 + 16 * j)];
     };
     // C += conj(phase) T, T = 0
+    int swap = 0;
     auto flush = [&](const v2d* ph) {
+        if constexpr (PARTS == 2) {
+            // the other part of T by way of LDS; two buffers, so that one barrier
+            // per flush does
+            char* mine = lds + NS * Tl::kStage + (swap * Tl::kWaves + wave) * (RB * CB * 2048) + lane * 16;
+            const int other = part ? wave - Tl::kWR * Tl::kWC : wave + Tl::kWR * Tl::kWC;
+            const char* its = lds + NS * Tl::kStage + (swap * Tl::kWaves + other) * (RB * CB * 2048) + lane * 16;
+#pragma unroll
+            for (int i = 0; i < RB; ++i)
+#pragma unroll
+                for (int j = 0; j < CB; ++j) {
+                    *(v2d*)&mine[(i * CB + j) * 2048] = v2d{tr_[i][j][0], tr_[i][j][1]};
+                    *(v2d*)&mine[(i * CB + j) * 2048 + 1024] = v2d{tr_[i][j][2], tr_[i][j][3]};
+                }
+            __builtin_amdgcn_s_waitcnt(wait_vm(63, true));
+            asm volatile("s_barrier" ::: "memory");
+#pragma unroll
+            for (int i = 0; i < RB; ++i)
+#pragma unroll
+                for (int j = 0; j < CB; ++j)
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        const v2d o = *(const v2d*)&its[(i * CB + j) * 2048 + h * 1024];
+#pragma unroll
+                        for (int q = 2 * h; q < 2 * h + 2; ++q) {
+                            // part 0: a mine, b the other; part 1 the other way round
+                            const double m = tr_[i][j][q], v = h == 0 ? (q == 0 ? o.x : o.y) : (q == 2 ? o.x : o.y);
+                            cr[i][j][q] = __builtin_fma(part ? -ph[j].y : ph[j].y, v, __builtin_fma(ph[j].x, m, cr[i][j][q]));
+                            tr_[i][j][q] = 0.0;
+                        }
+                    }
+            swap ^= 1;
+            return;
+        }
 #pragma unroll
         for (int i = 0; i < RB; ++i)
 #pragma unroll
@@ -1131,11 +1170,13 @@ __device__ __forceinline__ void sphere_gemm_tile(const SphereArgs& p, int blk, c
 #pragma unroll
                 for (int j = 0; j < CB; ++j)
                     tr_[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[i].x, y[j], tr_[i][j], 0, 0, 0);
+            if constexpr (PARTS == 1) {
 #pragma unroll
-            for (int i = 0; i < RB; ++i)
+                for (int i = 0; i < RB; ++i)
 #pragma unroll
-                for (int j = 0; j < CB; ++j)
-                    ti_[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[i].y, y[j], ti_[i][j], 0, 0, 0);
+                    for (int j = 0; j < CB; ++j)
+                        ti_[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[i].y, y[j], ti_[i][j], 0, 0, 0);
+            }
         }
     };
     i8 en[NS];              // stage s's entries in en[s % NS]
@@ -1271,8 +1312,10 @@ __device__ __forceinline__ void sphere_gemm_tile(const SphereArgs& p, int blk, c
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
                     const int gj = R0 + wr * 16 * RB + i * 16 + q0 + 4 * q;
-                    if (gi < ng && gi >= gj)
-                        kp->H[(int64_t)gj * kp->ldH + gi] = make_double2(cr[i][j][q], gi == gj ? 0.0 : ci[i][j][q]);
+                    if (gi >= ng || gi < gj) continue;
+                    double2* h = kp->H + (int64_t)gj * kp->ldH + gi;
+                    if constexpr (PARTS == 2) *((double*)h + part) = part && gi == gj ? 0.0 : cr[i][j][q];
+                    else *h = make_double2(cr[i][j][q], gi == gj ? 0.0 : ci[i][j][q]);
                 }
             }
     } else {
@@ -1299,30 +1342,32 @@ __device__ __forceinline__ void sphere_gemm_tile(const SphereArgs& p, int blk, c
     }
 }
 
-template <int BR, int BC, int RB, int CB, int NS, int kMode>
-__global__ __launch_bounds__((SphereTile<BR, BC, RB, CB, NS>::kThreads), 4) void k_sphere_gemm(SphereArgs p)
+template <int BR, int BC, int RB, int CB, int NS, int kMode, int PARTS = 1>
+__global__ __launch_bounds__((SphereTile<BR, BC, RB, CB, NS, PARTS>::kThreads), 4) void k_sphere_gemm(SphereArgs p)
 {
     extern __shared__ __attribute__((aligned(1024))) char lds[];
     stamp(p, kMode == kTApp ? 1 : 2);
-    sphere_gemm_tile<BR, BC, RB, CB, NS, kMode>(p, (int)blockIdx.x, lds);
+    sphere_gemm_tile<BR, BC, RB, CB, NS, kMode, PARTS>(p, (int)blockIdx.x, lds);
 }
 
 // H tiles of 32 x 32 and S tiles of 16 M x 16 M in one launch, for triangles
 // whose H tiles leave CUs or the vector pipe idle: S costs no time of its own.
-template <int M>
+// PARTS 2: H tiles of 16 x 32.
+template <int M, int PARTS>
 __global__ __launch_bounds__(256, 4) void k_sphere_hs(SphereArgs p, int hblocks)
 {
     extern __shared__ __attribute__((aligned(1024))) char lds[];
     stamp(p, 2);
-    if ((int)blockIdx.x < hblocks) sphere_gemm_tile<32, 32, 1, 1, kSphereSmall, kLowerH>(p, (int)blockIdx.x, lds);
+    if ((int)blockIdx.x < hblocks)
+        sphere_gemm_tile<32 / PARTS, 32, 1, 1, kSphereSmall, kLowerH, PARTS>(p, (int)blockIdx.x, lds);
     else overlap_tile<M, M, false, false>(p, (int)blockIdx.x - hblocks, lds);
 }
 
-template <int BR, int BC, int RB, int CB, int NS, int kMode>
+template <int BR, int BC, int RB, int CB, int NS, int kMode, int PARTS = 1>
 static hipError_t launch_sphere_gemm(const SphereArgs& p, int64_t nblk, hipEvent_t stop, hipStream_t st)
 {
-    using Tl = SphereTile<BR, BC, RB, CB, NS>;
-    return launch(k_sphere_gemm<BR, BC, RB, CB, NS, kMode>, dim3((unsigned)nblk), Tl::kThreads, Tl::kLds, stop, st, p);
+    using Tl = SphereTile<BR, BC, RB, CB, NS, PARTS>;
+    return launch(k_sphere_gemm<BR, BC, RB, CB, NS, kMode, PARTS>, dim3((unsigned)nblk), Tl::kThreads, Tl::kLds, stop, st, p);
 }
 
 // rtiles: row tiles of all kinds for the tile's rows (tile 64: 32 x 64)
@@ -1335,28 +1380,34 @@ hipError_t launch_sphere_tapp(const SphereArgs& p, int tile, int rtiles, hipEven
     return launch_sphere_gemm<32, 64, 1, 2, 2, kTApp>(q, nblk, stop, st);
 }
 
-static int64_t hblocks(const SphereArgs& p, int tile) { return ((int64_t)p.nsquares * (tile == 48 ? 2 : 1) + 7) / 8 * 8; }
+static int64_t hblocks(const SphereArgs& p, int tile)
+{
+    return ((int64_t)p.nsquares * (tile == 48 || tile == 16 ? 2 : 1) + 7) / 8 * 8;
+}
 
-// tile: 64 (64 x 64), 48 (32 x 64) or 32 (32 x 32)
+// tile: 64 (64 x 64), 48 (32 x 64), 32 (32 x 32) or 16 (16 x 32, by parts)
 hipError_t launch_sphere_h(const SphereArgs& p, int tile, hipEvent_t stop, hipStream_t st)
 {
     const int64_t n = hblocks(p, tile);
+    if (tile == 16) return launch_sphere_gemm<16, 32, 1, 1, kSphereSmall, kLowerH, 2>(p, n, stop, st);
     if (tile == 32) return launch_sphere_gemm<32, 32, 1, 1, kSphereSmall, kLowerH>(p, n, stop, st);
     if (tile == 48) return launch_sphere_gemm<32, 64, 1, 2, 2, kLowerH>(p, n, stop, st);
     return launch_sphere_gemm<64, 64, 1, 2, 2, kLowerH>(p, n, stop, st);
 }
 
-template <int M>
+template <int M, int PARTS>
 static hipError_t launch_hs(const SphereArgs& p, int64_t nstiles, hipEvent_t stop, hipStream_t st)
 {
-    const int64_t n = hblocks(p, 32);
-    const size_t lds = std::max<size_t>(SphereTile<32, 32, 1, 1, kSphereSmall>::kLds, OverlapTile<M, M>::lds((p.nl + 15) / 16));
-    return launch(k_sphere_hs<M>, dim3((unsigned)(n + nstiles)), 256, lds, stop, st, p, (int)n);
+    const int64_t n = hblocks(p, 32 / PARTS);
+    const size_t lds = std::max<size_t>(SphereTile<32 / PARTS, 32, 1, 1, kSphereSmall, PARTS>::kLds,
+                                        OverlapTile<M, M>::lds((p.nl + 15) / 16));
+    return launch(k_sphere_hs<M, PARTS>, dim3((unsigned)(n + nstiles)), 256, lds, stop, st, p, (int)n);
 }
 
-hipError_t launch_sphere_hs(const SphereArgs& p, int stile, int64_t nstiles, hipEvent_t stop, hipStream_t st)
+hipError_t launch_sphere_hs(const SphereArgs& p, int tile, int stile, int64_t nstiles, hipEvent_t stop, hipStream_t st)
 {
-    return stile == 32 ? launch_hs<2>(p, nstiles, stop, st) : launch_hs<1>(p, nstiles, stop, st);
+    if (tile == 16) return launch_hs<1, 2>(p, nstiles, stop, st);
+    return stile == 32 ? launch_hs<2, 1>(p, nstiles, stop, st) : launch_hs<1, 1>(p, nstiles, stop, st);
 }
 
 // G of the sampled columns: block ki, lane j.

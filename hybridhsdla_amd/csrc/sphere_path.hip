@@ -430,9 +430,16 @@ SphereLayout sphere_layout(const hsgen_ctx* ctx, const hsgen_sys* s, const std::
     // 3001 (24 atoms, lmax 8-12) 1846 / 1720 / 1864, 4000 4231 / 3946 / 3854,
     // 6002 9583 / 8625 / 8566.
     l.htile = t64 < 3 * (int64_t)ncu ? 32 : t64 < 6 * (int64_t)ncu ? 48 : 64;
+    // Where 16 x 32 tiles leave every CU at most one, H is one chain of MFMAs per
+    // wave: real and imaginary parts then go to waves of their own.  Calls, us: 2
+    // atoms of lmax 8 at N_G 235 49 -> 47, 16 of lmax 12 at 100 190 -> 166, 64 of
+    // lmax 8 at 100 317 -> 268; with two tiles per CU (600) both take the same.
+    int64_t t32 = 0;
+    for (int ng : ngs) t32 += lower((ng + 31) / 32);
+    if (2 * t32 <= ncu) l.htile = 16;
     l.ttile = tapp_tile(ctx, s, l.gtot);
     l.stile = overlap_tile_size(t64, ncu);
-    const int hc = l.htile == 32 ? 32 : 64;
+    const int hc = l.htile <= 32 ? 32 : 64;
     for (int ng : ngs) {
         l.nsquares += lower((ng + hc - 1) / hc);
         l.nstiles += lower((ng + l.stile - 1) / l.stile);
@@ -490,7 +497,7 @@ std::vector<SphereK> sphere_ks(const SphereLayout& l, const std::vector<const hs
                                const std::vector<int64_t>& ldS)
 {
     std::vector<SphereK> ks(kps.size());
-    const int hc = l.htile == 32 ? 32 : 64;
+    const int hc = l.htile <= 32 ? 32 : 64;
     int64_t col = 0, g = 0, st = 0, hp = 0;
     for (size_t i = 0; i < kps.size(); ++i) {
         SphereK& k = ks[i];
@@ -552,7 +559,8 @@ hipError_t sphere_launch(const SphereArgs& p, const SphereLayout& l, const hsgen
     hipError_t e = launch_sphere_gen(p, do_h || do_s ? none : last, st);
     if (e == hipSuccess && do_h) e = launch_sphere_tapp(p, l.ttile, s->rt32, none, st);
     if (e != hipSuccess) return e;
-    if (do_h && do_s && l.htile == 32 && l.stile <= 32) return launch_sphere_hs(p, l.stile, l.nstiles, last, st);
+    if (do_h && do_s && l.htile <= 32 && l.stile <= (l.htile == 16 ? 16 : 32))
+        return launch_sphere_hs(p, l.htile, l.stile, l.nstiles, last, st);
     if (do_h) e = launch_sphere_h(p, l.htile, do_s ? none : last, st);
     if (e == hipSuccess && do_s) e = launch_overlap(p, l.stile, l.nstiles, last, st);
     return e;
