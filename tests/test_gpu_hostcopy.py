@@ -109,3 +109,32 @@ def test_batched_results(ctx):
         want = _device(ctx, h, k)
         assert np.array_equal(H, np.tril(want[0])) and np.array_equal(S, np.tril(want[1]))
     h.close()
+
+
+def test_two_contexts_in_two_threads(ctx):
+    """Contexts that share the GPU and a system, each with its own slots and
+    threads, at the same time."""
+    import threading
+    from hybridhsdla_amd import Context
+    s, kp = _system(1300)
+    small = KPoint(k=kp.k, g=np.ascontiguousarray(kp.g[:500]), kmax=kp.kmax)
+    h = ctx.upload(s)
+    want = [ctx.create_HS2(h, k) for k in (kp, small)]
+    other = Context(0)
+    bad = []
+
+    def work(c):
+        for _ in range(4):
+            for k, w in zip((kp, small), want):
+                got = c.create_HS2(h, k)
+                if not all(np.array_equal(a, b) for a, b in zip(got, w)):
+                    bad.append(k.ng)
+
+    threads = [threading.Thread(target=work, args=(c,)) for c in (ctx, other)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(60)
+    assert not any(t.is_alive() for t in threads) and not bad
+    other.close()
+    h.close()
