@@ -40,15 +40,16 @@ def _kpoint(kp: KPoint) -> Tuple[HsgenKpoint, np.ndarray]:
     return s, g
 
 
-def _results(ng: int, H, S, flags: int):
+def _results(ng: int, H, S, flags: int, largest: int = 0):
     """H and S, allocated where the caller gave none, and the call's flags.
     Memory that the library writes as a whole is left uninitialised: clearing
     it here would be a pass of one thread over memory that the copy of the
     results writes anyway.  Beyond 32 MiB the C library maps fresh pages, which
-    are zero by themselves."""
+    are zero by themselves.  A call over several k-points has one set of flags:
+    `largest`, the plane waves of its largest, decides for all of them."""
     shape = dict(shape=(ng, ng), dtype=np.complex128, order="F")
     whole = flags & HSGEN_FILL_UPPER
-    if not whole and H is None and S is None and 16 * ng * ng <= 32 << 20:
+    if not whole and H is None and S is None and 16 * max(ng, largest) ** 2 <= 32 << 20:
         flags |= HSGEN_CLEAR_UPPER
         whole = True
     if H is None:
@@ -258,9 +259,9 @@ class Context:
             keep.append(g)
         res = []
         if outputs is None:
-            asked = flags
+            asked, largest = flags, max((kp.ng for kp in kps), default=0)
             for kp in kps:
-                H, S, flags = _results(kp.ng, None, None, asked)
+                H, S, flags = _results(kp.ng, None, None, asked, largest)
                 res.append((H, S))
             hp = (C.c_void_p * nk)(*[_ptr(h) for h, _ in res])
             sp = (C.c_void_p * nk)(*[_ptr(s) for _, s in res])
