@@ -26,8 +26,8 @@ ORACLE_LIB = ORACLE_DIR / "liborc.so"
 
 HIP_SOURCES = ["sphere.hip", "abgen.hip", "zgemm.hip", "ozaki.hip", "context.hip", "fp64_path.hip", "sphere_path.hip",
                "split_path.hip", "tune_eig.hip", "noalloc.hip", "hostcopy.hip"]
-# host-only set-up code (radial solver, T assembly), linked into the same library
-HOST_SOURCES = ["radial.cpp", "tmat.cpp"]
+# host-only code (radial solver, T assembly, copying threads), linked into the same library
+HOST_SOURCES = ["radial.cpp", "tmat.cpp", "hostpool.cpp"]
 HOST_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-Wall", "-ffp-contract=off"]
 
 HIPCC_FLAGS = [

@@ -22,11 +22,10 @@
 // two lower triangles out) 7.7 -> 4.9 ms, 3.4 with M built on the GPU and S's copy
 // beside H.
 #include <sys/mman.h>
-#include <unistd.h>
 
 #include <algorithm>
 #include <cstring>
-#include <exception>
+#include <thread>
 
 #include "hsgen_host.h"
 
@@ -38,7 +37,6 @@ namespace {
 #define MADV_POPULATE_WRITE 23
 #endif
 
-constexpr unsigned kMaxThreads = 8;
 constexpr size_t kSlotBytes = (size_t)4 << 20;
 constexpr size_t kPieceBytes = (size_t)256 << 10;    // what a thread copies at a time
 constexpr size_t kThreadBytes = (size_t)512 << 10;   // one more thread per so many bytes
@@ -221,64 +219,6 @@ void add_range(std::vector<std::pair<char*, size_t>>& out, char* p, size_t n)
 // ---------------------------------------------------------------------------
 // Threads
 // ---------------------------------------------------------------------------
-HostPool::HostPool()
-{
-    const unsigned hw = std::thread::hardware_concurrency();
-    pid_ = getpid();
-    try {
-        current_.assign(kMaxThreads, nullptr);
-        for (unsigned t = 0; t + 1 < hw && t < kMaxThreads; ++t) threads_.emplace_back([this, t] { loop((int)t); });
-    } catch (const std::exception&) {    // fewer threads, or none
-    }
-}
-
-HostPool::~HostPool()
-{
-    if (getpid() != pid_) {              // a forked process has no such threads
-        for (auto& t : threads_) t.detach();
-        return;
-    }
-    {
-        std::lock_guard<std::mutex> lk(mu_);
-        quit_ = true;
-    }
-    wake_.notify_all();
-    for (auto& t : threads_) t.join();
-}
-
-void HostPool::loop(int me)
-{
-    std::unique_lock<std::mutex> lk(mu_);
-    for (;;) {
-        wake_.wait(lk, [this] { return quit_ || !tasks_.empty(); });
-        if (tasks_.empty()) return;
-        const Task t = std::move(tasks_.front());
-        tasks_.pop_front();
-        current_[me] = t.group;
-        lk.unlock();
-        t.run();
-        lk.lock();
-        current_[me] = nullptr;
-        done_.notify_all();
-    }
-}
-
-void HostPool::post(const void* group, const std::function<void()>& run, size_t n)
-{
-    {
-        std::lock_guard<std::mutex> lk(mu_);
-        for (size_t i = 0; i < n; ++i) tasks_.push_back(Task{group, run});
-    }
-    wake_.notify_all();
-}
-
-void HostPool::finish(const void* group)
-{
-    std::unique_lock<std::mutex> lk(mu_);
-    tasks_.remove_if([&](const Task& t) { return t.group == group; });
-    done_.wait(lk, [&] { return std::find(current_.begin(), current_.end(), group) == current_.end(); });
-}
-
 // the context's threads; null: the calling thread works alone
 static HostPool* pool(hsgen_ctx* ctx, size_t bytes)
 {

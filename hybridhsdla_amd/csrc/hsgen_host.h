@@ -25,21 +25,19 @@
 
 #include <atomic>
 #include <complex>
-#include <condition_variable>
 #include <cstdarg>
-#include <functional>
 #include <list>
 #include <map>
 #include <memory>
 #include <mutex>
 #include <string>
-#include <thread>
 #include <utility>
 #include <vector>
 
 #include <rocblas/rocblas.h>
 
 #include "../../include/hsgen.h"
+#include "hostpool.h"
 #include "hsgen_internal.h"
 #include "sphere.h"
 
@@ -92,33 +90,6 @@ inline HostCopy copy_matrix(const double2* dev, int n, double* host, int64_t ld,
     return {(char*)dev, (char*)host, e * n, (size_t)n, e * n, e * ld, !(flags & HSGEN_FILL_UPPER),
             (flags & HSGEN_CLEAR_UPPER) != 0};
 }
-
-// Threads of a context that copy host memory: started with its first large
-// copy, at most 8, joined with the context.  Tasks run in the order they are
-// posted; finish() withdraws a group's waiting tasks and waits for its running
-// ones.
-class HostPool {
-public:
-    HostPool();
-    ~HostPool();
-    size_t size() const { return threads_.size(); }
-    void post(const void* group, const std::function<void()>& run, size_t n);
-    void finish(const void* group);
-
-private:
-    struct Task {
-        const void* group;
-        std::function<void()> run;
-    };
-    void loop(int me);
-    std::mutex mu_;
-    std::condition_variable wake_, done_;
-    std::list<Task> tasks_;
-    std::vector<const void*> current_;     // per thread: the group it works for
-    std::vector<std::thread> threads_;
-    bool quit_ = false;
-    int pid_;
-};
 
 // Maps the pages of a call's host results in the background until they are
 // copied or the object goes.
