@@ -310,7 +310,7 @@ hsgen_status hsgen_release_workspace(hsgen_ctx* ctx)
     for (DevBuf* b : {&ctx->Z, &ctx->Zs, &ctx->W, &ctx->Htmp, &ctx->Stmp, &ctx->A, &ctx->B, &ctx->g,
                       &ctx->probs, &ctx->work, &ctx->lists, &ctx->pack, &ctx->oz_e, &ctx->oz_res,
                       &ctx->oz_out, &ctx->oz_fprob, &ctx->oz_probs, &ctx->oz_work, &ctx->oz_smp, &ctx->btmp,
-                      &ctx->ring_left, &ctx->m_in, &ctx->M, &ctx->eig_a, &ctx->eig_b, &ctx->eig_d, &ctx->sph_ph, &ctx->sph_rs, &ctx->sph_y, &ctx->sph_w, &ctx->sph_smp})
+                      &ctx->ring_left, &ctx->m_in, &ctx->M, &ctx->eig_a, &ctx->eig_b, &ctx->eig_d})
         release(*b);
     for (auto& bg : ctx->bgraphs) {
         if (bg.exec) (void)hipGraphExecDestroy(bg.exec);

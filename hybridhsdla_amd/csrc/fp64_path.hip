@@ -495,8 +495,8 @@ hsgen_status create_hs_sphere(hsgen_ctx* ctx, hsgen_sys* s, const hsgen_kpoint* 
     }
     hsgen_status st;
     const SphereLayout l = sphere_layout(ctx, s, {ng}, do_h);
-    if ((st = ensure(ctx, ctx->sph_ph, l.b_ph, false)) || (st = ensure(ctx, ctx->sph_rs, l.b_rs, false))) return st;
-    if (do_h && ((st = ensure(ctx, ctx->sph_y, l.b_y, false)) || (st = ensure(ctx, ctx->sph_w, l.b_w, false)))) return st;
+    SphereOperands op;
+    if ((st = sphere_operands(ctx, l, do_h, op))) return st;
     const bool hdev = !do_h || is_device_ptr(H), sdev = !do_s || is_device_ptr(S);
     double2* dH = (double2*)H;
     double2* dS = (double2*)S;
@@ -513,8 +513,7 @@ hsgen_status create_hs_sphere(hsgen_ctx* ctx, hsgen_sys* s, const hsgen_kpoint* 
         dS = (double2*)ctx->Stmp.p;
         ldS = ng;
     }
-    SphereArgs p = sphere_args(s, l, ctx->sph_ph.p, ctx->sph_rs.p, do_h ? ctx->sph_y.p : nullptr,
-                               do_h ? ctx->sph_w.p : nullptr);
+    SphereArgs p = sphere_args(s, l, op.ph, op.rs, op.y, op.w);
     p.one = sphere_ks(l, {kp}, {nullptr}, {dH}, {dS}, {ldH}, {ldS})[0];
     st = sphere_g(ctx, kp, nullptr, p.one);
     if (st) return st;
@@ -568,10 +567,10 @@ hsgen_status batched_fp64(hsgen_ctx* ctx, hsgen_sys* s, int nk, const hsgen_kpoi
     // batches: operands plus device copies of host outputs within 90% of the
     // memory the call may use (the rest of the call's device memory, the
     // graph's G lists, is small)
+    if (s->fold) release(ctx->Zs);   // only unfolded operands need it
     size_t fr = 0, tot = 0;
     HIPCHK(hipMemGetInfo(&fr, &tot));
-    size_t budget = (size_t)(0.9 * (double)(fr + ctx->sph_ph.bytes + ctx->sph_rs.bytes + ctx->sph_y.bytes +
-                                            ctx->sph_w.bytes + ctx->btmp.bytes));
+    size_t budget = (size_t)(0.9 * (double)(fr + ctx->Z.bytes + ctx->W.bytes + ctx->btmp.bytes));
     if (const char* e = std::getenv("HSGEN_BATCH_BYTES"))   // cap (tuning and tests)
         if (std::strtoull(e, nullptr, 10) > 0) budget = std::min<size_t>(budget, std::strtoull(e, nullptr, 10));
     std::vector<std::vector<int>> batches;
@@ -606,9 +605,8 @@ hsgen_status batched_fp64(hsgen_ctx* ctx, hsgen_sys* s, int nk, const hsgen_kpoi
             ntmp += (int64_t)kps[i].ng * kps[i].ng * ((!hdev[i]) + (!sdev[i]));
         }
         const SphereLayout l = sphere_layout(ctx, s, ngs, do_h);
-        if ((st = ensure(ctx, ctx->sph_ph, l.b_ph, false)) || (st = ensure(ctx, ctx->sph_rs, l.b_rs, false))) return st;
-        if (do_h && ((st = ensure(ctx, ctx->sph_y, l.b_y, false)) || (st = ensure(ctx, ctx->sph_w, l.b_w, false))))
-            return st;
+        SphereOperands op;
+        if ((st = sphere_operands(ctx, l, do_h, op))) return st;
         if (ntmp > 0) {
             st = ensure(ctx, ctx->btmp, sizeof(double2) * (size_t)ntmp, false);
             if (st) return st;
@@ -627,9 +625,8 @@ hsgen_status batched_fp64(hsgen_ctx* ctx, hsgen_sys* s, int nk, const hsgen_kpoi
             ldS[q] = ts ? kps[i].ng : ld[i];
         }
         // call signature
-        std::vector<int64_t> sig{(int64_t)s->serial, (int64_t)flags, (int64_t)(intptr_t)ctx->sph_ph.p,
-                                 (int64_t)(intptr_t)ctx->sph_rs.p, (int64_t)(intptr_t)ctx->sph_y.p,
-                                 (int64_t)(intptr_t)ctx->sph_w.p, (int64_t)(intptr_t)ctx->btmp.p, (int64_t)ks.size()};
+        std::vector<int64_t> sig{(int64_t)s->serial, (int64_t)flags, (int64_t)(intptr_t)op.ph, (int64_t)(intptr_t)op.w,
+                                 (int64_t)(intptr_t)ctx->btmp.p, (int64_t)ks.size()};
         for (size_t q = 0; q < ks.size(); ++q) {
             const int i = ks[q];
             int64_t kb[3];
@@ -668,8 +665,7 @@ hsgen_status batched_fp64(hsgen_ctx* ctx, hsgen_sys* s, int nk, const hsgen_kpoi
             HIPCHK(hipMemcpyAsync(bg.ks.p, sk.data(), sizeof(SphereK) * sk.size(), hipMemcpyHostToDevice, ctx->stream));
             // the host vectors must outlive the copies
             HIPCHK(hipStreamSynchronize(ctx->stream));
-            SphereArgs p = sphere_args(s, l, ctx->sph_ph.p, ctx->sph_rs.p, do_h ? ctx->sph_y.p : nullptr,
-                                       do_h ? ctx->sph_w.p : nullptr);
+            SphereArgs p = sphere_args(s, l, op.ph, op.rs, op.y, op.w);
             p.nk = (int32_t)sk.size();
             p.one = sk[0];
             p.many = (const SphereK*)bg.ks.p;

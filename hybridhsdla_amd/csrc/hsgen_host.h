@@ -117,9 +117,7 @@ struct hsgen_ctx {
     std::string err;
     // workspace
     hsgen::DevBuf Z, Zs, W, Htmp, Stmp, A, B, g, probs, work, pack, m_in, M, lists;
-    // FP64 from a system: phases, radial factors, real vectors (W, host-output copies above)
-    hsgen::DevBuf sph_ph, sph_rs, sph_y, sph_w, sph_smp;
-    // split precision
+    // split precision (oz_res: before the residues, the real vectors that W is formed from)
     hsgen::DevBuf oz_e, oz_res, oz_out, oz_probs, oz_work, oz_smp, oz_fprob;
     hipEvent_t oz_ev[2 * hsgen::kMaxModuli] = {};   // INT8 GEMM start/stop per residue group
     int n_cu = 0;                                    // compute units
@@ -298,7 +296,12 @@ struct SphereLayout {
     int htile = 64, ttile = 64, stile = 64;
     size_t b_ph = 0, b_rs = 0, b_y = 0, b_w = 0;   // bytes of the operand arrays
 };
+// Operands of a call: phases, radial factors, real vectors, W.
+struct SphereOperands {
+    void *ph, *rs, *y, *w;
+};
 hsgen_status sphere_setup(hsgen_ctx* ctx, hsgen_sys* s, const RadDev* rad);
+hsgen_status sphere_operands(hsgen_ctx* ctx, const SphereLayout& l, bool do_h, SphereOperands& o);
 SphereLayout sphere_layout(const hsgen_ctx* ctx, const hsgen_sys* s, const std::vector<int>& ngs, bool do_h);
 SphereArgs sphere_args(const hsgen_sys* s, const SphereLayout& l, void* ph, void* rs, void* y, void* w);
 std::vector<SphereK> sphere_ks(const SphereLayout& l, const std::vector<const hsgen_kpoint*>& kps,

@@ -323,7 +323,8 @@ hsgen_status sphere_split_setup(hsgen_ctx* ctx, hsgen_sys* s)
 
 // W of split precision (rows 2 off_a .. of every column, leading dimension ldw)
 // over the ncols padded columns of the k-points ks (k, g, ng, col0 set;
-// ks_dev: their device copy).  Column chunks bound the real vectors' memory.
+// ks_dev: their device copy).  Column chunks bound the real vectors' memory,
+// which with the sample's operands lies where the residues will.
 // cols: null, or per k-point kSampleCols columns (past its plane waves the last
 // again) whose H and, with do_s, S go to the k-points' H and S, in FP64: H from
 // W of the sampled columns and the chunk's real vectors, S by the addition
@@ -339,25 +340,30 @@ hsgen_status sphere_split_w(hsgen_ctx* ctx, hsgen_sys* s, const std::vector<Sphe
         if (std::strtoull(e, nullptr, 10) > 0) bytes = std::min<int64_t>(bytes, std::strtoll(e, nullptr, 10));
     const int64_t per = 8 * s->ldy + 16 * (int64_t)s->natoms + (cols ? 16 * (int64_t)s->ldr : 0);
     const int64_t chunk = std::min(ncols, std::max<int64_t>(kSphereCols, bytes / per / kSphereCols * kSphereCols));
-    if ((st = ensure(ctx, ctx->sph_ph, sizeof(double2) * (size_t)(chunk * s->natoms), false)) ||
-        (st = ensure(ctx, ctx->sph_y, sizeof(double) * (size_t)(chunk * s->ldy), false)) ||
-        (cols && (st = ensure(ctx, ctx->sph_rs, sizeof(double2) * (size_t)(chunk * s->ldr), false))))
-        return st;
+    auto up = [](size_t b) { return (size_t)roundup((int64_t)b, 256); };
+    const int nk = (int)ks.size();
+    const int64_t nsmp = cols ? (int64_t)kSampleCols * nk : 0;
+    // the chunk's operands and the sample's, in the residues' buffer
+    const size_t b_ph = up(sizeof(double2) * (size_t)(chunk * s->natoms)),
+                 b_rs = cols ? up(sizeof(double2) * (size_t)(chunk * s->ldr)) : 0,
+                 b_y = up(sizeof(double) * (size_t)(chunk * s->ldy));
+    const size_t s_k = up(sizeof(SphereK) * nk), s_c = up(sizeof(int32_t) * nsmp), s_g = up(3 * sizeof(int32_t) * nsmp),
+                 s_ph = up(sizeof(double2) * nsmp * s->natoms), s_rs = up(sizeof(double2) * nsmp * s->ldr),
+                 s_y = up(sizeof(double) * nsmp * s->ldy), s_w = up(sizeof(double2) * nsmp * s->ldw);
+    st = ensure(ctx, ctx->oz_res, b_ph + b_rs + b_y + (cols ? s_k + s_c + s_g + s_ph + s_rs + s_y + s_w : 0), false);
+    if (st) return st;
+    char* const d_ph = (char*)ctx->oz_res.p;
+    char* const d_rs = d_ph + b_ph;
+    char* const d_y = d_rs + b_rs;
     SphereArgs smp;
     std::vector<SphereK> sk;
     std::vector<char> tables;
     if (cols) {
         // the sampled columns as k-points of their own: operands and W
-        const int nk = (int)ks.size();
         SphereLayout l;
-        l.gtot = (int64_t)kSampleCols * nk;
-        auto up = [](size_t b) { return (size_t)roundup((int64_t)b, 256); };
-        const size_t b_k = up(sizeof(SphereK) * nk), b_c = up(sizeof(int32_t) * l.gtot), b_g = up(3 * sizeof(int32_t) * l.gtot),
-                     b_ph = up(sizeof(double2) * l.gtot * s->natoms), b_rs = up(sizeof(double2) * l.gtot * s->ldr),
-                     b_y = up(sizeof(double) * l.gtot * s->ldy), b_w = up(sizeof(double2) * l.gtot * s->ldw);
-        if ((st = ensure(ctx, ctx->sph_smp, b_k + b_c + b_g + b_ph + b_rs + b_y + b_w, false))) return st;
-        char* p = (char*)ctx->sph_smp.p;
-        int32_t* g = (int32_t*)(p + b_k + b_c);
+        l.gtot = nsmp;
+        char* p = d_y + b_y;
+        int32_t* g = (int32_t*)(p + s_k + s_c);
         for (int i = 0; i < nk; ++i) {
             SphereK k = ks[i];
             k.ng = std::min(ks[i].ng, kSampleCols);
@@ -368,16 +374,16 @@ hsgen_status sphere_split_w(hsgen_ctx* ctx, hsgen_sys* s, const std::vector<Sphe
             l.ngcols += k.ng;
             sk.push_back(k);
         }
-        tables.resize(b_k + b_c);
+        tables.resize(s_k + s_c);
         std::memcpy(tables.data(), sk.data(), sizeof(SphereK) * nk);
-        std::memcpy(tables.data() + b_k, cols->data(), sizeof(int32_t) * l.gtot);
+        std::memcpy(tables.data() + s_k, cols->data(), sizeof(int32_t) * l.gtot);
         HIPCHK(hipMemcpyAsync(p, tables.data(), tables.size(), hipMemcpyHostToDevice, ctx->stream));
-        char* a = p + b_k + b_c + b_g;
-        smp = sphere_args(s, l, a, a + b_ph, a + b_ph + b_rs, a + b_ph + b_rs + b_y);
+        char* a = p + s_k + s_c + s_g;
+        smp = sphere_args(s, l, a, a + s_ph, a + s_ph + s_rs, a + s_ph + s_rs + s_y);
         smp.nk = nk;
         smp.one = ks[0];
         smp.many = ks_dev;
-        HIPCHK(launch_sample_g(smp, (const int32_t*)(p + b_k), g, ctx->stream));
+        HIPCHK(launch_sample_g(smp, (const int32_t*)(p + s_k), g, ctx->stream));
         smp.one = sk[0];
         smp.many = (const SphereK*)p;
         HIPCHK(launch_sphere_gen(smp, nullptr, ctx->stream));
@@ -388,7 +394,7 @@ hsgen_status sphere_split_w(hsgen_ctx* ctx, hsgen_sys* s, const std::vector<Sphe
         SphereLayout l;
         l.gtot = std::min(chunk, ncols - c0);
         l.ngcols = l.gtot;
-        SphereArgs p = sphere_args(s, l, ctx->sph_ph.p, cols ? ctx->sph_rs.p : nullptr, ctx->sph_y.p, W + c0 * ldw);
+        SphereArgs p = sphere_args(s, l, d_ph, cols ? d_rs : nullptr, d_y, W + c0 * ldw);
         p.mt = (const double2*)s->d_split;
         p.mtoff = s->d_split_off;
         p.rowdst = s->d_split_rows;
@@ -451,6 +457,21 @@ SphereLayout sphere_layout(const hsgen_ctx* ctx, const hsgen_sys* s, const std::
     l.b_y = do_h ? sizeof(double) * g * (size_t)s->ldy : 0;
     l.b_w = do_h ? sizeof(double2) * g * (size_t)s->ldw : 0;
     return l;
+}
+
+// The operands of a call in the buffers that the general ones have too (a
+// context that uses both holds one set): W in W, the others in Z.
+hsgen_status sphere_operands(hsgen_ctx* ctx, const SphereLayout& l, bool do_h, SphereOperands& o)
+{
+    auto up = [](size_t b) { return (size_t)roundup((int64_t)b, 256); };
+    hsgen_status st = ensure(ctx, ctx->Z, up(l.b_ph) + up(l.b_rs) + l.b_y, false);
+    if (st) return st;
+    if (do_h && (st = ensure(ctx, ctx->W, l.b_w, false))) return st;
+    o.ph = ctx->Z.p;
+    o.rs = (char*)o.ph + up(l.b_ph);
+    o.y = do_h ? (char*)o.rs + up(l.b_rs) : nullptr;
+    o.w = do_h ? ctx->W.p : nullptr;
+    return HSGEN_OK;
 }
 
 SphereArgs sphere_args(const hsgen_sys* s, const SphereLayout& l, void* ph, void* rs, void* y, void* w)
