@@ -370,7 +370,7 @@ hsgen_status finish_hs(hsgen_ctx* ctx, hsgen_sys* s, const Geometry& geo, int ng
             k.ng = ng;
             std::vector<OzK> ks(1);
             ks[0].ng = ng;
-            if ((st = oz_sample(ctx, geo, ks, smp))) return st;
+            if ((st = oz_sample(ctx, geo, ks, false, smp))) return st;
             k.H = smp.H;
             k.S = smp.S;
             k.ldH = k.ldS = ng;

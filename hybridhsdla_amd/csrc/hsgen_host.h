@@ -359,7 +359,9 @@ struct OzSample {
     // kSampleCols columns per k-point, the last again past nb
     std::vector<int32_t> padded() const;
 };
-hsgen_status oz_sample(hsgen_ctx* ctx, const Geometry& geo, const std::vector<OzK>& ks, OzSample& smp);
+// operands: whether run_ozaki forms it from the operands (with memory for their
+// gathered columns and the depth chunks' products), or sphere_split_w does.
+hsgen_status oz_sample(hsgen_ctx* ctx, const Geometry& geo, const std::vector<OzK>& ks, bool operands, OzSample& smp);
 
 // capture: the INT8 launch sequence of each modulus count runs as cached
 // hipGraphs (the batched path), else eagerly.  sample: null, or the call's

@@ -491,7 +491,7 @@ hsgen_status oz_execute(hsgen_ctx* ctx, const Geometry& geo, const std::vector<O
 }  // namespace
 
 
-hsgen_status oz_sample(hsgen_ctx* ctx, const Geometry& geo, const std::vector<OzK>& ks, OzSample& smp)
+hsgen_status oz_sample(hsgen_ctx* ctx, const Geometry& geo, const std::vector<OzK>& ks, bool operands, OzSample& smp)
 {
     const ZgemmLaunchCfg sc = zgemm_cfg(kSampleTile);
     smp = OzSample{};
@@ -512,12 +512,13 @@ hsgen_status oz_sample(hsgen_ctx* ctx, const Geometry& geo, const std::vector<Oz
     // summed in chunk order afterwards.  nsplit depends on the depth only, so
     // a k-point's sample is the same in single and batched calls.
     smp.nsplit = (int)std::max<int64_t>(1, std::min<int64_t>(8, geo.kpad / 2048));
+    const size_t products = operands ? 2 * smp.gath_total + 2 * smp.total * (smp.nsplit - 1) : 0;
     const hsgen_status st =
-        ensure(ctx, ctx->oz_smp, sizeof(double2) * std::max<size_t>(2 * (smp.total + smp.gath_total) + 2 * smp.total * (smp.nsplit - 1), 1),
-               false);
+        ensure(ctx, ctx->oz_smp, sizeof(double2) * std::max<size_t>(2 * smp.total + products, 1), false);
     if (st) return st;
     smp.S = (double2*)ctx->oz_smp.p;
     smp.H = smp.S + smp.total;
+    if (!operands) return HSGEN_OK;
     smp.gath_s = smp.H + smp.total;
     smp.gath_h = smp.gath_s + smp.gath_total;
     smp.parts = smp.gath_h + smp.gath_total;     // chunks 1 .. nsplit-1 of S and H, 2 total each
@@ -566,7 +567,7 @@ hsgen_status run_ozaki(hsgen_ctx* ctx, const Geometry& geo, const std::vector<Oz
     hsgen_status st = HSGEN_OK;
     OzSample own;
     if (!sample) {
-        if ((st = oz_sample(ctx, geo, ks, own))) return st;
+        if ((st = oz_sample(ctx, geo, ks, true, own))) return st;
         sample = &own;
     }
     const std::vector<int>& nb = sample->nb;
@@ -852,7 +853,7 @@ hsgen_status batched_split(hsgen_ctx* ctx, hsgen_sys* s, int nk, const hsgen_kpo
         sdev[i] = !do_s || is_device_ptr(S[i]);
     }
     // batches within ~70% of the memory the call may use: operands Z, Zs, W,
-    // device copies of host outputs, the stored residue outputs (2 bytes per
+    // device copies of host outputs, the FP64 sample, the stored residue outputs (2 bytes per
     // element of every S/H tile and modulus, counted for 14 moduli or the
     // requested count) and the residue arrays of as many moduli as one
     // residue pass converts when the moduli take two passes of at most 16
@@ -860,6 +861,7 @@ hsgen_status batched_split(hsgen_ctx* ctx, hsgen_sys* s, int nk, const hsgen_kpo
     // one pass per batch saves those reads but needs more, smaller batches,
     // which cost as much again at 64 k-points)
     if (g0.fold) release(ctx->Zs);   // folded operands need no Zs
+    if (do_h && (st = sphere_split_setup(ctx, s))) return st;   // the system keeps these: not of the budget
     size_t fr = 0, tot = 0;
     HIPCHK(hipMemGetInfo(&fr, &tot));
     size_t held = 0;
@@ -885,6 +887,7 @@ hsgen_status batched_split(hsgen_ctx* ctx, hsgen_sys* s, int nk, const hsgen_kpo
         for (size_t bi = 0; bi < ntr; ++bi)
             tiles += std::min(ntc, ((bi + 1) * ic.bm + ic.bn - 1) / ic.bn);
         need[i] = n_operands(g0) * sizeof(double2) * (size_t)g0.ldz * gp + sizeof(double2) * ng * ng * ((!hdev[i]) + (!sdev[i])) +
+                  2 * sizeof(double2) * ng * std::min<size_t>(ng, kSampleCols) +
                   (size_t)(do_s + do_h) * tiles * 2 * ic.bm * ic.bn * nmod_est + (size_t)gslots * narr * 2 * ic.esize * kd * gp;
         total += need[i];
     }
@@ -987,7 +990,7 @@ hsgen_status batched_split(hsgen_ctx* ctx, hsgen_sys* s, int nk, const hsgen_kpo
         OzSample smp;
         if (do_h) {
             // T application over every column of the batch from the real vectors
-            if ((st = oz_sample(ctx, geo, ks, smp))) return st;
+            if ((st = oz_sample(ctx, geo, ks, false, smp))) return st;
             std::vector<SphereK> sk(bk.size());
             for (size_t q = 0; q < bk.size(); ++q) {
                 std::memset(&sk[q], 0, sizeof sk[q]);

@@ -69,3 +69,28 @@ def test_real_vectors_of_split_precision_take_no_memory_of_their_own(ctx):
         h.close()
     print(f"shared {held[0] / MIB:.0f} own {held[1] / MIB:.0f} MiB", flush=True)
     assert abs(held[1] - held[0]) <= 32 * MIB
+
+
+def test_sample_of_a_system_takes_no_products_memory(ctx):
+    """Twelve k-points of 64 plane waves, 128 columns each in 128 x 128 tiles:
+    Y, W and the residues of ten moduli (of Y and of W) are what the
+    call keeps.  Gathered columns for a sample from the operands would be 190 MB."""
+    s, kp = _workload(100)
+    h = ctx.upload(s)
+    kps = [KPoint(k=kp.k + 0.001 * i, g=kp.g[:64], kmax=kp.kmax) for i in range(12)]
+    out = [_matrices(64) for _ in kps]
+    outputs = [(H.data_ptr(), S.data_ptr(), 64) for H, S in out]
+
+    def held():
+        ctx.release_workspace()
+        before = _used()
+        ctx.create_HS2_batched(h, kps, precision=HSGEN_PREC_OZAKI_INT8, slices=10, tile=14, outputs=outputs)
+        return _used() - before
+
+    held()
+    rows, cols = 2 * 121 * 32, 12 * 128
+    kept = held()
+    want = 2 * 16 * rows * cols + 10 * 2 * 2 * rows * cols
+    print(f"kept {kept / MIB:.0f} of {want / MIB:.0f} MiB", flush=True)
+    assert kept <= 1.02 * want + 64 * MIB
+    h.close()
