@@ -189,8 +189,6 @@ hsgen_status upload_M(hsgen_ctx* ctx, hsgen_sys* s, const int32_t* nlm, const do
 hsgen_status ensure_M(hsgen_ctx* ctx, hsgen_sys* s, int bk, int bm)
 {
     std::lock_guard<std::mutex> lk(s->m_mu);
-    s->pad_bk = bk;
-    s->pad_bm = bm;
     if (s->d_M && s->m_bk == bk && s->m_bm == bm) return HSGEN_OK;
     const int na = s->natoms;
     std::vector<const double*> pa(na), pb(na), pc(na);
@@ -464,9 +462,6 @@ hsgen_status hsgen_system_create(hsgen_ctx* ctx, const hsgen_system* d, hsgen_sy
         cp(xtab[a], d->t_ab[a]);
         cp(xtbb[a], d->t_bb[a]);
     }
-    const Geometry geo = geometry(0, s->kdim, 1);
-    s->pad_bk = geo.t.bk;
-    s->pad_bm = geo.t.bm;
     st = sphere_setup(ctx, s, rad.data());
     if (st != HSGEN_OK) {
         hsgen_system_destroy(ctx, s);

@@ -306,14 +306,7 @@ hsgen_status finish_hs(hsgen_ctx* ctx, hsgen_sys* s, const Geometry& geo, int ng
         dS = (double2*)ctx->Stmp.p;
         ldS = ng;
     }
-    if (kp) {
-        std::lock_guard<std::mutex> lk(s->m_mu);
-        s->pad_bk = geo.t.bk;
-        s->pad_bm = geo.t.bm;
-    } else {
-        st = ensure_M(ctx, s, geo.t.bk, geo.t.bm);
-        if (st) return st;
-    }
+    if (!kp && (st = ensure_M(ctx, s, geo.t.bk, geo.t.bm))) return st;
 
     const bool do_s = !(flags & HSGEN_SKIP_S);
     std::vector<HostCopy> out_h, out_s;
@@ -488,11 +481,6 @@ hsgen_status create_hs_sphere(hsgen_ctx* ctx, hsgen_sys* s, const hsgen_kpoint* 
     const int ng = kp->ng;
     const bool do_h = !(o.flags & HSGEN_SKIP_H), do_s = !(o.flags & HSGEN_SKIP_S);
     const Geometry geo = geometry(o.tile, s->kdim, ng);
-    {
-        std::lock_guard<std::mutex> lk(s->m_mu);
-        s->pad_bk = geo.t.bk;
-        s->pad_bm = geo.t.bm;
-    }
     hsgen_status st;
     const SphereLayout l = sphere_layout(ctx, s, {ng}, do_h);
     SphereOperands op;
@@ -548,11 +536,6 @@ hsgen_status batched_fp64(hsgen_ctx* ctx, hsgen_sys* s, int nk, const hsgen_kpoi
     int max_ng = 1;
     for (int i = 0; i < nk; ++i) max_ng = std::max(max_ng, kps[i].ng);
     const Geometry geo = geometry(o.tile, s->kdim, max_ng);
-    {
-        std::lock_guard<std::mutex> lk(s->m_mu);
-        s->pad_bk = geo.t.bk;
-        s->pad_bm = geo.t.bm;
-    }
     hsgen_status st;
     // largest k first; k-points without G-vectors have nothing to compute
     std::vector<int> order;

@@ -170,10 +170,8 @@ struct hsgen_sys {
     std::vector<int32_t> m_cols;       // per atom: padded column count
     int m_bk = 0, m_bm = 0;            // tile geometry M was padded for
     // M is built by the first call that reads it (calls on contexts that share
-    // the system may be the first together); pad_bk, pad_bm: the tile geometry
-    // of the last call, which the allocation-free entry point asks for
+    // the system may be the first together)
     std::mutex m_mu;
-    int pad_bk = 0, pad_bm = 0;
     int64_t sum_nlm2 = 0;              // sum_a nlm_a^2
     // folded operands: Y = [A_a; sqrt(N_a) B_a] per atom (S = Y^H Y,
     // H = Y^H M' Y) when every N_l = ||u_dot_l||^2 is positive; otherwise

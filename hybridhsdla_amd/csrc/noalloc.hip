@@ -106,18 +106,6 @@ extern "C" hsgen_status hsgen_create_hs_noalloc(hsgen_ctx* ctx, const hsgen_sys*
     geo.fold = s->fold;
     const int tc = tapp_cfg(geo);
     const ZgemmLaunchCfg tcc = zgemm_cfg(tc);
-    int pad_bk, pad_bm;
-    {
-        hsgen_sys* sm = const_cast<hsgen_sys*>(s);
-        std::lock_guard<std::mutex> lk(sm->m_mu);
-        pad_bk = s->pad_bk;
-        pad_bm = s->pad_bm;
-    }
-    if (pad_bk != geo.t.bk || pad_bm != geo.t.bm)
-        return fail(ctx, HSGEN_ERR_UNSUPPORTED,
-                    "the system's T blocks are padded for tiles with BK %d, BM %d, tile %d needs %d, %d (a "
-                    "hsgen_create_hs call with this tile pads them once)",
-                    pad_bk, pad_bm, geo.cfg, geo.t.bk, geo.t.bm);
     // the general operands and their work lists, which set the limit
     const int na = s->natoms;
     const int ntn = (int)((geo.gp + tcc.bn - 1) / tcc.bn);

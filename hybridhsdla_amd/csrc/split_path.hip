@@ -836,11 +836,6 @@ hsgen_status batched_split(hsgen_ctx* ctx, hsgen_sys* s, int nk, const hsgen_kpo
     const int64_t kd = roundup(g0.kpad, ic.bk);
     const int narr = oz_slots(ic, g0.fold).narr;
     hsgen_status st;
-    {
-        std::lock_guard<std::mutex> lk(s->m_mu);
-        s->pad_bk = g0.t.bk;
-        s->pad_bm = g0.t.bm;
-    }
     if (rep) std::memset(rep, 0, sizeof(hsgen_report) * nk);
     // largest k first; k-points without G-vectors have nothing to compute
     std::vector<int> order;

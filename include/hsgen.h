@@ -228,9 +228,7 @@ hsgen_status hsgen_contract_hs(hsgen_ctx* ctx, int32_t L, int32_t a, int32_t G,
  * ||u_dot||^2) pass HSGEN_NOALLOC_SCRATCH_BYTES is HSGEN_ERR_ARG.  H and S must be device memory (HSGEN_ERR_ARG
  * otherwise); kp->g may be host or device memory.  opts->precision must be
  * HSGEN_PREC_FP64 (HSGEN_ERR_UNSUPPORTED otherwise); flags and tile as for
- * hsgen_create_hs, with the tile's T-block padding already in place (the
- * default tile's is made by hsgen_system_create).  Results equal
- * hsgen_create_hs's bit for bit.  Calls on one GPU share its array: calls
+ * hsgen_create_hs.  Results equal hsgen_create_hs's bit for bit.  Calls on one GPU share its array: calls
  * that overlap on one GPU, from any contexts, race. */
 hsgen_status hsgen_create_hs_noalloc(hsgen_ctx* ctx, const hsgen_sys* sys,
                                      const hsgen_kpoint* kp, const hsgen_opts* opts,
