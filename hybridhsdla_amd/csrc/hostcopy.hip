@@ -40,7 +40,7 @@ namespace {
 constexpr size_t kSlotBytes = (size_t)4 << 20;
 constexpr size_t kPieceBytes = (size_t)256 << 10;    // what a thread copies at a time
 constexpr size_t kThreadBytes = (size_t)512 << 10;   // one more thread per so many bytes
-constexpr size_t kFlagBytes = 64 * kRingSlots;       // one line per slot, after the slots
+constexpr size_t kFlagBytes = 64 * (kRingSlots + 1); // one line per slot, after the slots, and one for the start
 constexpr size_t kGrid = 24;                         // workgroups of a copy kernel
 constexpr int kGroup = kRingSlots / 2;               // slots of one launch
 constexpr size_t kRange = (size_t)2 << 20;           // memory that Prefault maps at a time
@@ -70,6 +70,7 @@ typedef double v2d __attribute__((ext_vector_type(2)));
 
 struct SlotGroup {
     SlotCopy c[kGroup];
+    uint64_t* begun;        // pinned: takes the first block's seq as the kernel starts
     int32_t n;
 };
 
@@ -92,6 +93,8 @@ __device__ __forceinline__ void copy_units(const char* src, char* dst, uint32_t 
 template <bool kToHost>
 __global__ __launch_bounds__(256) void k_slot_copy(SlotGroup g)
 {
+    if (blockIdx.x == 0 && threadIdx.x == 0)
+        __hip_atomic_store(g.begun, g.c[0].seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     for (int b = 0; b < g.n; ++b) {
         const SlotCopy& p = g.c[b];
         const uint32_t w = (uint32_t)(p.width / 16);
@@ -327,6 +330,7 @@ hsgen_status host_copy(hsgen_ctx* ctx, const std::vector<HostCopy>& list, bool t
     // launches the kernel of blocks b .. b + m - 1
     auto move = [&](int b, int m) {
         SlotGroup g{};
+        g.begun = (uint64_t*)((char*)ctx->ring_dev + kSlotBytes * kN + 64 * kN);
         size_t most = 0;
         for (g.n = 0; g.n < m; ++g.n) {
             const Block& k = blocks[b + g.n];
@@ -342,12 +346,13 @@ hsgen_status host_copy(hsgen_ctx* ctx, const std::vector<HostCopy>& list, bool t
         else hipLaunchKernelGGL(k_slot_copy<false>, grid, dim3(256), 0, stream, g);
         return hipGetLastError();
     };
-    auto landed = [&](int b) {
-        const uint64_t* f = (const uint64_t*)(ctx->ring + kSlotBytes * kN + 64 * (b % kN));
-        return __atomic_load_n(f, __ATOMIC_ACQUIRE) >= seq0 + b;
+    auto flag = [&](int i) {
+        return __atomic_load_n((const uint64_t*)(ctx->ring + kSlotBytes * kN + 64 * i), __ATOMIC_ACQUIRE);
     };
+    auto landed = [&](int b) { return flag(b % kN) >= seq0 + b; };
 
-    // kernels first, then the threads that would wait for them
+    // The threads to the host start with the first kernel, not before: it waits
+    // for what the stream computes, and they would spin meanwhile.
     hipError_t e = hipSuccess;
     int issued = 0, nready = 0, freed = 0;
     unsigned idle = 0;
@@ -366,9 +371,13 @@ hsgen_status host_copy(hsgen_ctx* ctx, const std::vector<HostCopy>& list, bool t
         ready.store(nready, std::memory_order_release);
     }
     HostPool* threads = pool(ctx, plan.bytes);
-    if (to_host && ctx->prefault) ctx->prefault->stop();
-    if (threads && e == hipSuccess) threads->post(&plan, worker, std::min(threads->size(), plan.bytes / kThreadBytes));
+    bool posted = false;
     while (e == hipSuccess && (to_host ? freed < n : issued < n)) {
+        if (!posted && (!to_host || flag(kN) >= seq0 || landed(0))) {
+            if (to_host && ctx->prefault) ctx->prefault->stop();
+            if (threads) threads->post(&plan, worker, std::min(threads->size(), plan.bytes / kThreadBytes));
+            posted = true;
+        }
         if (to_host) {
             send();
         } else {
