@@ -28,19 +28,21 @@ std::string kind_key(const hsgen_sys* s, int a, const RadDev* rad, bool rot)
 }
 
 // Two rotations give the same cosines between plane waves: their R R^T (of
-// kb = R^T K) agree to the rounding of the products, 4 units of the largest.
+// kb = R^T K) agree to the rounding of the products, 4 units of each entry's own
+// scale |R_i| |R_j| (in a long cell the axes' differ by orders of magnitude).
 bool same_cosines(const double* r, const double* q)
 {
-    double g[2][9], big = 0.0;
+    double g[2][9];
     for (int w = 0; w < 2; ++w) {
         const double* m = w ? q : r;
         for (int i = 0; i < 3; ++i)
             for (int j = 0; j < 3; ++j)
                 g[w][3 * i + j] = m[i] * m[j] + m[3 + i] * m[3 + j] + m[6 + i] * m[6 + j];
     }
-    for (int i = 0; i < 9; ++i) big = std::max(big, std::fabs(g[0][i]));
-    for (int i = 0; i < 9; ++i)
-        if (!(std::fabs(g[0][i] - g[1][i]) <= 4.0 * 2.220446049250313e-16 * big)) return false;   // NaN too
+    for (int i = 0; i < 9; ++i) {
+        const double scale = std::sqrt(g[0][i / 3 * 4]) * std::sqrt(g[0][i % 3 * 4]);
+        if (!(std::fabs(g[0][i] - g[1][i]) <= 4.0 * 2.220446049250313e-16 * scale)) return false;   // NaN too
+    }
     return true;
 }
 
