@@ -195,6 +195,8 @@ struct hsgen_sys {
     hsgen::SphereStage* d_stages = nullptr;
     int64_t* d_mtoff = nullptr;
     std::vector<int32_t> h_order;      // atoms in kind order
+    std::vector<hsgen::OverlapGroup> h_groups;
+    std::vector<int32_t> h_group_kind; // first kind of each, and the end
     // split precision (built by its first call): matrices, their offsets per
     // atom in kind order, rows of W
     void* d_split = nullptr;
@@ -293,6 +295,9 @@ struct SphereLayout {
     int64_t ngcols = 0, nsquares = 0, nstiles = 0;
     int htile = 64, ttile = 64, stile = 64;
     size_t b_ph = 0, b_rs = 0, b_y = 0, b_w = 0;   // bytes of the operand arrays
+    // a call in parts (sphere_parts), or empty and 0
+    std::vector<int> sparts;                // first groups of S's parts, and the end
+    int64_t wcols = 0;                      // columns of W at a time
 };
 // Operands of a call: phases, radial factors, real vectors, W.
 struct SphereOperands {
@@ -301,6 +306,9 @@ struct SphereOperands {
 hsgen_status sphere_setup(hsgen_ctx* ctx, hsgen_sys* s, const RadDev* rad);
 hsgen_status sphere_operands(hsgen_ctx* ctx, const SphereLayout& l, bool do_h, SphereOperands& o);
 SphereLayout sphere_layout(const hsgen_ctx* ctx, const hsgen_sys* s, const std::vector<int>& ngs, bool do_h);
+// Lays a call of one k-point out for `bytes` of memory that do not hold its
+// operands at once (all of it from SphereArgs::ph on); false if it cannot be.
+bool sphere_parts(const hsgen_sys* s, SphereLayout& l, bool do_h, bool do_s, size_t bytes);
 SphereArgs sphere_args(const hsgen_sys* s, const SphereLayout& l, void* ph, void* rs, void* y, void* w);
 std::vector<SphereK> sphere_ks(const SphereLayout& l, const std::vector<const hsgen_kpoint*>& kps,
                                const std::vector<const int32_t*>& gs, const std::vector<double2*>& H,

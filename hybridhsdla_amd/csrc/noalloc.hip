@@ -16,7 +16,9 @@
 // call's own operands need less for the l cutoffs in use, but up to 9/4 as
 // much where atoms have lmax 0 and each is of a kind of its own (144 bytes per
 // plane wave: phase 16, radial factors 32, y and W of two rows padded to the
-// MFMA depth of four 32 and 64; general operands 64), hence the array's size.
+// MFMA depth of four 32 and 64; general operands 64), and 3/2 for S alone.
+// Those calls go in parts: S over some groups of atoms at a time, then H from
+// some columns of W at a time (phases and y 48 bytes, the rest for W).
 //
 // The call copies nothing from host memory except a host G list (a short one is
 // read from pinned memory).  Every value
@@ -33,7 +35,7 @@
 namespace hsgen {
 
 constexpr size_t kScratchLimit = HSGEN_NOALLOC_SCRATCH_BYTES;      // of the general operands
-constexpr size_t kScratchBytes = kScratchLimit / 4 * 9 + ((size_t)1 << 20);   // the array
+constexpr size_t kScratchBytes = kScratchLimit + ((size_t)1 << 20);   // the array
 constexpr int kScratchDevices = 64;
 
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
@@ -136,11 +138,11 @@ extern "C" hsgen_status hsgen_create_hs_noalloc(hsgen_ctx* ctx, const hsgen_sys*
                     "(use hsgen_create_hs)",
                     ng, s->kdim, off, kScratchLimit);
     // the call's own layout
-    const SphereLayout l = sphere_layout(ctx, s, {ng}, do_h);
+    SphereLayout l = sphere_layout(ctx, s, {ng}, do_h);
     off = 0;
     const size_t o_g = gdev ? 0 : take(sizeof(int32_t) * 3 * (size_t)ng);
     const size_t o_ph = take(l.b_ph), o_rs = take(l.b_rs), o_y = take(l.b_y), o_w = take(l.b_w);
-    if (off > kScratchBytes)
+    if (off > kScratchBytes && (o_ph >= kScratchBytes || !sphere_parts(s, l, do_h, do_s, kScratchBytes - o_ph)))
         return fail(ctx, HSGEN_ERR_ARG, "N_G %d with K %d needs %zu bytes of scratch; the array has %zu", ng, s->kdim, off,
                     kScratchBytes);
     SphereArgs p = sphere_args(s, l, base + o_ph, base + o_rs, do_h ? base + o_y : nullptr, do_h ? base + o_w : nullptr);

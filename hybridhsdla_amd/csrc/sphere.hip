@@ -335,7 +335,8 @@ struct OverlapTile {
 };
 
 // kSample: the sampled columns of S, all rows of a chunk's columns.
-template <int M, int MJ, bool kAhead, bool kSample>
+// kAdd: S of some of the groups, added (p.sadd) to that of the ones before.
+template <int M, int MJ, bool kAhead, bool kSample, bool kAdd = false>
 __device__ __forceinline__ void overlap_tile(const SphereArgs& p, int blk, char* lds)
 {
     // one rounding per written operation: every tile gives the same bits
@@ -414,6 +415,14 @@ __device__ __forceinline__ void overlap_tile(const SphereArgs& p, int blk, char*
             si[m][n] = 0.0;
             t[m][n] = 0.0;
             sg[m][n] = 1.0;
+            if constexpr (kAdd) {
+                const int i = I0 + tx + 16 * m, j = J0 + ty + TY * n;
+                if (p.sadd && i < ng && i >= j) {
+                    const double2 v = kp->S[(int64_t)j * kp->ldS + i];
+                    sr[m][n] = v.x;
+                    si[m][n] = v.y;
+                }
+            }
         }
     // 1 / (l + 1) in lane l: read from there, not by a load that a step would wait for
     const double inv_l = kLegendre.v[min(lane, kMaxLmax)];
@@ -427,7 +436,7 @@ __device__ __forceinline__ void overlap_tile(const SphereArgs& p, int blk, char*
     for (int kk = 0; kk < p.ngroups; ++kk) {
         const auto& kd = groups[kk];
         const int nlk = kd.lmax + 1, count = kd.count, rb = kk & 1;
-        if (kd.newdir) {
+        if ((kAdd && kk == 0) || kd.newdir) {
             // unit vectors [side][3][T] where the next group's radial factors will be
             double* s_n = (double*)(lds + (rb ^ 1) * 2 * planes * Ov::kPlane);
             __syncthreads();
@@ -597,6 +606,13 @@ __global__ __launch_bounds__(256) void k_overlap_sample(SphereArgs p)
     overlap_tile<2, 2, true, true>(p, (int)blockIdx.x, lds);
 }
 
+__global__ __launch_bounds__(256) void k_overlap_part(SphereArgs p)
+{
+    extern __shared__ __attribute__((aligned(1024))) char lds[];
+    stamp(p, 3);
+    overlap_tile<2, 2, true, false, true>(p, (int)blockIdx.x, lds);
+}
+
 int overlap_tile_size(int64_t tiles64, int n_cu)
 {
     // 64 x 64 tiles, one workgroup per CU, once every CU has eight; 32 x 32 once
@@ -622,6 +638,13 @@ hipError_t launch_overlap(const SphereArgs& p, int tile, int64_t ntiles, hipEven
     if (tile == 64) return launch_overlap_tile<4, 2>(p, ntiles, stop, st);
     if (tile == 32) return launch_overlap_tile<2, 2>(p, ntiles, stop, st);
     return launch_overlap_tile<1, 1>(p, ntiles, stop, st);
+}
+
+hipError_t launch_overlap_part(const SphereArgs& p, hipEvent_t stop, hipStream_t st)
+{
+    const int64_t n = (p.one.ng + 31) / 32;
+    return launch(k_overlap_part, dim3((unsigned)(n * (n + 1) / 2)), 256, (size_t)OverlapTile<2, 2>::lds((p.nl + 15) / 16),
+                  stop, st, p);
 }
 
 // ---------------------------------------------------------------------------
@@ -957,7 +980,7 @@ __device__ __forceinline__ void sphere_gemm_tile(const SphereArgs& p, int blk, c
         }
         C0 = uni((pi * P + bi) * BC);
         R0 = uni(bj * BC + (t0 + at) % kRat * BR);
-        if (R0 >= kp->ng) return;
+        if (R0 >= kp->ng || R0 < p.hcol0 || R0 >= p.hcol1) return;
         nsteps = p.nksteps;
     } else {
         // Columns in groups of P tiles; per group the tiles of rows of all
@@ -965,7 +988,7 @@ __device__ __forceinline__ void sphere_gemm_tile(const SphereArgs& p, int blk, c
         // in turn: what an XCD reads of the group's y stays in its L2 while the
         // rows pass.
         constexpr int P = kSphereColumns / BC;
-        const int ntc = (int)(p.gtot / BC);
+        const int ntc = p.tcols / BC;
         const int cg = (int)(blk / ((int64_t)P * p.rtiles));
         const int u = (int)(blk - (int64_t)cg * P * p.rtiles);
         const int h = min(P, ntc - cg * P);                   // the group's columns
@@ -1375,7 +1398,7 @@ hipError_t launch_sphere_tapp(const SphereArgs& p, int tile, int rtiles, hipEven
 {
     SphereArgs q = p;
     q.rtiles = rtiles;
-    const int64_t nblk = (int64_t)rtiles * (p.gtot / (tile == 32 ? 32 : 64));
+    const int64_t nblk = (int64_t)rtiles * (p.tcols / (tile == 32 ? 32 : 64));
     if (tile == 32) return launch_sphere_gemm<32, 32, 1, 1, 2, kTApp>(q, nblk, stop, st);
     return launch_sphere_gemm<32, 64, 1, 2, 2, kTApp>(q, nblk, stop, st);
 }

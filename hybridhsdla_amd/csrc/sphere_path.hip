@@ -150,6 +150,7 @@ hsgen_status sphere_setup(hsgen_ctx* ctx, hsgen_sys* s, const RadDev* rad)
             g.newdir = i == 0 || members[i].cos != members[i - 1].cos;
             std::memcpy(g.rot, s->atoms[cos_rep[members[i].cos]].rot, sizeof g.rot);
             groups.push_back(g);
+            s->h_group_kind.push_back((int32_t)i);
             rr += 2 * (at.lmax + 1);
         }
         groups.back().count += k.count;
@@ -184,6 +185,8 @@ hsgen_status sphere_setup(hsgen_ctx* ctx, hsgen_sys* s, const RadDev* rad)
     s->nkinds = (int)kinds.size();
     s->h_order = order;
     s->ngroups = (int)groups.size();
+    s->h_groups = groups;
+    s->h_group_kind.push_back(s->nkinds);
     s->ldr = (int)rr;
     s->rt32 = (int)rt32;
     // whole stages of 16 rows can be read at the end of a column, from any
@@ -498,6 +501,8 @@ SphereArgs sphere_args(const hsgen_sys* s, const SphereLayout& l, void* ph, void
     p.nk = 1;
     p.ngcols = (int32_t)l.ngcols;
     p.gtot = l.gtot;
+    p.tcols = (int32_t)l.gtot;
+    p.hcol1 = INT32_MAX;
     p.ph = (double2*)ph;
     p.rs = (double2*)rs;
     p.ldr = s->ldr;
@@ -573,11 +578,88 @@ hsgen_status sphere_g(hsgen_ctx* ctx, const hsgen_kpoint* kp, int32_t* dev, Sphe
     return HSGEN_OK;
 }
 
+// Bytes of the phases and radial factors of groups g0 .. g1 - 1.
+static size_t part_bytes(const hsgen_sys* s, const SphereLayout& l, int g0, int g1)
+{
+    const int atoms = (g1 < s->ngroups ? s->h_groups[g1].first : s->natoms) - s->h_groups[g0].first;
+    const int rows = (g1 < s->ngroups ? s->h_groups[g1].rsoff : s->ldr) - s->h_groups[g0].rsoff;
+    return sizeof(double2) * (size_t)l.gtot * ((size_t)atoms + rows);
+}
+
+bool sphere_parts(const hsgen_sys* s, SphereLayout& l, bool do_h, bool do_s, size_t bytes)
+{
+    for (int g0 = 0; do_s && g0 < s->ngroups;) {
+        int g1 = g0 + 1;
+        while (g1 < s->ngroups && part_bytes(s, l, g0, g1 + 1) <= bytes) ++g1;
+        if (part_bytes(s, l, g0, g1) > bytes) return false;
+        l.sparts.push_back(g0);
+        g0 = g1;
+    }
+    l.sparts.push_back(s->ngroups);
+    const size_t column = sizeof(double2) * (size_t)s->ldw;
+    if (l.b_ph + l.b_y >= bytes) return !do_h;
+    l.wcols = std::min(l.gtot, (int64_t)((bytes - l.b_ph - l.b_y) / column) / kSphereCols * kSphereCols);
+    return !do_h || l.wcols > 0;
+}
+
+// The launches of one k-point in parts: S over its groups in turn, then H from
+// W a few columns at a time, in the same memory.  The same kernels in the same
+// order of sums, so the same bits.
+static hipError_t sphere_launch_parts(const SphereArgs& p, const SphereLayout& l, const hsgen_sys* s, bool do_h, bool do_s,
+                                      hipEvent_t stop, hipStream_t st)
+{
+    if (!do_h && !do_s) return stop ? hipEventRecord(stop, st) : hipSuccess;
+    hipError_t e = hipSuccess;
+    const int nparts = do_s ? (int)l.sparts.size() - 1 : 0;
+    for (int i = 0; i < nparts; ++i) {
+        const int g0 = l.sparts[i], g1 = l.sparts[i + 1];
+        const int first = s->h_groups[g0].first, rs0 = s->h_groups[g0].rsoff;
+        SphereArgs q = p;
+        q.y = nullptr;
+        q.groups += g0;
+        q.ngroups = g1 - g0;
+        q.kinds += s->h_group_kind[g0];
+        q.nkinds = s->h_group_kind[g1] - s->h_group_kind[g0];
+        q.order += first;
+        q.natoms = (g1 < s->ngroups ? s->h_groups[g1].first : s->natoms) - first;
+        q.ldr = (g1 < s->ngroups ? s->h_groups[g1].rsoff : s->ldr) - rs0;
+        // rows of the whole call: the part's begin at rs0, its atoms at `first`
+        q.rs = (double2*)((uintptr_t)(p.ph + (int64_t)q.natoms * l.gtot) - sizeof(double2) * (size_t)rs0);
+        if ((e = launch_sphere_gen(q, nullptr, st)) != hipSuccess) return e;
+        q.ph = (double2*)((uintptr_t)p.ph - sizeof(double2) * (size_t)first * (size_t)l.gtot);
+        q.sadd = i > 0;
+        e = launch_overlap_part(q, i + 1 < nparts || do_h ? nullptr : stop, st);
+        if (e != hipSuccess) return e;
+    }
+    if (!do_h) return e;
+    SphereArgs q = p;
+    q.rs = nullptr;
+    q.y = (double*)((char*)p.ph + l.b_ph);
+    double2* const w = (double2*)((char*)q.y + l.b_y);
+    e = launch_sphere_gen(q, nullptr, st);
+    for (int64_t c0 = 0; c0 < l.gtot && e == hipSuccess; c0 += l.wcols) {
+        const int64_t n = std::min(l.wcols, l.gtot - c0);
+        SphereArgs t = q;
+        t.tcols = (int32_t)n;
+        t.y += c0 * p.ldy;
+        t.ph += c0;
+        t.W = w;
+        if ((e = launch_sphere_tapp(t, l.ttile, s->rt32, nullptr, st)) != hipSuccess) return e;
+        t = q;
+        t.W = (double2*)((uintptr_t)w - sizeof(double2) * (size_t)(c0 * p.ldw));   // addressed by the call's columns
+        t.hcol0 = (int32_t)c0;
+        t.hcol1 = (int32_t)(c0 + n);
+        e = launch_sphere_h(t, l.htile, c0 + n < l.gtot ? nullptr : stop, st);
+    }
+    return e;
+}
+
 // The launches of one call.  stop: null, or an event that takes the end of the
 // last of them.
 hipError_t sphere_launch(const SphereArgs& p, const SphereLayout& l, const hsgen_sys* s, bool do_h, bool do_s,
                          hipEvent_t stop, hipStream_t st)
 {
+    if (!l.sparts.empty()) return sphere_launch_parts(p, l, s, do_h, do_s, stop, st);
     const hipEvent_t none = nullptr, last = stop;
     hipError_t e = launch_sphere_gen(p, do_h || do_s ? none : last, st);
     if (e == hipSuccess && do_h) e = launch_sphere_tapp(p, l.ttile, s->rt32, none, st);

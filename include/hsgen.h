@@ -221,7 +221,7 @@ hsgen_status hsgen_contract_hs(hsgen_ctx* ctx, int32_t L, int32_t a, int32_t G,
 /* hsgen_create_hs in FP64 with no device allocation.  No counterpart in the
  * reference: for callers that cannot allocate device memory (code under HIP
  * graph capture, tight serving loops, harnesses that forbid hipMalloc).  The
- * call's workspaces live in one device array per GPU (577 MiB), held by the
+ * call's workspaces live in one device array per GPU (257 MiB), held by the
  * library until the process ends.  A problem whose general operands (a host G
  * list's device copy, the grouped-GEMM work lists and 2 x 16 B x (2K + 32) x
  * roundup(ng, 128) for the default tile, 3 x for a system with a zero
