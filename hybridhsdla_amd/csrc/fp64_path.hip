@@ -432,8 +432,9 @@ hsgen_status finish_hs(hsgen_ctx* ctx, hsgen_sys* s, const Geometry& geo, int ng
     return HSGEN_OK;
 }
 
-// create_hs on the general operands: A/B generator -> T application -> S and
-// H.  o.tile is the call's tile; ng > 0.
+// create_hs on the general operands (split precision, the autotuner, systems
+// whose columns are too long for the real vectors): A/B generator -> T
+// application -> S and H.  o.tile is the call's tile; ng > 0.
 hsgen_status create_hs_general(hsgen_ctx* ctx, hsgen_sys* s, const hsgen_kpoint* kp, const hsgen_opts& o, double* H,
                                double* S, int64_t ld, hsgen_report* rep)
 {
@@ -459,7 +460,7 @@ hsgen_status create_hs_general(hsgen_ctx* ctx, hsgen_sys* s, const hsgen_kpoint*
     HIPCHK(hipEventRecord(ctx->ev[0], ctx->stream));
     HIPCHK(launch_abgen(p, true, ctx->stream));
     HIPCHK(hipEventRecord(ctx->ev[1], ctx->stream));
-    st = finish_hs(ctx, s, geo, ng, o, H, S, ld, rep, 0.0, is_split(o.precision) ? kp : nullptr);
+    st = finish_hs(ctx, s, geo, ng, o, H, S, ld, rep, 0.0, is_split(o.precision) && s->real_vectors ? kp : nullptr);
     if (st) return st;
     if (rep) {
         float t0 = 0;
@@ -537,6 +538,18 @@ hsgen_status batched_fp64(hsgen_ctx* ctx, hsgen_sys* s, int nk, const hsgen_kpoi
     for (int i = 0; i < nk; ++i) max_ng = std::max(max_ng, kps[i].ng);
     const Geometry geo = geometry(o.tile, s->kdim, max_ng);
     hsgen_status st;
+    if (!s->real_vectors) {     // one k-point after the other
+        double total = 0.0;
+        for (int i = 0; i < nk; ++i) {
+            hsgen_report r;
+            std::memset(&r, 0, sizeof r);
+            if (kps[i].ng > 0 && (st = create_hs_general(ctx, s, &kps[i], o, H[i], S[i], ld[i], &r))) return st;
+            total += r.ms_total;
+            if (rep) rep[i] = r;
+        }
+        if (rep) rep[0].ms_total = total;
+        return HSGEN_OK;
+    }
     // largest k first; k-points without G-vectors have nothing to compute
     std::vector<int> order;
     for (int i = 0; i < nk; ++i)
@@ -774,7 +787,7 @@ hsgen_status hsgen_create_hs(hsgen_ctx* ctx, const hsgen_sys* sc, const hsgen_kp
     if (rep) std::memset(rep, 0, sizeof *rep);
     if (ng == 0) return HSGEN_OK;
     HIPCHK(hipSetDevice(ctx->device));
-    if (is_split(o.precision)) return create_hs_general(ctx, s, kp, o, H, S, ld, rep);
+    if (is_split(o.precision) || !s->real_vectors) return create_hs_general(ctx, s, kp, o, H, S, ld, rep);
     return create_hs_sphere(ctx, s, kp, o, H, S, ld, rep);
 }
 

@@ -204,6 +204,7 @@ struct hsgen_sys {
     int32_t* d_split_rows = nullptr;
     int nkinds = 0, ngroups = 0, nksteps = 0, ldr = 0, rt32 = 0;
     int64_t ldy = 0, ldw = 0;
+    bool real_vectors = true;          // calls take the path of sphere.h, else the general operands
     // first atom of each rotation class and of each rmt class (AtomDev::cls)
     std::vector<int32_t> rot_rep, rmt_rep;
 };

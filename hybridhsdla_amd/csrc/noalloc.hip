@@ -101,6 +101,7 @@ extern "C" hsgen_status hsgen_create_hs_noalloc(hsgen_ctx* ctx, const hsgen_sys*
     if (rep) std::memset(rep, 0, sizeof *rep);
     if (ng == 0) return HSGEN_OK;
     HIPCHK(hipSetDevice(ctx->device));
+    if (!s->real_vectors) return fail(ctx, HSGEN_ERR_ARG, "K %d is beyond the allocation-free entry point", s->kdim);
     char* base = (char*)scratch_of(ctx->device);
     if (!base) return fail(ctx, HSGEN_ERR_UNSUPPORTED, "no scratch array on device %d", ctx->device);
     o.tile = pick_tile(ctx, o, ng, s->kdim);

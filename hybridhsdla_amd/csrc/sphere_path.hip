@@ -194,6 +194,10 @@ hsgen_status sphere_setup(hsgen_ctx* ctx, hsgen_sys* s, const RadDev* rad)
     // memory channels
     s->ldy = (roundup(ry, 16) + 16) | 16;
     s->ldw = roundup(rw, 16) | 16;
+    // the products address 4 columns of W and 8 of y with 32-bit offsets; longer
+    // columns (44 million rows of coefficients) take the general operands
+    const char* env = std::getenv("HSGEN_REAL_VECTORS");      // 0: general operands (tests and comparisons)
+    s->real_vectors = 64 * s->ldw < (int64_t(1) << 32) && 64 * s->ldy < (int64_t(1) << 32) && !(env && env[0] == '0');
     // T blocks in real harmonics, one per distinct T (h_owner)
     std::vector<int64_t> off(na, 0);
     int64_t total = 0;

@@ -856,7 +856,8 @@ hsgen_status batched_split(hsgen_ctx* ctx, hsgen_sys* s, int nk, const hsgen_kpo
     // one pass per batch saves those reads but needs more, smaller batches,
     // which cost as much again at 64 k-points)
     if (g0.fold) release(ctx->Zs);   // folded operands need no Zs
-    if (do_h && (st = sphere_split_setup(ctx, s))) return st;   // the system keeps these: not of the budget
+    // the system keeps these: not of the budget
+    if (do_h && (st = s->real_vectors ? sphere_split_setup(ctx, s) : ensure_M(ctx, s, g0.t.bk, g0.t.bm))) return st;
     size_t fr = 0, tot = 0;
     HIPCHK(hipMemGetInfo(&fr, &tot));
     size_t held = 0;
@@ -983,7 +984,15 @@ hsgen_status batched_split(hsgen_ctx* ctx, hsgen_sys* s, int nk, const hsgen_kpo
             HIPCHK(launch_abgen(p, true, ctx->stream));
         }
         OzSample smp;
-        if (do_h) {
+        if (do_h && !s->real_vectors) {
+            std::vector<GemmProblem> probs;
+            std::vector<TileWork> work;
+            const int tc = tapp_cfg(geo);
+            add_tmul_problems(probs, work, s, geo, zgemm_cfg(tc), ncols, Z, W);
+            st = run_grouped(ctx, tc, probs, work);
+            if (st) return st;
+            HIPCHK(launch_clear_rows(W, geo.ldz, 2 * (int64_t)s->kdim, geo.ldz, (int)ncols, ctx->stream));
+        } else if (do_h) {
             // T application over every column of the batch from the real vectors
             if ((st = oz_sample(ctx, geo, ks, false, smp))) return st;
             std::vector<SphereK> sk(bk.size());
@@ -1015,7 +1024,7 @@ hsgen_status batched_split(hsgen_ctx* ctx, hsgen_sys* s, int nk, const hsgen_kpo
         }
         Prefault pages(ctx, out);
         std::vector<OzResult> ozr;
-        st = run_ozaki(ctx, geo, ks, flags, icfg, o.slices, o.target_rel_err, ozr, true, do_h ? &smp : nullptr);
+        st = run_ozaki(ctx, geo, ks, flags, icfg, o.slices, o.target_rel_err, ozr, true, do_h && s->real_vectors ? &smp : nullptr);
         if (st) return st;
         for (size_t q = 0; q < bk.size() && (flags & HSGEN_FILL_UPPER); ++q) {
             if (do_h) HIPCHK(launch_fill_upper(ks[q].dH, ks[q].ldH, ks[q].ng, ctx->stream));
