@@ -17,7 +17,7 @@
 // 15 GB/s, eight at 65, more not faster.  The last slot's host side overlaps
 // nothing, so slots are small.
 // Measured, whole calls, the runtime's copies before: A and B of 16 atoms at
-// N_G 1500 (62 MB) 5.0 -> 1.3 ms; H and S at N_G 1201 (46 MB, both triangles)
+// N_G 1500 (62 MB) 5.0-5.8 -> 1.3-1.7 ms (over boards); H and S at N_G 1201 (46 MB, both triangles)
 // 2.87 -> 1.45 ms; the contraction of given coefficients at N_G 1500 (62 MB in,
 // two lower triangles out) 7.7 -> 4.9 ms, 3.4 with M built on the GPU and S's copy
 // beside H.

@@ -849,8 +849,8 @@ hipError_t launch_split_mt(const SplitMtJob* jobs, int njobs, int64_t max_elems,
 // 26.9) at N_G 600, 12.5 (13.7) at 235, 1075 (1121) at 2003; four stages and
 // three workgroups per CU 21.3, 12.7 and 1112.  The T application, with depths of
 // 10 to 20 stages, loses with a third stage what it loses in workgroups.
-// Rate of the H tiles: 0.87 of the FP64 peak at N_G 16000 and 25000, 0.85 at
-// 10000, 0.82 at 6002 (32 atoms, lmax 10).
+// Rate of the H tiles: 0.86 of the FP64 peak at N_G 12009, 16000 and 24995 (0.84
+// on the slowest board), 0.85 at 10025, 0.82 at 6002 (32 atoms, lmax 10).
 // Measured (whole call, complex-by-complex contraction of S and H before, now):
 // 714 -> 202 ms at N_G 12007 (128 atoms, lmax 12), 33.5 -> 10.0 ms at 6002 and
 // 5.41 -> 1.37 ms at 2003 (32 atoms, lmax 10), with S and all else since.

@@ -107,15 +107,19 @@ int pick_tile(const hsgen_ctx* ctx, const hsgen_opts& o, int ng, int kdim, const
     if (o.precision == HSGEN_PREC_FP64) return fp64_tile_by_size(ctx, ng, kps, nk);
     const int64_t t = call_tiles(ng, kps, nk, 256, 192);
     if (o.precision == HSGEN_PREC_OZAKI_INT8) {
-        // A CU holds one workgroup of the larger tiles, so a launch takes whole
-        // rounds of n_cu tiles; a 128 x 256 round takes about 0.72 of a 256 x 192
-        // one.  128 x 128 tiles where they make one round; else, up to three
-        // rounds of 256 x 192 (where the rounding counts), the fewer.  INT8 GEMM
-        // ms of a call, 256 x 192 / 128 x 256 / 128 x 128 tiles (12 moduli; k-points
-        // of 48 atoms): 2 of 1200 plane waves 2.15 / 1.60 / 1.09, 2 of 1900 4.48 /
-        // 3.63 / 4.23, 4 of 1900 8.94 / 6.75 / 6.97, 8 of 1900 13.77 / 11.77 / 13.44;
-        // (32 atoms, N_G) 2500 3.02 / 2.34 / 2.95, 3000 3.38 / 4.33 / 4.30, 3500 6.47 /
-        // 4.95 / 6.18, 4000 6.53 / 7.25 / 7.70, 5000 9.94 / 9.88 / 11.23.
+        // A CU holds one workgroup of the larger tiles; a 128 x 256 tile takes about
+        // 0.72 of a 256 x 192 one.  128 x 128 tiles where one modulus's make one
+        // round of the CUs; else, up to three rounds of 256 x 192, the fewer rounds.
+        // The rounds are one modulus's.  All moduli share a launch, which levels
+        // most of the rounding out, so the rule's lines are no longer sharp: INT8
+        // GEMM ms of a call, 256 x 192 / 128 x 256 / 128 x 128 tiles (12 moduli;
+        // k-points of 48 atoms): 2 of 1200 plane waves 1.61 / 1.47 / 1.73, 2 of 1900
+        // 3.60 / 3.31 / 3.93, 4 of 1900 6.32 / 5.94 / 7.09, 8 of 1900 11.88 / 11.58 /
+        // 13.08; (32 atoms, N_G) 2003 1.32 / 1.33 / 1.56, 2500 2.15 / 2.16 / 2.51, 3000
+        // 3.06 / 3.04 / 3.75, 3500 4.11 / 4.27 / 5.26, 4000 5.26 / 5.60 / 6.62, 5000
+        // 7.88 / 8.55 / 10.12, 6002 11.18 / 11.51 / 13.93.  It is within 4% of the
+        // best but at 2 of 1200 (18% of the GEMMs) and 5000 (8%); whole calls differ
+        // by less, as the smaller tiles pad less (3500: 6.40 and 6.39 ms).
         const int64_t ncu = std::max(ctx->n_cu, 1);
         auto rounds = [&](int64_t n) { return (n + ncu - 1) / ncu; };
         if (call_tiles(ng, kps, nk, 128, 128) <= ncu) return kInt8SmallCfg;

@@ -123,7 +123,9 @@ typedef struct {
     int32_t ng;                /* G */
     int32_t kdim;              /* K = sum_a L_a */
     int32_t slices_used;       /* split precision: slices actually used */
-    int32_t tile_used;         /* contraction tile config id actually used */
+    int32_t tile_used;         /* split precision, and FP64 from given coefficients: contraction
+                                  tile config id used.  FP64 from a system, whose kernels have no
+                                  tile id: the id that the call asked for or that goes with its size */
     double err_est_h;          /* split precision: estimated relative Frobenius error of H */
     double err_est_s;          /* ... and of S (0 in FP64) */
     double ms_igemm;           /* split precision: GPU time of the residue (INT8 or BF16) GEMM launches alone
@@ -181,11 +183,13 @@ hsgen_status hsgen_create_hs_batched(hsgen_ctx* ctx, const hsgen_sys* sys,
                                      double* const* S, const int64_t* ld,
                                      hsgen_report* report);
 
-/* Autotuner: time every tile configuration of the contraction (FP64 GEMM,
- * or the INT8 GEMM of split precision at a fixed 10 moduli) on this
- * k-point and remember the fastest for problems of its size (half-octave
- * buckets of G and K).  Later calls with opts.tile = 0 use the remembered
- * configuration; explicit opts.tile values still win.  No reference
+/* Autotuner: time every tile configuration of the contraction (FP64 GEMM of
+ * the complex operands, or the INT8 or BF16 GEMM of split precision at a fixed
+ * 10 moduli) on this k-point and remember the fastest for problems of its size
+ * (half-octave buckets of G and K).  Later calls with opts.tile = 0 that run
+ * such a contraction use the remembered configuration (FP64: hsgen_contract_hs;
+ * calls from a system pick their kernels by size and only report it); explicit
+ * opts.tile values still win.  No reference
  * counterpart: it takes the place of the reference's per-machine GPU/CPU
  * split-ratio tuning (compute_ratio.cpp, wrappers.cpp:73-109).  *best_tile
  * and *best_ms (contraction GPU time of the winner) may be NULL. */
