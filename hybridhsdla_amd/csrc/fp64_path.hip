@@ -404,7 +404,9 @@ hsgen_status finish_hs(hsgen_ctx* ctx, hsgen_sys* s, const Geometry& geo, int ng
     if (apart) HIPCHK(hipStreamWaitEvent(ctx->stream, ctx->ev[5], 0));
     HIPCHK(hipEventRecord(ctx->ev[4], ctx->stream));
     if (apart) {
-        if ((st = host_copy(ctx, out_s, true, ctx->stream2)) || (st = host_copy(ctx, out_h, true, ctx->stream))) return st;
+        if ((st = host_copy(ctx, out_s, true, ctx->stream2, false)) ||
+            (st = host_copy(ctx, out_h, true, ctx->stream, false)))
+            return st;
     } else {
         HIPCHK(hipEventSynchronize(ctx->ev[4]));
         if ((st = host_copy(ctx, out, true, ctx->stream))) return st;
@@ -760,6 +762,7 @@ hsgen_status hsgen_construct_ab(hsgen_ctx* ctx, const hsgen_sys* s, const hsgen_
     if (!bdev) out.push_back(copy_run(dB, B, sizeof(double2) * n));
     Prefault pages(ctx, out);
     HIPCHK(launch_abgen(p, false, ctx->stream));
+    // a hundredth of the copy's time: as good as computed
     st = host_copy(ctx, out, true, ctx->stream);
     if (st) return st;
     HIPCHK(hipStreamSynchronize(ctx->stream));

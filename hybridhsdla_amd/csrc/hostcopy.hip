@@ -271,7 +271,7 @@ Prefault::~Prefault()
     ctx_->prefault = nullptr;
 }
 
-hsgen_status host_copy(hsgen_ctx* ctx, const std::vector<HostCopy>& list, bool to_host, hipStream_t stream)
+hsgen_status host_copy(hsgen_ctx* ctx, const std::vector<HostCopy>& list, bool to_host, hipStream_t stream, bool computed)
 {
     constexpr int kN = kRingSlots;
     Plan plan;
@@ -351,8 +351,10 @@ hsgen_status host_copy(hsgen_ctx* ctx, const std::vector<HostCopy>& list, bool t
     };
     auto landed = [&](int b) { return flag(b % kN) >= seq0 + b; };
 
-    // The threads to the host start with the first kernel, not before: it waits
-    // for what the stream computes, and they would spin meanwhile.
+    // While the stream still computes what is to be copied the threads sleep until
+    // the first kernel starts: they would spin meanwhile.  Where it is done they
+    // start at once, with the kernel's launch (H and S at N_G 1201: 1.44 ms, 1.51
+    // with the kernel's start).
     hipError_t e = hipSuccess;
     int issued = 0, nready = 0, freed = 0;
     unsigned idle = 0;
@@ -373,7 +375,7 @@ hsgen_status host_copy(hsgen_ctx* ctx, const std::vector<HostCopy>& list, bool t
     HostPool* threads = pool(ctx, plan.bytes);
     bool posted = false;
     while (e == hipSuccess && (to_host ? freed < n : issued < n)) {
-        if (!posted && (!to_host || flag(kN) >= seq0 || landed(0))) {
+        if (!posted && (!to_host || computed || flag(kN) >= seq0 || landed(0))) {
             if (to_host && ctx->prefault) ctx->prefault->stop();
             if (threads) threads->post(&plan, worker, std::min(threads->size(), plan.bytes / kThreadBytes));
             posted = true;

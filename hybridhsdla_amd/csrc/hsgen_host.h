@@ -244,7 +244,9 @@ hsgen_status check_kpoint(hsgen_ctx* ctx, const hsgen_kpoint* kp);
 hsgen_status upload_g(hsgen_ctx* ctx, const hsgen_kpoint* kp);
 // Copies of a call, started on `stream` and complete on return (to the device:
 // the host side is; calls with different streams order their slots' use).
-hsgen_status host_copy(hsgen_ctx* ctx, const std::vector<HostCopy>& list, bool to_host, hipStream_t stream);
+// computed: to the host, what is copied is there already.
+hsgen_status host_copy(hsgen_ctx* ctx, const std::vector<HostCopy>& list, bool to_host, hipStream_t stream,
+                       bool computed = true);
 
 // ---- fp64_path.hip ----
 struct Geometry {
