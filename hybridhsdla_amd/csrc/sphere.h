@@ -123,9 +123,10 @@ struct SphereArgs {
     SphereK one;
     const SphereK* many;
     int64_t gtot;              // columns of the operand arrays
-    // a call in parts (sphere_launch_parts): columns of the T application, H
-    // columns of the launch, and whether S adds to what an earlier launch left
-    int32_t tcols, hcol0, hcol1, sadd;
+    int32_t tcols;             // columns of the T application
+    // a call in parts (sphere_launch_parts): H columns of the launch, and whether
+    // S adds to what an earlier launch left
+    int32_t hcol0, hcol1, sadd;
     double2* ph;               // [natoms][gtot] phases, kind order
     double2* rs;               // [gtot][ldr] radial factors per overlap group: (a_l, b_l), then with S's weights
     int32_t ldr;
@@ -163,6 +164,7 @@ hipError_t launch_sphere_h(const SphereArgs& p, int tile, hipEvent_t stop, hipSt
 // S tile side by the number of lower tiles; the bits do not depend on it
 int overlap_tile_size(int64_t tiles64, int n_cu);
 hipError_t launch_overlap(const SphereArgs& p, int tile, int64_t ntiles, hipEvent_t stop, hipStream_t st);
+hipError_t launch_sphere_h_part(const SphereArgs& p, hipEvent_t stop, hipStream_t st);
 // S of one k-point from the groups of p, added to S as it is where p.sadd
 hipError_t launch_overlap_part(const SphereArgs& p, hipEvent_t stop, hipStream_t st);
 // H tiles of 32 x 32 (or 16 x 32: tile 16, S tile 16) and S tiles of 16 or 32 in one launch

@@ -913,9 +913,9 @@ __device__ __forceinline__ int64_t uni(int64_t v)
     return (int64_t)(((uint64_t)(uint32_t)uni((int)(v >> 32)) << 32) | (uint32_t)uni((int)v));
 }
 
-// What a product computes: W (T application), the lower triangle of H, or the
-// sampled columns of H.
-enum SphereMode { kTApp, kLowerH, kSampleH };
+// What a product computes: W (T application), the lower triangle of H, the
+// sampled columns of H, or the triangle's columns hcol0 .. hcol1 - 1.
+enum SphereMode { kTApp, kLowerH, kSampleH, kPartH };
 
 template <int BR, int BC, int RB, int CB, int NS, int kMode, int PARTS = 1>
 __device__ __forceinline__ void sphere_gemm_tile(const SphereArgs& p, int blk, char* lds)
@@ -980,7 +980,8 @@ __device__ __forceinline__ void sphere_gemm_tile(const SphereArgs& p, int blk, c
         }
         C0 = uni((pi * P + bi) * BC);
         R0 = uni(bj * BC + (t0 + at) % kRat * BR);
-        if (R0 >= kp->ng || R0 < p.hcol0 || R0 >= p.hcol1) return;
+        if (R0 >= kp->ng) return;
+        if (kMode == kPartH && (R0 < p.hcol0 || R0 >= p.hcol1)) return;
         nsteps = p.nksteps;
     } else {
         // Columns in groups of P tiles; per group the tiles of rows of all
@@ -999,7 +1000,7 @@ __device__ __forceinline__ void sphere_gemm_tile(const SphereArgs& p, int blk, c
         C0 = uni((cg * P + u - tr * h) * BC);
         nsteps = uni(kd->r4 / 4);
     }
-    const int64_t col0 = kMode == kLowerH ? uni(kp->col0) : 0;
+    const int64_t col0 = kMode == kLowerH || kMode == kPartH ? uni(kp->col0) : 0;
     const double2* const X = kMode == kSampleH ? p.smp_W + (int64_t)xcol * p.smp_ldw : p.W + col0 * p.ldw;
     const int64_t ldx = kMode == kSampleH ? p.smp_ldw : p.ldw;
     const int nst = uni((nsteps + 3) / 4);
@@ -1416,6 +1417,15 @@ hipError_t launch_sphere_h(const SphereArgs& p, int tile, hipEvent_t stop, hipSt
     if (tile == 32) return launch_sphere_gemm<32, 32, 1, 1, kSphereSmall, kLowerH>(p, n, stop, st);
     if (tile == 48) return launch_sphere_gemm<32, 64, 1, 2, 2, kLowerH>(p, n, stop, st);
     return launch_sphere_gemm<64, 64, 1, 2, 2, kLowerH>(p, n, stop, st);
+}
+
+// H of one k-point's columns hcol0 .. hcol1 - 1, multiples of 64
+hipError_t launch_sphere_h_part(const SphereArgs& p, hipEvent_t stop, hipStream_t st)
+{
+    SphereArgs q = p;
+    const int n = (p.one.ng + 31) / 32;
+    q.nsquares = n * (n + 1) / 2;
+    return launch_sphere_gemm<32, 32, 1, 1, kSphereSmall, kPartH>(q, (q.nsquares + 7) / 8 * 8, stop, st);
 }
 
 template <int M, int PARTS>

@@ -506,7 +506,6 @@ SphereArgs sphere_args(const hsgen_sys* s, const SphereLayout& l, void* ph, void
     p.ngcols = (int32_t)l.ngcols;
     p.gtot = l.gtot;
     p.tcols = (int32_t)l.gtot;
-    p.hcol1 = INT32_MAX;
     p.ph = (double2*)ph;
     p.rs = (double2*)rs;
     p.ldr = s->ldr;
@@ -653,7 +652,7 @@ static hipError_t sphere_launch_parts(const SphereArgs& p, const SphereLayout& l
         t.W = (double2*)((uintptr_t)w - sizeof(double2) * (size_t)(c0 * p.ldw));   // addressed by the call's columns
         t.hcol0 = (int32_t)c0;
         t.hcol1 = (int32_t)(c0 + n);
-        e = launch_sphere_h(t, l.htile, c0 + n < l.gtot ? nullptr : stop, st);
+        e = launch_sphere_h_part(t, c0 + n < l.gtot ? nullptr : stop, st);
     }
     return e;
 }
