@@ -324,6 +324,7 @@ hsgen_status hsgen_release_workspace(hsgen_ctx* ctx)
 hsgen_status hsgen_finalize(hsgen_ctx* ctx)
 {
     if (!ctx) return HSGEN_ERR_ARG;
+    if (getpid() != ctx->pid) return HSGEN_OK;    // a forked process owns none of it and must not call HIP
     (void)hipSetDevice(ctx->device);
     (void)hipStreamSynchronize(ctx->stream);
     hsgen_release_workspace(ctx);
@@ -474,6 +475,7 @@ hsgen_status hsgen_system_create(hsgen_ctx* ctx, const hsgen_system* d, hsgen_sy
 hsgen_status hsgen_system_destroy(hsgen_ctx* ctx, hsgen_sys* s)
 {
     if (!s) return HSGEN_ERR_ARG;
+    if (ctx && getpid() != ctx->pid) return HSGEN_OK;
     if (ctx) (void)hipSetDevice(ctx->device);
     if (s->d_atoms) (void)hipFree(s->d_atoms);
     if (s->d_rad) (void)hipFree(s->d_rad);

@@ -23,6 +23,8 @@
 // element is zero so the kernels need no bounds checks along k.
 #pragma once
 
+#include <unistd.h>
+
 #include <atomic>
 #include <complex>
 #include <cstdarg>
@@ -111,6 +113,7 @@ private:
 
 struct hsgen_ctx {
     int device = 0;
+    pid_t pid = getpid();                            // of the process whose GPU resources these are
     hipStream_t stream = nullptr;
     hipStream_t stream2 = nullptr;                   // S beside the T application and H
     hipEvent_t ev[8] = {};

@@ -136,7 +136,9 @@ typedef struct {
 } hsgen_report;
 
 /* Context: bind GPU `device` (HIP ordinal), create its stream.
- * Replaces dev_init()/dev_finalize() (flapw_opt/src/include/acc/wrappers.h:6-7). */
+ * Replaces dev_init()/dev_finalize() (flapw_opt/src/include/acc/wrappers.h:6-7).
+ * In a process forked from the one that made them, hsgen_finalize and
+ * hsgen_system_destroy leave the context and its systems as they are. */
 hsgen_status hsgen_init(hsgen_ctx** ctx, int32_t device);
 hsgen_status hsgen_finalize(hsgen_ctx* ctx);
 const char* hsgen_last_error(const hsgen_ctx* ctx);   /* never NULL */
