@@ -1,5 +1,6 @@
 // Host-side state and helpers shared by the hsgen C-ABI translation units:
-//   context.hip     contexts, device-resident systems, workspace, host copies
+//   context.hip     contexts, device-resident systems, workspace
+//   hostcopy.hip    copies from and to host memory (threads: hostpool.cpp)
 //   fp64_path.hip   tiling, the single-k and batched FP64 paths, construct_ab,
 //                   create_hs, create_hs_batched, contract_hs
 //   split_path.hip  split precision (Ozaki scheme II on INT8 MFMA), single-k
